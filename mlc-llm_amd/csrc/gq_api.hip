@@ -338,9 +338,29 @@ int64_t mi355gq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits
   return linear_workspace_need(M, N, K, bits, group_size, true);
 }
 
+// q4f32_1 linears: rows that run on the kernel on unscaled weight operands (K % 256 == 0; five per pass over the weights), the
+// rest on the GEMM over three bfloat16 planes of x.  One row of K up to 8192 stays on the dot-product GEMV (4096 x 4096 9.2 us
+// against 11.5, 28672 x 4096 27.4 / 27.8, 128256 x 4096 81 / 91); 6..10 rows take two passes from 64 M weights on (28672 x 4096 at 8
+// rows 50 against the GEMM's 60, 128256 x 4096 176 / 230; 4096 x 4096 23 / 17.7 and 4096 x 14336 37 / 35.7 stay with the GEMM).
+static bool f32_rows_by_midrow(int64_t M, int64_t N, int64_t K) {
+  if ((K & 255) != 0) return false;
+  if (M == 1) return K > 8192;
+  return M <= 5 || (M <= 10 && N * K >= (64ll << 20));
+}
+// one row of K up to 8192, and two where that kernel does not apply: the dot-product GEMV (4096 x 4096 at two rows 15.5 us
+// against the GEMM's 17.6 with its scratch, 74 without)
+static bool f32_rows_by_gemv(int64_t M, int64_t N, int64_t K) {
+  return M <= 2 && K <= 8192 && !f32_rows_by_midrow(M, N, K);
+}
+
 int64_t mi355gq_linear_dt_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group_size,
                                           int model_dtype) {
   if (model_dtype == MI355GQ_F16) return mi355gq_linear_workspace_bytes(M, N, K, bits, group_size);
+  if (model_dtype == MI355GQ_F32 && check_scheme(bits, group_size) == MI355GQ_OK && bits == 4 && M >= 1 && N >= 1 && K >= 1 &&
+      M < kMaxDim && N < kMaxDim && K < kMaxDim)
+    return f32_rows_by_midrow(M, N, K) ? gq::midrow_workspace_bytes(M, N, K)
+           : f32_rows_by_gemv(M, N, K) ? 0
+                                       : gq::gemm_f32_workspace_bytes(M, N, K);
   if (model_dtype != MI355GQ_BF16 || check_scheme(bits, group_size) != MI355GQ_OK || M < 2 || N < 0 || K < 0 ||
       M >= kMaxDim || N >= kMaxDim || K >= kMaxDim)
     return 0;
@@ -762,6 +782,27 @@ static int linear_dt_impl(const void* x, const void* q_weight, const void* q_sca
                                          : aligned2(x) && aligned2(q_scale) && aligned2(bias) && aligned2(residual)) &&
                  (out_dtype == MI355GQ_F32 ? aligned4(y) : aligned2(y)),
              "linear_dt: q_weight must be 16-byte aligned, the other tensors naturally aligned");
+  // (overrides: gemv_variant 0 the dot-product kernels, 10 the mid-row kernel, any other the GEMM)
+  const int gv32 = gq::options().gemv_variant;
+  if (f32 && bits == 4 && aligned16(x) && gv32 != 0 && !(gv32 < 0 && f32_rows_by_gemv(M, N, K))) {
+    gq::GemmArgs g{};
+    g.x = static_cast<const uint16_t*>(x);
+    g.q_weight = static_cast<const uint32_t*>(q_weight);
+    g.q_scale = static_cast<const uint16_t*>(q_scale);
+    g.bias = static_cast<const uint16_t*>(bias);
+    g.residual = static_cast<const uint16_t*>(residual);
+    g.y = y;
+    g.rows = M; g.N = N; g.K = K; g.num_experts = 1;
+    g.bits = bits; g.group_size = group_size; g.out_f32 = 1;
+    g.workspace = workspace; g.workspace_bytes = workspace ? workspace_bytes : 0;
+    g.f32 = 1;
+    if (gv32 == 10 || (gv32 < 0 && f32_rows_by_midrow(M, N, K))) {
+      const hipError_t e = gq::launch_midrow(g, static_cast<int>(M), as_stream(stream));
+      if (e != hipErrorNotSupported) return hip_result(e, "linear_dt mid-row launch");
+    }
+    const hipError_t e = gq::launch_gemm_f32(g, as_stream(stream));
+    if (e != hipErrorNotSupported) return hip_result(e, "linear_dt float32 gemm launch");
+  }
   if (model_dtype == MI355GQ_BF16 && M == 2 && bits == 4 && (K & 7) == 0 && aligned16(x) && gq::options().gemm_variant < 0 &&
       (gq::options().gemv_variant < 0 || gq::options().gemv_variant == 9)) {
     // two rows of q4: the few-row kernel with x in registers, as in the float16 linear (28672 x 4096 14.6 us against 17.4
@@ -1154,6 +1195,22 @@ static int moe_gemv_dt_impl(const void* x, int64_t x_rows, const void* q_weight,
                  (f32 ? aligned4(x) && aligned4(q_scale) && aligned4(out)
                       : aligned2(x) && aligned2(q_scale) && aligned2(out)),
              "moe_gemv_dt: q_weight must be 16-byte aligned, the other tensors naturally aligned");
+  // (float32, a K the dot-product kernel does not reach: 2 of 8 experts of 4096 x 14336 1139 us on the float32 GEMM -> 38; a
+  //  shorter K stays, 2 of 8 experts of 28672 x 4096 42 us against 44.5)
+  if (f32 && bits == 4 && aligned16(x) && (gq::options().gemv_variant == 10 || (gq::options().gemv_variant < 0 && K > 8192))) {
+    gq::GemmArgs g{};
+    g.x = static_cast<const uint16_t*>(x);
+    g.q_weight = static_cast<const uint32_t*>(q_weight);
+    g.q_scale = static_cast<const uint16_t*>(q_scale);
+    g.y = out;
+    g.rows = top_k; g.N = N; g.K = K; g.num_experts = num_experts;
+    g.bits = bits; g.group_size = group_size; g.out_f32 = 1;
+    g.f32 = 1;
+    g.expert_ids = static_cast<const int32_t*>(expert_ids);
+    g.x_one_row = x_rows == 1;
+    const hipError_t e = gq::launch_midrow(g, 1, as_stream(stream));
+    if (e != hipErrorNotSupported) return hip_result(e, "moe_gemv_dt mid-row launch");
+  }
   if (model_dtype == MI355GQ_BF16 && aligned16(x) && (x_rows == 1 || (K % 8) == 0)) {
     gq::GemvArgs a{};
     a.x = static_cast<const uint16_t*>(x);
@@ -1222,6 +1279,30 @@ static int moe_group_gemm_dt_impl(const void* x, int64_t rows, const void* q_wei
                  (f32 ? aligned4(x) && aligned4(q_scale) && aligned4(out)
                       : aligned2(x) && aligned2(q_scale) && aligned2(out)),
              "moe_group_gemm_dt: q_weight must be 16-byte aligned, the other tensors naturally aligned");
+  // float32: fewer than one row for every second expert on the dot-product kernel (64 experts of 2816 x 2048 at 12 / 24 rows 28 /
+  // 37 us against 64 / 60; 8 experts of 28672 x 4096 at 4 rows 112 / 135, at 8 rows 230 / 138), up to four rows per expert on
+  // average, eight with few experts, on the kernel on unscaled weight operands (passes of five rows: 8 experts of 28672 x 4096
+  // at 8 / 32 / 64 rows 138 / 275 / 416 us, 64 of 2816 x 2048 at 3 / 6 rows per expert 118 / 178), more on the three-plane
+  // GEMM (285 / 430 / 437, 149 / 161)
+  const bool f32_gemv = 2 * rows <= num_experts && rows <= 32 && K <= 8192;
+  if (f32 && bits == 4 && aligned16(x) && gq::options().gemv_variant != 0 && !(gq::options().gemv_variant < 0 && f32_gemv)) {
+    gq::GemmArgs g{};
+    g.x = static_cast<const uint16_t*>(x);
+    g.q_weight = static_cast<const uint32_t*>(q_weight);
+    g.q_scale = static_cast<const uint16_t*>(q_scale);
+    g.y = out;
+    g.indptr = indptr; g.indptr_i64 = indptr_dtype == MI355GQ_I64;
+    g.rows = rows; g.N = N; g.K = K; g.num_experts = num_experts;
+    g.bits = bits; g.group_size = group_size; g.out_f32 = 1;
+    g.f32 = 1;
+    const int gv = gq::options().gemv_variant;
+    if (gv == 10 || (gv < 0 && rows <= (num_experts <= 16 ? 8 : 4) * num_experts)) {
+      const hipError_t e = gq::launch_midrow(g, 5, as_stream(stream));
+      if (e != hipErrorNotSupported) return hip_result(e, "moe_group_gemm_dt mid-row launch");
+    }
+    const hipError_t e = gq::launch_gemm_f32(g, as_stream(stream));
+    if (e != hipErrorNotSupported) return hip_result(e, "moe_group_gemm_dt float32 gemm launch");
+  }
   if (model_dtype == MI355GQ_BF16 && rows > 1 && (K & 7) == 0 && aligned16(x) && aligned16(out)) {
     // the float16 grouped GEMM's tiles on the bf16 matrix instruction (as in linear_dt, faster than the
     // dot-product kernel from two rows on)

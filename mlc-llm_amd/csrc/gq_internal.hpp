@@ -82,6 +82,9 @@ struct GemmArgs {
   const int32_t* x_rows = nullptr; // the MoE gather folded in: activation row r reads x[x_rows[r]] (x has x_src_rows rows)
   int64_t x_src_rows = 0;
   int bf16 = 0;                    // bfloat16 model: x, q_scale, bias and a 16-bit y are bf16 (plain linear only)
+  int f32 = 0;                     // float32 model: x, q_scale, bias, residual and y are float32 (the pointers above are casts)
+  const int32_t* expert_ids = nullptr;  // float32 model: row i uses expert expert_ids[i] (dequantize_gemv), reading row 0 of x
+  int x_one_row = 0;                    //   when x_one_row is set, row i otherwise
 };
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t s);
 // scratch the split-K form of the GEMM wants for this shape (0 when it does not split)
@@ -102,6 +105,13 @@ hipError_t launch_quadreg(const GemmArgs& a, int rows_max, hipStream_t s);
 // does not fit.
 hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s);
 int64_t midrow_workspace_bytes(int64_t rows, int64_t N, int64_t K);
+
+// float32 models (q4f32_1, K % 8 == 0), plain linears and expert segments: three bfloat16 planes of x on the bfloat16
+// matrix cores; hipErrorNotSupported otherwise.  Its split of K wants gemm_f32_workspace_bytes of scratch.
+hipError_t launch_gemm_f32(const GemmArgs& a, hipStream_t s);
+int64_t gemm_f32_workspace_bytes(int64_t rows, int64_t N, int64_t K);
+hipError_t launch_splitk_reduce_f32(const float* part, int slices, int64_t rows, int64_t N, const float* bias,
+                                    const float* residual, float* y, hipStream_t s);
 
 // KN-layout tensors (q_weight [nw, N], q_scale [ng, N]): both tensors transposed in one call (src_rows_w / src_rows_s rows
 // of src_cols columns each), the dequantisation to [K, N], and the decode GEMV (M <= 8, N % 4 == 0) with its workspace

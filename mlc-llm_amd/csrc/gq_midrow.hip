@@ -33,7 +33,12 @@
 // is walked in phases: each phase loads its share of x and visits every tile again (its own K range of it: the weights
 // are still read once), adding to the sums in LDS.  Expert segments (moe_matmul.dequantize_group_gemm,
 // python/mlc_llm/op/moe_matmul.py:562-768): grid row = expert, rows from indptr, more rows than the batch tiles hold in
-// passes.  The fused gate/up form walks a gate tile and its up tile in consecutive rounds and folds silu(gate) * up into
+// passes.  Float32 models (q4f32_1): x = h + m + l, three bfloat16 planes that together are x exactly, so five activation
+// rows make fifteen rows of the bfloat16 operand; the weights are the integers q (v_cvt_scalef32_pk_bf16_fp8, two fields per
+// instruction), the offset -7 * sum(x), and the planes of a row meet where the K shares do: products and scales as exact as
+// float32 dot products make them (relative error 8e-8 against float64 at K = 4096), at the price of the weight stream
+// (4 rows: 28672 x 4096 76.7 us on the dot-product kernel's passes -> 26.8, 128256 x 4096 237 -> 91, 4096 x 14336 1168 -> 21.8).
+// The fused gate/up form walks a gate tile and its up tile in consecutive rounds and folds silu(gate) * up into
 // the step that adds the K shares.
 #include "gq_gemm_common.hpp"
 #include "gq_gemv_common.hpp"
@@ -51,6 +56,7 @@ struct MidParams {
   void* y;
   const void* indptr;      // null: one segment [0, rows)
   const int32_t* x_rows;   // null, or the row of x each activation row reads
+  const int32_t* ids;      // (float32) null, or one expert per row: grid row = activation row, its expert ids[row]
   int64_t expert_w_stride, expert_s_stride;
   int rows, N, K, ng, nw;
   int ntiles;              // tiles of 16 weight rows a walk visits: ceil(N / 16); the fused gate/up form: N / 32 pairs
@@ -61,6 +67,7 @@ struct MidParams {
                            // K and leaves fp32 partial sums [slice][rows][N] in y for the reduction kernel)
   int kw_log2;             // log2 of the waves that share a tile's K
   int out_f32, paired, indptr_i64, x_src_rows;
+  int num_experts, x_one_row;  // with ids: experts in the stack; every row reads row 0 of x
 };
 
 // T[j][m] (register m of the lanes 16 j .. 16 j + 15) -> T[m][j]
@@ -84,6 +91,17 @@ __device__ __forceinline__ float4_t mid_mfma(const mid_u4 a, const mid_u4 b, con
   }
 }
 
+// the eight fields of a storage word as bfloat16 integers, fields (0, 2) (4, 6) (1, 3) (5, 7): a byte 0 .. 15 read as an
+// fp8 (e4m3) number is that many 2^-9 (subnormals, then the first binade, whose steps are the same), so the scaled
+// conversion delivers two fields per instruction
+__device__ __forceinline__ mid_u4 mid_word_bf16(uint32_t w) {
+  const uint32_t t0 = w & 0x0f0f0f0fu, t1 = (w >> 4) & 0x0f0f0f0fu;
+  return mid_u4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t0, 512.0f, false)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t0, 512.0f, true)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t1, 512.0f, false)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t1, 512.0f, true))};
+}
+
 // NBT: batch tiles of 16 rows; U: groups of K a wave owns (4 or 8); RT: tiles of loads in flight per wave;
 // BF: bfloat16 model (x, scales, bias, residual and the 16-bit result are bfloat16): 0x4300 | q is the bfloat16 128 + q, so
 // every field is shifted down to bit 0 of its half (no x16 trick, x is not rescaled) and all carry the offset 128 + 7;
@@ -91,11 +109,19 @@ __device__ __forceinline__ float4_t mid_mfma(const mid_u4 a, const mid_u4 b, con
 // PHASED: K takes more than one phase (the sums of all of a wave's rounds stay in LDS between phases: one chunk of rounds);
 // else a wave's rounds come in chunks of p.rounds, each followed by the step that adds the K shares and stores, with x
 // and the ring of loads carried across
-template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, bool BF = false>
+template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16>
 __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
+  constexpr bool BF = DT == MODEL_BF16, F32 = DT == MODEL_F32;
   constexpr int STEPS = U / 4;
+  constexpr int EL = F32 ? 4 : 2;     // bytes of an activation, a scale
+  constexpr int BR = F32 ? 5 : 16;    // activation rows a batch tile holds
+  constexpr int SW = F32 ? U : U / 2; // registers of a row's U scales
   constexpr uint32_t kMagic = BF ? 0x43004300u : 0x64006400u;
-  auto to_f32 = [](uint16_t bits) { return BF ? bf2f(bits) : h2f(bits); };
+  // element i of a tensor in the model dtype
+  auto elem = [](const uint16_t* t, int64_t i) -> float {
+    if constexpr (F32) return reinterpret_cast<const float*>(t)[i];
+    else return BF ? bf2f(t[i]) : h2f(t[i]);
+  };
   extern __shared__ float4 res_lds[];  // [round][wave][NBT][64 lanes]
 
   // (the wave index in a scalar register: everything derived from it - K share, tiles, the loads' scalar offsets - is
@@ -109,9 +135,13 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
   const int half_tiles = p.N >> 5;        // (the fused form: tiles of gate rows)
 
   // ---- this workgroup's expert and rows
-  const int expert = blockIdx.y;
+  int expert = blockIdx.y;
   int seg_lo = 0, seg_hi = p.rows;
-  if (p.indptr != nullptr) {
+  if (F32 && p.ids != nullptr) {
+    seg_lo = expert;
+    seg_hi = seg_lo + 1;
+    expert = min(max(p.ids[seg_lo], 0), p.num_experts - 1);
+  } else if (p.indptr != nullptr) {
     if (p.indptr_i64) {
       seg_lo = static_cast<int>(static_cast<const int64_t*>(p.indptr)[expert]);
       seg_hi = static_cast<int>(static_cast<const int64_t*>(p.indptr)[expert + 1]);
@@ -131,12 +161,12 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
   const uint32_t w_bytes = static_cast<uint32_t>(p.N) * static_cast<uint32_t>(p.nw) * 4u;
-  const uint32_t s_bytes = static_cast<uint32_t>(p.N) * static_cast<uint32_t>(p.ng) * 2u;
+  const uint32_t s_bytes = static_cast<uint32_t>(p.N) * static_cast<uint32_t>(p.ng) * EL;
   const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint32_t*>(p.qw + expert * p.expert_w_stride), short(0), static_cast<int>(w_bytes), 0x00020000);
   const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(p.qs + expert * p.expert_s_stride), short(0), static_cast<int>(s_bytes), 0x00020000);
-  const uint32_t w_tile = 16u * static_cast<uint32_t>(p.nw) * 4u, s_tile = 16u * static_cast<uint32_t>(p.ng) * 2u;
+      const_cast<uint16_t*>(p.qs + expert * p.expert_s_stride * (EL / 2)), short(0), static_cast<int>(s_bytes), 0x00020000);
+  const uint32_t w_tile = 16u * static_cast<uint32_t>(p.nw) * 4u, s_tile = 16u * static_cast<uint32_t>(p.ng) * EL;
   // round r of this wave -> tile (the fused form: rounds 2 i, 2 i + 1 = gate tile, up tile of pair i); -1 past the end.
   // Straight-line scalar arithmetic: a branch here would sit inside the walk, where every join makes the wait for one
   // tile's loads a wait for all of them.
@@ -150,18 +180,19 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
 
   constexpr uint32_t kLoLo = 0x05040100u, kHiHi = 0x07060302u;
   const half2_t r16 = {static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)};
-  const mid_u4 neg_off = BF ? mid_u4{0xc307c307u /* -135 */, 0xc307c307u, 0xc307c307u, 0xc307c307u}
-                            : mid_u4{0xe407e407u /* -1031 */, 0xe407e407u, 0xe470e470u /* -16 * 71 */, 0xe470e470u};
+  const mid_u4 neg_off = F32  ? mid_u4{0xc0e0c0e0u /* -7 */, 0xc0e0c0e0u, 0xc0e0c0e0u, 0xc0e0c0e0u}
+                         : BF ? mid_u4{0xc307c307u /* -135 */, 0xc307c307u, 0xc307c307u, 0xc307c307u}
+                              : mid_u4{0xe407e407u /* -1031 */, 0xe407e407u, 0xe470e470u /* -16 * 71 */, 0xe470e470u};
 
-  for (int pass_lo = seg_lo; pass_lo < seg_hi; pass_lo += 16 * NBT) {
+  for (int pass_lo = seg_lo; pass_lo < seg_hi; pass_lo += BR * NBT) {
     for (int ph = 0; ph < (PHASED ? p.phases : 1); ++ph) {
       const int ga_raw = ((static_cast<int>(blockIdx.z) + ph) * kw + ks) * U;  // (slices > 1: one phase each)
       const bool k_live = ga_raw < p.ng;  // (uniform; ng % U == 0: a share is whole or empty)
       const int ga = k_live ? ga_raw : p.ng - U;
-      const int w_lane = (c * p.nw + 4 * (ga + j)) * 4, s_lane = (c * p.ng + ga) * 2;
+      const int w_lane = (c * p.nw + 4 * (ga + j)) * 4, s_lane = (c * p.ng + ga) * EL;
       u32x4 w[RT][STEPS];  // (kept as whole register tuples until the point of use, see walk_tile)
-      uint32_t sc[RT][U / 2];  // the U scales of this lane's row (two per register)
-      auto issue = [&](int r, u32x4 (&wv)[STEPS], uint32_t (&sv)[U / 2]) {
+      uint32_t sc[RT][SW];  // the U scales of this lane's row (16-bit: two per register)
+      auto issue = [&](int r, u32x4 (&wv)[STEPS], uint32_t (&sv)[SW]) {
         const int tile = tile_of(r);
         const int w_off = static_cast<int>(tile >= 0 ? static_cast<uint32_t>(tile) * w_tile : w_bytes);
         const int s_off = static_cast<int>(tile >= 0 ? static_cast<uint32_t>(tile) * s_tile : s_bytes);
@@ -169,7 +200,13 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
         for (int st = 0; st < STEPS; ++st) {
           wv[st] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_lane + 64 * st, w_off, 0);
         }
-        if constexpr (U == 8) {
+        if constexpr (F32) {
+#pragma unroll
+          for (int q = 0; q < U / 4; ++q) {
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, s_lane + 16 * q, s_off, 0);
+            sv[4 * q] = v.x; sv[4 * q + 1] = v.y; sv[4 * q + 2] = v.z; sv[4 * q + 3] = v.w;
+          }
+        } else if constexpr (U == 8) {
           const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, s_lane, s_off, 0);
           sv[0] = v.x; sv[1] = v.y; sv[2] = v.z; sv[3] = v.w;
         } else {
@@ -177,44 +214,87 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
           sv[0] = v.x; sv[1] = v.y;
         }
       };
-      // ---- this wave's share of x goes out first (it is needed first, and loads retire in issue order): lane (i = c, j)
-      //      of batch tile bt reads x[row 16 bt + i][32 g + 8 j .. + 7]
-      uint4 xraw[NBT][U];
-      bool x_ok[NBT];
-#pragma unroll
-      for (int bt = 0; bt < NBT; ++bt) {
-        const int b = pass_lo + 16 * bt + c;
-        x_ok[bt] = k_live && b < seg_hi;
-        const uint16_t* xrow = p.x + x_row(p.x_rows, p.x_src_rows, x_ok[bt] ? b : seg_lo) * p.K + ga * 32 + 8 * j;
-#pragma unroll
-        for (int u = 0; u < U; ++u) xraw[bt][u] = *reinterpret_cast<const uint4*>(xrow + u * 32);
-      }
-#pragma unroll
-      for (int r = 0; r < RT; ++r) issue(r, w[r], sc[r]);
-
-      // ---- x in operand order, (x0, x4) (x2, x6) (x1, x5) / 16 (x3, x7) / 16, and the offset terms
       mid_u4 xa[NBT][U];
       float4_t cc[KEEP_C ? NBT : 1][KEEP_C ? U : 1];
+      if constexpr (F32) {
+        // ---- x as three bfloat16 planes, x = h + m + l: the leading 8 bits of the significand, the next 8, the last 8
+        //      (differences of float32 values that share their exponent range are exact, so the planes lose nothing).  A
+        //      batch tile's matrix rows are (activation row, plane): row i of the operand is plane i % 3 of row i / 3.
+        const int pl = c % 3;
 #pragma unroll
-      for (int bt = 0; bt < NBT; ++bt) {
+        for (int bt = 0; bt < NBT; ++bt) {
+          const int b = pass_lo + BR * bt + c / 3;
+          const bool ok = k_live && c < 3 * BR && b < seg_hi;
+          const int64_t xr = p.x_one_row ? 0 : x_row(p.x_rows, p.x_src_rows, ok ? b : seg_lo);
+          const float* const xrow = reinterpret_cast<const float*>(p.x) + xr * p.K + ga * 32 + 8 * j;
+          uint4 lo[U], hi[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          uint4 v = xraw[bt][u];
-          if (!x_ok[bt]) v = make_uint4(0, 0, 0, 0);
-          xa[bt][u][0] = __builtin_amdgcn_perm(v.z, v.x, kLoLo);
-          xa[bt][u][1] = __builtin_amdgcn_perm(v.w, v.y, kLoLo);
-          xa[bt][u][2] = __builtin_amdgcn_perm(v.z, v.x, kHiHi);
-          xa[bt][u][3] = __builtin_amdgcn_perm(v.w, v.y, kHiHi);
-          if constexpr (!BF) {
-            xa[bt][u][2] = as_u32(as_half2(xa[bt][u][2]) * r16);
-            xa[bt][u][3] = as_u32(as_half2(xa[bt][u][3]) * r16);
+          for (int u = 0; u < U; ++u) {
+            lo[u] = *reinterpret_cast<const uint4*>(xrow + u * 32);
+            hi[u] = *reinterpret_cast<const uint4*>(xrow + u * 32 + 4);
           }
-          if constexpr (KEEP_C) cc[bt][u] = mid_mfma<BF>(xa[bt][u], neg_off, float4_t{0.f, 0.f, 0.f, 0.f});
+          if (bt == NBT - 1) {  // (behind the loads of x: those are needed first, and loads retire in issue order)
+#pragma unroll
+            for (int r = 0; r < RT; ++r) issue(r, w[r], sc[r]);
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const uint32_t raw[8] = {lo[u].x, lo[u].y, lo[u].z, lo[u].w, hi[u].x, hi[u].y, hi[u].z, hi[u].w};
+            uint32_t v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float x = __builtin_bit_cast(float, ok ? raw[e] : 0u);
+              const float h = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xffff0000u);
+              const float r1 = x - h;
+              const float m = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r1) & 0xffff0000u);
+              v[e] = __builtin_bit_cast(uint32_t, pl == 0 ? h : (pl == 1 ? m : r1 - m));
+            }
+            // fields (0, 2) (4, 6) (1, 3) (5, 7): the order in which the conversion delivers a word
+            xa[bt][u][0] = __builtin_amdgcn_perm(v[2], v[0], kHiHi);
+            xa[bt][u][1] = __builtin_amdgcn_perm(v[6], v[4], kHiHi);
+            xa[bt][u][2] = __builtin_amdgcn_perm(v[3], v[1], kHiHi);
+            xa[bt][u][3] = __builtin_amdgcn_perm(v[7], v[5], kHiHi);
+            if constexpr (KEEP_C) cc[bt][u] = mid_mfma<true>(xa[bt][u], neg_off, float4_t{0.f, 0.f, 0.f, 0.f});
+          }
+        }
+      } else {
+        // ---- this wave's share of x goes out first (it is needed first, and loads retire in issue order): lane (i = c, j)
+        //      of batch tile bt reads x[row 16 bt + i][32 g + 8 j .. + 7]
+        uint4 xraw[NBT][U];
+        bool x_ok[NBT];
+#pragma unroll
+        for (int bt = 0; bt < NBT; ++bt) {
+          const int b = pass_lo + 16 * bt + c;
+          x_ok[bt] = k_live && b < seg_hi;
+          const uint16_t* xrow = p.x + x_row(p.x_rows, p.x_src_rows, x_ok[bt] ? b : seg_lo) * p.K + ga * 32 + 8 * j;
+#pragma unroll
+          for (int u = 0; u < U; ++u) xraw[bt][u] = *reinterpret_cast<const uint4*>(xrow + u * 32);
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r) issue(r, w[r], sc[r]);
+
+        // ---- x in operand order, (x0, x4) (x2, x6) (x1, x5) / 16 (x3, x7) / 16, and the offset terms
+#pragma unroll
+        for (int bt = 0; bt < NBT; ++bt) {
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            uint4 v = xraw[bt][u];
+            if (!x_ok[bt]) v = make_uint4(0, 0, 0, 0);
+            xa[bt][u][0] = __builtin_amdgcn_perm(v.z, v.x, kLoLo);
+            xa[bt][u][1] = __builtin_amdgcn_perm(v.w, v.y, kLoLo);
+            xa[bt][u][2] = __builtin_amdgcn_perm(v.z, v.x, kHiHi);
+            xa[bt][u][3] = __builtin_amdgcn_perm(v.w, v.y, kHiHi);
+            if constexpr (!BF) {
+              xa[bt][u][2] = as_u32(as_half2(xa[bt][u][2]) * r16);
+              xa[bt][u][3] = as_u32(as_half2(xa[bt][u][3]) * r16);
+            }
+            if constexpr (KEEP_C) cc[bt][u] = mid_mfma<BF>(xa[bt][u], neg_off, float4_t{0.f, 0.f, 0.f, 0.f});
+          }
         }
       }
 
       // one tile from a ring slot; round `next` goes into the registers it leaves
-      auto walk_tile = [&](int next, u32x4 (&wv)[STEPS], uint32_t (&sv)[U / 2], float4_t (&acc)[NBT]) __attribute__((always_inline)) {
+      auto walk_tile = [&](int next, u32x4 (&wv)[STEPS], uint32_t (&sv)[SW], float4_t (&acc)[NBT]) __attribute__((always_inline)) {
 #pragma unroll
         for (int bt = 0; bt < NBT; ++bt) acc[bt] = float4_t{0.f, 0.f, 0.f, 0.f};
         // (a zero the compiler cannot see through: the offset instruction would otherwise be hoisted out of the walk,
@@ -235,15 +315,22 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
           for (int m = 0; m < 4; ++m) {
             const int u = 4 * st + m;
             const uint32_t w8 = r[m] >> 8;
-            const mid_u4 bw = BF ? mid_u4{and_or_c(r[m], 0x000f000fu, kMagic), and_or_c(w8, 0x000f000fu, kMagic),
-                                          and_or_c(r[m] >> 4, 0x000f000fu, kMagic), and_or_c(r[m] >> 12, 0x000f000fu, kMagic)}
-                                 : mid_u4{and_or_c(r[m], 0x000f000fu, kMagic), and_or_c(w8, 0x000f000fu, kMagic),
-                                          and_or_c(r[m], 0x00f000f0u, kMagic), and_or_c(w8, 0x00f000f0u, kMagic)};
-            const float s = to_f32(static_cast<uint16_t>((u & 1) ? sv[u >> 1] >> 16 : sv[u >> 1] & 0xffffu));
+            const mid_u4 bw = F32  ? mid_word_bf16(r[m])
+                              : BF ? mid_u4{and_or_c(r[m], 0x000f000fu, kMagic), and_or_c(w8, 0x000f000fu, kMagic),
+                                            and_or_c(r[m] >> 4, 0x000f000fu, kMagic), and_or_c(r[m] >> 12, 0x000f000fu, kMagic)}
+                                   : mid_u4{and_or_c(r[m], 0x000f000fu, kMagic), and_or_c(w8, 0x000f000fu, kMagic),
+                                            and_or_c(r[m], 0x00f000f0u, kMagic), and_or_c(w8, 0x00f000f0u, kMagic)};
+            float s;
+            if constexpr (F32) {
+              s = __builtin_bit_cast(float, sv[u]);
+            } else {
+              const uint16_t sb = static_cast<uint16_t>((u & 1) ? sv[u >> 1] >> 16 : sv[u >> 1] & 0xffffu);
+              s = BF ? bf2f(sb) : h2f(sb);
+            }
             // (float16 without the kept offsets: the offsets come off the weight operand instead, exactly - 1024 + q - 1031
             //  and 1024 + 16 q - 16 * 71 are small integers -, four packed adds per group whatever the batch tiles, in place
             //  of one more matrix instruction per group and batch tile)
-            constexpr bool SUB = !KEEP_C && !BF;
+            constexpr bool SUB = !KEEP_C && DT == MODEL_F16;
             mid_u4 bo = bw;
             if constexpr (SUB) {
               const half2_t o_lo = {static_cast<_Float16>(-1031.f), static_cast<_Float16>(-1031.f)};
@@ -256,8 +343,8 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
               float4_t c0;
               if constexpr (KEEP_C) c0 = cc[bt][u];
               else if constexpr (SUB) c0 = float4_t{0.f, 0.f, 0.f, 0.f};
-              else c0 = mid_mfma<BF>(xa[bt][u], neg_off, zero4);
-              const float4_t d = mid_mfma<BF>(xa[bt][u], SUB ? bo : bw, c0);
+              else c0 = mid_mfma<BF || F32>(xa[bt][u], neg_off, zero4);
+              const float4_t d = mid_mfma<BF || F32>(xa[bt][u], SUB ? bo : bw, c0);
 #pragma unroll
               for (int q = 0; q < 4; ++q) acc[bt][q] = fmaf(s, d[q], acc[bt][q]);
             }
@@ -273,10 +360,20 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
       auto finish = [&](int r0) __attribute__((always_inline)) {
         const float* const res = reinterpret_cast<const float*>(res_lds);
         const int sub = threadIdx.x & 255, cq = sub & 15, jq = sub >> 4;
-        const int at = (((jq >> 2) * 16 + cq) << 2) + (jq & 3);  // lane (cq, jq / 4), value jq % 4
+        auto at_row = [&](int r) { return (((r >> 2) * 16 + cq) << 2) + (r & 3); };  // lane (cq, r / 4), value r % 4
+        const int at = at_row(F32 ? 0 : jq);
+        if (jq >= BR) return;
         auto share_sum = [&](int round, int tl, int bt) {
           float v = 0.f;
-          for (int k = 0; k < kw; ++k) v += res[(((round * 16 + (tl << p.kw_log2) + k) * NBT + bt) << 8) + at];
+          if constexpr (F32) {  // the row's three planes, the smallest first
+#pragma unroll
+            for (int pl = 2; pl >= 0; --pl) {
+              const int ap = at_row(3 * jq + pl);
+              for (int k = 0; k < kw; ++k) v += res[(((round * 16 + (tl << p.kw_log2) + k) * NBT + bt) << 8) + ap];
+            }
+          } else {
+            for (int k = 0; k < kw; ++k) v += res[(((round * 16 + (tl << p.kw_log2) + k) * NBT + bt) << 8) + at];
+          }
           return v;
         };
         if (p.paired) {
@@ -285,17 +382,17 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
           for (int it = threadIdx.x >> 8; it < items; it += 4) {
             const int bt = it % NBT, rest = it / NBT, tl = rest % tw, pr = rest / tw;
             const int pair = blockIdx.x * tw + tl + ((r0 >> 1) + pr) * tstride;
-            const int col = pair * 16 + cq, b = pass_lo + 16 * bt + jq;
+            const int col = pair * 16 + cq, b = pass_lo + BR * bt + jq;
             if (pair >= p.ntiles || b >= seg_hi) continue;
             const float gate = share_sum(2 * pr, tl, bt), up = share_sum(2 * pr + 1, tl, bt);
-            static_cast<uint16_t*>(p.y)[static_cast<int64_t>(b) * half + col] = silu_mul_t<BF>(gate, up);
+            if constexpr (!F32) static_cast<uint16_t*>(p.y)[static_cast<int64_t>(b) * half + col] = silu_mul_t<BF>(gate, up);
           }
         } else {
           const int items = p.rounds * tw * NBT;
           for (int it = threadIdx.x >> 8; it < items; it += 4) {
             const int bt = it % NBT, rest = it / NBT, tl = rest % tw, round = rest / tw;
             const int t = blockIdx.x * tw + tl + (r0 + round) * tstride;
-            const int col = t * 16 + cq, b = pass_lo + 16 * bt + jq;
+            const int col = t * 16 + cq, b = pass_lo + BR * bt + jq;
             if (t >= p.ntiles || col >= p.N || b >= seg_hi) continue;
             float v = share_sum(round, tl, bt);
             const int64_t oi = static_cast<int64_t>(b) * p.N + col;
@@ -303,9 +400,9 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
               static_cast<float*>(p.y)[static_cast<int64_t>(blockIdx.z) * p.rows * p.N + oi] = v;
               continue;
             }
-            if (p.bias != nullptr) v += to_f32(p.bias[col]);
-            if (p.residual != nullptr) v += to_f32(p.residual[oi]);
-            if (p.out_f32) static_cast<float*>(p.y)[oi] = v;
+            if (p.bias != nullptr) v += elem(p.bias, col);
+            if (p.residual != nullptr) v += elem(p.residual, oi);
+            if (F32 || p.out_f32) static_cast<float*>(p.y)[oi] = v;
             else static_cast<uint16_t*>(p.y)[oi] = BF ? f2bf(v) : f2h(v);
           }
         }
@@ -363,22 +460,22 @@ __global__ __launch_bounds__(256) void mid_reduce_silu_kernel(const float* __res
   }
 }
 
-template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, bool BF = false>
+template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16>
 hipError_t launch_mid(const MidParams& p, int wgx, int experts, hipStream_t s) {
   const size_t lds = static_cast<size_t>(p.rounds) * 16 * NBT * 1024;
   if (lds > 160 * 1024) return hipErrorNotSupported;
   if (lds > 64 * 1024) {
     static bool raised = false;  // (idempotent; a race sets the same attribute twice)
     if (!raised) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&midrow_kernel<NBT, U, RT, KEEP_C, PHASED, BF>),
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
       if (e != hipSuccess) return e;
       raised = true;
     }
   }
   note_kernel("gq::midrow_kernel<%d,%d,%d,%d,%d%s> rounds=%d chunks=%d phases=%d slices=%d kw=%d", NBT, U, RT, int(KEEP_C),
-              int(PHASED), BF ? ",true" : "", p.rounds, p.chunks, p.phases, p.slices, 1 << p.kw_log2);
-  hipLaunchKernelGGL((midrow_kernel<NBT, U, RT, KEEP_C, PHASED, BF>), dim3(wgx, experts, p.slices), dim3(1024), lds, s, p);
+              int(PHASED), DT == MODEL_BF16 ? ",2" : (DT == MODEL_F32 ? ",1" : ""), p.rounds, p.chunks, p.phases, p.slices, 1 << p.kw_log2);
+  hipLaunchKernelGGL((midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT>), dim3(wgx, experts, p.slices), dim3(1024), lds, s, p);
   return hipGetLastError();
 }
 
@@ -399,11 +496,15 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
       (reinterpret_cast<uintptr_t>(a.q_scale) & 15) != 0)
     return hipErrorNotSupported;
   if (a.N * (a.K / 8) >= (int64_t(1) << 29)) return hipErrorNotSupported;  // (32-bit byte offsets with room to add)
-  const int experts = grouped ? static_cast<int>(a.num_experts) : 1;
+  // (workgroup rows: one per expert, or per activation row where each names its expert)
+  const int experts = grouped ? static_cast<int>(a.num_experts) : (a.expert_ids != nullptr ? static_cast<int>(a.rows) : 1);
   if (experts < 1 || experts > 65535) return hipErrorNotSupported;
+  if (a.f32 && (a.paired || a.bf16)) return hipErrorNotSupported;
+  if (a.expert_ids != nullptr && (!a.f32 || grouped || (a.N & 15) != 0)) return hipErrorNotSupported;
   MidParams p{};
   p.x = a.x; p.qw = a.q_weight; p.qs = a.q_scale; p.bias = a.bias; p.residual = a.residual; p.y = a.y;
   p.indptr = a.indptr; p.indptr_i64 = a.indptr_i64; p.x_rows = a.x_rows; p.x_src_rows = static_cast<int>(a.x_src_rows);
+  p.ids = a.expert_ids; p.x_one_row = a.x_one_row; p.num_experts = static_cast<int>(a.num_experts);
   p.rows = static_cast<int>(a.rows); p.N = static_cast<int>(a.N); p.K = static_cast<int>(a.K);
   p.ng = p.K / 32; p.nw = 4 * p.ng;
   p.expert_w_stride = static_cast<int64_t>(p.N) * p.nw;
@@ -412,7 +513,7 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   p.ntiles = a.paired ? p.N / 32 : (p.N + 15) / 16;
   p.out_f32 = a.out_f32;
   // batch tiles per pass: one for up to 16 rows per segment, else two (more rows: passes)
-  const int nbt = rows_max <= 16 ? 1 : 2;
+  const int nbt = rows_max <= 16 || a.f32 ? 1 : 2;  // (float32: one, of five rows)
   constexpr int U = 8;
   // waves that share a tile's K: the power of two that covers K's shares of U groups, at most 16 (a wave whose share lies
   // past K idles: one phase with 14 of 16 waves at work is ahead of two phases of 8)
@@ -428,7 +529,7 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   // folds the activation in.  Tuning override: gemv_ksplit 0 keeps the phases.
   p.slices = 1;
   bool fold_silu = false;
-  if (p.phases > 1 && !grouped && p.phases <= 64 && options().gemv_ksplit != 0 && a.workspace != nullptr &&
+  if (p.phases > 1 && experts == 1 && !grouped && p.phases <= 64 && options().gemv_ksplit != 0 && a.workspace != nullptr &&
       a.workspace_bytes >= static_cast<int64_t>(p.phases) * p.rows * p.N * 4 &&
       (reinterpret_cast<uintptr_t>(a.workspace) & 15) == 0) {
     p.slices = p.phases;
@@ -465,12 +566,17 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   p.chunks = (rounds + max_rounds - 1) / max_rounds;
   p.rounds = ((rounds + p.chunks - 1) / p.chunks + unit - 1) / unit * unit;
   auto run = [&]() -> hipError_t {
+    if (a.f32) {
+      if (p.phases > 1)
+        return launch_mid<1, 8, 2, false, true, MODEL_F32>(p, wgx, experts, s);
+      return launch_mid<1, 8, 2, false, false, MODEL_F32>(p, wgx, experts, s);
+    }
     if (a.bf16) {  // (the bfloat16 instances: q4bf16_*)
       if (p.phases > 1)
-        return nbt == 2 ? launch_mid<2, 8, 2, false, true, true>(p, wgx, experts, s)
-                        : launch_mid<1, 8, 2, true, true, true>(p, wgx, experts, s);
-      return nbt == 2 ? launch_mid<2, 8, 2, false, false, true>(p, wgx, experts, s)
-                      : launch_mid<1, 8, 2, true, false, true>(p, wgx, experts, s);
+        return nbt == 2 ? launch_mid<2, 8, 2, false, true, MODEL_BF16>(p, wgx, experts, s)
+                        : launch_mid<1, 8, 2, true, true, MODEL_BF16>(p, wgx, experts, s);
+      return nbt == 2 ? launch_mid<2, 8, 2, false, false, MODEL_BF16>(p, wgx, experts, s)
+                      : launch_mid<1, 8, 2, true, false, MODEL_BF16>(p, wgx, experts, s);
     }
     if (p.phases > 1) {
       if (form == 2) return hipErrorNotSupported;
@@ -485,6 +591,9 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   const hipError_t e = run();
   if (e != hipSuccess || p.slices == 1) return e;
   const int64_t count = static_cast<int64_t>(p.rows) * p.N;
+  if (a.f32)
+    return launch_splitk_reduce_f32(static_cast<const float*>(a.workspace), p.slices, p.rows, p.N, reinterpret_cast<const float*>(a.bias),
+                                    reinterpret_cast<const float*>(a.residual), static_cast<float*>(a.y), s);
   if (fold_silu) {
     const int64_t outs = count / 2;
     hipLaunchKernelGGL(mid_reduce_silu_kernel, dim3(static_cast<unsigned>((outs + 255) / 256 > 4096 ? 4096 : (outs + 255) / 256)),
