@@ -339,12 +339,13 @@ int64_t mi355gq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits
 }
 
 // q4f32_1 linears: rows that run on the kernel on unscaled weight operands (K % 256 == 0; five per pass over the weights), the
-// rest on the GEMM over three bfloat16 planes of x.  One row of K up to 8192 stays on the dot-product GEMV (4096 x 4096 9.2 us
-// against 11.5, 28672 x 4096 27.4 / 27.8, 128256 x 4096 81 / 91); 6..10 rows take two passes from 64 M weights on (28672 x 4096 at 8
-// rows 50 against the GEMM's 60, 128256 x 4096 176 / 230; 4096 x 4096 23 / 17.7 and 4096 x 14336 37 / 35.7 stay with the GEMM).
+// rest on the GEMM over three bfloat16 planes of x.  One row of K up to 8192 and fewer than 64 M weights stays on the dot-product
+// GEMV (4096 x 4096 9.2 us against 11.5, 6144 x 4096 10.7 / 12.9; 28672 x 4096 27.4 / 23, 128256 x 4096 81 / 77); 6..10 rows take
+// two passes from 64 M weights on (28672 x 4096 at 8 rows 46 against the GEMM's 60, 128256 x 4096 150 / 230; 4096 x 4096 21 / 17.7
+// and 4096 x 14336 35 / 35.7 stay with the GEMM).
 static bool f32_rows_by_midrow(int64_t M, int64_t N, int64_t K) {
   if ((K & 255) != 0) return false;
-  if (M == 1) return K > 8192;
+  if (M == 1) return K > 8192 || N * K >= (64ll << 20);
   return M <= 5 || (M <= 10 && N * K >= (64ll << 20));
 }
 // one row of K up to 8192, and two where that kernel does not apply: the dot-product GEMV (4096 x 4096 at two rows 15.5 us

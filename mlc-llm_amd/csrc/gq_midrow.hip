@@ -37,7 +37,7 @@
 // rows make fifteen rows of the bfloat16 operand; the weights are the integers q (v_cvt_scalef32_pk_bf16_fp8, two fields per
 // instruction), the offset -7 * sum(x), and the planes of a row meet where the K shares do: products and scales as exact as
 // float32 dot products make them (relative error 8e-8 against float64 at K = 4096), at the price of the weight stream
-// (4 rows: 28672 x 4096 76.7 us on the dot-product kernel's passes -> 26.8, 128256 x 4096 237 -> 91, 4096 x 14336 1168 -> 21.8).
+// (4 rows: 28672 x 4096 76.7 us on the dot-product kernel's passes -> 23, 128256 x 4096 237 -> 77, 4096 x 14336 1168 -> 18.4).
 // The fused gate/up form walks a gate tile and its up tile in consecutive rounds and folds silu(gate) * up into
 // the step that adds the K shares.
 #include "gq_gemm_common.hpp"
@@ -112,8 +112,10 @@ __device__ __forceinline__ mid_u4 mid_word_bf16(uint32_t w) {
 template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16>
 __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
   constexpr bool BF = DT == MODEL_BF16, F32 = DT == MODEL_F32;
+  static_assert(U == 8 && RT % 2 == 0, "eight scales per row and share; float32 loads them for pairs of tiles");
   constexpr int STEPS = U / 4;
   constexpr int EL = F32 ? 4 : 2;     // bytes of an activation, a scale
+  constexpr bool PAIR = F32;        // scales come for pairs of tiles (see issue_scales)
   constexpr int BR = F32 ? 5 : 16;    // activation rows a batch tile holds
   constexpr int SW = F32 ? U : U / 2; // registers of a row's U scales
   constexpr uint32_t kMagic = BF ? 0x43004300u : 0x64006400u;
@@ -159,7 +161,6 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
   //      zeros, and a tile past the end (a wave's last rounds issue for tiles that do not exist) gets the tensor's size
   //      as its offset, which puts every lane out of range: zeros, and no memory traffic.  Nothing of either is kept.
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
   const uint32_t w_bytes = static_cast<uint32_t>(p.N) * static_cast<uint32_t>(p.nw) * 4u;
   const uint32_t s_bytes = static_cast<uint32_t>(p.N) * static_cast<uint32_t>(p.ng) * EL;
   const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -189,29 +190,44 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
       const int ga_raw = ((static_cast<int>(blockIdx.z) + ph) * kw + ks) * U;  // (slices > 1: one phase each)
       const bool k_live = ga_raw < p.ng;  // (uniform; ng % U == 0: a share is whole or empty)
       const int ga = k_live ? ga_raw : p.ng - U;
-      const int w_lane = (c * p.nw + 4 * (ga + j)) * 4, s_lane = (c * p.ng + ga) * EL;
+      const int w_lane = (c * p.nw + 4 * (ga + j)) * 4;
       u32x4 w[RT][STEPS];  // (kept as whole register tuples until the point of use, see walk_tile)
-      uint32_t sc[RT][SW];  // the U scales of this lane's row (16-bit: two per register)
-      auto issue = [&](int r, u32x4 (&wv)[STEPS], uint32_t (&sv)[SW]) {
+      auto issue = [&](int r, u32x4 (&wv)[STEPS]) {
         const int tile = tile_of(r);
         const int w_off = static_cast<int>(tile >= 0 ? static_cast<uint32_t>(tile) * w_tile : w_bytes);
-        const int s_off = static_cast<int>(tile >= 0 ? static_cast<uint32_t>(tile) * s_tile : s_bytes);
 #pragma unroll
         for (int st = 0; st < STEPS; ++st) {
           wv[st] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_lane + 64 * st, w_off, 0);
         }
-        if constexpr (F32) {
-#pragma unroll
-          for (int q = 0; q < U / 4; ++q) {
-            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, s_lane + 16 * q, s_off, 0);
-            sv[4 * q] = v.x; sv[4 * q + 1] = v.y; sv[4 * q + 2] = v.z; sv[4 * q + 3] = v.w;
-          }
-        } else if constexpr (U == 8) {
-          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, s_lane, s_off, 0);
+      };
+      // scales: the U of this lane's row c.  float32 (PAIR): of the tiles of rounds r and r + 1 in one load, lane (c, j) taking
+      // half j % 2 of row c of tile j / 2, handed round when a tile's turn comes.  A lane's own 32 bytes would be two loads per
+      // tile, which all four lanes of a row make to the same addresses; the texture unit was busy for 67 % of the kernel and
+      // is what the exchange relieves (four rows: 128256 x 4096 88 -> 77 us, 28672 x 4096 28 -> 23, 4096 x 14336 20.1 -> 18.4; the
+      // 16-bit scales are one load per tile, and the exchange's registers spill there)
+      const int s_lane = (c * p.ng + ga) * EL + (PAIR ? (j & 1) * (U / 2 * EL) : 0);
+      constexpr int NS = PAIR ? RT / 2 : RT;
+      constexpr int SR = PAIR ? SW / 2 : SW;
+      uint32_t sraw[NS][SR];
+      auto issue_scales = [&](int r, uint32_t (&sv)[SR]) {
+        const int t0 = tile_of(r);
+        const uint32_t o0 = t0 >= 0 ? static_cast<uint32_t>(t0) * s_tile : s_bytes;
+        if constexpr (PAIR) {
+          const int t1 = tile_of(r + 1);
+          const uint32_t o1 = t1 >= 0 ? static_cast<uint32_t>(t1) * s_tile : s_bytes;
+          const u32x4 v =
+              __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, s_lane + static_cast<int>(j < 2 ? o0 : o1), 0, 0);
           sv[0] = v.x; sv[1] = v.y; sv[2] = v.z; sv[3] = v.w;
         } else {
-          const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(s_rsrc, s_lane, s_off, 0);
-          sv[0] = v.x; sv[1] = v.y;
+          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, s_lane, static_cast<int>(o0), 0);
+          sv[0] = v.x; sv[1] = v.y; sv[2] = v.z; sv[3] = v.w;
+        }
+      };
+      auto issue_all = [&]() {
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          issue(r, w[r]);
+          if (!PAIR || r % 2 == 0) issue_scales(r, sraw[PAIR ? r / 2 : r]);
         }
       };
       mid_u4 xa[NBT][U];
@@ -234,8 +250,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
             hi[u] = *reinterpret_cast<const uint4*>(xrow + u * 32 + 4);
           }
           if (bt == NBT - 1) {  // (behind the loads of x: those are needed first, and loads retire in issue order)
-#pragma unroll
-            for (int r = 0; r < RT; ++r) issue(r, w[r], sc[r]);
+            issue_all();
           }
 #pragma unroll
           for (int u = 0; u < U; ++u) {
@@ -270,8 +285,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
 #pragma unroll
           for (int u = 0; u < U; ++u) xraw[bt][u] = *reinterpret_cast<const uint4*>(xrow + u * 32);
         }
-#pragma unroll
-        for (int r = 0; r < RT; ++r) issue(r, w[r], sc[r]);
+        issue_all();
 
         // ---- x in operand order, (x0, x4) (x2, x6) (x1, x5) / 16 (x3, x7) / 16, and the offset terms
 #pragma unroll
@@ -294,7 +308,29 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
       }
 
       // one tile from a ring slot; round `next` goes into the registers it leaves
-      auto walk_tile = [&](int next, u32x4 (&wv)[STEPS], uint32_t (&sv)[SW], float4_t (&acc)[NBT]) __attribute__((always_inline)) {
+      // (PAIR: first: the first of a pair of tiles; `odd`: the pair's scales after the exchange that splits them by tile, kept for
+      //  the second)
+      uint32_t odd[SR];
+      auto walk_tile = [&](bool first, int next, u32x4 (&wv)[STEPS], uint32_t (&sp)[SR], float4_t (&acc)[NBT]) __attribute__((always_inline)) {
+        uint32_t sv[SW];
+        if constexpr (PAIR) {
+          // to every lane: rows of 16 lanes hold (tile 0 half 0, tile 0 half 1, tile 1 half 0, tile 1 half 1)
+#pragma unroll
+          for (int q = 0; q < SW / 2; ++q) {
+            uint32_t mine = first ? sp[q] : odd[q];
+            if (first) {
+              auto e = __builtin_amdgcn_permlane32_swap(mine, mine, false, false);  // (0 0, 0 1, 0 0, 0 1) (1 0, 1 1, 1 0, 1 1)
+              mine = e[0];
+              odd[q] = e[1];
+            }
+            auto e = __builtin_amdgcn_permlane16_swap(mine, mine, false, false);  // half 0 everywhere, half 1 everywhere
+            sv[q] = e[0];
+            sv[SW / 2 + q] = e[1];
+          }
+        } else {
+#pragma unroll
+          for (int q = 0; q < SW; ++q) sv[q] = sp[q];
+        }
 #pragma unroll
         for (int bt = 0; bt < NBT; ++bt) acc[bt] = float4_t{0.f, 0.f, 0.f, 0.f};
         // (a zero the compiler cannot see through: the offset instruction would otherwise be hoisted out of the walk,
@@ -352,7 +388,8 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
         }
         // (after the arithmetic: the loads then land in the very registers the tile has left, with no copies whose
         //  wait would drain the queue)
-        issue(next, wv, sv);
+        issue(next, wv);
+        if (!PAIR || first) issue_scales(next, sp);
       };
 
       // ---- the K shares of a tile meet: 256 values per (round, tile lane, batch tile); thread (jq, cq) takes row
@@ -417,7 +454,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
 #pragma unroll
           for (int slot = 0; slot < RT; ++slot) {
             float4_t acc[NBT];
-            walk_tile(r0 + round + slot + RT, w[slot], sc[slot], acc);
+            walk_tile((slot & 1) == 0, r0 + round + slot + RT, w[slot], sraw[PAIR ? slot / 2 : slot], acc);
 #pragma unroll
             for (int bt = 0; bt < NBT; ++bt) {
               float4* const at = res_lds + (((round + slot) * 16 + wave) * NBT + bt) * 64 + lane;
@@ -474,7 +511,7 @@ hipError_t launch_mid(const MidParams& p, int wgx, int experts, hipStream_t s) {
     }
   }
   note_kernel("gq::midrow_kernel<%d,%d,%d,%d,%d%s> rounds=%d chunks=%d phases=%d slices=%d kw=%d", NBT, U, RT, int(KEEP_C),
-              int(PHASED), DT == MODEL_BF16 ? ",2" : (DT == MODEL_F32 ? ",1" : ""), p.rounds, p.chunks, p.phases, p.slices, 1 << p.kw_log2);
+              int(PHASED), DT == MODEL_BF16 ? ",true" : (DT == MODEL_F32 ? ",f32" : ""), p.rounds, p.chunks, p.phases, p.slices, 1 << p.kw_log2);
   hipLaunchKernelGGL((midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT>), dim3(wgx, experts, p.slices), dim3(1024), lds, s, p);
   return hipGetLastError();
 }
@@ -545,7 +582,7 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   const bool paired_walk = p.paired != 0;
   const int tw = 16 >> kwl;
   const int form = options().gemv_rows_per_wave;  // (tuning override: which one-batch-tile instance)
-  const int rt = form == 2 ? 4 : (form == 4 ? 3 : 2);
+  const int rt = form == 2 ? 4 : 2;
   // workgroups in all: one per CU (sixteen waves of up to 128 registers fill it), each with at most 128 KiB of sums in LDS
   const int want_wg = options().gemv_waves > 0 ? options().gemv_waves / 16 : 256;
   int wgx = want_wg / (experts * p.slices);
@@ -585,7 +622,6 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
     }
     if (nbt == 2) return launch_mid<2, 8, 2, false, false>(p, wgx, experts, s);
     if (form == 2) return launch_mid<1, 8, 4, false, false>(p, wgx, experts, s);
-    if (form == 4) return launch_mid<1, 8, 3, true, false>(p, wgx, experts, s);
     return launch_mid<1, 8, 2, true, false>(p, wgx, experts, s);
   };
   const hipError_t e = run();
