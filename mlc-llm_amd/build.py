@@ -1,6 +1,6 @@
-"""Build libmi355gq.so (gfx950 code only) with hipcc, in tree.
+"""Build libmi355gq.so (gfx950 code only) with hipcc and _mi355gq_torch.so (host code only) with g++, in tree.
 
-    python mlc-llm_amd/build.py            # compile every csrc/*.hip and link lib/libmi355gq.so
+    python mlc-llm_amd/build.py            # compile every csrc/*.hip and link lib/libmi355gq.so, then csrc/gq_torch.cc
 
 The TVM-FFI adapter (csrc/tvm_ffi_adapter.cc) is compiled in only when the
 `tvm_ffi` Python package (which ships tvm/ffi/c_api.h) is importable.
@@ -14,12 +14,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 OBJDIR = os.path.join(HERE, "build")
 LIB = os.path.join(LIBDIR, "libmi355gq.so")
+TORCH_EXT = os.path.join(LIBDIR, "_mi355gq_torch.so")
 
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 FLAGS = [
@@ -65,6 +67,24 @@ def _compile(src: str, extra: list[str]) -> str:
     return obj
 
 
+def _build_torch_ext() -> None:
+    """The native call path of the dense operators: a Python extension module on torch's C++ interface, linked to the library."""
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
+    includes = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f for i in includes for f in ("-isystem", i)), os.path.join(CSRC, "gq_torch.cc"), "-o", TORCH_EXT,
+           "-L" + os.path.join(root, "lib"), "-L" + LIBDIR, "-l:libmi355gq.so", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for gq_torch.cc:\n{r.stdout}\n{r.stderr}")
+
+
 def build(verbose: bool = True) -> str:
     os.makedirs(LIBDIR, exist_ok=True)
     os.makedirs(OBJDIR, exist_ok=True)
@@ -82,6 +102,7 @@ def build(verbose: bool = True) -> str:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
+    _build_torch_ext()
     if verbose:
         print(f"built {LIB} from {len(objs)} objects" + (" (+tvm_ffi adapter)" if ffi_inc else ""))
     return LIB

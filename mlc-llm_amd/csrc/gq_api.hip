@@ -18,13 +18,9 @@ Options& options() {
   return o;
 }
 
-static thread_local char g_last_kernel[160] = "";
-
-void note_kernel(const char* fmt, ...) {
-  va_list ap;
-  va_start(ap, fmt);
-  vsnprintf(g_last_kernel, sizeof(g_last_kernel), fmt, ap);
-  va_end(ap);
+Note& last_note() {
+  static thread_local Note note;
+  return note;
 }
 
 // Raises a kernel's dynamic-LDS limit to the CU's 160 KiB, once per (kernel, device).  Called on every launch that
@@ -154,7 +150,13 @@ int mi355gq_check_device(void) {
   return MI355GQ_OK;
 }
 
-const char* mi355gq_testing_last_kernel(void) { return gq::g_last_kernel; }
+const char* mi355gq_testing_last_kernel(void) {
+  static thread_local char text[160];
+  const gq::Note& n = gq::last_note();
+  text[0] = 0;
+  if (n.fmt != nullptr) n.render(n, text, sizeof(text));
+  return text;
+}
 
 int mi355gq_testing_set_option(const char* name, int value) {
   GQ_REQUIRE(name != nullptr, "option name is null");

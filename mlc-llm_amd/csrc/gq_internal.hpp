@@ -4,6 +4,11 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <stdio.h>
+
+#include <new>
+#include <tuple>
+#include <type_traits>
 
 namespace gq {
 
@@ -23,9 +28,28 @@ struct Options {
 };
 Options& options();
 
-// Records which kernel instantiation the calling thread launched last (thread-local text, read back through the
-// test hook mi355gq_testing_last_kernel): measurement code names the kernel it timed from the run itself.
-void note_kernel(const char* fmt, ...);
+// Records which kernel instantiation the calling thread launched last (thread-local, read back through the test hook
+// mi355gq_testing_last_kernel): measurement code names the kernel it timed from the run itself.  A launch keeps the format
+// and its arguments (integers and string literals); the text is made when it is asked for, because formatting it took as
+// long as a tenth of a small launch.
+struct Note {
+  const char* fmt = nullptr;
+  void (*render)(const Note&, char*, size_t) = nullptr;
+  alignas(8) unsigned char args[128];
+};
+Note& last_note();
+
+template <class... A>
+void note_kernel(const char* fmt, A... a) {
+  using Args = std::tuple<A...>;
+  static_assert(sizeof(Args) <= sizeof(Note::args) && (std::is_trivially_copyable_v<A> && ...), "plain arguments");
+  Note& n = last_note();
+  n.fmt = fmt;
+  new (n.args) Args(a...);
+  n.render = [](const Note& note, char* out, size_t size) {
+    std::apply([&](const auto&... v) { snprintf(out, size, note.fmt, v...); }, *reinterpret_cast<const Args*>(note.args));
+  };
+}
 
 // hipFuncAttributeMaxDynamicSharedMemorySize = the CU's whole LDS, set once per (kernel, device) and remembered;
 // kernels whose dynamic LDS may exceed 64 KiB call it before launching.

@@ -1,4 +1,5 @@
-"""ctypes binding of libmi355gq.so (the C ABI declared in include/mi355gq.h).
+"""ctypes binding of libmi355gq.so (the C ABI declared in include/mi355gq.h), and the native call path of the dense
+operators beside it (_mi355gq_torch.so, csrc/gq_torch.cc).
 
 There is no fallback: if the shared library is missing or a call fails, an
 exception is raised.  Tensors are torch tensors on the ROCm device; only their
@@ -8,12 +9,15 @@ exception is raised.  Tensors are torch tensors on the ROCm device; only their
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import re
 from ctypes import c_char_p, c_int, c_int64, c_void_p
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_HERE), "lib", "libmi355gq.so")
+TORCH_PATH = os.path.join(os.path.dirname(_HERE), "lib", "_mi355gq_torch.so")
 HEADER_PATH = os.path.join(os.path.dirname(os.path.dirname(_HERE)), "include", "mi355gq.h")
 
 OK = 0
@@ -105,6 +109,7 @@ class Mi355gqError(RuntimeError):
 
 
 _LIB = None
+_TORCH = None
 
 
 def declared_symbols() -> list[str]:
@@ -132,12 +137,30 @@ def lib() -> ctypes.CDLL:
     return _LIB
 
 
+def native():
+    """The native call path of the dense operators (loaded once).  Raises if it has not been built."""
+    global _TORCH
+    if _TORCH is None:
+        lib()  # the library it is linked to
+        if not os.path.exists(TORCH_PATH):
+            raise RuntimeError(f"{TORCH_PATH} is missing: build it with `python mlc-llm_amd/build.py`")
+        loader = importlib.machinery.ExtensionFileLoader("_mi355gq_torch", TORCH_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_mi355gq_torch", loader))
+        loader.exec_module(module)
+        _TORCH = module
+    return _TORCH
+
+
+def failed(name: str, rc: int) -> "Mi355gqError":
+    """The error of an entry point that returned `rc` on this thread."""
+    return Mi355gqError(name, rc, lib().mi355gq_last_error().decode("utf-8", "replace"))
+
+
 def call(name: str, *args) -> None:
     """Invoke an int-returning entry point; raise Mi355gqError on failure."""
-    handle = lib()
-    rc = getattr(handle, name)(*args)
+    rc = getattr(lib(), name)(*args)
     if rc != OK:
-        raise Mi355gqError(name, rc, handle.mi355gq_last_error().decode("utf-8", "replace"))
+        raise failed(name, rc)
 
 
 def last_kernel() -> str:

@@ -4,6 +4,9 @@ Each function plays the role the Relax VM plays around `call_dps_packed`: it
 checks shapes and dtypes, allocates the output tensor(s) and hands raw pointers
 plus the current HIP stream to the C ABI.  uint32 storage is held in int32
 torch tensors (same bits; torch's uint32 support on device is partial).
+
+linear, linear_silu_mul and embedding_take first offer their arguments to the native call path (csrc/gq_torch.cc), which does the
+same checks, allocation and call in one step; it declines (None) whatever it does not recognise, and the Python below decides.
 """
 
 from __future__ import annotations
@@ -16,7 +19,7 @@ from . import _lib
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _lib.native().stream()
 
 
 def _chk(t: torch.Tensor, dtype, name: str) -> torch.Tensor:
@@ -95,6 +98,11 @@ def _check_qshapes(q_weight, q_scale, lead, k, bits, group_size):
 
 def embedding_take(ids: torch.Tensor, q_weight: torch.Tensor, q_scale: torch.Tensor, k: int,
                    bits: int, group_size: int) -> torch.Tensor:
+    done = _lib.native().embedding_take(ids, q_weight, q_scale, k, bits, group_size)
+    if isinstance(done, torch.Tensor):
+        return done
+    if done is not None:
+        raise _lib.failed("mi355gq_embedding_take_dt", done)
     _chk(ids, torch.int32, "ids")
     _chk(q_weight, _STORAGE, "q_weight")
     _chk(q_scale, _FLOATS, "q_scale")
@@ -118,6 +126,11 @@ def linear(x: torch.Tensor, q_weight: torch.Tensor, q_scale: torch.Tensor, bits:
 
     `residual` (fp16, the shape of y) is added inside the kernel; passing the same tensor as `out`
     updates it in place."""
+    done = _lib.native().linear(x, q_weight, q_scale, bits, group_size, bias, out_dtype, out, residual)
+    if isinstance(done, torch.Tensor):
+        return done
+    if done is not None:
+        raise _lib.failed("mi355gq_linear_dt" if residual is None else "mi355gq_linear_residual_dt", done)
     _chk(x, _FLOATS, "x")
     if x.dtype != torch.float16:
         return _linear_other_dtype(x, q_weight, q_scale, bits, group_size, bias, out_dtype, out, residual)
@@ -280,6 +293,11 @@ def linear_silu_mul(x: torch.Tensor, q_weight: torch.Tensor, q_scale: torch.Tens
     """silu(x1) * x2 with x1, x2 = split(linear(x), 2, axis=-1): the gate_up projection of an MLP
     with its activation folded into the matmul kernel.  Bit-identical to linear then silu_mul;
     shapes without a fused kernel run exactly those two calls."""
+    done = _lib.native().linear_silu_mul(x, q_weight, q_scale, bits, group_size)
+    if isinstance(done, torch.Tensor):
+        return done
+    if done is not None and done != _lib.ERR_UNSUPPORTED:
+        raise _lib.failed("mi355gq_linear_silu_mul_dt", done)
     _chk(x, _FLOATS, "x")
     _chk(q_weight, _STORAGE, "q_weight")
     _chk(q_scale, x.dtype, "q_scale")

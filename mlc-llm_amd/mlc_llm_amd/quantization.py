@@ -255,8 +255,7 @@ class GroupQuantizeLinear(nn.Module):
         model_dtype = _TORCH_DTYPE[self.config.model_dtype]
         out_dtype = model_dtype if self.out_dtype is None else _TORCH_DTYPE[self.out_dtype]
         bias = self.bias
-        rows = x.numel() // max(x.shape[-1], 1)
-        if (self.config.linear_weight_layout == "KN" and model_dtype == torch.float16 and rows <= 8
+        if (self.config.linear_weight_layout == "KN" and model_dtype == torch.float16 and x.numel() // max(x.shape[-1], 1) <= 8
                 and self.out_features % 4 == 0 and (bias is None or bias.dtype == model_dtype)):
             # decode batches of a KN-layout model: the stored tensors are streamed as they are
             return ops.linear_kn(x, self.q_weight, self.q_scale, self.config.bits, self.config.group_size, bias, out_dtype)
@@ -296,10 +295,8 @@ class GroupQuantizeEmbedding(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         self.config._require_built(matmul=False)
-        ids = x.reshape(-1).to(torch.int32).contiguous()
-        out = ops.embedding_take(ids, self.q_weight, self.q_scale, self.dim, self.config.bits,
-                                 self.config.group_size)
-        return out.reshape(*x.shape, self.dim)
+        return ops.embedding_take(x.to(torch.int32).contiguous(), self.q_weight, self.q_scale, self.dim, self.config.bits,
+                                  self.config.group_size)
 
     def lm_head_forward(self, x: torch.Tensor) -> torch.Tensor:
         """Dequantize the table and multiply: logits in float32."""
