@@ -370,7 +370,7 @@ int64_t mi355gq_linear_dt_workspace_bytes(int64_t M, int64_t N, int64_t K, int b
   // bfloat16: every batch from two rows on may run the few-row GEMM (there are no bf16 skinny kernels); 9..16 rows of a
   // long K: the K slices of the kernel on unscaled weight operands
   const int64_t mid = (bits == 4 && M <= 16 && (M > 8 || (M > 4 && K > 8192))) ? gq::midrow_workspace_bytes(M, N, K) : 0;
-  const int64_t gemm = gq::gemm_workspace_bytes(M, N, K, bits, group_size);
+  const int64_t gemm = gq::gemm_workspace_bytes(M, N, K, bits, group_size, 1);
   return gemm > mid ? gemm : mid;
 }
 

@@ -226,15 +226,17 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
   }
   if (a.rows == 0 || a.N == 0) return hipSuccess;
   const int variant = options().gemm_variant;
-  if (variant < 0 || a.bf16) {
-    const SplitPlan plan = plan_split_k(a.rows, a.N, a.K, a.bits, a.group_size, a.indptr != nullptr);
-    p.bm_hint = plan.bm;
-    const int64_t need = static_cast<int64_t>(plan.split) * a.rows * a.N * 4;
-    // without (enough) scratch the same tiles run unsplit: slower, never wrong
+  {
     // (fused gate/up form: the partial sums keep the tile's column order, which only lines up with
     //  rows of N floats when the gate half is whole 32-row blocks)
-    if (plan.bm > 0 && plan.split > 1 && a.workspace != nullptr && a.workspace_bytes >= need &&
-        (reinterpret_cast<uintptr_t>(a.workspace) & 15) == 0 && (!a.paired || (a.N % 64) == 0)) {
+    const bool may_split = (variant < 0 || a.bf16) && a.workspace != nullptr && (reinterpret_cast<uintptr_t>(a.workspace) & 15) == 0 &&
+                           (!a.paired || (a.N % 64) == 0);
+    const int64_t scratch = may_split ? a.workspace_bytes : 0;
+    const SplitPlan plan = plan_split_k(a.rows, a.N, a.K, a.bits, a.group_size, a.indptr != nullptr, a.bf16, scratch);
+    p.bm_hint = plan.bm;
+    p.bn_hint = plan.bn;
+    // without (enough) scratch the same tiles run unsplit: slower, never wrong
+    if (plan.bm > 0 && plan.split > 1 && scratch >= static_cast<int64_t>(plan.split) * a.rows * a.N * 4) {
       p.partial = static_cast<float*>(a.workspace);
       p.kt_per_split = plan.kt_per_split;
     }
@@ -271,9 +273,9 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
   return launch_cfg<3, 128, 128, 64, 64>(p, s);
 }
 
-int64_t gemm_workspace_bytes(int64_t rows, int64_t N, int64_t K, int bits, int group_size) {
+int64_t gemm_workspace_bytes(int64_t rows, int64_t N, int64_t K, int bits, int group_size, int bf16) {
   if (options().gemm_variant >= 0) return 0;
-  const SplitPlan plan = plan_split_k(rows, N, K, bits, group_size, false);
+  const SplitPlan plan = plan_split_k(rows, N, K, bits, group_size, false, bf16, kMaxSplitBytes);
   return plan.bm > 0 && plan.split > 1 ? static_cast<int64_t>(plan.split) * rows * N * 4 : 0;
 }
 

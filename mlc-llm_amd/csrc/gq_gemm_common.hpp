@@ -34,7 +34,8 @@ struct GemmParams {
   // `partial` is set, leaves its fp32 tile in partial[z][rows][N] for the reduction kernel
   float* partial;
   int kt_per_split;
-  int bm_hint;  // rows per tile chosen by plan_split_k (0: regular tiles)
+  int bm_hint;  // rows, columns per tile chosen by plan_split_k (0: regular tiles)
+  int bn_hint = 0;
   // Fused gate/up form: y[rows, N / 2] = silu(x . W[j]) * (x . W[N / 2 + j]).  A tile's columns walk
   // the stored rows in blocks of 32 gate rows then the matching 32 up rows, so both halves of an
   // output element sit in the same lane and register of neighbouring 32 x 32 accumulators (blocks of
@@ -70,13 +71,15 @@ __global__ void splitk_reduce_silu_kernel(const float* partial, int split, int64
 // gate rows per column block (32 | 16) of the tile launch_gemm_pipe picks for these parameters
 int gemm_pipe_pair_block(const GemmParams& p, int bits);
 
-// How a few-row GEMM is cut so that every CU streams weights: rows per tile and K splits.
+// How a plain GEMM is cut: its tile and K splits.
 struct SplitPlan {
-  int bm;            // 0: not a few-row problem, use the regular tiles
+  int bm, bn;        // 0: no plan, use the regular tiles
   int split;         // workgroups along K (1: no reduction pass)
   int kt_per_split;  // K tiles (2 groups each) per workgroup
 };
-SplitPlan plan_split_k(int64_t rows, int64_t N, int64_t K, int bits, int group_size, bool grouped);
+// scratch_bytes: what the partial sums of a split may take
+SplitPlan plan_split_k(int64_t rows, int64_t N, int64_t K, int bits, int group_size, bool grouped, int bf16, int64_t scratch_bytes);
+constexpr int64_t kMaxSplitBytes = int64_t(32) << 20;  // no plan of the q4 cost model asks for more
 
 // One group (4 storage words) -> G halves in natural k order, (q - m) * s with fp16 rounding.
 template <int BITS>

@@ -602,9 +602,83 @@ __global__ __launch_bounds__(256) void splitk_reduce_silu_kernel(const float* __
   }
 }
 
-SplitPlan plan_split_k(int64_t rows, int64_t N, int64_t K, int bits, int group_size, bool grouped) {
-  SplitPlan plan{0, 1, 1 << 28};
+// The plain q4 GEMM's tiles beyond 64 rows, each with its fitted cost (us): a launch of `tiles x split` workgroups of `kt` K
+// tiles takes
+//   base + whole * kt * pairs + odd * kt * odd_one + filled * kt * per_cu + live * kt * per_cu * (rows / tile rows) + round * rounds
+//        + (split: reduce + 1e-6 * traffic * split * rows * N) + 1e-6 * store * rows * N
+// per_cu = workgroups / 256 (fractional), rounds = per_cu rounded up; the tiles of four waves sit two on a CU (pairs = rounds / 2, a
+// lone one `odd_one`), the others one (pairs = rounds).  The last, partly filled round is what decides between tiles; the terms in
+// the fractional per_cu are the part's power limit (a round on half the CUs runs faster than a full one) and, for the tiles whose waves
+// skip row blocks past the last row, the matrix work that is left out.
+struct TileCost {
+  int bm, bn;
+  int skip;  // waves skip the 32-row blocks past the last row (256-row tiles: for a row count that leaves such blocks)
+  float base, whole, odd, filled, live, round, reduce, traffic, store;
+};
+// Least squares (non-negative) over 22 shapes (N 2048..37888, K 2048..28672, the projections of 1.5B to 70B models) x 19 row counts from
+// 72 to 4096 x splits of 1 to 16: 7500 timings, 5-6 % rms.  Choosing by it instead of by the rules it replaced (128 x 128 tiles split up to
+// 256 workgroups to 1024 rows, three unsplit tiles beyond) makes those launches 7.3 % (bfloat16 10.8 %) faster on average, where
+// the best of all measured choices would make 8.1 % (11.3 %).  For instance (us): 4096 x 14336 at 160 / 300 / 640 / 777 rows 43.6 / 77.8 /
+// 113.5 / 129 -> 36.9 / 62 / 89.8 / 117 (bfloat16 46.3 / 85.2 / 122.5 / 143 -> 37.0 / 61.2 / 91.9 / 113), 4096 x 4096 at 300 rows 37.1 -> 27.2, 28672 x
+// 4096 at 160 / 300 / 777 rows 66.3 / 112.5 / 219.8 -> 54.3 / 92.7 / 207.4; from 1536 rows on the choice is mostly the old one.
+constexpr TileCost kTilesF16[] = {
+    {128, 128, 0, 6.83f, 0.593f, 0.37f, 0.219f, 0, 0, 2.51f, 0.862f, 0.333f},
+    {128, 256, 0, 5.43f, 0.549f, 0, 0.419f, 0, 2.18f, 2.62f, 0.72f, 0.15f},
+    {256, 256, 0, 0, 0.922f, 0, 0.681f, 0, 11.9f, 2.65f, 0.371f, 0.0433f},
+    {256, 256, 1, 1.01f, 0.933f, 0, 0, 0.712f, 10.6f, 3.66f, 0.405f, 0},
+    {256, 128, 1, 7.72f, 0.57f, 0, 0, 0.437f, 1.25f, 2.89f, 0.57f, 0},
+    {64, 128, 0, 6.12f, 0.458f, 0.31f, 0.104f, 0, 0.000585f, 1.35f, 1.63f, 0.153f},
+};
+constexpr TileCost kTilesBf16[] = {  // (more vector instructions per weight: the tiles that dequantise it less often are ahead)
+    {128, 128, 0, 8.01f, 0.62f, 0.4f, 0.224f, 0, 0, 2.5f, 0.731f, 0.371f},
+    {128, 256, 0, 6.06f, 0.625f, 0, 0.386f, 0, 2.48f, 2.62f, 0.578f, 0.225f},
+    {256, 256, 0, 0.54f, 1.01f, 0, 0.574f, 0, 10.2f, 3.73f, 0.396f, 0.151f},
+    {256, 256, 1, 6.62f, 0.969f, 0, 0, 0.692f, 4.42f, 4.4f, 0.384f, 0.0966f},
+    {256, 128, 1, 7.17f, 0.552f, 0, 0, 0.411f, 2.2f, 2.86f, 0.517f, 0},
+    {64, 128, 0, 7.4f, 0.509f, 0.348f, 0.115f, 0, 0, 1.12f, 1.3f, 0.235f},
+};
+
+static SplitPlan plan_by_cost(int64_t rows, int64_t N, int nk, int bf16, int64_t scratch_bytes) {
+  SplitPlan best{0, 0, 1, 1 << 28};
+  float best_us = 0.f;
+  if (scratch_bytes > kMaxSplitBytes) scratch_bytes = kMaxSplitBytes;
+  const float mn = 1e-6f * static_cast<float>(rows) * static_cast<float>(N);
+  for (int t = 0; t < 6; ++t) {
+    const TileCost& c = bf16 ? kTilesBf16[t] : kTilesF16[t];
+    if (c.bm == 256 && (c.skip != 0) != (c.bn == 128 || rows % 256 != 0)) continue;
+    const int64_t mt = (rows + c.bm - 1) / c.bm, tiles = mt * ((N + c.bn - 1) / c.bn);
+    const float live = static_cast<float>(rows) / static_cast<float>(mt * c.bm);
+    const bool pairs = c.bm * c.bn <= 128 * 128;  // (four waves: two workgroups on a CU)
+    int last = 0;
+    for (int want = 1; want <= 16; ++want) {
+      const int kt = ((nk + want - 1) / want + 3) / 4 * 4;  // (the K loop advances four tiles at a time)
+      const int split = (nk + kt - 1) / kt;
+      // at least four K tiles per workgroup, and no more workgroups than two and a half rounds of one per CU
+      if (split > 1 && (want > nk / 4 || tiles * split > 640 || split * rows * N * 4 > scratch_bytes)) break;
+      if (split == last) continue;
+      last = split;
+      const int64_t wgs = tiles * split, rounds = (wgs + 255) / 256;
+      const float ktf = static_cast<float>(split > 1 ? kt : (nk + 3) / 4 * 4), per_cu = static_cast<float>(wgs) / 256.f;
+      float us = c.base + ktf * (c.whole * static_cast<float>(pairs ? rounds / 2 : rounds) + (pairs ? c.odd * static_cast<float>(rounds % 2) : 0.f) +
+                                 per_cu * (c.filled + c.live * live)) +
+                 c.round * static_cast<float>(rounds) + c.store * mn;
+      // (a split has to be 2 % ahead on paper)
+      if (split > 1) us = (us + c.reduce + c.traffic * static_cast<float>(split) * mn) * 1.02f;
+      if (best.bm == 0 || us < best_us) {
+        best_us = us;
+        best = SplitPlan{c.bm, c.bn, split, split > 1 ? kt : 1 << 28};
+      }
+    }
+  }
+  return best;
+}
+
+SplitPlan plan_split_k(int64_t rows, int64_t N, int64_t K, int bits, int group_size, bool grouped, int bf16, int64_t scratch_bytes) {
+  SplitPlan plan{0, 0, 1, 1 << 28};
   if (grouped || rows <= 0 || N <= 0 || K <= 0 || (K & 7) != 0) return plan;
+  const int ng = static_cast<int>((K + group_size - 1) / group_size);
+  const int nk = (ng + 1) / 2;
+  if (bits == 4 && rows > 64 && options().gemm_split_k <= 0) return plan_by_cost(rows, N, nk, bf16, scratch_bytes);
   // few rows: the GEMM is bound by streaming the weights, and 128-wide column tiles alone leave
   // most CUs idle (o_proj / down have 32 of them).  Match the tile height to the rows and cut K
   // until about one workgroup per CU exists.
@@ -614,8 +688,7 @@ SplitPlan plan_split_k(int64_t rows, int64_t N, int64_t K, int bits, int group_s
   const int64_t tiles = ((rows + bm - 1) / bm) * ((N + 127) / 128);
   if (rows > 128 && tiles >= 200) return plan;  // the regular tiles already fill the chip
   plan.bm = bm;
-  const int ng = static_cast<int>((K + group_size - 1) / group_size);
-  const int nk = (ng + 1) / 2;
+  plan.bn = 128;
   // Splitting K pays with partial sums (split * rows * N * 8 bytes written and read back): only
   // when the tiles alone leave CUs idle, and never beyond about twice the weight bytes.
   int split = 1;
@@ -636,34 +709,33 @@ SplitPlan plan_split_k(int64_t rows, int64_t N, int64_t K, int bits, int group_s
 }
 
 int gemm_pipe_pair_block(const GemmParams& p, int bits) {
-  return (p.bm_hint == 32 && options().gemm_variant < 0) ? 16 : 32;  // the 32 x 128 tile below
+  return p.bm_hint == 32 ? 16 : 32;  // the 32 x 128 tile below
 }
 
-// Which of the three regular tiles a plain matmul of this shape should run: 2 = 256 x 256, 1 = 128 x 256,
-// 0 = 128 x 128.  A launch costs rounds x (time of one tile), rounds = ceil(tiles / resident workgroups) (256 for
-// the two large tiles, 512 for 128 x 128), tile times from the per-tile rates measured with balanced rounds (q4:
-// 1035 / 870 / 806 TFLOP/s; q3, whose K tile does not fit the largest one: 739 / 566).  What the model is for is the
-// last, partly filled round: 300 tiles of 256 x 256 take two rounds where 540 of 128 x 256 take three half-sized
-// ones (13B qkv at 1025 rows: 584 -> 621 TFLOP/s; gate_up at 1025 rows: 699 -> 785; qkv 6144 x 4096 at 1536 rows, the
-// other way round: 568 -> 706).
-int pick_regular_tile(int64_t rows, int64_t N, int bits) {
-  const int64_t ntw = (N + 255) / 256, ntn = (N + 127) / 128;
-  const int64_t big = ((rows + 255) / 256) * ntw, mid = ((rows + 127) / 128) * ntw, small = ((rows + 127) / 128) * ntn;
-  const double t_big = 65536.0 / (1035.0 / 256), t_mid = 32768.0 / ((bits == 4 ? 870.0 : 739.0) / 256),
-               t_small = 16384.0 / ((bits == 4 ? 806.0 : 566.0) / 512);
-  const double c_big = bits == 4 ? static_cast<double>((big + 255) / 256) * t_big : 1e30;
-  const double c_mid = static_cast<double>((mid + 255) / 256) * t_mid;
-  // 128 x 128: two workgroups share a CU; one on its own runs faster than its half of a pair (0.72 of the
-  // pair's time fits 13B o_proj at 640 rows, 200 such tiles: 539 TFLOP/s against 420 on 100 tiles of 128 x 256)
+// q3: 128 x 256 tiles rather than 128 x 128 (a K tile is 80 wide and the 256 x 256 tile does not fit LDS)?  A launch costs rounds x
+// (time of one tile), rounds = ceil(tiles / resident workgroups) (256, 512 for 128 x 128), tile times from the rates measured with
+// balanced rounds, 739 / 566 TFLOP/s.
+static bool q3_wide_tile(int64_t rows, int64_t N) {
+  const int64_t mid = ((rows + 127) / 128) * ((N + 255) / 256), small = ((rows + 127) / 128) * ((N + 127) / 128);
+  const double t_mid = 32768.0 / (739.0 / 256), t_small = 16384.0 / (566.0 / 512);
+  // 128 x 128: two workgroups share a CU; one on its own runs faster than its half of a pair (0.72 of the pair's time)
   const int64_t per_cu = (small + 255) / 256;
   const double c_small = static_cast<double>(per_cu / 2) * t_small + static_cast<double>(per_cu % 2) * 0.72 * t_small;
   // a partly filled last round runs faster than a full one (the part is power-limited), which favours the larger
-  // tile: a smaller tile has to win by 8 % on paper
-  int pick = 2;
-  double best = c_big;
-  if (c_mid < 0.92 * best) { pick = 1; best = c_mid; }
-  if (c_small < 0.92 * best) pick = 0;
-  return pick;
+  // tile: the smaller one has to win by 8 % on paper
+  return c_small >= 0.92 * static_cast<double>((mid + 255) / 256) * t_mid;
+}
+
+// the planned tile of a plain q4 matmul (see plan_split_k)
+template <bool BF>
+static hipError_t launch_planned_q4(const GemmParams& p, hipStream_t s) {
+  if (p.bm_hint == 32) return launch_pipe_cfg<4, 32, 128, 32, 32, 4, BF>(p, s);
+  if (p.bm_hint == 64) return launch_pipe_cfg<4, 64, 128, 32, 64, 4, BF>(p, s);
+  if (p.bm_hint == 128 && p.bn_hint == 256) return launch_pipe_cfg<4, 128, 256, 64, 64, 2, BF>(p, s);
+  if (p.bm_hint == 256 && p.bn_hint == 128) return launch_pipe_cfg<4, 256, 128, 64, 64, 2, BF, true, 2>(p, s);
+  if (p.bm_hint == 256)
+    return p.rows % 256 != 0 ? launch_pipe_cfg<4, 256, 256, 128, 64, 2, BF, true, 2>(p, s) : launch_pipe_cfg<4, 256, 256, 128, 64, 2, BF>(p, s);
+  return launch_pipe_cfg<4, 128, 128, 64, 64, 2, BF>(p, s);
 }
 
 hipError_t launch_gemm_pipe(const GemmParams& p, int bits, hipStream_t s) {
@@ -672,10 +744,8 @@ hipError_t launch_gemm_pipe(const GemmParams& p, int bits, hipStream_t s) {
   if (p.paired && (p.N & 1)) return hipErrorNotSupported;
   if (p.bf16) {
     // bfloat16 models: plain and grouped matmul (no folded activation)
+    if (p.indptr == nullptr && bits == 4) return launch_planned_q4<true>(p, s);
     if (p.bm_hint > 0 && p.indptr == nullptr) {  // few rows, K possibly split (see plan_split_k)
-      if (bits == 4 && p.bm_hint == 32) return launch_pipe_cfg<4, 32, 128, 32, 32, 4, true>(p, s);
-      if (bits == 4 && p.bm_hint == 64) return launch_pipe_cfg<4, 64, 128, 32, 64, 4, true>(p, s);
-      if (bits == 4) return launch_pipe_cfg<4, 128, 128, 64, 64, 2, true>(p, s);
       if (p.bm_hint == 32) return launch_pipe_cfg<3, 32, 128, 32, 32, 4, true>(p, s);
       if (p.bm_hint == 64) return launch_pipe_cfg<3, 64, 128, 32, 64, 4, true>(p, s);
       return launch_pipe_cfg<3, 128, 128, 64, 64, 2, true>(p, s);
@@ -694,22 +764,11 @@ hipError_t launch_gemm_pipe(const GemmParams& p, int bits, hipStream_t s) {
       return wide ? launch_pipe_cfg<3, 128, 256, 64, 64, 2, true>(p, s)
                   : launch_pipe_cfg<3, 128, 128, 64, 64, 2, true>(p, s);
     }
-    if (bits == 4) {
-      // few rows: tile height follows the rows (the float16 path's few-row tiles, unsplit)
-      if (p.rows <= 32) return launch_pipe_cfg<4, 32, 128, 32, 32, 4, true>(p, s);
-      if (p.rows <= 64) return launch_pipe_cfg<4, 64, 128, 32, 64, 4, true>(p, s);
-      const int tile = pick_regular_tile(p.rows, p.N, 4);
-      if (tile == 2) return launch_pipe_cfg<4, 256, 256, 128, 64, 2, true>(p, s);
-      if (tile == 1) return launch_pipe_cfg<4, 128, 256, 64, 64, 2, true>(p, s);
-      return launch_pipe_cfg<4, 128, 128, 64, 64, 2, true>(p, s);
-    }
-    if (pick_regular_tile(p.rows, p.N, 3) == 1) return launch_pipe_cfg<3, 128, 256, 64, 64, 2, true>(p, s);
+    if (q3_wide_tile(p.rows, p.N)) return launch_pipe_cfg<3, 128, 256, 64, 64, 2, true>(p, s);
     return launch_pipe_cfg<3, 128, 128, 64, 64, 2, true>(p, s);
   }
+  if (p.indptr == nullptr && bits == 4 && variant != 6 && variant != 7 && variant != 9) return launch_planned_q4<false>(p, s);
   if (p.bm_hint > 0 && variant < 0) {
-    if (bits == 4 && p.bm_hint == 32) return launch_pipe_cfg<4, 32, 128, 32, 32, 4>(p, s);
-    if (bits == 4 && p.bm_hint == 64) return launch_pipe_cfg<4, 64, 128, 32, 64, 4>(p, s);
-    if (bits == 4) return launch_pipe_cfg<4, 128, 128, 64, 64>(p, s);
     if (p.bm_hint == 32) return launch_pipe_cfg<3, 32, 128, 32, 32, 4>(p, s);
     if (p.bm_hint == 64) return launch_pipe_cfg<3, 64, 128, 32, 64, 4>(p, s);
     return launch_pipe_cfg<3, 128, 128, 64, 64>(p, s);
@@ -754,12 +813,9 @@ hipError_t launch_gemm_pipe(const GemmParams& p, int bits, hipStream_t s) {
       if (p.rows <= 16 * p.num_experts) return launch_pipe_cfg<4, 32, 128, 32, 32, 4>(p, s);
       if (p.rows <= 48 * p.num_experts) return launch_pipe_cfg<4, 64, 128, 32, 64, 4>(p, s);
     }
-    // plain matmul: the tile whose rounds of workgroups cost least (variants 6 / 7 / 9 force one)
-    const int tile = p.indptr != nullptr ? 0 : pick_regular_tile(p.rows, p.N, 4);
-    const bool big = variant == 7 ? true : (variant == 6 ? false : tile == 2);
+    // plain matmul, tuning override: variants 6 / 7 / 9 force one tile
     if (variant == 9) return launch_pipe_cfg<4, 128, 256, 64, 64>(p, s);
-    if (big) return launch_pipe_cfg<4, 256, 256, 128, 64>(p, s);
-    if (variant != 6 && tile == 1) return launch_pipe_cfg<4, 128, 256, 64, 64>(p, s);
+    if (variant == 7) return launch_pipe_cfg<4, 256, 256, 128, 64>(p, s);
     // grouped: the wider tile once the experts' row tiles alone make several rounds of workgroups
     if (variant != 6 && p.indptr != nullptr && p.rows >= 96 * p.num_experts &&
         (static_cast<int64_t>(p.rows) / 128 + p.num_experts) * ((p.N + 255) / 256) >= 768)
@@ -771,7 +827,7 @@ hipError_t launch_gemm_pipe(const GemmParams& p, int bits, hipStream_t s) {
     if (p.rows <= 48 * p.num_experts) return launch_pipe_cfg<3, 64, 128, 32, 64, 4>(p, s);
   }
   // q3: a K tile is 80 wide, so the 256 x 256 tile does not fit LDS; 128 x 256 does
-  const bool plain_wide = p.indptr == nullptr && pick_regular_tile(p.rows, p.N, 3) == 1;
+  const bool plain_wide = p.indptr == nullptr && q3_wide_tile(p.rows, p.N);
   const bool grouped_wide = p.indptr != nullptr && p.rows >= 96 * p.num_experts &&
                             (static_cast<int64_t>(p.rows) / 128 + p.num_experts) * ((p.N + 255) / 256) >= 768;
   if (variant == 9 || (variant != 6 && (plain_wide || grouped_wide)))

@@ -1,0 +1,49 @@
+"""The plain q4 GEMM beyond 64 rows: every tile that the cost model chooses between, whole and split along K, at sizes that leave
+ragged rows, columns and K tiles, against the float64 product of the dequantised weights (whose packing has tests of its own)."""
+
+import pytest
+import torch
+
+import mlc_llm_amd as gq
+from mlc_llm_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+# rows, N, K, tile, split along K
+CASES = [(65, 256, 256, "64,128", False), (65, 256, 1000, "64,128", True), (65, 6000, 4096, "128", True),
+         (333, 6000, 1000, "128,128", False), (513, 8200, 320, "128,256", False), (129, 4096, 4104, None, None), (160, 4096, 14336, "256,128", True),
+         (257, 4100, 2048, None, None), (777, 4096, 8192, "256,128", None), (300, 28672, 1024, "256,256", False),
+         (512, 28680, 512, "256,256", False), (1025, 2056, 4096, None, None)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k,tile,split", CASES)
+def test_planned_tiles(dtype, m, n, k, tile, split):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    w = (torch.randn((n, k), generator=g, device="cuda") * 0.02).to(dtype)
+    qw, qs = ops.quantize(w, 4, 32)
+    x = torch.randn((m, k), generator=g, device="cuda").to(dtype)
+    bias = torch.randn((n,), generator=g, device="cuda").to(dtype)
+    residual = torch.randn((m, n), generator=g, device="cuda").to(dtype)
+    want = x.double() @ ops.dequantize(qw, qs, k, 4, 32).double().t().contiguous()
+    # one rounding of the output (2^-11, bfloat16 2^-9 of the element), and float32 sums of K terms (sqrt(K) 2^-24 of the norm)
+    tol = (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -9) + 1e-5
+    full = want + bias.double() + residual.double()
+    got = ops.linear(x, qw, qs, 4, 32, bias, residual=residual)
+    kernel = gq._lib.last_kernel()
+    assert (got.double() - full).norm() / full.norm() <= tol, kernel
+    got32 = ops.linear(x, qw, qs, 4, 32, None, torch.float32)
+    assert (got32.double() - want).norm() / want.norm() <= 1e-5, kernel
+    need = gq._lib.lib().mi355gq_linear_dt_workspace_bytes(m, n, k, 4, 32, ops._MODEL_DTYPES[dtype])
+    assert need <= 32 << 20
+    if dtype == torch.float16:
+        assert split is None or (need > 0) == split, need
+        assert tile is None or f"gemm_pipe_kernel<4,{tile}," in kernel, kernel
+    # without scratch: another plan, unsplit
+    out = torch.empty((m, n), dtype=dtype, device="cuda")
+    gq._lib.call("mi355gq_linear_dt", x.data_ptr(), qw.data_ptr(), qs.data_ptr(), bias.data_ptr(), m, n, k, 4, 32,
+                 ops._MODEL_DTYPES[dtype], ops._MODEL_DTYPES[dtype], out.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream)
+    full = want + bias.double()
+    assert (out.double() - full).norm() / full.norm() <= tol, gq._lib.last_kernel()
+    if n % 64 == 0:  # the fused gate/up form adds in the same order: the same bits as the two steps
+        assert torch.equal(ops.linear_silu_mul(x, qw, qs, 4, 32), ops.silu_mul(ops.linear(x, qw, qs, 4, 32)))
