@@ -326,7 +326,8 @@ MI355GQ_API int mi355gq_moe_experts(const void* x, int64_t x_rows, const void* x
  * them: weights fp16 [T, top_k], ids int32 [T, top_k], token_indices / reverse_indices int32
  * [T * top_k], indptr [num_experts + 1] (exclusive form, indptr[0] = 0); plus slot_positions int32
  * [T * top_k], the inverse of reverse_indices (slot t * top_k + j is row slot_positions[...] of the
- * expert-sorted order), which lets mi355gq_moe_combine_sorted read the experts' output where it lies.
+ * expert-sorted order; -1 for a slot that repeats an expert of its token, which counts once and has no row), which lets
+ * mi355gq_moe_combine_sorted read the experts' output where it lies (a negative position adds nothing).
  * The [num_experts, T] cumsum table is not materialised.
  */
 MI355GQ_API int mi355gq_moe_route(const void* logits, int64_t T, int64_t num_experts, int64_t top_k,

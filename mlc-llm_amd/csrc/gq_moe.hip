@@ -229,8 +229,14 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const void* __restrict_
   const int lane = tid & 63, wave = tid >> 6, nwaves = nthreads >> 6;
   for (int t = tid; t < T; t += nthreads) {
     topk_softmax_token<DT>(logits, t, ne, k, w, ids);
-    if (ids_in_lds)
-      for (int j = 0; j < k; ++j) ids_lds[t * k + j] = ids[static_cast<int64_t>(t) * k + j];  // own writes
+    for (int j = 0; j < k; ++j) {  // own writes
+      const int64_t s = static_cast<int64_t>(t) * k + j;
+      const int id = ids[s];
+      if (ids_in_lds) ids_lds[s] = id;
+      bool repeated = false;
+      for (int jj = 0; jj < j; ++jj) repeated |= ids[s - j + jj] == id;
+      if (repeated) pos_of_slot[s] = -1;  // (counted once below: this slot has no row)
+    }
   }
   __syncthreads();  // ids written above are read back by other threads below
   const int32_t* id_src = ids_in_lds ? ids_lds : ids;
@@ -324,6 +330,7 @@ __global__ __launch_bounds__(1024) void moe_route_slots_kernel(const void* __res
         for (int jj = 0; jj < kMaxTopK - 1; ++jj)  // unconditional loads (its own id past j), all in flight together
           repeated |= (ids[s - j + (jj < j ? jj : j)] == id) & (jj < j);
         if (!repeated) myid[r] = id;
+        else pos_of_slot[s] = -1;
       }
       if (ne > 16) {
         // many experts: the lanes compare ids pairwise instead (64 lane broadcasts whatever the expert count);
@@ -520,7 +527,8 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const void* __restrict__ 
 }
 
 // out[t, h] = sum_j fp16(y[t, j, h] * w[t, j]), fp16 adds left to right
-// pos: where slot t * k + j sits among the rows of y (expert-sorted order), or null for y in slot order
+// pos: where slot t * k + j sits among the rows of y (expert-sorted order; negative: it has no row and adds nothing), or null
+// for y in slot order
 template <int DT>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const void* __restrict__ y, const void* __restrict__ w,
                                                           const int32_t* __restrict__ pos, int64_t T, int k,
@@ -533,9 +541,9 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const void* __restrict
     int64_t row = t * k + j;
     if (pos != nullptr) {
       row = pos[row];
-      row = row < 0 ? 0 : (row >= T * k ? T * k - 1 : row);
+      row = row >= T * k ? T * k - 1 : row;
     }
-    const float prod = Elem<DT>::rnd(Elem<DT>::load(y, row * H + h) * Elem<DT>::load(w, t * k + j));
+    const float prod = Elem<DT>::rnd((row < 0 ? 0.f : Elem<DT>::load(y, row * H + h)) * Elem<DT>::load(w, t * k + j));
     acc = (j == 0) ? prod : Elem<DT>::rnd(acc + prod);
   }
   Elem<DT>::store(out, i, acc);
@@ -555,15 +563,17 @@ __global__ __launch_bounds__(256) void moe_combine_vec_kernel(const void* __rest
   float acc[VEC];
   for (int j = 0; j < k; ++j) {
     int64_t row = t * k + j;
+    bool none = false;
     if (pos != nullptr) {
       row = pos[row];
-      row = row < 0 ? 0 : (row >= T * k ? T * k - 1 : row);
+      none = row < 0;
+      row = none ? 0 : (row >= T * k ? T * k - 1 : row);
     }
     const Pack yv = *reinterpret_cast<const Pack*>(static_cast<const uint16_t*>(y) + row * H + h);
     const float wj = Elem<DT>::load(w, t * k + j);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
-      const float ye = DT == MODEL_BF16 ? bf2f(yv.v[e]) : h2f(yv.v[e]);
+      const float ye = none ? 0.f : (DT == MODEL_BF16 ? bf2f(yv.v[e]) : h2f(yv.v[e]));
       const float prod = Elem<DT>::rnd(ye * wj);
       acc[e] = (j == 0) ? prod : Elem<DT>::rnd(acc[e] + prod);
     }

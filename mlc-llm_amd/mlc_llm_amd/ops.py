@@ -429,9 +429,11 @@ def moe_gemv(x: torch.Tensor, q_weight: torch.Tensor, q_scale: torch.Tensor,
 
 
 def moe_group_gemm(x: torch.Tensor, q_weight: torch.Tensor, q_scale: torch.Tensor,
-                   indptr: torch.Tensor, bits: int, group_size: int, silu_mul_halves: bool = False
+                   indptr: torch.Tensor, bits: int, group_size: int, silu_mul_halves: bool = False, *, rows_covered: bool = False
                    ) -> torch.Tensor:
-    """x, q_scale and the result share the model dtype (float16, float32 or bfloat16)."""
+    """x, q_scale and the result share the model dtype (float16, float32 or bfloat16).  Rows outside the experts' segments
+    come back as zeros; rows_covered: the caller reads no such row, and they are left as they are."""
+    new = torch.empty if rows_covered else torch.zeros
     _chk(x, _FLOATS, "x")
     _chk(q_weight, _STORAGE, "q_weight")
     _chk(q_scale, x.dtype, "q_scale")
@@ -448,15 +450,15 @@ def moe_group_gemm(x: torch.Tensor, q_weight: torch.Tensor, q_scale: torch.Tenso
         if silu_mul_halves:
             if n % 2:
                 raise ValueError(f"moe_group_gemm: {n} rows cannot be split into gate and up halves")
-            out = torch.zeros((rows, n // 2), dtype=x.dtype, device=x.device)
+            out = new((rows, n // 2), dtype=x.dtype, device=x.device)
             try:
                 _lib.call("mi355gq_moe_group_gemm_silu_mul_dt", *dt_args, out.data_ptr(), _stream())
                 return out
             except _lib.Mi355gqError as err:
                 if not _unsupported(err):
                     raise
-                return silu_mul(moe_group_gemm(x, q_weight, q_scale, indptr, bits, group_size))
-        out = torch.zeros((rows, n), dtype=x.dtype, device=x.device)
+                return silu_mul(moe_group_gemm(x, q_weight, q_scale, indptr, bits, group_size, rows_covered=rows_covered))
+        out = new((rows, n), dtype=x.dtype, device=x.device)
         _lib.call("mi355gq_moe_group_gemm_dt", *dt_args, out.data_ptr(), _stream())
         return out
     args = (x.data_ptr(), rows, q_weight.data_ptr(), q_scale.data_ptr(), indptr.data_ptr(),
@@ -464,22 +466,22 @@ def moe_group_gemm(x: torch.Tensor, q_weight: torch.Tensor, q_scale: torch.Tenso
     if silu_mul_halves:
         if n % 2:
             raise ValueError(f"moe_group_gemm: {n} rows cannot be split into gate and up halves")
-        out = torch.zeros((rows, n // 2), dtype=torch.float16, device=x.device)
+        out = new((rows, n // 2), dtype=torch.float16, device=x.device)
         try:
             _lib.call("mi355gq_moe_group_gemm_silu_mul", *args, out.data_ptr(), _stream())
             return out
         except _lib.Mi355gqError as err:
             if not _unsupported(err):
                 raise
-            return silu_mul(moe_group_gemm(x, q_weight, q_scale, indptr, bits, group_size))
-    out = torch.zeros((rows, n), dtype=torch.float16, device=x.device)
+            return silu_mul(moe_group_gemm(x, q_weight, q_scale, indptr, bits, group_size, rows_covered=rows_covered))
+    out = new((rows, n), dtype=torch.float16, device=x.device)
     _lib.call("mi355gq_moe_group_gemm", *args, out.data_ptr(), _stream())
     return out
 
 
 def moe_experts(x: torch.Tensor, x_row_index: Optional[torch.Tensor], q_weight: torch.Tensor,
                 q_scale: torch.Tensor, indptr: torch.Tensor, bits: int, group_size: int,
-                silu_mul_halves: bool = False) -> torch.Tensor:
+                silu_mul_halves: bool = False, *, rows_covered: bool = False) -> torch.Tensor:
     """moe_group_gemm on x[x_row_index] (the layer's gather folded into the matmul's row addressing);
     x_row_index None: x is already in expert order.  Float16 and bfloat16 models; anything without such a
     kernel (float32 models, odd shapes) runs take_rows and moe_group_gemm."""
@@ -498,7 +500,8 @@ def moe_experts(x: torch.Tensor, x_row_index: Optional[torch.Tensor], q_weight: 
         rows = x_row_index.numel()
     if silu_mul_halves and n % 2:
         raise ValueError(f"moe_experts: {n} rows cannot be split into gate and up halves")
-    out = torch.zeros((rows, n // 2 if silu_mul_halves else n), dtype=x.dtype, device=x.device)
+    new = torch.empty if rows_covered else torch.zeros
+    out = new((rows, n // 2 if silu_mul_halves else n), dtype=x.dtype, device=x.device)
     try:
         _lib.call("mi355gq_moe_experts_dt", x.data_ptr(), x_rows,
                   x_row_index.data_ptr() if x_row_index is not None else None, rows, q_weight.data_ptr(),
@@ -509,7 +512,7 @@ def moe_experts(x: torch.Tensor, x_row_index: Optional[torch.Tensor], q_weight: 
         if not _unsupported(err):
             raise
         gathered = take_rows(x, x_row_index) if x_row_index is not None else x
-        return moe_group_gemm(gathered, q_weight, q_scale, indptr, bits, group_size, silu_mul_halves)
+        return moe_group_gemm(gathered, q_weight, q_scale, indptr, bits, group_size, silu_mul_halves, rows_covered=rows_covered)
     return out
 
 
@@ -599,11 +602,13 @@ def get_indptr(cumsum: torch.Tensor, num_local_experts: int, batch_size: int, in
     return out
 
 
-def take_rows(x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
+def take_rows(x: torch.Tensor, indices: torch.Tensor, *, rows_covered: bool = False) -> torch.Tensor:
+    """x[indices]; an index outside x gives a row of zeros (rows_covered: a row that is left as it is and that the caller
+    does not read)."""
     _chk(x, _FLOATS, "x")
     _chk(indices, torch.int32, "indices")
     r, h = indices.numel(), x.shape[1]
-    out = torch.zeros((r, h), dtype=x.dtype, device=x.device)
+    out = (torch.empty if rows_covered else torch.zeros)((r, h), dtype=x.dtype, device=x.device)
     _lib.call("mi355gq_take_rows_dt", x.data_ptr(), indices.data_ptr(), r, h, x.shape[0],
               out.data_ptr(), _MODEL_DTYPES[x.dtype], _stream())
     return out

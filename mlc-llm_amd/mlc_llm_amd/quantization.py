@@ -352,10 +352,11 @@ class GroupQuantizeMixtralExperts(nn.Module):
             device=src.weight.device,
         )
 
-    def forward(self, x: torch.Tensor, indptr: torch.Tensor, silu_mul_halves: bool = False) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, indptr: torch.Tensor, silu_mul_halves: bool = False, *,
+                rows_covered: bool = False) -> torch.Tensor:
         """2-D `indptr` [1, k] holds the selected expert ids (single token); 1-D is a true indptr.
         silu_mul_halves: return silu(x1) * x3 of the two halves of the output (the e1_e3 stack of
-        mixtral_model.py:64-68) from the same kernel."""
+        mixtral_model.py:64-68) from the same kernel.  rows_covered: see ops.moe_group_gemm."""
         assert x.dim() == 2
         if self.config.model_dtype not in MOE_MODEL_DTYPES:
             raise NotImplementedError(f"{self.config.name}: the expert matmuls are built for {MOE_MODEL_DTYPES} models")
@@ -365,7 +366,7 @@ class GroupQuantizeMixtralExperts(nn.Module):
                                 self.group_size, silu_mul_halves)
         assert indptr.dim() == 1
         return ops.moe_group_gemm(x, self.q_weight, self.q_scale, indptr, self.config.bits,
-                                  self.group_size, silu_mul_halves)
+                                  self.group_size, silu_mul_halves, rows_covered=rows_covered)
 
 
 def _group(name: str, group_size: int, qdtype: str, layout: str, model_dtype: str = "float16",
