@@ -233,10 +233,19 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
                            (!a.paired || (a.N % 64) == 0);
     const int64_t scratch = may_split ? a.workspace_bytes : 0;
     const SplitPlan plan = plan_split_k(a.rows, a.N, a.K, a.bits, a.group_size, a.indptr != nullptr, a.bf16, scratch);
+    if (plan.n_head > 0 && (variant < 0 || a.bf16)) {
+      GemmParams head = p;
+      head.bm_hint = plan.head_bm;
+      head.bn_hint = plan.head_bn;
+      head.n_end = static_cast<int>(plan.n_head);
+      const hipError_t e = launch_gemm_pipe(head, a.bits, s);
+      if (e != hipSuccess) return e;
+      p.n_begin = head.n_end;
+    }
     p.bm_hint = plan.bm;
     p.bn_hint = plan.bn;
     // without (enough) scratch the same tiles run unsplit: slower, never wrong
-    if (plan.bm > 0 && plan.split > 1 && scratch >= static_cast<int64_t>(plan.split) * a.rows * a.N * 4) {
+    if (plan.bm > 0 && plan.split > 1 && scratch >= static_cast<int64_t>(plan.split) * a.rows * (a.N - plan.n_head) * 4) {
       p.partial = static_cast<float*>(a.workspace);
       p.kt_per_split = plan.kt_per_split;
     }
@@ -244,19 +253,20 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
   if (a.bf16 || (variant != 3 && variant != 4 && variant != 5)) {
     const hipError_t e = launch_gemm_pipe(p, a.bits, s);
     if (e == hipSuccess && p.partial != nullptr) {
-      const int64_t count = a.rows * a.N;
+      const int cols = p.N - p.n_begin;
+      const int64_t count = a.rows * cols;
       const int nk = (p.ng + 1) / 2;
       const int split = (nk + p.kt_per_split - 1) / p.kt_per_split;
       int64_t blocks = (count / 4 + 255) / 256;
       blocks = blocks < 1 ? 1 : (blocks > 2048 ? 2048 : blocks);
       if (p.paired) {
         hipLaunchKernelGGL(splitk_reduce_silu_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s,
-                           p.partial, split, a.rows, p.N, gemm_pipe_pair_block(p, a.bits),
+                           p.partial, split, a.rows, cols, p.N, gemm_pipe_pair_block(p, a.bits),
                            static_cast<uint16_t*>(p.y), p.bf16);
         return hipGetLastError();
       }
       hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s,
-                         p.partial, split, count, p.N, p.bias, p.residual, p.y, p.out_f32, p.bf16);
+                         p.partial, split, count, cols, p.N, p.bias, p.residual, p.y, p.out_f32, p.bf16);
       return hipGetLastError();
     }
     if (e != hipErrorNotSupported || a.bf16) return e;  // (bfloat16 models: the pipelined kernel or nothing)
@@ -276,7 +286,7 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
 int64_t gemm_workspace_bytes(int64_t rows, int64_t N, int64_t K, int bits, int group_size, int bf16) {
   if (options().gemm_variant >= 0) return 0;
   const SplitPlan plan = plan_split_k(rows, N, K, bits, group_size, false, bf16, kMaxSplitBytes);
-  return plan.bm > 0 && plan.split > 1 ? static_cast<int64_t>(plan.split) * rows * N * 4 : 0;
+  return plan.bm > 0 && plan.split > 1 ? static_cast<int64_t>(plan.split) * rows * (N - plan.n_head) * 4 : 0;
 }
 
 }  // namespace gq

@@ -31,7 +31,7 @@ struct GemmParams {
   int num_experts;
   int out_f32, indptr_i64;
   // split-K: workgroup z multiplies K tiles [z * kt_per_split, (z + 1) * kt_per_split) and, when
-  // `partial` is set, leaves its fp32 tile in partial[z][rows][N] for the reduction kernel
+  // `partial` is set, leaves its fp32 tile in partial[z][rows][N - n_begin] for the reduction kernel
   float* partial;
   int kt_per_split;
   int bm_hint;  // rows, columns per tile chosen by plan_split_k (0: regular tiles)
@@ -63,10 +63,12 @@ __device__ __forceinline__ int gate_up_row_blk(int c, int N) {
   return (c & PB) ? half + o : o;
 }
 
-__global__ void splitk_reduce_kernel(const float* partial, int split, int64_t count, int N,
+// partial[split][count / cols][cols] -> columns [N - cols, N) of y [rows, N]
+__global__ void splitk_reduce_kernel(const float* partial, int split, int64_t count, int cols, int N,
                                      const uint16_t* bias, const uint16_t* residual, void* y, int out_f32, int bf16);
-// fused gate/up form: partial[split][rows][N] in the block-interleaved column order -> y fp16 [rows, N / 2]
-__global__ void splitk_reduce_silu_kernel(const float* partial, int split, int64_t rows, int N, int pb,
+// fused gate/up form: partial[split][rows][cols] in the block-interleaved column order -> the last cols / 2 columns of
+// y [rows, N / 2]
+__global__ void splitk_reduce_silu_kernel(const float* partial, int split, int64_t rows, int cols, int N, int pb,
                                           uint16_t* y, int bf16);
 // gate rows per column block (32 | 16) of the tile launch_gemm_pipe picks for these parameters
 int gemm_pipe_pair_block(const GemmParams& p, int bits);
@@ -76,6 +78,9 @@ struct SplitPlan {
   int bm, bn;        // 0: no plan, use the regular tiles
   int split;         // workgroups along K (1: no reduction pass)
   int kt_per_split;  // K tiles (2 groups each) per workgroup
+  // columns [0, n_head) run first, unsplit, as whole rounds of workgroups on a tile of their own; bm, bn and split are for the rest
+  int64_t n_head = 0;
+  int head_bm = 0, head_bn = 0;
 };
 // scratch_bytes: what the partial sums of a split may take
 SplitPlan plan_split_k(int64_t rows, int64_t N, int64_t K, int bits, int group_size, bool grouped, int bf16, int64_t scratch_bytes);

@@ -21,7 +21,7 @@
 // instructions) was 4 to 10 % slower than the compiler's own order.
 //
 // Measured against the float32 matrix instruction's kernel it replaced (us; rows, then N x K): 16 x 4096 x 4096 317 -> 18,
-// 64 x 28672 x 4096 352 -> 97, 300 x 4096 x 14336 1197 -> 167, 300 x 28672 x 4096 1189 -> 370 (200 TFLOP/s), 1024 x 28672 x 4096
+// 64 x 28672 x 4096 352 -> 97, 300 x 4096 x 14336 1197 -> 167, 300 x 28672 x 4096 1189 -> 272 (259 TFLOP/s), 1024 x 28672 x 4096
 // 867 (277 TFLOP/s; the float32 matrix instruction's peak is 157).  Relative error against float64 products 1.0e-7 .. 2.1e-7,
 // before 8e-7 .. 1.9e-6.
 #include "gq_gemm_common.hpp"
@@ -40,11 +40,12 @@ struct F32Params {
   const float* bias;      // [N] or null (plain linear only)
   const float* residual;  // [rows, N] or null, may be y (plain linear only)
   float* y;
-  float* partial;         // split K: [split][rows][N] sums, else null
+  float* partial;         // split K: [split][rows][N - n_begin] sums, else null
   const void* indptr;     // [num_experts + 1] or null
   int rows, N, K, ng, nw;
   int num_experts, indptr_i64;
   int kt_per_split;
+  int n_begin, n_end;     // columns of this launch
 };
 
 constexpr int kRow = 40;  // halves per LDS row: 32 + 8 of padding
@@ -106,7 +107,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_f32_kernel(co
     }
     if (!found) return;  // (uniform: before any barrier)
   }
-  const int m0 = seg_lo + mt * BM, n0 = blockIdx.x * BN;
+  const int m0 = seg_lo + mt * BM, n0 = p.n_begin + blockIdx.x * BN;
   const uint32_t* const qw = p.qw + static_cast<int64_t>(expert) * p.N * p.nw;
   const float* const qs = p.qs + static_cast<int64_t>(expert) * p.N * p.ng;
 
@@ -249,10 +250,10 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_f32_kernel(co
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = m0 + wm0 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row < seg_hi && col < p.N) {
+        if (row < seg_hi && col < p.n_end) {
           const int64_t oi = static_cast<int64_t>(row) * p.N + col;
           if (p.partial != nullptr) {
-            p.partial[static_cast<int64_t>(blockIdx.z) * p.rows * p.N + oi] = acc[i][j][r];
+            p.partial[(static_cast<int64_t>(blockIdx.z) * p.rows + row) * (p.N - p.n_begin) + (col - p.n_begin)] = acc[i][j][r];
           } else {
             float v = acc[i][j][r] + bias;
             if (p.residual != nullptr) v += p.residual[oi];
@@ -274,13 +275,14 @@ hipError_t launch_tile(const F32Params& p, int split, hipStream_t s) {
   const int m_tiles = (p.rows + BM - 1) / BM + (p.indptr != nullptr ? p.num_experts : 0);
   if (m_tiles > 65535) return hipErrorNotSupported;
   note_kernel("gq::gemm_f32_kernel<%d,%d,%d,%d> split=%d", BM, BN, WM, WN, split);
-  hipLaunchKernelGGL(kern, dim3((p.N + BN - 1) / BN, m_tiles, split), dim3(64 * (BM / WM) * (BN / WN)), lds, s, p);
+  hipLaunchKernelGGL(kern, dim3((p.n_end - p.n_begin + BN - 1) / BN, m_tiles, split), dim3(64 * (BM / WM) * (BN / WN)), lds, s, p);
   return hipGetLastError();
 }
 
 // rows of the tile a problem runs on, and how its K is cut so that most CUs have a workgroup
 struct F32Plan {
   int bm, split, kt_per_split;
+  int64_t n_head = 0;  // columns that run first, unsplit, as whole rounds of workgroups
 };
 F32Plan plan_f32(int64_t rows, int64_t N, int64_t K, int64_t num_experts, bool grouped) {
   const int64_t per = grouped ? (rows + num_experts - 1) / num_experts : rows;
@@ -293,6 +295,21 @@ F32Plan plan_f32(int64_t rows, int64_t N, int64_t K, int64_t num_experts, bool g
   const int64_t want = plan.bm == 32 ? 512 : 256;
   int64_t split = want / tiles;
   if (split > ng / 8) split = ng / 8;  // at least eight K tiles per workgroup
+  if (plan.bm == 128 && tiles > 256) {
+    // A last round of workgroups costs a whole round however few they are (28672 x 4096: 224 tiles 178 us, 336 tiles 334).  The
+    // columns of the whole rounds then run on their own, and the K of the rest is cut so that it fills the chip once: worth it
+    // while that shorter round, the sums it writes and reads back and the two more launches stay below 0.85 of a round
+    // (a round: 1.3 us per K tile; 28672 x 4096 at 300 / 640 / 777 rows: one launch 334 / 535 / 708 us, so 272 / 453 / 625).
+    const int64_t mt = (rows + 127) / 128, nt = (N + 255) / 256, head = tiles / 256 * 256 / mt, rest = mt * (nt - head);
+    const int64_t cut = rest > 0 ? (256 / rest < ng / 8 ? 256 / rest : ng / 8) : 0;
+    if (head > 0 && cut > 1) {
+      const double round_us = 1.3 * ng, sums_us = 10.0 + 2e-6 * static_cast<double>(cut * rows * (N - head * 256));
+      if (round_us / static_cast<double>(cut) + sums_us < 0.85 * round_us) {
+        plan.n_head = head * 256;
+        split = cut;
+      }
+    }
+  }
   if (split <= 1) return plan;
   plan.kt_per_split = (ng + static_cast<int>(split) - 1) / static_cast<int>(split);
   plan.split = (ng + plan.kt_per_split - 1) / plan.kt_per_split;
@@ -301,31 +318,33 @@ F32Plan plan_f32(int64_t rows, int64_t N, int64_t K, int64_t num_experts, bool g
 
 }  // namespace
 
-// y = sum over slices of part[slice][count] + bias + residual, all float32 (y may be the residual)
-__global__ __launch_bounds__(256) void splitk_reduce_f32_kernel(const float* __restrict__ part, int slices, int64_t count, int N,
+// columns [N - cols, N) of y [rows, N] = sum over slices of part[slice][rows][cols] + bias + residual, all float32 (y may be the
+// residual)
+__global__ __launch_bounds__(256) void splitk_reduce_f32_kernel(const float* __restrict__ part, int slices, int64_t count, int cols, int N,
                                                                 const float* __restrict__ bias, const float* residual, float* y) {
   const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < count; i += stride) {
     float v = part[i];
     for (int sl = 1; sl < slices; ++sl) v += part[sl * count + i];
-    if (bias != nullptr) v += bias[i % N];
-    if (residual != nullptr) v += residual[i];
-    y[i] = v;
+    const int64_t o = cols == N ? i : (i / cols) * N + (N - cols) + i % cols;
+    if (bias != nullptr) v += bias[o % N];
+    if (residual != nullptr) v += residual[o];
+    y[o] = v;
   }
 }
 
-hipError_t launch_splitk_reduce_f32(const float* part, int slices, int64_t rows, int64_t N, const float* bias,
+hipError_t launch_splitk_reduce_f32(const float* part, int slices, int64_t rows, int64_t cols, int64_t N, const float* bias,
                                     const float* residual, float* y, hipStream_t s) {
-  const int64_t count = rows * N, blocks = (count + 255) / 256;
+  const int64_t count = rows * cols, blocks = (count + 255) / 256;
   hipLaunchKernelGGL(splitk_reduce_f32_kernel, dim3(static_cast<unsigned>(blocks > 8192 ? 8192 : blocks)), dim3(256), 0, s, part,
-                     slices, count, static_cast<int>(N), bias, residual, y);
+                     slices, count, static_cast<int>(cols), static_cast<int>(N), bias, residual, y);
   return hipGetLastError();
 }
 
 int64_t gemm_f32_workspace_bytes(int64_t rows, int64_t N, int64_t K) {
   if (rows < 1 || N < 1 || K < 1 || (K & 7) != 0) return 0;
   const F32Plan plan = plan_f32(rows, N, K, 1, false);
-  return plan.split > 1 ? static_cast<int64_t>(plan.split) * rows * N * 4 : 0;
+  return plan.split > 1 ? static_cast<int64_t>(plan.split) * rows * (N - plan.n_head) * 4 : 0;
 }
 
 hipError_t launch_gemm_f32(const GemmArgs& a, hipStream_t s) {
@@ -345,19 +364,30 @@ hipError_t launch_gemm_f32(const GemmArgs& a, hipStream_t s) {
   F32Plan plan = plan_f32(a.rows, a.N, a.K, a.num_experts, a.indptr != nullptr);
   if (plan.split > 1) {
     if (a.workspace != nullptr && (reinterpret_cast<uintptr_t>(a.workspace) & 3) == 0 &&
-        a.workspace_bytes >= static_cast<int64_t>(plan.split) * a.rows * a.N * 4) {
+        a.workspace_bytes >= static_cast<int64_t>(plan.split) * a.rows * (a.N - plan.n_head) * 4) {
       p.partial = static_cast<float*>(a.workspace);
     } else {
       plan.split = 1;
       plan.kt_per_split = p.ng;
+      plan.n_head = 0;
     }
+  }
+  p.n_end = p.N;
+  if (plan.n_head > 0) {
+    F32Params head = p;
+    head.partial = nullptr;
+    head.kt_per_split = p.ng;
+    head.n_end = static_cast<int>(plan.n_head);
+    const hipError_t e = launch_tile<128, 256, 64, 64>(head, 1, s);
+    if (e != hipSuccess) return e;
+    p.n_begin = head.n_end;
   }
   p.kt_per_split = plan.kt_per_split;
   const hipError_t e = plan.bm == 32   ? launch_tile<32, 128, 32, 32>(p, plan.split, s)
                        : plan.bm == 64 ? launch_tile<64, 128, 32, 64>(p, plan.split, s)
                                        : launch_tile<128, 256, 64, 64>(p, plan.split, s);
   if (e != hipSuccess || p.partial == nullptr) return e;
-  return launch_splitk_reduce_f32(p.partial, plan.split, a.rows, a.N, p.bias, p.residual, p.y, s);
+  return launch_splitk_reduce_f32(p.partial, plan.split, a.rows, a.N - plan.n_head, a.N, p.bias, p.residual, p.y, s);
 }
 
 }  // namespace gq

@@ -474,8 +474,9 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_pipe_kernel(c
     }
   };
   if (p.partial != nullptr) {
-    float* part = p.partial + static_cast<int64_t>(blockIdx.z) * p.rows * p.N;
-    for_each([&](int row, int col, float v) { part[static_cast<int64_t>(row) * p.N + col] = v; });
+    const int cols = p.N - p.n_begin;
+    float* part = p.partial + static_cast<int64_t>(blockIdx.z) * p.rows * cols - p.n_begin;
+    for_each([&](int row, int col, float v) { part[static_cast<int64_t>(row) * cols + col] = v; });
   } else if (p.bias == nullptr && p.residual == nullptr) {
     if (p.out_f32)
       for_each([&](int row, int col, float v) { static_cast<float*>(p.y)[static_cast<int64_t>(row) * p.N + col] = v; });
@@ -537,68 +538,72 @@ static hipError_t launch_pipe_cfg(const GemmParams& p, hipStream_t s) {
 // y = sum over splits of partial[s] + bias + residual, in the output type (y may be the residual
 // buffer itself: every element is read before the same thread writes it)
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ partial, int split,
-                                                            int64_t count /* rows * N */, int N,
+                                                            int64_t count /* rows * cols */, int cols, int N,
                                                             const uint16_t* __restrict__ bias,
                                                             const uint16_t* residual, void* y, int out_f32, int bf16) {
   // bias, residual and a 16-bit y carry the model dtype: float16, or bfloat16 when bf16 is set
   auto in = [bf16](uint16_t bits) { return bf16 ? bf2f(bits) : h2f(bits); };
   auto out = [bf16](float v) { return bf16 ? f2bf(v) : f2h(v); };
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  if ((N & 3) == 0) {  // rows are 16-byte aligned: four columns per thread
+  // element i of the sums -> element of y
+  auto at = [&](int64_t i) -> int64_t { return cols == N ? i : (i / cols) * N + (N - cols) + i % cols; };
+  if (((N | cols) & 3) == 0) {  // rows are 16-byte aligned: four columns per thread
     for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; 4 * i < count; i += stride) {
       float4 a = *reinterpret_cast<const float4*>(partial + 4 * i);
       for (int sidx = 1; sidx < split; ++sidx) {
         const float4 b = *reinterpret_cast<const float4*>(partial + sidx * count + 4 * i);
         a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
       }
+      const int64_t o4 = at(4 * i);
       if (bias != nullptr) {
-        const int col = static_cast<int>((4 * i) % N);
+        const int col = static_cast<int>(o4 % N);
         const uint2 bb = *reinterpret_cast<const uint2*>(bias + col);
         a.x += in(static_cast<uint16_t>(bb.x & 0xffffu)); a.y += in(static_cast<uint16_t>(bb.x >> 16));
         a.z += in(static_cast<uint16_t>(bb.y & 0xffffu)); a.w += in(static_cast<uint16_t>(bb.y >> 16));
       }
       if (residual != nullptr) {
-        const uint2 rr = *reinterpret_cast<const uint2*>(residual + 4 * i);
+        const uint2 rr = *reinterpret_cast<const uint2*>(residual + o4);
         a.x += in(static_cast<uint16_t>(rr.x & 0xffffu)); a.y += in(static_cast<uint16_t>(rr.x >> 16));
         a.z += in(static_cast<uint16_t>(rr.y & 0xffffu)); a.w += in(static_cast<uint16_t>(rr.y >> 16));
       }
       if (out_f32) {
-        *reinterpret_cast<float4*>(static_cast<float*>(y) + 4 * i) = a;
+        *reinterpret_cast<float4*>(static_cast<float*>(y) + o4) = a;
       } else {
         uint2 o;
         o.x = static_cast<uint32_t>(out(a.x)) | (static_cast<uint32_t>(out(a.y)) << 16);
         o.y = static_cast<uint32_t>(out(a.z)) | (static_cast<uint32_t>(out(a.w)) << 16);
-        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + 4 * i) = o;
+        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + o4) = o;
       }
     }
   } else {
     for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < count; i += stride) {
       float a = partial[i];
       for (int sidx = 1; sidx < split; ++sidx) a += partial[sidx * count + i];
-      if (bias != nullptr) a += in(bias[i % N]);
-      if (residual != nullptr) a += in(residual[i]);
-      if (out_f32) static_cast<float*>(y)[i] = a;
-      else static_cast<uint16_t*>(y)[i] = out(a);
+      const int64_t o = at(i);
+      if (bias != nullptr) a += in(bias[o % N]);
+      if (residual != nullptr) a += in(residual[o]);
+      if (out_f32) static_cast<float*>(y)[o] = a;
+      else static_cast<uint16_t*>(y)[o] = out(a);
     }
   }
 }
 
 __global__ __launch_bounds__(256) void splitk_reduce_silu_kernel(const float* __restrict__ partial, int split,
-                                                                 int64_t rows, int N, int pb,
+                                                                 int64_t rows, int cols, int N, int pb,
                                                                  uint16_t* __restrict__ y, int bf16) {
-  const int half = N >> 1;
-  const int64_t count = rows * N, outs = rows * half;
+  const int half = cols >> 1;
+  const int64_t count = rows * cols, outs = rows * half;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < outs; i += stride) {
     const int64_t row = i / half;
     const int oc = static_cast<int>(i - row * half);
-    const int64_t at = row * N + (oc / pb) * 2 * pb + oc % pb;  // pb gate columns, then their pb up columns
+    const int64_t at = row * cols + (oc / pb) * 2 * pb + oc % pb;  // pb gate columns, then their pb up columns
     float g = partial[at], u = partial[at + pb];
     for (int sidx = 1; sidx < split; ++sidx) {
       g += partial[sidx * count + at];
       u += partial[sidx * count + at + pb];
     }
-    y[i] = bf16 ? silu_mul_bf(g, u) : silu_mul_h(g, u);
+    y[row * (N >> 1) + ((N - cols) >> 1) + oc] = bf16 ? silu_mul_bf(g, u) : silu_mul_h(g, u);
   }
 }
 
@@ -616,39 +621,48 @@ struct TileCost {
   float base, whole, odd, filled, live, round, reduce, traffic, store;
 };
 // Least squares (non-negative) over 22 shapes (N 2048..37888, K 2048..28672, the projections of 1.5B to 70B models) x 19 row counts from
-// 72 to 4096 x splits of 1 to 16: 7500 timings, 5-6 % rms.  Choosing by it instead of by the rules it replaced (128 x 128 tiles split up to
-// 256 workgroups to 1024 rows, three unsplit tiles beyond) makes those launches 7.3 % (bfloat16 10.8 %) faster on average, where
-// the best of all measured choices would make 8.1 % (11.3 %).  For instance (us): 4096 x 14336 at 160 / 300 / 640 / 777 rows 43.6 / 77.8 /
+// 72 to 4096 x splits of 1 to 16: 7700 timings, 5-6 % rms.  Choosing by it instead of by the rules it replaced (128 x 128 tiles split up to
+// 256 workgroups to 1024 rows, three unsplit tiles beyond) makes those launches 7.5 % (bfloat16 11 %) faster on average, where
+// the best of all measured choices would make 8.3 % (11.3 %).  For instance (us): 4096 x 14336 at 160 / 300 / 640 / 777 rows 43.6 / 77.8 /
 // 113.5 / 129 -> 36.9 / 62 / 89.8 / 117 (bfloat16 46.3 / 85.2 / 122.5 / 143 -> 37.0 / 61.2 / 91.9 / 113), 4096 x 4096 at 300 rows 37.1 -> 27.2, 28672 x
 // 4096 at 160 / 300 / 777 rows 66.3 / 112.5 / 219.8 -> 54.3 / 92.7 / 207.4; from 1536 rows on the choice is mostly the old one.
 constexpr TileCost kTilesF16[] = {
-    {128, 128, 0, 6.83f, 0.593f, 0.37f, 0.219f, 0, 0, 2.51f, 0.862f, 0.333f},
-    {128, 256, 0, 5.43f, 0.549f, 0, 0.419f, 0, 2.18f, 2.62f, 0.72f, 0.15f},
-    {256, 256, 0, 0, 0.922f, 0, 0.681f, 0, 11.9f, 2.65f, 0.371f, 0.0433f},
-    {256, 256, 1, 1.01f, 0.933f, 0, 0, 0.712f, 10.6f, 3.66f, 0.405f, 0},
-    {256, 128, 1, 7.72f, 0.57f, 0, 0, 0.437f, 1.25f, 2.89f, 0.57f, 0},
-    {64, 128, 0, 6.12f, 0.458f, 0.31f, 0.104f, 0, 0.000585f, 1.35f, 1.63f, 0.153f},
+    {128, 128, 0, 6.83f, 0.593f, 0.37f, 0.219f, 0, 0, 2.51f, 0.858f, 0.33f},
+    {128, 256, 0, 5.43f, 0.549f, 0, 0.419f, 0, 2.18f, 2.62f, 0.719f, 0.149f},
+    {256, 256, 0, 0, 0.922f, 0, 0.681f, 0, 11.9f, 2.66f, 0.37f, 0.0425f},
+    {256, 256, 1, 0.992f, 0.934f, 0, 0, 0.712f, 10.5f, 3.68f, 0.405f, 0},
+    {256, 128, 1, 7.7f, 0.57f, 0, 0, 0.437f, 1.24f, 2.91f, 0.569f, 0},
+    {64, 128, 0, 5.69f, 0.446f, 0.298f, 0.119f, 0, 0.175f, 2.0f, 1.22f, 0.604f},
 };
 constexpr TileCost kTilesBf16[] = {  // (more vector instructions per weight: the tiles that dequantise it less often are ahead)
-    {128, 128, 0, 8.01f, 0.62f, 0.4f, 0.224f, 0, 0, 2.5f, 0.731f, 0.371f},
-    {128, 256, 0, 6.06f, 0.625f, 0, 0.386f, 0, 2.48f, 2.62f, 0.578f, 0.225f},
-    {256, 256, 0, 0.54f, 1.01f, 0, 0.574f, 0, 10.2f, 3.73f, 0.396f, 0.151f},
-    {256, 256, 1, 6.62f, 0.969f, 0, 0, 0.692f, 4.42f, 4.4f, 0.384f, 0.0966f},
-    {256, 128, 1, 7.17f, 0.552f, 0, 0, 0.411f, 2.2f, 2.86f, 0.517f, 0},
-    {64, 128, 0, 7.4f, 0.509f, 0.348f, 0.115f, 0, 0, 1.12f, 1.3f, 0.235f},
+    {128, 128, 0, 8.01f, 0.621f, 0.4f, 0.224f, 0, 0, 2.51f, 0.73f, 0.371f},
+    {128, 256, 0, 6.05f, 0.625f, 0, 0.385f, 0, 2.47f, 2.64f, 0.578f, 0.23f},
+    {256, 256, 0, 0.544f, 1.01f, 0, 0.574f, 0, 10.2f, 3.75f, 0.395f, 0.152f},
+    {256, 256, 1, 6.61f, 0.969f, 0, 0, 0.692f, 4.4f, 4.43f, 0.384f, 0.0978f},
+    {256, 128, 1, 7.17f, 0.552f, 0, 0, 0.412f, 2.2f, 2.87f, 0.518f, 0},
+    {64, 128, 0, 6.81f, 0.507f, 0.338f, 0.128f, 0, 0.183f, 1.99f, 0.916f, 0.339f},
 };
 
-static SplitPlan plan_by_cost(int64_t rows, int64_t N, int nk, int bf16, int64_t scratch_bytes) {
+static float tile_us(const TileCost& c, int64_t rows, int64_t N, int nk, int kt, int split) {
+  const int64_t mt = (rows + c.bm - 1) / c.bm, wgs = mt * ((N + c.bn - 1) / c.bn) * split, rounds = (wgs + 255) / 256;
+  const float live = static_cast<float>(rows) / static_cast<float>(mt * c.bm), mn = 1e-6f * static_cast<float>(rows) * static_cast<float>(N);
+  const bool pairs = c.bm * c.bn <= 128 * 128;  // (four waves: two workgroups on a CU)
+  const float ktf = static_cast<float>(split > 1 ? kt : (nk + 3) / 4 * 4), per_cu = static_cast<float>(wgs) / 256.f;
+  const float us = c.base + ktf * (c.whole * static_cast<float>(pairs ? rounds / 2 : rounds) + (pairs ? c.odd * static_cast<float>(rounds % 2) : 0.f) +
+                                   per_cu * (c.filled + c.live * live)) +
+                   c.round * static_cast<float>(rounds) + c.store * mn;
+  // (a split has to be 2 % ahead on paper)
+  return split > 1 ? (us + c.reduce + c.traffic * static_cast<float>(split) * mn) * 1.02f : us;
+}
+static bool tile_applies(const TileCost& c, int64_t rows) { return c.bm < 256 || (c.skip != 0) == (c.bn == 128 || rows % 256 != 0); }
+
+// one launch for all columns
+static SplitPlan plan_one(const TileCost* costs, int64_t rows, int64_t N, int nk, int64_t scratch_bytes, float* best_us) {
   SplitPlan best{0, 0, 1, 1 << 28};
-  float best_us = 0.f;
-  if (scratch_bytes > kMaxSplitBytes) scratch_bytes = kMaxSplitBytes;
-  const float mn = 1e-6f * static_cast<float>(rows) * static_cast<float>(N);
   for (int t = 0; t < 6; ++t) {
-    const TileCost& c = bf16 ? kTilesBf16[t] : kTilesF16[t];
-    if (c.bm == 256 && (c.skip != 0) != (c.bn == 128 || rows % 256 != 0)) continue;
-    const int64_t mt = (rows + c.bm - 1) / c.bm, tiles = mt * ((N + c.bn - 1) / c.bn);
-    const float live = static_cast<float>(rows) / static_cast<float>(mt * c.bm);
-    const bool pairs = c.bm * c.bn <= 128 * 128;  // (four waves: two workgroups on a CU)
+    const TileCost& c = costs[t];
+    if (!tile_applies(c, rows)) continue;
+    const int64_t tiles = ((rows + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
     int last = 0;
     for (int want = 1; want <= 16; ++want) {
       const int kt = ((nk + want - 1) / want + 3) / 4 * 4;  // (the K loop advances four tiles at a time)
@@ -657,17 +671,42 @@ static SplitPlan plan_by_cost(int64_t rows, int64_t N, int nk, int bf16, int64_t
       if (split > 1 && (want > nk / 4 || tiles * split > 640 || split * rows * N * 4 > scratch_bytes)) break;
       if (split == last) continue;
       last = split;
-      const int64_t wgs = tiles * split, rounds = (wgs + 255) / 256;
-      const float ktf = static_cast<float>(split > 1 ? kt : (nk + 3) / 4 * 4), per_cu = static_cast<float>(wgs) / 256.f;
-      float us = c.base + ktf * (c.whole * static_cast<float>(pairs ? rounds / 2 : rounds) + (pairs ? c.odd * static_cast<float>(rounds % 2) : 0.f) +
-                                 per_cu * (c.filled + c.live * live)) +
-                 c.round * static_cast<float>(rounds) + c.store * mn;
-      // (a split has to be 2 % ahead on paper)
-      if (split > 1) us = (us + c.reduce + c.traffic * static_cast<float>(split) * mn) * 1.02f;
-      if (best.bm == 0 || us < best_us) {
-        best_us = us;
+      const float us = tile_us(c, rows, N, nk, kt, split);
+      if (best.bm == 0 || us < *best_us) {
+        *best_us = us;
         best = SplitPlan{c.bm, c.bn, split, split > 1 ? kt : 1 << 28};
       }
+    }
+  }
+  return best;
+}
+
+// ... or two: a last round of workgroups that is far from full costs about what a full one does, so the columns of the whole rounds run
+// first on one of the large tiles and the rest on whatever suits it (a smaller tile, K split).  Taken where the model puts it 7 % ahead
+// (it is some 5 % too optimistic about two launches).  Measured (us, one launch -> two): 6144 x 4096 at 2700 rows 181 -> 147, 22016 x 4096 at
+// 1536 326 -> 268, 10240 x 8192 at 2048 377 -> 329, 15360 x 5120 at 1200 230 -> 205, 37888 x 3584 at 450 164 -> 145; 28672 x 4096 at 2048 (3.5
+// rounds) within the noise either way, and left alone by the 7 %.
+static SplitPlan plan_by_cost(int64_t rows, int64_t N, int nk, int bf16, int64_t scratch_bytes) {
+  if (scratch_bytes > kMaxSplitBytes) scratch_bytes = kMaxSplitBytes;
+  const TileCost* const costs = bf16 ? kTilesBf16 : kTilesF16;
+  float one_us = 0.f;
+  SplitPlan best = plan_one(costs, rows, N, nk, scratch_bytes, &one_us);
+  float best_us = one_us / 1.07f;
+  for (int t = 1; t <= 4; ++t) {  // (the tiles of one workgroup per CU)
+    const TileCost& c = costs[t];
+    const int64_t mt = (rows + c.bm - 1) / c.bm, nt = (N + c.bn - 1) / c.bn, head = mt * nt / 256 * 256 / mt;  // column tiles of the whole rounds
+    if (!tile_applies(c, rows) || head < 1 || head >= nt) continue;
+    const int64_t n_head = head * c.bn;
+    const float head_us = tile_us(c, rows, n_head, nk, 0, 1) - 3.f;  // (its launch overlaps the other's)
+    if (head_us >= best_us) continue;
+    float rest_us = 0.f;
+    SplitPlan rest = plan_one(costs, rows, N - n_head, nk, scratch_bytes, &rest_us);
+    if (head_us + rest_us < best_us) {
+      best_us = head_us + rest_us;
+      best = rest;
+      best.n_head = n_head;
+      best.head_bm = c.bm;
+      best.head_bn = c.bn;
     }
   }
   return best;

@@ -134,7 +134,7 @@ int64_t midrow_workspace_bytes(int64_t rows, int64_t N, int64_t K);
 // matrix cores; hipErrorNotSupported otherwise.  Its split of K wants gemm_f32_workspace_bytes of scratch.
 hipError_t launch_gemm_f32(const GemmArgs& a, hipStream_t s);
 int64_t gemm_f32_workspace_bytes(int64_t rows, int64_t N, int64_t K);
-hipError_t launch_splitk_reduce_f32(const float* part, int slices, int64_t rows, int64_t N, const float* bias,
+hipError_t launch_splitk_reduce_f32(const float* part, int slices, int64_t rows, int64_t cols, int64_t N, const float* bias,
                                     const float* residual, float* y, hipStream_t s);
 
 // KN-layout tensors (q_weight [nw, N], q_scale [ng, N]): both tensors transposed in one call (src_rows_w / src_rows_s rows

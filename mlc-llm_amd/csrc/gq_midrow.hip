@@ -628,7 +628,7 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   if (e != hipSuccess || p.slices == 1) return e;
   const int64_t count = static_cast<int64_t>(p.rows) * p.N;
   if (a.f32)
-    return launch_splitk_reduce_f32(static_cast<const float*>(a.workspace), p.slices, p.rows, p.N, reinterpret_cast<const float*>(a.bias),
+    return launch_splitk_reduce_f32(static_cast<const float*>(a.workspace), p.slices, p.rows, p.N, p.N, reinterpret_cast<const float*>(a.bias),
                                     reinterpret_cast<const float*>(a.residual), static_cast<float*>(a.y), s);
   if (fold_silu) {
     const int64_t outs = count / 2;
@@ -638,7 +638,7 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   } else {
     const int64_t blocks = ((p.N & 3) == 0 ? (count / 4 + 255) / 256 : (count + 255) / 256);
     hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>(blocks > 4096 ? 4096 : blocks)), dim3(256), 0, s,
-                       static_cast<const float*>(a.workspace), p.slices, count, p.N, a.bias, a.residual, a.y, a.out_f32, a.bf16);
+                       static_cast<const float*>(a.workspace), p.slices, count, p.N, p.N, a.bias, a.residual, a.y, a.out_f32, a.bf16);
   }
   return hipGetLastError();
 }

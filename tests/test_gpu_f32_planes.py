@@ -46,6 +46,7 @@ def _close(y, ref, k, what):
     (6, 16400, 4096, "midrow"), (10, 16400, 4096, "midrow"),
     (5, 100, 1000, "gemm"), (6, 129, 8, "gemm"), (31, 130, 1544, "gemm"), (32, 128, 4096, "gemm"), (33, 300, 360, "gemm"),
     (64, 128, 288, "gemm"), (65, 256, 4096, "gemm"), (128, 257, 64, "gemm"), (129, 16, 5632, "gemm"), (300, 520, 1544, "gemm"),
+    (300, 22300, 1024, "split=4"),  # whole rounds of columns first, the K of the rest cut
 ])
 def test_linear_f32_tiles(m, n, k, kernel):
     x, qw, qs, rng = _case(m, n, k, m * 7919 + n + k)
