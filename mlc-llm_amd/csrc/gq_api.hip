@@ -1055,24 +1055,26 @@ static hipError_t moe_row_gemv(const gq::GemmArgs& g, hipStream_t s) {
 // Expert segments on the kernel that scales the matrix instruction's result (gq_midrow.hip): rows per pass (16 or 32), or
 // 0 where the quad-row kernel (fewer rows) or the GEMM's tiles (more) stay ahead.  A segment longer than a pass takes
 // another pass over its expert's weights while the other experts' workgroups are done, so the bounds keep the longest
-// segment inside one pass: with 8 experts 4 to 8 rows per expert on average for 16-row passes, with 64 experts (whose
-// longest segment is further above the average: 12 at an average of 6, 17 at 9) 2 to 6; beyond that, up to 24 resp. 16 on
-// average, the two-tile instance where K is one phase.  Measured, 8 experts x top-2 (Mixtral, e1_e3 / e2 in us): 24 tokens
-// 156 / 102 -> 115 / 76, 32 tokens 170 / 106 -> 117 / 78, 16 tokens 118 / 75 against the quad-row kernel's 122 / 74, 40 tokens
-// with 16-row passes 203 / 131 against the GEMM's 166 / 104; two tiles at 40 / 64 / 96 tokens 166 / 167 / 195 -> 140 / 143 / 153
-// for e1_e3 (e2, K = 14336 in phases, 113-131 against 96-112: stays with the GEMM).  64 experts x top-6, 2816 x 2048 / 2048 x
-// 1536 / 5120 x 3584 at 144..384 rows: 55-64 / 46-49 / 142-197 -> 51-53 / 34-35 / 142-145; at 576 rows (two tiles) 83 / 49 / 211
-// -> 69 / 48 / 191.
+// segment inside one pass: 16-row passes up to 8 rows per expert on average, from 4 on with few experts (Mixtral, e1_e3 / e2
+// in us: 24 tokens 156 / 102 -> 115 / 76, 32 tokens 170 / 106 -> 117 / 78, 16 tokens 118 / 75 against the quad-row kernel's 122 / 74),
+// from 2 on with 16 and more (16 experts of 4096 x 2048 at 4 rows 19.5 against 24.0; 64 of 2816 x 2048, 128 of 1536 x 2048 and of 2048 x 768 at
+// 8 rows 48 / 49 / 32 against 59 / 58 / 46 for 32-row passes and 61 / 64 / 38 for the GEMM's 32-row tiles, at 10 rows 84 / 88 / 55; a K below 768, not measured
+// there, keeps 6).  Beyond
+// that, up to 24 resp. 16 on average, 32-row passes where K is one phase whose shares of 256 keep most of the waves busy: K = 2048
+// and 3584 (8 of 8, 14 of 16 waves) 58 / 178 against 62 / 219 for the GEMM's tiles, K = 2560 and 768 (10 of 16, 3 of 4) 125 / 47
+// against 102 / 38.  (e2 of Mixtral, K = 14336 in phases, 113-131 against 96-112: the GEMM.)
 static int midrow_rows_per_pass(int64_t rows, int64_t num_experts, int64_t K, int bits) {
   const int gv = gq::options().gemv_variant;
   if (gv == 10) return 16;  // (forced)
   if (gv == 11) return 32;
   if (gv >= 0 || bits != 4 || gq::options().gemm_variant >= 0) return 0;
-  const bool many = num_experts > 16;
-  const int64_t lo = (many ? 2 : 4) * num_experts, mid = (many ? 6 : 8) * num_experts,
-                hi = (many ? 16 : 24) * num_experts;
-  if (rows > lo && rows <= mid) return 16;
-  if (rows > mid && rows <= hi && K <= 4096) return 32;
+  const bool many = num_experts >= 16;
+  const int64_t mid = (many && K < 768 ? 6 : 8) * num_experts;
+  if (rows > (many ? 2 : 4) * num_experts && rows <= mid) return 16;
+  int64_t waves = 1;
+  while (waves * 256 < K) waves *= 2;
+  const bool busy = 4 * K > 3 * 256 * waves;
+  if (rows > mid && rows <= (many ? 16 : 24) * num_experts && K <= 4096 && busy) return 32;
   return 0;
 }
 
@@ -1123,12 +1125,14 @@ static int moe_group_gemm_impl(const void* x, int64_t rows, const void* q_weight
   //  282 / 292 / 301 / 307 / 343: the skinny kernel, once the step between the two, is behind both since the GEMM reads
   //  its scales in bulk, and only a forced variant runs it on expert segments.  The same rows per expert hold for many
   //  experts: 64 experts x top-6 (2048 x 1408 projections), whole layer at 144 / 192 / 288 / 384 / 432 routed rows
-  //  112 / 115 / 117 / 127 / 142 us against 137 / 141 / 146 / 143 / 144 on the GEMM's tiles)
   if (const int per_pass = midrow_rows_per_pass(rows, num_experts, K, bits)) {
     const hipError_t q = gq::launch_midrow(g, per_pass, as_stream(stream));
     if (q != hipErrorNotSupported) return hip_result(q, "moe mid-row launch");
   }
-  const int64_t quad_rows = 7 * num_experts > 32 ? 7 * num_experts : 32;
+  //  112 / 115 / 117 / 127 / 142 us against 137 / 141 / 146 / 143 / 144 on the GEMM's tiles as they were; since a tile finds its expert in
+  //  one step, 64 experts of 2048 x 1408 at 4 / 6 rows take 43 / 53 here and 38 / 38 there, and q4 hands over at three from K = 768 on, the shortest K measured)
+  const int64_t quad_per = bits == 4 && num_experts > 16 && K >= 768 ? 3 : 7;
+  const int64_t quad_rows = quad_per * num_experts > 32 ? quad_per * num_experts : 32;
   if ((rows <= 128 || rows <= 8 * num_experts) && gq::options().gemm_variant != 1 &&
       ((gv < 0 && rows <= quad_rows) || (gv >= 6 && gv <= 8))) {
     const hipError_t q = gq::launch_quadrow(g, static_cast<int>(rows), as_stream(stream));

@@ -199,33 +199,60 @@ __device__ __forceinline__ void dequant_group_bf16(const uint4 w4, const uint16_
     }
 }
 
-// Which activation rows [seg_lo, seg_hi) and which expert the m-tile `t` of a launch belongs to.
-// Plain linear: one segment.  Grouped: walk indptr (python/mlc_llm/op/moe_matmul.py:653-679 of
-// the reference does the same walk per tile).  Returns false when the tile does not exist.
+// The t-th row tile of BM rows among the experts' segments, taken one after another (python/mlc_llm/op/moe_matmul.py:653-679 of
+// the reference does the same walk per tile): its segment [seg_lo, seg_hi), its number mt within the segment, its expert.  False
+// when there are fewer tiles; the launch has one row of workgroups per tile that there could be, and most of the surplus ends
+// here.  Every wave looks at 64 experts at a time, a lane each: walked expert by expert, each step waits for its own two loads,
+// and that walk was longer than the multiplication for many small experts (128 experts of 2048 x 768, 24 rows each: 147 us on
+// 32-row tiles for 100 MB of weights, so 57).
+template <int BM>
+__device__ __forceinline__ bool locate_segment(const void* indptr, int indptr_i64, int num_experts, int rows, int t, int& seg_lo,
+                                               int& seg_hi, int& mt, int& expert) {
+  const int lane = threadIdx.x & 63;
+  for (int e0 = 0; e0 < num_experts; e0 += 64) {
+    int lo = 0, hi = 0;
+    if (e0 + lane < num_experts) {
+      int64_t l, h;
+      if (indptr_i64) {
+        l = static_cast<const int64_t*>(indptr)[e0 + lane];
+        h = static_cast<const int64_t*>(indptr)[e0 + lane + 1];
+      } else {
+        l = static_cast<const int32_t*>(indptr)[e0 + lane];
+        h = static_cast<const int32_t*>(indptr)[e0 + lane + 1];
+      }
+      l = l < 0 ? 0 : (l > rows ? rows : l);  // a corrupt indptr must not leave the tensors
+      h = h < l ? l : (h > rows ? rows : h);
+      lo = static_cast<int>(l);
+      hi = static_cast<int>(h);
+    }
+    const int tiles = (hi - lo + BM - 1) / BM;
+    int upto = tiles;  // tiles of this block's experts up to and including this lane's
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(upto, off);
+      if (lane >= off) upto += o;
+    }
+    const unsigned long long past = __ballot(upto > t);
+    if (past != 0) {
+      const int l = __builtin_ctzll(past);
+      seg_lo = __builtin_amdgcn_readlane(lo, l);
+      seg_hi = __builtin_amdgcn_readlane(hi, l);
+      mt = t - (__builtin_amdgcn_readlane(upto, l) - __builtin_amdgcn_readlane(tiles, l));
+      expert = e0 + l;
+      return true;
+    }
+    t -= __builtin_amdgcn_readlane(upto, 63);
+  }
+  return false;
+}
+
+// the same for a launch's parameters; plain linear: one segment
 template <int BM>
 __device__ __forceinline__ bool locate_tile(const GemmParams& p, int t, int& seg_lo, int& seg_hi,
                                             int& mt, int& expert) {
   seg_lo = 0; seg_hi = p.rows; mt = t; expert = 0;
   if (p.indptr == nullptr) return t * BM < p.rows;
-  for (int e = 0; e < p.num_experts; ++e) {
-    int64_t lo, hi;
-    if (p.indptr_i64) {
-      lo = static_cast<const int64_t*>(p.indptr)[e];
-      hi = static_cast<const int64_t*>(p.indptr)[e + 1];
-    } else {
-      lo = static_cast<const int32_t*>(p.indptr)[e];
-      hi = static_cast<const int32_t*>(p.indptr)[e + 1];
-    }
-    lo = lo < 0 ? 0 : (lo > p.rows ? p.rows : lo);  // a corrupt indptr must not leave the tensors
-    hi = hi < lo ? lo : (hi > p.rows ? p.rows : hi);
-    const int tiles = static_cast<int>((hi - lo + BM - 1) / BM);
-    if (t < tiles) {
-      seg_lo = static_cast<int>(lo); seg_hi = static_cast<int>(hi); mt = t; expert = e;
-      return true;
-    }
-    t -= tiles;
-  }
-  return false;
+  return locate_segment<BM>(p.indptr, p.indptr_i64, p.num_experts, p.rows, t, seg_lo, seg_hi, mt, expert);
 }
 
 // software-pipelined kernel family (needs K % 8 == 0); hipErrorNotSupported otherwise

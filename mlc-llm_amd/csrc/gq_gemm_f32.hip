@@ -85,26 +85,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_f32_kernel(co
   // ---- segment and row tile (grouped: the tiles of the experts' segments one after another)
   int seg_lo = 0, seg_hi = p.rows, mt = blockIdx.y, expert = 0;
   if (p.indptr != nullptr) {
-    bool found = false;
-    for (int e = 0; e < p.num_experts && !found; ++e) {
-      int64_t lo, hi;
-      if (p.indptr_i64) {
-        lo = static_cast<const int64_t*>(p.indptr)[e];
-        hi = static_cast<const int64_t*>(p.indptr)[e + 1];
-      } else {
-        lo = static_cast<const int32_t*>(p.indptr)[e];
-        hi = static_cast<const int32_t*>(p.indptr)[e + 1];
-      }
-      lo = lo < 0 ? 0 : (lo > p.rows ? p.rows : lo);  // a corrupt indptr must not leave the tensors
-      hi = hi < lo ? lo : (hi > p.rows ? p.rows : hi);
-      const int tiles = static_cast<int>((hi - lo + BM - 1) / BM);
-      if (mt < tiles) {
-        found = true;
-        seg_lo = static_cast<int>(lo); seg_hi = static_cast<int>(hi); expert = e;
-      } else {
-        mt -= tiles;
-      }
-    }
+    const bool found = locate_segment<BM>(p.indptr, p.indptr_i64, p.num_experts, p.rows, mt, seg_lo, seg_hi, mt, expert);
     if (!found) return;  // (uniform: before any barrier)
   }
   const int m0 = seg_lo + mt * BM, n0 = p.n_begin + blockIdx.x * BN;

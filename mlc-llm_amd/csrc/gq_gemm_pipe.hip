@@ -777,6 +777,42 @@ static hipError_t launch_planned_q4(const GemmParams& p, hipStream_t s) {
   return launch_pipe_cfg<4, 128, 128, 64, 64, 2, BF>(p, s);
 }
 
+// Expert segments of a q4 model: the tile height follows the rows per expert on average, r.  Measured on 8 / 16 / 64 / 128 experts of 768
+// x 2048 to 28672 x 4096 (f16, us; tiles of 32 / 64 / 128 / 256 rows): 64 experts of 2816 x 2048 at r = 20 63.7 / 81.0 / 107 / 108, at r =
+// 32 93.9 / 84.0 / 111 / 125, at r = 64 145 / 121 / 116 / 125, at r = 96 - / 163 / 120 / 140, at r = 128 - / 194 / 175 / 151; 8 experts of 4096 x
+// 14336 at r = 20 89.5 / 103, r = 64 183 / 158 / 142 / 170, r = 96 - / 177 / 150 / 185, r = 128 - / 258 / 232 / 189.  Beyond r = 100 a segment no longer fits
+// 128 rows, and 256-row tiles whose waves skip the 32-row blocks past the segment's end are ahead: matrix work is the segment's rows
+// rounded up to 32, and the expert's weights are dequantised once.  bfloat16 the same (64 experts of 5120 x 3584 at r = 128 / 192: 468 / 561
+// against 560 / 728 for 128 rows).
+template <bool BF>
+static hipError_t launch_grouped_q4(const GemmParams& p, hipStream_t s) {
+  const int64_t rows = p.rows, experts = p.num_experts;
+  if (rows <= 24 * experts) return launch_pipe_cfg<4, 32, 128, 32, 32, 4, BF>(p, s);
+  if (rows <= 48 * experts) return launch_pipe_cfg<4, 64, 128, 32, 64, 4, BF>(p, s);
+  if (rows <= 100 * experts && p.K >= 768) return launch_pipe_cfg<4, 128, 128, 64, 64, 2, BF>(p, s);  // (the shortest K measured)
+  // 256 columns per tile while that gives every CU a workgroup, else 128 (e2 of a Mixtral layer, 128 wide tiles: r = 128 189
+  // against 270 us; 16 experts of 4096 x 2048, 256 of them: 53 against 63)
+  const int64_t tiles_x = (p.N + 255) / 256, live = experts > rows / 256 ? experts : rows / 256;  // row tiles that hold rows
+  if (tiles_x * live < 256) return launch_pipe_cfg<4, 256, 128, 64, 64, 2, BF, true, 2>(p, s);
+  // A last round of workgroups that is at most about half full costs a whole round here (the kernel waits on
+  // memory, not on the matrix pipe): its columns go to a second launch on the narrow tile, whose workgroups take
+  // half as long.  (Mixtral's e1_e3, 112 column tiles x 8 experts = 3.5 rounds of 256.)
+  const int64_t rounds = tiles_x * live / 256, rest = tiles_x * live % 256;
+  if (rest > 0 && rest <= 144) {
+    GemmParams a = p, b = p;
+    a.n_end = static_cast<int>(rounds * 256 / live * 256);
+    b.n_begin = a.n_end;
+    if (a.n_end > 0 && a.n_end < p.N) {
+      const hipError_t e = launch_pipe_cfg<4, 256, 256, 128, 64, 2, BF, true, 2>(a, s);
+      if (e != hipSuccess) return e;
+      return launch_pipe_cfg<4, 256, 128, 64, 64, 2, BF, true, 2>(b, s);
+    }
+  }
+  // (both tiles' weight loads run two more K tiles ahead than their activation loads: Mixtral's e2 on the narrow tile
+  // at 64 / 128 / 256 rows per expert 201 -> 177, 236 -> 213, 320 -> 305 us; e1_e3 on the wide one 1-2 %)
+  return launch_pipe_cfg<4, 256, 256, 128, 64, 2, BF, true, 2>(p, s);
+}
+
 hipError_t launch_gemm_pipe(const GemmParams& p, int bits, hipStream_t s) {
   if ((p.K & 7) != 0 || p.ng == 0) return hipErrorNotSupported;
   const int variant = options().gemm_variant;
@@ -791,15 +827,9 @@ hipError_t launch_gemm_pipe(const GemmParams& p, int bits, hipStream_t s) {
     }
     if (p.partial != nullptr) return hipErrorNotSupported;
     if (p.indptr != nullptr) {
+      if (bits == 4) return launch_grouped_q4<true>(p, s);
       const bool wide = p.rows >= 96 * p.num_experts &&
                         (static_cast<int64_t>(p.rows) / 128 + p.num_experts) * ((p.N + 255) / 256) >= 768;
-      if (bits == 4) {
-        // few rows per expert: the tile height follows them (there are no bf16 few-row kernels)
-        if (p.rows <= 16 * p.num_experts) return launch_pipe_cfg<4, 32, 128, 32, 32, 4, true>(p, s);
-        if (p.rows <= 48 * p.num_experts) return launch_pipe_cfg<4, 64, 128, 32, 64, 4, true>(p, s);
-        return wide ? launch_pipe_cfg<4, 128, 256, 64, 64, 2, true>(p, s)
-                    : launch_pipe_cfg<4, 128, 128, 64, 64, 2, true>(p, s);
-      }
       return wide ? launch_pipe_cfg<3, 128, 256, 64, 64, 2, true>(p, s)
                   : launch_pipe_cfg<3, 128, 128, 64, 64, 2, true>(p, s);
     }
@@ -812,56 +842,23 @@ hipError_t launch_gemm_pipe(const GemmParams& p, int bits, hipStream_t s) {
     if (p.bm_hint == 64) return launch_pipe_cfg<3, 64, 128, 32, 64, 4>(p, s);
     return launch_pipe_cfg<3, 128, 128, 64, 64>(p, s);
   }
-  // Grouped, from about 64 rows per expert on: 256-row tiles whose waves skip the 32-row blocks past the end of
-  // the expert's segment.  A ragged segment then costs its rows rounded up to 32 in matrix work, and the expert's
-  // weights are dequantised once per 256 rows instead of once per (often nearly empty) 128-row tile.  256 columns
-  // per tile while that still makes two workgroups per CU, else 128 (e2 of a Mixtral layer: 32 column tiles).
-  if (p.indptr != nullptr && ((variant < 0 && p.rows > 48 * p.num_experts) || variant == 10 || variant == 11)) {
-    const int64_t mt = p.rows / 256 + p.num_experts;
-    const bool wide = variant == 10 || (variant != 11 && bits == 4 && mt * ((p.N + 255) / 256) >= 512);
-    if (bits == 4) {
-      if (wide) {
-        // A last round of workgroups that is at most about half full costs a whole round here (the kernel waits on
-        // memory, not on the matrix pipe): its columns go to a second launch on the narrow tile, whose workgroups take
-        // half as long.  (Mixtral's e1_e3, 112 column tiles x 8 experts = 3.5 rounds of 256.)
-        const int64_t tiles_x = (p.N + 255) / 256;
-        const int64_t live = p.num_experts > p.rows / 256 ? p.num_experts : p.rows / 256;  // row tiles that hold rows
-        const int64_t rounds = tiles_x * live / 256, rest = tiles_x * live % 256;
-        if (variant != 10 && rounds >= 1 && rest > 0 && rest <= 144 && p.n_end == 0 && p.n_begin == 0) {
-          GemmParams a = p, b = p;
-          a.n_end = static_cast<int>(rounds * 256 / live * 256);
-          b.n_begin = a.n_end;
-          if (a.n_end > 0 && a.n_end < p.N) {
-            const hipError_t e = launch_pipe_cfg<4, 256, 256, 128, 64, 2, false, true, 2>(a, s);
-            if (e != hipSuccess) return e;
-            return launch_pipe_cfg<4, 256, 128, 64, 64, 2, false, true, 2>(b, s);
-          }
-        }
-        return launch_pipe_cfg<4, 256, 256, 128, 64, 2, false, true, 2>(p, s);
-      }
-      // both tiles' weight loads run two more K tiles ahead than their activation loads (Mixtral's e2 on the narrow tile
-      // at 64 / 128 / 256 rows per expert: 201 -> 177, 236 -> 213, 320 -> 305 us; e1_e3 on the wide one 1-2 %)
-      return launch_pipe_cfg<4, 256, 128, 64, 64, 2, false, true, 2>(p, s);
-    }
-    return launch_pipe_cfg<3, 256, 128, 64, 64, 2, false, true>(p, s);
+  if (p.indptr != nullptr && bits == 4) {
+    // (tuning override: 6 / 9 / 10 / 11 force 128 x 128, 128 x 256, 256 x 256 and 256 x 128 tiles)
+    if (variant == 6) return launch_pipe_cfg<4, 128, 128, 64, 64>(p, s);
+    if (variant == 9) return launch_pipe_cfg<4, 128, 256, 64, 64>(p, s);
+    if (variant == 10) return launch_pipe_cfg<4, 256, 256, 128, 64, 2, false, true, 2>(p, s);
+    if (variant == 11) return launch_pipe_cfg<4, 256, 128, 64, 64, 2, false, true, 2>(p, s);
+    if (variant != 7) return launch_grouped_q4<false>(p, s);
   }
-  if (bits == 4) {
-    // grouped, few rows per expert: the tile height follows them (Mixtral layer, 8 experts: 144-384 routed
-    // rows 18-20 % faster than on 128-row tiles)
-    if (p.indptr != nullptr && (variant < 0 || variant == 1)) {
-      if (p.rows <= 16 * p.num_experts) return launch_pipe_cfg<4, 32, 128, 32, 32, 4>(p, s);
-      if (p.rows <= 48 * p.num_experts) return launch_pipe_cfg<4, 64, 128, 32, 64, 4>(p, s);
-    }
-    // plain matmul, tuning override: variants 6 / 7 / 9 force one tile
+  // q3, from about 64 rows per expert on: 256-row tiles whose waves skip the row blocks past the segment's end
+  if (p.indptr != nullptr && ((variant < 0 && p.rows > 48 * p.num_experts) || variant == 10 || variant == 11))
+    return launch_pipe_cfg<3, 256, 128, 64, 64, 2, false, true>(p, s);
+  if (bits == 4) {  // (tuning override: the forced tiles of a plain matmul)
     if (variant == 9) return launch_pipe_cfg<4, 128, 256, 64, 64>(p, s);
     if (variant == 7) return launch_pipe_cfg<4, 256, 256, 128, 64>(p, s);
-    // grouped: the wider tile once the experts' row tiles alone make several rounds of workgroups
-    if (variant != 6 && p.indptr != nullptr && p.rows >= 96 * p.num_experts &&
-        (static_cast<int64_t>(p.rows) / 128 + p.num_experts) * ((p.N + 255) / 256) >= 768)
-      return launch_pipe_cfg<4, 128, 256, 64, 64>(p, s);
     return launch_pipe_cfg<4, 128, 128, 64, 64>(p, s);
   }
-  if (p.indptr != nullptr && (variant < 0 || variant == 1)) {  // grouped, few rows per expert: as q4 above
+  if (p.indptr != nullptr && (variant < 0 || variant == 1)) {  // grouped, few rows per expert
     if (p.rows <= 16 * p.num_experts) return launch_pipe_cfg<3, 32, 128, 32, 32, 4>(p, s);
     if (p.rows <= 48 * p.num_experts) return launch_pipe_cfg<3, 64, 128, 32, 64, 4>(p, s);
   }

@@ -1,0 +1,44 @@
+"""Row tiles of expert segments: a wave finds its tile's expert among 64 at a time, so expert counts around 64 and its multiples, empty
+segments at the ends and in between, tiles that do not exist; the tile heights by rows per expert.  Against the float64 product of
+the dequantised weights."""
+
+import pytest
+import torch
+
+import mlc_llm_amd as gq
+from mlc_llm_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("experts", [1, 63, 64, 65, 130])
+@pytest.mark.parametrize("average", [22, 40, 70, 150])
+def test_every_row_meets_its_expert(dtype, experts, average):
+    n, k = 72, 768
+    g = torch.Generator().manual_seed(experts * average)
+    sizes = torch.randint(0, 2 * average, (experts,), generator=g)
+    sizes[torch.rand((experts,), generator=g) < 0.2] = 0
+    if experts > 1:
+        sizes[0] = sizes[-1] = 0
+        sizes[experts // 2] += max(0, average * experts - int(sizes.sum()))  # one long segment brings the average up
+    else:
+        sizes[0] = average
+    indptr = torch.cat([torch.zeros(1, dtype=torch.int64), sizes.cumsum(0)])
+    rows = int(indptr[-1])
+    gd = torch.Generator(device="cuda").manual_seed(experts + average)
+    w = (torch.randn((experts, n, k), generator=gd, device="cuda") * 0.05).to(dtype)
+    qw, qs = ops.quantize(w, 4, 32)
+    full = ops.dequantize(qw, qs, k, 4, 32).double()
+    x = torch.randn((rows, k), generator=gd, device="cuda").to(dtype)
+    want = torch.empty((rows, n), dtype=torch.float64, device="cuda")
+    for e in range(experts):
+        want[indptr[e]:indptr[e + 1]] = x[indptr[e]:indptr[e + 1]].double() @ full[e].t().contiguous()
+    got = ops.moe_group_gemm(x, qw, qs, indptr.int().cuda(), 4, 32)
+    # one rounding of the output and float32 sums (a wrong expert is off by its whole row)
+    tol = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -9, torch.float32: 0}[dtype] + 1e-5
+    err = (got.double() - want).norm(dim=1) / want.norm(dim=1)
+    assert err.max().item() <= 2 * tol, gq._lib.last_kernel()  # (2: a row of 72 elements, where the bound is for the mean)
+    assert torch.equal(got, ops.moe_group_gemm(x, qw, qs, indptr.cuda(), 4, 32))
+    short = ops.moe_group_gemm(torch.cat([x, x[:5]]), qw, qs, indptr.int().cuda(), 4, 32)  # rows behind the last segment
+    assert (short[rows:] == 0).all() and (short[:rows].double() - want).norm() <= 2 * tol * want.norm()
