@@ -204,7 +204,7 @@ __device__ __forceinline__ void dequant_group_bf16(const uint4 w4, const uint16_
 // when there are fewer tiles; the launch has one row of workgroups per tile that there could be, and most of the surplus ends
 // here.  Every wave looks at 64 experts at a time, a lane each: walked expert by expert, each step waits for its own two loads,
 // and that walk was longer than the multiplication for many small experts (128 experts of 2048 x 768, 24 rows each: 147 us on
-// 32-row tiles for 100 MB of weights, so 57).
+// 32-row tiles for 113 MB of weights, so 44).
 template <int BM>
 __device__ __forceinline__ bool locate_segment(const void* indptr, int indptr_i64, int num_experts, int rows, int t, int& seg_lo,
                                                int& seg_hi, int& mt, int& expert) {
