@@ -4,7 +4,7 @@
 // What it replaces took 13 us of interpreter time per projection (a torch.cuda.Stream object, three Python checks per tensor, two
 // ctypes calls), which is more than a decode projection takes on the GPU: a one-row 4096 x 4096 linear took 14.0 us per call for
 // a 4.3 us kernel (7.3 us this way), and every decode step of one to a few rows was bound by it (34 linears of an 8-layer step with
-one row: 455 -> 332 us, with 3-bit weights 449 -> 277).
+// one row: 455 -> 332 us, with 3-bit weights 449 -> 277).
 //
 // A function returns the output tensor, or the C ABI's (negative) code as an int, or None where the arguments are not what it
 // expects: plain strided tensors on the GPU of the types and shapes that the operator takes, no torch function mode.  The caller
