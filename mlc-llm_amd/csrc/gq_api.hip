@@ -158,6 +158,8 @@ const char* mi355gq_testing_last_kernel(void) {
   return text;
 }
 
+int mi355gq_testing_x_chunk(int k, int end) { return gq::x_chunk(k, end); }
+
 int mi355gq_testing_set_option(const char* name, int value) {
   GQ_REQUIRE(name != nullptr, "option name is null");
   gq::Options& o = gq::options();

@@ -94,14 +94,14 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_f32_kernel(co
 
   // ---- this thread's share of a K tile (rows past the segment and columns past N read valid rows: they reach no live
   //      result and the epilogue drops theirs)
-  const float* a_src[A_CH];
+  const float* a_src[A_CH];  // the start of the chunk's row
   int a_k[A_CH], a_dst[A_CH];
   const bool a_active = A_ALL || tid < BM * 4;  // (wave-uniform)
 #pragma unroll
   for (int i = 0; i < A_CH; ++i) {
     const int idx = a_active ? tid + NT * i : 0;
     const int r = idx >> 2, ch = idx & 3;
-    a_src[i] = p.x + static_cast<int64_t>(min(m0 + r, seg_hi - 1)) * p.K + 8 * ch;
+    a_src[i] = p.x + static_cast<int64_t>(min(m0 + r, seg_hi - 1)) * p.K;
     a_k[i] = 8 * ch;
     a_dst[i] = r * kRow + 8 * ch;
   }
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_f32_kernel(co
     const int kt = min(kt_raw, kt1 - 1);  // (tiles past the end re-read the last one: never multiplied)
 #pragma unroll
     for (int i = 0; i < A_CH; ++i) {
-      const float* const src = a_src[i] + (kt * 32 + a_k[i] < p.K ? kt * 32 : 0);  // K % 8 == 0: a chunk is inside or outside
+      const float* const src = a_src[i] + x_chunk(kt * 32 + a_k[i], p.K);
       r.a[i][0] = *reinterpret_cast<const float4*>(src);
       r.a[i][1] = *reinterpret_cast<const float4*>(src + 4);
     }

@@ -28,6 +28,11 @@ struct Options {
 };
 Options& options();
 
+// Where in its row the eight activations at k are loaded from by a kernel that loads whatever the tile covers and masks the
+// values later: at k, or at the row's start where k lies at or past `end` (K % 8 == 0 and end % 8 == 0, so a chunk is inside
+// or outside; every row has a first chunk, and no other address is sure to be the caller's).
+__host__ __device__ inline int x_chunk(int k, int end) { return k < end ? k : 0; }
+
 // Records which kernel instantiation the calling thread launched last (thread-local, read back through the test hook
 // mi355gq_testing_last_kernel): measurement code names the kernel it timed from the run itself.  A launch keeps the format
 // and its arguments (integers and string literals); the text is made when it is asked for, because formatting it took as

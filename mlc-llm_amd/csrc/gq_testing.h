@@ -42,6 +42,10 @@ __attribute__((visibility("default"))) const char* mi355gq_testing_last_kernel(v
 __attribute__((visibility("default"))) int mi355gq_testing_stream_read(const void* a, int64_t a_bytes, const void* b,
                                                                        int64_t b_bytes, void* sink, void* stream);
 
+/* The load address rule of the GEMMs' activation chunks (x_chunk in csrc/gq_internal.hpp): the element of its row at which the
+ * eight activations at k are read when a row has `end` of them. */
+__attribute__((visibility("default"))) int mi355gq_testing_x_chunk(int k, int end);
+
 #ifdef __cplusplus
 }
 #endif

@@ -96,6 +96,7 @@ TEST_HOOKS = {
     "mi355gq_testing_set_option": (_I, [c_char_p, _I]),
     "mi355gq_testing_last_kernel": (c_char_p, []),
     "mi355gq_testing_stream_read": (_I, [_P, _L, _P, _L, _P, _P]),
+    "mi355gq_testing_x_chunk": (_I, [_I, _I]),
 }
 
 

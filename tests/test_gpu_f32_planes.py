@@ -44,7 +44,7 @@ def _close(y, ref, k, what):
 @pytest.mark.parametrize("m,n,k,kernel", [
     (1, 48, 14336, "midrow"), (2, 16, 256, "midrow"), (3, 1000, 1280, "midrow"), (5, 257, 4096, "midrow"), (4, 144, 8448, "midrow"),
     (6, 16400, 4096, "midrow"), (10, 16400, 4096, "midrow"),
-    (5, 100, 1000, "gemm"), (6, 129, 8, "gemm"), (31, 130, 1544, "gemm"), (32, 128, 4096, "gemm"), (33, 300, 360, "gemm"),
+    (5, 100, 1000, "gemm"), (6, 129, 8, "gemm"), (5, 40, 16, "gemm"), (33, 130, 24, "gemm"), (31, 130, 1544, "gemm"), (32, 128, 4096, "gemm"), (33, 300, 360, "gemm"),
     (64, 128, 288, "gemm"), (65, 256, 4096, "gemm"), (128, 257, 64, "gemm"), (129, 16, 5632, "gemm"), (300, 520, 1544, "gemm"),
     (300, 22300, 1024, "split=4"),  # whole rounds of columns first, the K of the rest cut
 ])

@@ -296,3 +296,14 @@ def test_other_model_dtypes_carry_their_dtype_in_the_parameters():
         assert lin.q_scale.dtype == dt and lin.bias.dtype == dt and lin.q_weight.shape == (24, 8)
         emb = gq.GroupQuantizeEmbedding(10, 64, gq.QUANTIZATION[name])
         assert emb.q_scale.dtype == dt
+
+
+def test_activation_chunks_are_loaded_from_inside_their_row():
+    """Kernels load every chunk of eight activations that a K tile covers and mask what lies past K: the load itself stays in the
+    row for every K, tiles wider than K included (a K of 8 under tiles of 32, 64 and 80)."""
+    chunk = _lib.lib().mi355gq_testing_x_chunk
+    for tile in (32, 64, 80):
+        for k_total in list(range(8, 200, 8)) + [1544, 4104, 14336]:
+            for k in range(0, (k_total // tile + 2) * tile, 8):  # one tile past the last, as the K loops run ahead
+                at = chunk(k, k_total)
+                assert at == k if k < k_total else 0 <= at <= k_total - 8, (tile, k_total, k, at)
