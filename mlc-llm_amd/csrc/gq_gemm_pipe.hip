@@ -211,8 +211,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_pipe_kernel(c
     const int k_base = kt * BK;
 #pragma unroll
     for (int i = 0; i < A_CHUNKS; ++i) {
-      const bool ok = k_base + a_k[i] < k_lim;  // K % 8 == 0: a chunk is entirely inside or outside
-      st.a[i] = *reinterpret_cast<const uint4*>(ok ? a_src[i] + k_base : a_src[i]);
+      st.a[i] = *reinterpret_cast<const uint4*>(a_src[i] + (x_chunk(k_base + a_k[i], k_lim) - a_k[i]));
     }
   };
   auto load_w = [&](int kt, StageW& st) {

@@ -14,6 +14,8 @@ CASES = [(65, 256, 256, "64,128", False), (65, 256, 1000, "64,128", True), (65, 
          (333, 6000, 1000, "128,128", False), (513, 8200, 320, "128,256", False), (129, 4096, 4104, None, None), (160, 4096, 14336, "256,128", True),
          (257, 4100, 2048, None, None), (777, 4096, 8192, "256,128", None), (300, 28672, 1024, "256,256", False),
          (512, 28680, 512, "256,256", False), (1025, 2056, 4096, None, None),
+         # a K shorter than a K tile, whose chunks past K are loaded from the row's start
+         (65, 256, 8, None, False), (130, 200, 24, None, False), (300, 130, 56, None, False),
          # columns of the whole rounds first, the rest on another tile or split
          (300, 25000, 2048, None, None), (450, 37888, 1024, None, None), (1536, 12288, 1024, None, None)]
 
