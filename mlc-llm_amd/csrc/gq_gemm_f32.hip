@@ -6,7 +6,7 @@
 //
 // The float32 matrix instruction runs at a sixteenth of the bfloat16 one's rate and was what bounded these models.  Here x is cut
 // into three bfloat16 planes, x = h + m + l: the leading 8 bits of the significand, the next 8 and the last 8, which is all
-// 24 of them (the differences are exact), and the weights enter as the integers q - 7, which a bfloat16 holds exactly.  The
+// 24 of them (the differences are exact), and the weights enter as the integers q - 7 (times 2^-9), which a bfloat16 holds exactly.  The
 // three products of a group of 32 weights then carry no rounding but that of the float32 accumulator, smallest plane first,
 // and the group's float32 scale multiplies the group's sum: one rounding per group where the kernel this replaced rounded
 // every weight.  Three bfloat16 instructions per product instead of one float32 instruction: up to 16 / 3 = 5.3 times the rate.
@@ -54,14 +54,16 @@ __device__ __forceinline__ uint32_t hi_pair(float a, float b) {  // upper halves
   return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
 }
 
-// one storage word -> 8 bfloat16 integers q - 7 in the order (0, 2) (4, 6) (1, 3) (5, 7).  A byte 0 .. 15 read as an fp8
-// (e4m3) number is that many 2^-9: the subnormals, then the first binade, whose steps are the same.
+// one storage word -> 8 bfloat16 numbers (q - 7) 2^-9 in the order (0, 2) (4, 6) (1, 3) (5, 7).  A byte 0 .. 15 read as an fp8
+// (e4m3) number is that many 2^-9: the subnormals, then the first binade, whose steps are the same.  The 2^-9 stays on until
+// the result is stored: a group's sum is then at most half the largest |x| in it and cannot overflow before its scale is applied.
 __device__ __forceinline__ uint4 word_minus7(uint32_t w) {
+  constexpr float k7 = 7.0f / 512.0f;
   const uint32_t t0 = w & 0x0f0f0f0fu, t1 = (w >> 4) & 0x0f0f0f0fu;
-  const f3_f2 a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t0, 512.0f, false), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t0, 512.0f, true);
-  const f3_f2 c = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t1, 512.0f, false), d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t1, 512.0f, true);
-  return make_uint4(hi_pair(a.x - 7.0f, a.y - 7.0f), hi_pair(b.x - 7.0f, b.y - 7.0f), hi_pair(c.x - 7.0f, c.y - 7.0f),
-                    hi_pair(d.x - 7.0f, d.y - 7.0f));
+  const f3_f2 a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t0, 1.0f, false), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t0, 1.0f, true);
+  const f3_f2 c = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t1, 1.0f, false), d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t1, 1.0f, true);
+  return make_uint4(hi_pair(a.x - k7, a.y - k7), hi_pair(b.x - k7, b.y - k7), hi_pair(c.x - k7, c.y - k7),
+                    hi_pair(d.x - k7, d.y - k7));
 }
 
 template <int BM, int BN, int WM, int WN>
@@ -141,7 +143,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_f32_kernel(co
           const uint32_t xb = __builtin_bit_cast(uint32_t, raw[e]) & keep;
           const float x = __builtin_bit_cast(float, xb);
           h[e] = __builtin_bit_cast(float, xb & 0xffff0000u);
-          const float r1 = x - h[e];
+          const float r1 = __builtin_isinf(x) ? 0.0f : x - h[e];  // (inf - inf: an infinity is all in the first plane)
           m[e] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r1) & 0xffff0000u);
           l[e] = r1 - m[e];
         }
@@ -233,10 +235,11 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_f32_kernel(co
         const int row = m0 + wm0 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
         if (row < seg_hi && col < p.n_end) {
           const int64_t oi = static_cast<int64_t>(row) * p.N + col;
+          const float sum = 512.0f * acc[i][j][r];
           if (p.partial != nullptr) {
-            p.partial[(static_cast<int64_t>(blockIdx.z) * p.rows + row) * (p.N - p.n_begin) + (col - p.n_begin)] = acc[i][j][r];
+            p.partial[(static_cast<int64_t>(blockIdx.z) * p.rows + row) * (p.N - p.n_begin) + (col - p.n_begin)] = sum;
           } else {
-            float v = acc[i][j][r] + bias;
+            float v = sum + bias;
             if (p.residual != nullptr) v += p.residual[oi];
             p.y[oi] = v;
           }
