@@ -31,7 +31,6 @@ namespace gq {
 namespace {
 
 typedef __bf16 f3_bf8 __attribute__((ext_vector_type(8)));
-typedef float f3_f2 __attribute__((ext_vector_type(2)));
 
 struct F32Params {
   const float* x;
@@ -49,22 +48,6 @@ struct F32Params {
 };
 
 constexpr int kRow = 40;  // halves per LDS row: 32 + 8 of padding
-
-__device__ __forceinline__ uint32_t hi_pair(float a, float b) {  // upper halves of two float32: (a, b) as bfloat16, truncated
-  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
-}
-
-// one storage word -> 8 bfloat16 numbers (q - 7) 2^-9 in the order (0, 2) (4, 6) (1, 3) (5, 7).  A byte 0 .. 15 read as an fp8
-// (e4m3) number is that many 2^-9: the subnormals, then the first binade, whose steps are the same.  The 2^-9 stays on until
-// the result is stored: a group's sum is then at most half the largest |x| in it and cannot overflow before its scale is applied.
-__device__ __forceinline__ uint4 word_minus7(uint32_t w) {
-  constexpr float k7 = 7.0f / 512.0f;
-  const uint32_t t0 = w & 0x0f0f0f0fu, t1 = (w >> 4) & 0x0f0f0f0fu;
-  const f3_f2 a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t0, 1.0f, false), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t0, 1.0f, true);
-  const f3_f2 c = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t1, 1.0f, false), d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(t1, 1.0f, true);
-  return make_uint4(hi_pair(a.x - k7, a.y - k7), hi_pair(b.x - k7, b.y - k7), hi_pair(c.x - k7, c.y - k7),
-                    hi_pair(d.x - k7, d.y - k7));
-}
 
 template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_f32_kernel(const F32Params p) {

@@ -34,8 +34,8 @@
 // are still read once), adding to the sums in LDS.  Expert segments (moe_matmul.dequantize_group_gemm,
 // python/mlc_llm/op/moe_matmul.py:562-768): grid row = expert, rows from indptr, more rows than the batch tiles hold in
 // passes.  Float32 models (q4f32_1): x = h + m + l, three bfloat16 planes that together are x exactly, so five activation
-// rows make fifteen rows of the bfloat16 operand; the weights are the integers q (v_cvt_scalef32_pk_bf16_fp8, two fields per
-// instruction), the offset -7 * sum(x), and the planes of a row meet where the K shares do: products and scales as exact as
+// rows make fifteen rows of the bfloat16 operand; the weights are the integers q, times 2^-9 (v_cvt_scalef32_pk_bf16_fp8, two
+// fields per instruction), the offset -7 * sum(x), and the planes of a row meet where the K shares do: products and scales as exact as
 // float32 dot products make them (relative error 8e-8 against float64 at K = 4096), at the price of the weight stream
 // (4 rows: 28672 x 4096 76.7 us on the dot-product kernel's passes -> 23, 128256 x 4096 237 -> 77, 4096 x 14336 1168 -> 18.4).
 // The fused gate/up form walks a gate tile and its up tile in consecutive rounds and folds silu(gate) * up into
@@ -91,15 +91,16 @@ __device__ __forceinline__ float4_t mid_mfma(const mid_u4 a, const mid_u4 b, con
   }
 }
 
-// the eight fields of a storage word as bfloat16 integers, fields (0, 2) (4, 6) (1, 3) (5, 7): a byte 0 .. 15 read as an
+// the eight fields of a storage word as bfloat16 numbers q 2^-9, fields (0, 2) (4, 6) (1, 3) (5, 7): a byte 0 .. 15 read as an
 // fp8 (e4m3) number is that many 2^-9 (subnormals, then the first binade, whose steps are the same), so the scaled
-// conversion delivers two fields per instruction
+// conversion delivers two fields per instruction.  The 2^-9 stays on until the K shares meet: a group's sum, offset
+// included, then stays below the largest |x| in it and cannot overflow before its scale is applied.
 __device__ __forceinline__ mid_u4 mid_word_bf16(uint32_t w) {
   const uint32_t t0 = w & 0x0f0f0f0fu, t1 = (w >> 4) & 0x0f0f0f0fu;
-  return mid_u4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t0, 512.0f, false)),
-                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t0, 512.0f, true)),
-                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t1, 512.0f, false)),
-                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t1, 512.0f, true))};
+  return mid_u4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t0, 1.0f, false)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t0, 1.0f, true)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t1, 1.0f, false)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t1, 1.0f, true))};
 }
 
 // NBT: batch tiles of 16 rows; U: groups of K a wave owns (4 or 8); RT: tiles of loads in flight per wave;
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
 
   constexpr uint32_t kLoLo = 0x05040100u, kHiHi = 0x07060302u;
   const half2_t r16 = {static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)};
-  const mid_u4 neg_off = F32  ? mid_u4{0xc0e0c0e0u /* -7 */, 0xc0e0c0e0u, 0xc0e0c0e0u, 0xc0e0c0e0u}
+  const mid_u4 neg_off = F32  ? mid_u4{0xbc60bc60u /* -7 2^-9 */, 0xbc60bc60u, 0xbc60bc60u, 0xbc60bc60u}
                          : BF ? mid_u4{0xc307c307u /* -135 */, 0xc307c307u, 0xc307c307u, 0xc307c307u}
                               : mid_u4{0xe407e407u /* -1031 */, 0xe407e407u, 0xe470e470u /* -16 * 71 */, 0xe470e470u};
 
@@ -231,46 +232,56 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
         }
       };
       mid_u4 xa[NBT][U];
+      bool any_odd = false;  // (float32, uniform) this wave's share of x holds an infinity or a NaN
       float4_t cc[KEEP_C ? NBT : 1][KEEP_C ? U : 1];
       if constexpr (F32) {
         // ---- x as three bfloat16 planes, x = h + m + l: the leading 8 bits of the significand, the next 8, the last 8
         //      (differences of float32 values that share their exponent range are exact, so the planes lose nothing).  A
         //      batch tile's matrix rows are (activation row, plane): row i of the operand is plane i % 3 of row i / 3.
+        //      An infinity has to count as zero here, because its products and their offset would be inf - inf, and so does a NaN
+        //      (add_infinities below brings both in); one of them is told by x - h, which is NaN for it, once per wave.
         const int pl = c % 3;
+        float odd = 0.f;  // NaN: an infinity or a NaN among this lane's activations
+        static_assert(!F32 || (NBT == 1 && !KEEP_C), "one batch tile, offsets from the operand");
+        const int b = pass_lo + c / 3;
+        const bool ok = k_live && c < 3 * BR && b < seg_hi;
+        const int64_t xr = p.x_one_row ? 0 : x_row(p.x_rows, p.x_src_rows, ok ? b : seg_lo);
+        const float* const xrow = reinterpret_cast<const float*>(p.x) + xr * p.K + ga * 32 + 8 * j;
+        uint4 lo[U], hi[U];
 #pragma unroll
-        for (int bt = 0; bt < NBT; ++bt) {
-          const int b = pass_lo + BR * bt + c / 3;
-          const bool ok = k_live && c < 3 * BR && b < seg_hi;
-          const int64_t xr = p.x_one_row ? 0 : x_row(p.x_rows, p.x_src_rows, ok ? b : seg_lo);
-          const float* const xrow = reinterpret_cast<const float*>(p.x) + xr * p.K + ga * 32 + 8 * j;
-          uint4 lo[U], hi[U];
+        for (int u = 0; u < U; ++u) {
+          lo[u] = *reinterpret_cast<const uint4*>(xrow + u * 32);
+          hi[u] = *reinterpret_cast<const uint4*>(xrow + u * 32 + 4);
+        }
+        issue_all();  // (behind the loads of x: those are needed first, and loads retire in issue order)
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            lo[u] = *reinterpret_cast<const uint4*>(xrow + u * 32);
-            hi[u] = *reinterpret_cast<const uint4*>(xrow + u * 32 + 4);
+        for (int u = 0; u < U; ++u) {
+          const uint32_t raw[8] = {lo[u].x, lo[u].y, lo[u].z, lo[u].w, hi[u].x, hi[u].y, hi[u].z, hi[u].w};
+          uint32_t v[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float x = __builtin_bit_cast(float, ok ? raw[e] : 0u);
+            const float h = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xffff0000u);
+            const float r1 = x - h;
+            const float m = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r1) & 0xffff0000u);
+            odd = fmaf(r1, 0.f, odd);
+            v[e] = __builtin_bit_cast(uint32_t, pl == 0 ? h : (pl == 1 ? m : r1 - m));
           }
-          if (bt == NBT - 1) {  // (behind the loads of x: those are needed first, and loads retire in issue order)
-            issue_all();
-          }
+          // fields (0, 2) (4, 6) (1, 3) (5, 7): the order in which the conversion delivers a word
+          xa[0][u][0] = __builtin_amdgcn_perm(v[2], v[0], kHiHi);
+          xa[0][u][1] = __builtin_amdgcn_perm(v[6], v[4], kHiHi);
+          xa[0][u][2] = __builtin_amdgcn_perm(v[3], v[1], kHiHi);
+          xa[0][u][3] = __builtin_amdgcn_perm(v[7], v[5], kHiHi);
+        }
+        any_odd = __ballot(odd != odd) != 0;
+        if (any_odd) {  // (uniform, rare; no plane of a finite activation has an exponent of all ones)
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const uint32_t raw[8] = {lo[u].x, lo[u].y, lo[u].z, lo[u].w, hi[u].x, hi[u].y, hi[u].z, hi[u].w};
-            uint32_t v[8];
+          for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const float x = __builtin_bit_cast(float, ok ? raw[e] : 0u);
-              const float h = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xffff0000u);
-              const float r1 = x - h;
-              const float m = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r1) & 0xffff0000u);
-              v[e] = __builtin_bit_cast(uint32_t, pl == 0 ? h : (pl == 1 ? m : r1 - m));
+            for (int i = 0; i < 4; ++i) {
+              const uint32_t v = xa[0][u][i];
+              xa[0][u][i] = ((v & 0x7f80u) == 0x7f80u ? 0u : v & 0xffffu) | ((v & 0x7f800000u) == 0x7f800000u ? 0u : v & 0xffff0000u);
             }
-            // fields (0, 2) (4, 6) (1, 3) (5, 7): the order in which the conversion delivers a word
-            xa[bt][u][0] = __builtin_amdgcn_perm(v[2], v[0], kHiHi);
-            xa[bt][u][1] = __builtin_amdgcn_perm(v[6], v[4], kHiHi);
-            xa[bt][u][2] = __builtin_amdgcn_perm(v[3], v[1], kHiHi);
-            xa[bt][u][3] = __builtin_amdgcn_perm(v[7], v[5], kHiHi);
-            if constexpr (KEEP_C) cc[bt][u] = mid_mfma<true>(xa[bt][u], neg_off, float4_t{0.f, 0.f, 0.f, 0.f});
-          }
         }
       } else {
         // ---- this wave's share of x goes out first (it is needed first, and loads retire in issue order): lane (i = c, j)
@@ -392,6 +403,51 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
         if (!PAIR || first) issue_scales(next, sp);
       };
 
+      // (float32) what the infinities and NaNs of this wave's share of x add to its sums of a chunk of rounds, from the weights with
+      // their offset taken off.  They are rare, so the tiles are read a second time and x with them, and the walk above stays as
+      // it is (tested for once per chunk).
+      auto add_infinities = [&](int r0) {
+        const int b = pass_lo + c / 3;
+        const bool ok = k_live && c < 3 * BR && b < seg_hi && c % 3 == 0;
+        const int64_t xr = p.x_one_row ? 0 : x_row(p.x_rows, p.x_src_rows, ok ? b : seg_lo);
+        const uint32_t* const xrow = reinterpret_cast<const uint32_t*>(p.x) + xr * p.K + ga * 32 + 8 * j;
+        const uint32_t keep = ok ? 0x7fffffffu : 0u;
+#pragma unroll 1
+        for (int round = 0; round < p.rounds; ++round) {
+          const int tile = tile_of(r0 + round);
+          if (tile < 0) break;
+          float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int st = 0; st < STEPS; ++st) {
+            const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_lane + 64 * st, static_cast<int>(static_cast<uint32_t>(tile) * w_tile), 0);
+            const u32x4 sv = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, ((c * p.ng + ga) + 4 * st) * 4,
+                                                                   static_cast<int>(static_cast<uint32_t>(tile) * s_tile), 0);
+            uint32_t r[4] = {t.x, t.y, t.z, t.w};
+            mid_transpose(r[0], r[1], r[2], r[3]);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+              uint32_t v[8];
+#pragma unroll
+              for (int e = 0; e < 8; ++e) {
+                const uint32_t raw = xrow[(4 * st + m) * 32 + e];
+                const uint32_t quiet = (raw & 0x7fffffu) != 0 ? raw | 0x400000u : raw;  // (a NaN's upper half is to stay a NaN)
+                v[e] = (raw & keep) >= 0x7f800000u ? quiet : 0u;
+              }
+              const mid_u4 xi = {__builtin_amdgcn_perm(v[2], v[0], kHiHi), __builtin_amdgcn_perm(v[6], v[4], kHiHi),
+                                 __builtin_amdgcn_perm(v[3], v[1], kHiHi), __builtin_amdgcn_perm(v[7], v[5], kHiHi)};
+              const uint4 w7 = word_minus7(r[m]);
+              const float4_t d = mid_mfma<true>(xi, mid_u4{w7.x, w7.y, w7.z, w7.w}, float4_t{0.f, 0.f, 0.f, 0.f});
+              const float s = __builtin_bit_cast(float, m == 0 ? sv.x : (m == 1 ? sv.y : (m == 2 ? sv.z : sv.w)));
+#pragma unroll
+              for (int q = 0; q < 4; ++q) acc[q] = d[q] != 0.f ? fmaf(s, d[q], acc[q]) : acc[q];
+            }
+          }
+          float4* const at = res_lds + (round * 16 + wave) * 64 + lane;
+          const float4 old = *at;
+          *at = make_float4(old.x + acc[0], old.y + acc[1], old.z + acc[2], old.w + acc[3]);
+        }
+      };
+
       // ---- the K shares of a tile meet: 256 values per (round, tile lane, batch tile); thread (jq, cq) takes row
       //      16 bt + jq of column cq, so that 16 neighbouring threads store 16 neighbouring columns
       auto finish = [&](int r0) __attribute__((always_inline)) {
@@ -411,7 +467,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
           } else {
             for (int k = 0; k < kw; ++k) v += res[(((round * 16 + (tl << p.kw_log2) + k) * NBT + bt) << 8) + at];
           }
-          return v;
+          return F32 ? 512.0f * v : v;
         };
         if (p.paired) {
           const int items = (p.rounds >> 1) * tw * NBT;
@@ -469,6 +525,9 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
             }
             __builtin_amdgcn_sched_barrier(0);  // (each refill stays ahead of the next tile's arithmetic)
           }
+        }
+        if constexpr (F32) {
+          if (any_odd) add_infinities(r0);  // (uniform; the sums are this wave's own until the barrier)
         }
         if (!PHASED || ph + 1 == p.phases) {  // (uniform)
           __syncthreads();

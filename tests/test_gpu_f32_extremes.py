@@ -61,17 +61,32 @@ def _check(y, x, w, k, what):
 @pytest.mark.parametrize("m,n,k,kernel", [
     (12, 70, 40, "gemm_f32_kernel<32"), (40, 130, 1544, "gemm_f32_kernel<64"), (70, 300, 1024, "gemm_f32_kernel<128"),
     (16, 128, 4096, "gemm_f32_kernel<32"),  # K split over workgroups
+    (1, 48, 14336, "midrow"), (3, 1000, 1280, "midrow"), (5, 257, 4096, "midrow"), (4, 144, 8448, "midrow"),
+    (2, 1000, 1280, "chunks=4"),  # one workgroup, whose sums meet several times
 ])
 def test_linear(kind, m, n, k, kernel):
     x, qw, qs, rng = _operands(m, n, k, m + n + k)
     KINDS[kind](x[m // 2], rng.choice(k, 2, replace=False))
-    y = ops.linear(_dev(x), _dev(qw), _dev(qs), 4, 32)
+    args = (_dev(x), _dev(qw), _dev(qs))
+    gq._lib.set_option("gemv_waves", 16 if "chunks" in kernel else -1)
+    try:
+        y = ops.linear(*args, 4, 32)
+    finally:
+        gq._lib.set_option("gemv_waves", -1)
     assert kernel in gq._lib.last_kernel(), gq._lib.last_kernel()
+    if k > 4096:  # without scratch: K in phases
+        out = torch.empty_like(y)
+        gq._lib.call("mi355gq_linear_dt", *(t.data_ptr() for t in args), None, m, n, k, 4, 32, gq._lib.F32, gq._lib.F32, out.data_ptr(),
+                     None, 0, torch.cuda.current_stream().cuda_stream)
+        assert "midrow_kernel<1,8,2,0,1" in gq._lib.last_kernel(), gq._lib.last_kernel()
+        _check(out.double().cpu().numpy(), x, o.dequantize_dt(qw, qs, S, k, "float32").astype(np.float64), k, kind)
     _check(y.double().cpu().numpy(), x, o.dequantize_dt(qw, qs, S, k, "float32").astype(np.float64), k, kind)
 
 
 @pytest.mark.parametrize("kind", KINDS)
-@pytest.mark.parametrize("experts,n,k,sizes,kernel", [(3, 144, 256, [40, 0, 33], "gemm_f32_kernel")])
+@pytest.mark.parametrize("experts,n,k,sizes,kernel", [
+    (3, 144, 256, [40, 0, 33], "gemm_f32_kernel"), (4, 48, 512, [0, 1, 6, 4], "midrow"), (4, 32, 8448, [3, 0, 2, 1], "midrow"),
+])
 def test_experts(kind, experts, n, k, sizes, kernel):
     m = sum(sizes)
     x, qw, qs, rng = _operands(m, n, k, m + n + k, experts)
@@ -83,3 +98,16 @@ def test_experts(kind, experts, n, k, sizes, kernel):
     for e in range(experts):
         w = o.dequantize_dt(qw[e], qs[e], S, k, "float32").astype(np.float64)
         _check(y[ip[e]:ip[e + 1]], x[ip[e]:ip[e + 1]], w, k, (kind, e))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_expert_per_row(kind):
+    experts, n, k = 5, 48, 8448
+    x, qw, qs, rng = _operands(3, n, k, 3, experts)
+    KINDS[kind](x[1], rng.choice(k, 2, replace=False))
+    ids = np.array([[4, 0, 4]], dtype=np.int32)
+    y = ops.moe_gemv(_dev(x), _dev(qw), _dev(qs), _dev(ids), 4, 32)
+    assert "midrow" in gq._lib.last_kernel(), gq._lib.last_kernel()
+    for i, e in enumerate(ids[0]):
+        w = o.dequantize_dt(qw[e], qs[e], S, k, "float32").astype(np.float64)
+        _check(y[i:i + 1].double().cpu().numpy(), x[i:i + 1], w, k, (kind, i))
