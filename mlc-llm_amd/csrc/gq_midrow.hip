@@ -232,16 +232,13 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
         }
       };
       mid_u4 xa[NBT][U];
-      bool any_odd = false;  // (float32, uniform) this wave's share of x holds an infinity or a NaN
       float4_t cc[KEEP_C ? NBT : 1][KEEP_C ? U : 1];
       if constexpr (F32) {
         // ---- x as three bfloat16 planes, x = h + m + l: the leading 8 bits of the significand, the next 8, the last 8
         //      (differences of float32 values that share their exponent range are exact, so the planes lose nothing).  A
         //      batch tile's matrix rows are (activation row, plane): row i of the operand is plane i % 3 of row i / 3.
-        //      An infinity has to count as zero here, because its products and their offset would be inf - inf, and so does a NaN
-        //      (add_infinities below brings both in); one of them is told by x - h, which is NaN for it, once per wave.
+        //      The products of an infinity and their offset are inf - inf: such rows are made anew in redo_odd_rows below.
         const int pl = c % 3;
-        float odd = 0.f;  // NaN: an infinity or a NaN among this lane's activations
         static_assert(!F32 || (NBT == 1 && !KEEP_C), "one batch tile, offsets from the operand");
         const int b = pass_lo + c / 3;
         const bool ok = k_live && c < 3 * BR && b < seg_hi;
@@ -254,34 +251,25 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
           hi[u] = *reinterpret_cast<const uint4*>(xrow + u * 32 + 4);
         }
         issue_all();  // (behind the loads of x: those are needed first, and loads retire in issue order)
+        // (masks: selects become branches behind the loads, which wait for all of them, the ring's included)
+        uint32_t live_x = ok ? 0xffffffffu : 0u, minus_h = pl > 0 ? 0xffff0000u : 0u, minus_m = pl > 1 ? 0xffff0000u : 0u;
+        asm volatile("" : "+v"(live_x), "+v"(minus_h), "+v"(minus_m));
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const uint32_t raw[8] = {lo[u].x, lo[u].y, lo[u].z, lo[u].w, hi[u].x, hi[u].y, hi[u].z, hi[u].w};
           uint32_t v[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const float x = __builtin_bit_cast(float, ok ? raw[e] : 0u);
-            const float h = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xffff0000u);
-            const float r1 = x - h;
-            const float m = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r1) & 0xffff0000u);
-            odd = fmaf(r1, 0.f, odd);
-            v[e] = __builtin_bit_cast(uint32_t, pl == 0 ? h : (pl == 1 ? m : r1 - m));
+            const uint32_t xb = raw[e] & live_x;
+            const float r = __builtin_bit_cast(float, xb) - __builtin_bit_cast(float, xb & minus_h);
+            const float l = r - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & minus_m);
+            v[e] = __builtin_bit_cast(uint32_t, l);
           }
           // fields (0, 2) (4, 6) (1, 3) (5, 7): the order in which the conversion delivers a word
           xa[0][u][0] = __builtin_amdgcn_perm(v[2], v[0], kHiHi);
           xa[0][u][1] = __builtin_amdgcn_perm(v[6], v[4], kHiHi);
           xa[0][u][2] = __builtin_amdgcn_perm(v[3], v[1], kHiHi);
           xa[0][u][3] = __builtin_amdgcn_perm(v[7], v[5], kHiHi);
-        }
-        any_odd = __ballot(odd != odd) != 0;
-        if (any_odd) {  // (uniform, rare; no plane of a finite activation has an exponent of all ones)
-#pragma unroll
-          for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const uint32_t v = xa[0][u][i];
-              xa[0][u][i] = ((v & 0x7f80u) == 0x7f80u ? 0u : v & 0xffffu) | ((v & 0x7f800000u) == 0x7f800000u ? 0u : v & 0xffff0000u);
-            }
         }
       } else {
         // ---- this wave's share of x goes out first (it is needed first, and loads retire in issue order): lane (i = c, j)
@@ -403,48 +391,59 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
         if (!PAIR || first) issue_scales(next, sp);
       };
 
-      // (float32) what the infinities and NaNs of this wave's share of x add to its sums of a chunk of rounds, from the weights with
-      // their offset taken off.  They are rare, so the tiles are read a second time and x with them, and the walk above stays as
-      // it is (tested for once per chunk).
-      auto add_infinities = [&](int r0) {
+      // (float32) the sums of a chunk of rounds in the rows whose shares of x hold infinities or NaNs, which are then all that
+      // counts: from the weights with their offset taken off, an infinity's products are infinities and, with a weight of zero, NaN.
+      // Rare, so the tiles are read a second time and x with them.  What calls for it is a NaN in the sums of the walk's last round, a
+      // tile past the end included: whatever the tile, the offset alone makes one.  (Tests of x ahead of the walk cost the
+      // phases 4 to 9 % of their time.)
+      auto redo_odd_rows = [&](int r0) {
+        int lane_here = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane_here));  // (what follows from it is made here, not kept in registers through the walk)
+        const int c = lane_here & 15, j = lane_here >> 4;
         const int b = pass_lo + c / 3;
-        const bool ok = k_live && c < 3 * BR && b < seg_hi && c % 3 == 0;
+        const bool ok = c < 3 * BR && b < seg_hi;
         const int64_t xr = p.x_one_row ? 0 : x_row(p.x_rows, p.x_src_rows, ok ? b : seg_lo);
-        const uint32_t* const xrow = reinterpret_cast<const uint32_t*>(p.x) + xr * p.K + ga * 32 + 8 * j;
         const uint32_t keep = ok ? 0x7fffffffu : 0u;
 #pragma unroll 1
         for (int round = 0; round < p.rounds; ++round) {
           const int tile = tile_of(r0 + round);
           if (tile < 0) break;
-          float4_t acc = {0.f, 0.f, 0.f, 0.f};
+          float4_t acc = {0.f, 0.f, 0.f, 0.f}, odd_x = {0.f, 0.f, 0.f, 0.f};  // odd_x: NaN in the rows in question
+#pragma unroll 1
+          for (int g = (static_cast<int>(blockIdx.z) * kw + ks) * U, ph2 = 0; ph2 <= ph && g < p.ng; ++ph2, g += kw * U) {
+            const uint32_t* const xrow = reinterpret_cast<const uint32_t*>(p.x) + xr * p.K + g * 32 + 8 * j;
 #pragma unroll
-          for (int st = 0; st < STEPS; ++st) {
-            const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_lane + 64 * st, static_cast<int>(static_cast<uint32_t>(tile) * w_tile), 0);
-            const u32x4 sv = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, ((c * p.ng + ga) + 4 * st) * 4,
-                                                                   static_cast<int>(static_cast<uint32_t>(tile) * s_tile), 0);
-            uint32_t r[4] = {t.x, t.y, t.z, t.w};
-            mid_transpose(r[0], r[1], r[2], r[3]);
+            for (int st = 0; st < STEPS; ++st) {
+              const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, (c * p.nw + 4 * (g + j)) * 4 + 64 * st,
+                                                                    static_cast<int>(static_cast<uint32_t>(tile) * w_tile), 0);
+              const u32x4 sv = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, (c * p.ng + g + 4 * st) * 4,
+                                                                     static_cast<int>(static_cast<uint32_t>(tile) * s_tile), 0);
+              uint32_t r[4] = {t.x, t.y, t.z, t.w};
+              mid_transpose(r[0], r[1], r[2], r[3]);
 #pragma unroll
-            for (int m = 0; m < 4; ++m) {
-              uint32_t v[8];
+              for (int m = 0; m < 4; ++m) {
+                uint32_t v[8];
 #pragma unroll
-              for (int e = 0; e < 8; ++e) {
-                const uint32_t raw = xrow[(4 * st + m) * 32 + e];
-                const uint32_t quiet = (raw & 0x7fffffu) != 0 ? raw | 0x400000u : raw;  // (a NaN's upper half is to stay a NaN)
-                v[e] = (raw & keep) >= 0x7f800000u ? quiet : 0u;
+                for (int e = 0; e < 8; ++e) {
+                  const uint32_t raw = xrow[(4 * st + m) * 32 + e];
+                  const uint32_t quiet = (raw & 0x7fffffu) != 0 ? raw | 0x400000u : raw;  // (a NaN's upper half is to stay a NaN)
+                  v[e] = (raw & keep) >= 0x7f800000u ? quiet : 0u;
+                }
+                const mid_u4 xi = {__builtin_amdgcn_perm(v[2], v[0], kHiHi), __builtin_amdgcn_perm(v[6], v[4], kHiHi),
+                                   __builtin_amdgcn_perm(v[3], v[1], kHiHi), __builtin_amdgcn_perm(v[7], v[5], kHiHi)};
+                odd_x = mid_mfma<true>(xi, mid_u4{0u, 0u, 0u, 0u}, odd_x);
+                const uint4 w7 = word_minus7(r[m]);
+                const float4_t d = mid_mfma<true>(xi, mid_u4{w7.x, w7.y, w7.z, w7.w}, float4_t{0.f, 0.f, 0.f, 0.f});
+                const float s = __builtin_bit_cast(float, m == 0 ? sv.x : (m == 1 ? sv.y : (m == 2 ? sv.z : sv.w)));
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[q] = d[q] != 0.f ? fmaf(s, d[q], acc[q]) : acc[q];
               }
-              const mid_u4 xi = {__builtin_amdgcn_perm(v[2], v[0], kHiHi), __builtin_amdgcn_perm(v[6], v[4], kHiHi),
-                                 __builtin_amdgcn_perm(v[3], v[1], kHiHi), __builtin_amdgcn_perm(v[7], v[5], kHiHi)};
-              const uint4 w7 = word_minus7(r[m]);
-              const float4_t d = mid_mfma<true>(xi, mid_u4{w7.x, w7.y, w7.z, w7.w}, float4_t{0.f, 0.f, 0.f, 0.f});
-              const float s = __builtin_bit_cast(float, m == 0 ? sv.x : (m == 1 ? sv.y : (m == 2 ? sv.z : sv.w)));
-#pragma unroll
-              for (int q = 0; q < 4; ++q) acc[q] = d[q] != 0.f ? fmaf(s, d[q], acc[q]) : acc[q];
             }
           }
-          float4* const at = res_lds + (round * 16 + wave) * 64 + lane;
-          const float4 old = *at;
-          *at = make_float4(old.x + acc[0], old.y + acc[1], old.z + acc[2], old.w + acc[3]);
+          float* const at = reinterpret_cast<float*>(res_lds + (round * 16 + wave) * 64 + lane_here);
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (odd_x[q] != odd_x[q]) at[q] = acc[q];
         }
       };
 
@@ -526,10 +525,12 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
             __builtin_amdgcn_sched_barrier(0);  // (each refill stays ahead of the next tile's arithmetic)
           }
         }
-        if constexpr (F32) {
-          if (any_odd) add_infinities(r0);  // (uniform; the sums are this wave's own until the barrier)
-        }
         if (!PHASED || ph + 1 == p.phases) {  // (uniform)
+          if constexpr (F32) {
+            const float4 last = res_lds[((p.rounds - 1) * 16 + wave) * 64 + lane];
+            const float sum = (last.x + last.y) + (last.z + last.w);
+            if (__ballot(sum != sum) != 0) redo_odd_rows(r0);  // (uniform; the sums are this wave's own until the barrier)
+          }
           __syncthreads();
           finish(r0);
           __syncthreads();  // (the next chunk, or the next pass, writes the same LDS slots)
