@@ -181,11 +181,13 @@ MI355GQ_API int mi355gq_linear_residual(const void* x, const void* q_weight, con
  * mi355gq_linear for the other model dtypes (see mi355gq_quantize_dt): x, q_scale and bias carry
  * model_dtype (MI355GQ_F32 or MI355GQ_BF16; MI355GQ_F16 forwards to mi355gq_linear), y carries
  * out_dtype = model_dtype or MI355GQ_F32.  Weights are dequantised as GroupQuantize._dequantize does
- * ((q - m) * scale rounded to the model dtype) and accumulated in fp32.  Exception: up to 8 bfloat16 rows run the
+ * ((q - m) * scale rounded to the model dtype) and accumulated in fp32.  Exceptions: up to 8 bfloat16 rows run the
  * float16 path's register GEMV / quad-row kernel, which scale each group's integer dot product in fp32 and so skip
- * that per-weight rounding (as mi355gq_linear does for float16).  No SiLU epilogue.
+ * that per-weight rounding (as mi355gq_linear does for float16); 4-bit float32 matmuls scale each group's sum of x (q - m) in
+ * fp32 likewise, one rounding per group and none per weight.  No SiLU epilogue.
  * workspace: device scratch of at least mi355gq_linear_dt_workspace_bytes(M, N, K, ...) bytes, 16-byte aligned,
- * or null (then few-row bfloat16 matmuls run unsplit: slower, same result up to summation order).
+ * or null (then matmuls that would split K, bfloat16 and float32 ones of few workgroups, run unsplit or on another kernel:
+ * slower, same result up to summation order).
  */
 /* mi355gq_linear_residual for the other model dtypes: residual [M, N] carries model_dtype (it may be y itself when
  * out_dtype == model_dtype). */

@@ -358,6 +358,19 @@ static bool f32_rows_by_gemv(int64_t M, int64_t N, int64_t K) {
   return M <= 2 && K <= 8192 && !f32_rows_by_midrow(M, N, K);
 }
 
+// Without the scratch that the GEMM's split of K wants, its few workgroups take 3.6 us + 0.55 per group whatever the rows.  Up to ten
+// rows the mid-row kernel's two passes need none (us, 8 rows, against the unsplit GEMM: 4096 x 4096 21 / 74, 28672 x 1024 20 / 22, 4096 x 14336 in
+// phases 61 / 249).  Where that kernel does not apply (K % 256 != 0), up to eight rows go in passes of two over the
+// dot-product kernel while those are shorter; a pass, fitted to 64 shapes of N 1024..32768 and K 264..8184: for K up to 4096 a start and
+// the weight stream, beyond that four groups per lane, where up to 4096 weight rows are in flight at once and more take turns.  (4 rows, passes against
+// the GEMM: 2056 x 1544 15 / 30, 20008 x 1544 29 / 31, 28680 x 1544 36 / 31, 4104 x 4104 80 / 74; 6 rows: 8208 x 1544 28 / 30, 14344 x 1544 35 / 31.)
+static bool f32_unsplit_by_gemv(int64_t M, int64_t N, int64_t K) {
+  if (M > 8 || K > 8192) return false;
+  const double k = static_cast<double>(K), nk = static_cast<double>(N) * k;
+  const double pass_us = K <= 4096 ? 3.0 + 2.4e-3 * k + 2.4e-7 * nk : N <= 4096 ? 13.4 + 1.9e-3 * k : 18.0 + 2.8e-3 * k + 5.5e-7 * nk;
+  return static_cast<double>((M + 1) / 2) * pass_us < 3.6 + 0.55 * static_cast<double>((K + 31) / 32);
+}
+
 int64_t mi355gq_linear_dt_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group_size,
                                           int model_dtype) {
   if (model_dtype == MI355GQ_F16) return mi355gq_linear_workspace_bytes(M, N, K, bits, group_size);
@@ -801,10 +814,15 @@ static int linear_dt_impl(const void* x, const void* q_weight, const void* q_sca
     g.bits = bits; g.group_size = group_size; g.out_f32 = 1;
     g.workspace = workspace; g.workspace_bytes = workspace ? workspace_bytes : 0;
     g.f32 = 1;
-    if (gv32 == 10 || (gv32 < 0 && f32_rows_by_midrow(M, N, K))) {
+    const bool lacking = gv32 < 0 && gq::gemm_f32_workspace_bytes(M, N, K) > g.workspace_bytes;  // (the GEMM would run unsplit)
+    if (gv32 == 10 || (gv32 < 0 && f32_rows_by_midrow(M, N, K)) || (lacking && M <= 10)) {
       const hipError_t e = gq::launch_midrow(g, static_cast<int>(M), as_stream(stream));
       if (e != hipErrorNotSupported) return hip_result(e, "linear_dt mid-row launch");
     }
+    if (lacking && f32_unsplit_by_gemv(M, N, K))
+      return hip_result(gq::launch_linear_dt(x, g.q_weight, q_scale, bias, residual, M, N, K, bits, group_size, model_dtype, out_dtype, y,
+                                             as_stream(stream)),
+                        "linear_dt launch");
     const hipError_t e = gq::launch_gemm_f32(g, as_stream(stream));
     if (e != hipErrorNotSupported) return hip_result(e, "linear_dt float32 gemm launch");
   }

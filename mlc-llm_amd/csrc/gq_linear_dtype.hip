@@ -494,6 +494,7 @@ hipError_t launch_dt(const LinParams& p, hipStream_t s) {
             const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kern));
             if (e != hipSuccess) return e;
           }
+          note_kernel("gq::gemv_dt_kernel<%d,%d,%d> passes=%d", BITS, DT, nb, passes);
           hipLaunchKernelGGL(kern, dim3(blocks, segments), dim3(256), lds, s, q, nsets);
           return hipGetLastError();
         };
@@ -523,6 +524,7 @@ hipError_t launch_dt(const LinParams& p, hipStream_t s) {
   // row tiles: one per one-row segment; grouped, every expert may add a partly filled one
   const int m_tiles = p.ids != nullptr ? p.M : (p.M + 127) / 128 + (p.indptr != nullptr ? p.num_experts : 0);
   if (m_tiles > 65535) return hipErrorNotSupported;
+  note_kernel("gq::gemm_dt_kernel<%d,%d>", BITS, DT);
   hipLaunchKernelGGL(kern, dim3((p.N + 127) / 128, m_tiles), dim3(256), lds, s, p);
   return hipGetLastError();
 }

@@ -109,3 +109,29 @@ def test_expert_per_row_f32(one_row):
     for i, e in enumerate(ids[0]):
         w = o.dequantize_dt(qw[e], qs[e], S, k, "float32").astype(np.float64)
         _close(y[i], x[0 if one_row else i].astype(np.float64) @ w.T, k, i)
+
+
+@pytest.mark.parametrize("m,n,k,kernel,with_scratch", [
+    (8, 130, 4096, "midrow_kernel<1,8,2,0,0,f32>", "gemm_f32"), (10, 64, 1024, "midrow_kernel<1,8,2,0,0,f32>", "gemm_f32"),
+    (6, 48, 14336, "midrow_kernel<1,8,2,0,", "gemm_f32"), (11, 130, 4096, "gemm_f32_kernel<32,128,32,32> split=1", "gemm_f32"),
+    (3, 200, 1544, "gemv_dt_kernel<4,1,2> passes=2", "gemm_f32"), (6, 1032, 4104, "gemv_dt_kernel<4,1,2> passes=3", "gemm_f32"),
+    (8, 64, 1000, "gemm_f32_kernel<32,128,32,32> split=1", "gemm_f32"), (4, 28680, 1544, "gemm_f32_kernel<32,128,32,32> split=1", "gemm_f32"),
+    (4, 4104, 4104, "gemm_f32_kernel<32,128,32,32> split=1", "gemm_f32"), (5, 40, 264, "gemm_f32", "gemm_f32"),  # (wants no scratch)
+])
+def test_linear_f32_without_scratch(m, n, k, kernel, with_scratch):
+    """Few rows whose split of K has no scratch: two passes of the mid-row kernel, passes of the dot-product kernel while they are
+    the shorter, the unsplit GEMM otherwise."""
+    x, qw, qs, rng = _case(m, n, k, m + n + k)
+    bias, res = rng.standard_normal(n).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    ref = x.astype(np.float64) @ o.dequantize_dt(qw, qs, S, k, "float32").astype(np.float64).T + bias + res
+    xd, wd, sd, bd, rd = map(_dev, (x, qw, qs, bias, res))
+    y = ops.linear(xd, wd, sd, 4, 32, bias=bd, residual=rd)
+    assert with_scratch in gq._lib.last_kernel(), gq._lib.last_kernel()
+    _close(y, ref, k, "with scratch")
+    need = gq._lib.lib().mi355gq_linear_dt_workspace_bytes(m, n, k, 4, 32, gq._lib.F32)
+    small = torch.empty(max(need - 4, 16), dtype=torch.uint8, device=DEV)
+    for ws, size in ((None, 0), (small.data_ptr(), max(need - 4, 0))):  # none, and less than asked for
+        gq._lib.call("mi355gq_linear_residual_dt", xd.data_ptr(), wd.data_ptr(), sd.data_ptr(), bd.data_ptr(), rd.data_ptr(), m, n, k, 4, 32,
+                     gq._lib.F32, gq._lib.F32, y.data_ptr(), ws, size, torch.cuda.current_stream().cuda_stream)
+        assert kernel in gq._lib.last_kernel(), gq._lib.last_kernel()
+        _close(y, ref, k, "without scratch")
