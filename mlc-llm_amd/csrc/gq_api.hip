@@ -1311,7 +1311,13 @@ static int moe_group_gemm_dt_impl(const void* x, int64_t rows, const void* q_wei
   // average, eight with few experts, on the kernel on unscaled weight operands (passes of five rows: 8 experts of 28672 x 4096
   // at 8 / 32 / 64 rows 138 / 275 / 416 us, 64 of 2816 x 2048 at 3 / 6 rows per expert 118 / 178), more on the three-plane
   // GEMM (285 / 430 / 437, 149 / 161)
-  const bool f32_gemv = 2 * rows <= num_experts && rows <= 32 && K <= 8192;
+  // Where the mid-row kernel does not apply (K % 256 != 0), the dot-product kernel's passes of two rows also stay ahead of the GEMM, whose
+  // 32-row tiles run all of K in one workgroup, while the stack is small: up to two rows per expert (K beyond 4096 one and a half) of
+  // 64 M weights in all (us, that kernel / the GEMM: 8 experts of 2816 x 1544 at 8 / 16 / 24 rows 15.5 / 31, 22 / 31, 42 / 31; 16 of 1000 x 1544 at 32
+  // rows 17 / 31; 8 of 1024 x 6152 at 12 rows 93 / 110, at 16 rows 124 / 111; 4 of 4104 x 4104, 67 M, at 4 rows 134 / 76).
+  const bool f32_gemv = rows <= 32 && K <= 8192 &&
+                        (2 * rows <= num_experts || ((K & 255) != 0 && num_experts * N * K <= (64ll << 20) &&
+                                                     (K > 4096 ? 2 * rows <= 3 * num_experts : rows <= 2 * num_experts)));
   if (f32 && bits == 4 && aligned16(x) && gq::options().gemv_variant != 0 && !(gq::options().gemv_variant < 0 && f32_gemv)) {
     gq::GemmArgs g{};
     g.x = static_cast<const uint16_t*>(x);

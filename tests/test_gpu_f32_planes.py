@@ -83,7 +83,11 @@ def test_planes_hold_every_bit_of_x():
 
 
 @pytest.mark.parametrize("experts,n,k,sizes,kernel", [
-    (4, 48, 512, [0, 1, 6, 4], "midrow"), (4, 32, 8448, [3, 0, 2, 1], "midrow"), (4, 40, 360, [3, 1, 0, 2], "gemm"),
+    (4, 48, 512, [0, 1, 6, 4], "midrow"), (4, 32, 8448, [3, 0, 2, 1], "midrow"), (4, 40, 360, [5, 3, 0, 2], "gemm"),
+    # K % 256 != 0 and up to two rows per expert (beyond K = 4096 one and a half): the dot-product kernel
+    (4, 40, 360, [3, 1, 0, 2], "gemv_dt"), (4, 40, 360, [3, 1, 0, 4], "gemv_dt"), (8, 24, 4104, [3, 1, 0, 4, 0, 2, 1, 1], "gemv_dt"),
+    (8, 24, 4104, [3, 1, 0, 4, 0, 3, 1, 1], "gemm"), (16, 1040, 4104, [1] * 9 + [0] * 7, "gemm"),  # (68 M weights)
+    (16, 1040, 4104, [1] * 8 + [0] * 8, "gemv_dt"),
     (3, 144, 256, [40, 0, 33], "gemm"), (3, 300, 1544, [130, 1, 64], "gemm"), (2, 256, 64, [200, 150], "gemm"),
 ])
 def test_experts_f32(experts, n, k, sizes, kernel):
