@@ -237,11 +237,16 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
       GemmParams head = p;
       head.bm_hint = plan.head_bm;
       head.bn_hint = plan.head_bn;
-      head.n_end = static_cast<int>(plan.n_head);
+      const bool halves = plan.halves && !a.paired;  // (the fused form's columns alternate between the halves in tile order)
+      if (halves) head.half_hi = static_cast<int>(plan.n_head / 2);
+      else head.n_end = static_cast<int>(plan.n_head);
       const hipError_t e = launch_gemm_pipe(head, a.bits, s);
       if (e != hipSuccess) return e;
       p.n_begin = head.n_end;
+      p.half_lo = head.half_hi;
+      p.half_hi = halves ? p.N / 2 : 0;
     }
+    p.part_cols = static_cast<int>(a.N - plan.n_head);
     p.bm_hint = plan.bm;
     p.bn_hint = plan.bn;
     // without (enough) scratch the same tiles run unsplit: slower, never wrong
@@ -253,7 +258,7 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
   if (a.bf16 || (variant != 3 && variant != 4 && variant != 5)) {
     const hipError_t e = launch_gemm_pipe(p, a.bits, s);
     if (e == hipSuccess && p.partial != nullptr) {
-      const int cols = p.N - p.n_begin;
+      const int cols = p.part_cols;
       const int64_t count = a.rows * cols;
       const int nk = (p.ng + 1) / 2;
       const int split = (nk + p.kt_per_split - 1) / p.kt_per_split;
@@ -265,7 +270,7 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
                            static_cast<uint16_t*>(p.y), p.bf16);
         return hipGetLastError();
       }
-      hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s,
+      hipLaunchKernelGGL((cols == p.N ? splitk_reduce_kernel<false> : splitk_reduce_kernel<true>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s,
                          p.partial, split, count, cols, p.N, p.bias, p.residual, p.y, p.out_f32, p.bf16);
       return hipGetLastError();
     }

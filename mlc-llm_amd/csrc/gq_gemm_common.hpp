@@ -31,7 +31,7 @@ struct GemmParams {
   int num_experts;
   int out_f32, indptr_i64;
   // split-K: workgroup z multiplies K tiles [z * kt_per_split, (z + 1) * kt_per_split) and, when
-  // `partial` is set, leaves its fp32 tile in partial[z][rows][N - n_begin] for the reduction kernel
+  // `partial` is set, leaves its fp32 tile in partial[z][rows][part_cols] for the reduction kernel
   float* partial;
   int kt_per_split;
   int bm_hint;  // rows, columns per tile chosen by plan_split_k (0: regular tiles)
@@ -46,11 +46,20 @@ struct GemmParams {
   int bf16;               // x, q_scale, bias and a 16-bit y are bfloat16 (q4bf16_* models), not float16
   // columns (in tile order) this launch covers: [n_begin, n_end), n_end = 0 for all; a launch can leave the columns
   // of its last, partly filled round of workgroups to a second launch with another tile
-  int n_begin = 0, n_end = 0;
+  int n_begin = 0;
+  // (set by the launcher, which knows the tile) the column tile from which on a launch of both halves of the N, below, is in the
+  // second one, and how far that one lies ahead; a launch of adjoining columns counts as all in the second
+  int hop_tile = 0, hop = 0;
+  int part_cols = 0;  // columns of this launch (the partial sums' row length)
   // every byte offset into x, one expert's q_weight and q_scale fits 32 bits, and K is whole K tiles of two groups
   // (set by the launcher; lets interior workgroups address with a uniform base plus a 32-bit lane offset)
   int fast_ok = 0;
   uint32_t x_bytes = 0;  // size of x (the form without zero-selects, whose offsets fit 32 bits)
+  int n_end = 0;
+  // columns [half_lo, half_hi) of both halves of the N of a plain matmul, half_hi = 0 for all.  Of a gate_up projection these are the
+  // columns [2 half_lo, 2 half_hi) in tile order, so that the fused form, whose launches are cut there, adds up every element in the
+  // order in which the plain matmul does.
+  int half_lo = 0, half_hi = 0;
 };
 
 // column c of the block-interleaved order above -> stored weight row (clamped into its half).
@@ -63,7 +72,8 @@ __device__ __forceinline__ int gate_up_row_blk(int c, int N) {
   return (c & PB) ? half + o : o;
 }
 
-// partial[split][count / cols][cols] -> columns [N - cols, N) of y [rows, N]
+// partial[split][count / cols][cols] -> y [rows, N]: all columns, or (HALVES, cols < N) the last cols / 2 of either half
+template <bool HALVES>
 __global__ void splitk_reduce_kernel(const float* partial, int split, int64_t count, int cols, int N,
                                      const uint16_t* bias, const uint16_t* residual, void* y, int out_f32, int bf16);
 // fused gate/up form: partial[split][rows][cols] in the block-interleaved column order -> the last cols / 2 columns of
@@ -78,8 +88,10 @@ struct SplitPlan {
   int bm, bn;        // 0: no plan, use the regular tiles
   int split;         // workgroups along K (1: no reduction pass)
   int kt_per_split;  // K tiles (2 groups each) per workgroup
-  // columns [0, n_head) run first, unsplit, as whole rounds of workgroups on a tile of their own; bm, bn and split are for the rest
+  // the first n_head columns, or the first n_head / 2 of either half, run first, unsplit, as whole rounds of workgroups on a tile of
+  // their own; bm, bn and split are for the rest
   int64_t n_head = 0;
+  bool halves = false;
   int head_bm = 0, head_bn = 0;
 };
 // scratch_bytes: what the partial sums of a split may take

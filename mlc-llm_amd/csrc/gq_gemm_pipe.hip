@@ -79,7 +79,8 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_pipe_kernel(c
   // 32-row blocks of this wave that hold rows of the segment: the others are skipped by the matrix core
   // (SKIP; a ragged expert segment or a last row tile leaves most of a tall tile empty)
   const int live = SKIP ? min(TM, max(0, (seg_hi - (m0 + wm0) + 31) / 32)) : TM;
-  const int n0 = p.n_begin + blockIdx.x * BN;
+  const bool second = static_cast<int>(blockIdx.x) >= p.hop_tile;
+  const int n0 = p.n_begin + blockIdx.x * BN + (second ? p.hop : 0);
   const uint32_t* qw = p.qw + expert * p.expert_w_stride;
   const uint16_t* qs = p.qs + expert * p.expert_s_stride;
 
@@ -458,6 +459,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_pipe_kernel(c
     return;
   }
   // (one loop nest per output form keeps each fully unrolled nest small)
+  const int n_lim = second ? p.N : p.N >> 1;  // (the launch of the first columns is whole tiles and stays below either)
   auto for_each = [&](auto&& body) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -467,15 +469,15 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_pipe_kernel(c
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int row = m0 + wm0 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-          if (row < seg_hi && col < p.N) body(row, col, acc[i][j][r]);
+          if (row < seg_hi && col < n_lim) body(row, col, acc[i][j][r]);
         }
       }
     }
   };
   if (p.partial != nullptr) {
-    const int cols = p.N - p.n_begin;
-    float* part = p.partial + static_cast<int64_t>(blockIdx.z) * p.rows * cols - p.n_begin;
-    for_each([&](int row, int col, float v) { part[static_cast<int64_t>(row) * cols + col] = v; });
+    const int part_at = second ? p.N - p.part_cols : p.n_begin;  // the column that the sums' first one would be
+    float* part = p.partial + static_cast<int64_t>(blockIdx.z) * p.rows * p.part_cols - part_at;
+    for_each([&](int row, int col, float v) { part[static_cast<int64_t>(row) * p.part_cols + col] = v; });
   } else if (p.bias == nullptr && p.residual == nullptr) {
     if (p.out_f32)
       for_each([&](int row, int col, float v) { static_cast<float*>(p.y)[static_cast<int64_t>(row) * p.N + col] = v; });
@@ -512,10 +514,23 @@ static hipError_t launch_pipe_form(const GemmParams& p, hipStream_t s) {
   const int n_cols = p.paired ? ((p.N / 2 + PB - 1) / PB) * 2 * PB : p.N;
   const int n_last = p.n_end > 0 ? p.n_end : n_cols;
   if (n_last <= p.n_begin) return hipSuccess;
-  const dim3 grid((n_last - p.n_begin + BN - 1) / BN, m_tiles, split);
-  note_kernel("gq::gemm_pipe_kernel<%d,%d,%d,%d,%d,%d,%s,%s,%d,%s>", BITS, BM, BN, WM, WN, DEPTH, BF ? "true" : "false",
-              SKIP ? "true" : "false", WX, FAST ? "true" : "false");
-  hipLaunchKernelGGL(kern, grid, dim3(64 * (BM / WM) * (BN / WN)), lds, s, p);
+  GemmParams q = p;
+  int n_tiles = (n_last - p.n_begin + BN - 1) / BN, first = p.n_begin;  // (first: columns that another launch has done)
+  if (p.half_hi > 0) {
+    q.hop_tile = (p.half_hi - p.half_lo + BN - 1) / BN;
+    q.hop = p.N / 2 - q.hop_tile * BN;
+    q.n_begin = p.half_lo;
+    n_tiles = 2 * q.hop_tile;
+    first = 2 * p.half_lo;
+  }
+  const dim3 grid(n_tiles, m_tiles, split);
+  if (first > 0)
+    note_kernel("gq::gemm_pipe_kernel<%d,%d,%d,%d,%d,%d,%s,%s,%d,%s> split=%d after %d columns", BITS, BM, BN, WM, WN, DEPTH,
+                BF ? "true" : "false", SKIP ? "true" : "false", WX, FAST ? "true" : "false", split, first);
+  else
+    note_kernel("gq::gemm_pipe_kernel<%d,%d,%d,%d,%d,%d,%s,%s,%d,%s>", BITS, BM, BN, WM, WN, DEPTH, BF ? "true" : "false",
+                SKIP ? "true" : "false", WX, FAST ? "true" : "false");
+  hipLaunchKernelGGL(kern, grid, dim3(64 * (BM / WM) * (BN / WN)), lds, s, q);
   return hipGetLastError();
 }
 
@@ -536,6 +551,7 @@ static hipError_t launch_pipe_cfg(const GemmParams& p, hipStream_t s) {
 
 // y = sum over splits of partial[s] + bias + residual, in the output type (y may be the residual
 // buffer itself: every element is read before the same thread writes it)
+template <bool HALVES>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ partial, int split,
                                                             int64_t count /* rows * cols */, int cols, int N,
                                                             const uint16_t* __restrict__ bias,
@@ -545,8 +561,13 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   auto out = [bf16](float v) { return bf16 ? f2bf(v) : f2h(v); };
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   // element i of the sums -> element of y
-  auto at = [&](int64_t i) -> int64_t { return cols == N ? i : (i / cols) * N + (N - cols) + i % cols; };
-  if (((N | cols) & 3) == 0) {  // rows are 16-byte aligned: four columns per thread
+  const int w = cols >> 1, half = N >> 1;
+  auto at = [&](int64_t i) -> int64_t {
+    if (!HALVES) return i;
+    const int c = static_cast<int>(i % cols);
+    return (i / cols) * N + (c < w ? half - w + c : N - w + (c - w));
+  };
+  if (((N | (HALVES ? cols : 0)) & (HALVES ? 7 : 3)) == 0) {  // runs of columns are 16-byte aligned: four per thread
     for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; 4 * i < count; i += stride) {
       float4 a = *reinterpret_cast<const float4*>(partial + 4 * i);
       for (int sidx = 1; sidx < split; ++sidx) {
@@ -586,6 +607,11 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     }
   }
 }
+
+template __global__ void splitk_reduce_kernel<false>(const float* __restrict__, int, int64_t, int, int, const uint16_t* __restrict__, const uint16_t*,
+                                                    void*, int, int);
+template __global__ void splitk_reduce_kernel<true>(const float* __restrict__, int, int64_t, int, int, const uint16_t* __restrict__, const uint16_t*,
+                                                   void*, int, int);
 
 __global__ __launch_bounds__(256) void splitk_reduce_silu_kernel(const float* __restrict__ partial, int split,
                                                                  int64_t rows, int cols, int N, int pb,
@@ -642,8 +668,11 @@ constexpr TileCost kTilesBf16[] = {  // (more vector instructions per weight: th
     {64, 128, 0, 6.81f, 0.507f, 0.338f, 0.128f, 0, 0.183f, 1.99f, 0.916f, 0.339f},
 };
 
-static float tile_us(const TileCost& c, int64_t rows, int64_t N, int nk, int kt, int split) {
-  const int64_t mt = (rows + c.bm - 1) / c.bm, wgs = mt * ((N + c.bn - 1) / c.bn) * split, rounds = (wgs + 255) / 256;
+// tiles of `bn` columns that N columns take, in one run of columns or in two of half of them
+static int64_t column_tiles(int64_t N, int bn, int runs) { return runs * ((N / runs + bn - 1) / bn); }
+
+static float tile_us(const TileCost& c, int64_t rows, int64_t N, int nk, int kt, int split, int runs) {
+  const int64_t mt = (rows + c.bm - 1) / c.bm, wgs = mt * column_tiles(N, c.bn, runs) * split, rounds = (wgs + 255) / 256;
   const float live = static_cast<float>(rows) / static_cast<float>(mt * c.bm), mn = 1e-6f * static_cast<float>(rows) * static_cast<float>(N);
   const bool pairs = c.bm * c.bn <= 128 * 128;  // (four waves: two workgroups on a CU)
   const float ktf = static_cast<float>(split > 1 ? kt : (nk + 3) / 4 * 4), per_cu = static_cast<float>(wgs) / 256.f;
@@ -655,13 +684,13 @@ static float tile_us(const TileCost& c, int64_t rows, int64_t N, int nk, int kt,
 }
 static bool tile_applies(const TileCost& c, int64_t rows) { return c.bm < 256 || (c.skip != 0) == (c.bn == 128 || rows % 256 != 0); }
 
-// one launch for all columns
-static SplitPlan plan_one(const TileCost* costs, int64_t rows, int64_t N, int nk, int64_t scratch_bytes, float* best_us) {
+// one launch for all of N columns
+static SplitPlan plan_one(const TileCost* costs, int64_t rows, int64_t N, int nk, int64_t scratch_bytes, int runs, float* best_us) {
   SplitPlan best{0, 0, 1, 1 << 28};
   for (int t = 0; t < 6; ++t) {
     const TileCost& c = costs[t];
     if (!tile_applies(c, rows)) continue;
-    const int64_t tiles = ((rows + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    const int64_t tiles = ((rows + c.bm - 1) / c.bm) * column_tiles(N, c.bn, runs);
     int last = 0;
     for (int want = 1; want <= 16; ++want) {
       const int kt = ((nk + want - 1) / want + 3) / 4 * 4;  // (the K loop advances four tiles at a time)
@@ -670,7 +699,7 @@ static SplitPlan plan_one(const TileCost* costs, int64_t rows, int64_t N, int nk
       if (split > 1 && (want > nk / 4 || tiles * split > 640 || split * rows * N * 4 > scratch_bytes)) break;
       if (split == last) continue;
       last = split;
-      const float us = tile_us(c, rows, N, nk, kt, split);
+      const float us = tile_us(c, rows, N, nk, kt, split, runs);
       if (best.bm == 0 || us < *best_us) {
         *best_us = us;
         best = SplitPlan{c.bm, c.bn, split, split > 1 ? kt : 1 << 28};
@@ -685,27 +714,35 @@ static SplitPlan plan_one(const TileCost* costs, int64_t rows, int64_t N, int nk
 // (it is some 5 % too optimistic about two launches).  Measured (us, one launch -> two): 6144 x 4096 at 2700 rows 181 -> 147, 22016 x 4096 at
 // 1536 326 -> 268, 10240 x 8192 at 2048 377 -> 329, 15360 x 5120 at 1200 230 -> 205, 37888 x 3584 at 450 164 -> 145; 28672 x 4096 at 2048 (3.5
 // rounds) within the noise either way, and left alone by the 7 %.
+// A rest that splits K takes the same columns of both halves of the N (runs = 2): of a gate_up projection those are whole pairs, as
+// the fused form needs them, and either form then adds up an element in the same order.  Unsplit, the order is the same everywhere and the
+// columns adjoin.  (The model puts this 0.1 % behind a rest of adjoining columns that may split.)
 static SplitPlan plan_by_cost(int64_t rows, int64_t N, int nk, int bf16, int64_t scratch_bytes) {
   if (scratch_bytes > kMaxSplitBytes) scratch_bytes = kMaxSplitBytes;
   const TileCost* const costs = bf16 ? kTilesBf16 : kTilesF16;
   float one_us = 0.f;
-  SplitPlan best = plan_one(costs, rows, N, nk, scratch_bytes, &one_us);
+  SplitPlan best = plan_one(costs, rows, N, nk, scratch_bytes, 1, &one_us);
   float best_us = one_us / 1.07f;
   for (int t = 1; t <= 4; ++t) {  // (the tiles of one workgroup per CU)
     const TileCost& c = costs[t];
-    const int64_t mt = (rows + c.bm - 1) / c.bm, nt = (N + c.bn - 1) / c.bn, head = mt * nt / 256 * 256 / mt;  // column tiles of the whole rounds
-    if (!tile_applies(c, rows) || head < 1 || head >= nt) continue;
-    const int64_t n_head = head * c.bn;
-    const float head_us = tile_us(c, rows, n_head, nk, 0, 1) - 3.f;  // (its launch overlaps the other's)
-    if (head_us >= best_us) continue;
-    float rest_us = 0.f;
-    SplitPlan rest = plan_one(costs, rows, N - n_head, nk, scratch_bytes, &rest_us);
-    if (head_us + rest_us < best_us) {
-      best_us = head_us + rest_us;
-      best = rest;
-      best.n_head = n_head;
-      best.head_bm = c.bm;
-      best.head_bn = c.bn;
+    if (!tile_applies(c, rows)) continue;
+    const int64_t mt = (rows + c.bm - 1) / c.bm;
+    for (int runs = 1; runs <= (N % 2 == 0 ? 2 : 1); ++runs) {
+      const int64_t nt = column_tiles(N, c.bn, runs), head = mt * nt / 256 * 256 / mt / runs * runs;  // column tiles of the whole rounds
+      if (head < 1 || head >= nt) continue;
+      const int64_t n_head = head * c.bn;
+      const float head_us = tile_us(c, rows, n_head, nk, 0, 1, runs) - 3.f;  // (its launch overlaps the other's)
+      if (head_us >= best_us) continue;
+      float rest_us = 0.f;
+      SplitPlan rest = plan_one(costs, rows, N - n_head, nk, runs == 2 ? scratch_bytes : 0, runs, &rest_us);
+      if (head_us + rest_us < best_us) {
+        best_us = head_us + rest_us;
+        best = rest;
+        best.n_head = n_head;
+        best.halves = runs == 2;
+        best.head_bm = c.bm;
+        best.head_bn = c.bn;
+      }
     }
   }
   return best;

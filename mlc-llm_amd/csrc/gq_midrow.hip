@@ -697,7 +697,7 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
                        static_cast<uint16_t*>(a.y), a.bf16);
   } else {
     const int64_t blocks = ((p.N & 3) == 0 ? (count / 4 + 255) / 256 : (count + 255) / 256);
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>(blocks > 4096 ? 4096 : blocks)), dim3(256), 0, s,
+    hipLaunchKernelGGL(splitk_reduce_kernel<false>, dim3(static_cast<unsigned>(blocks > 4096 ? 4096 : blocks)), dim3(256), 0, s,
                        static_cast<const float*>(a.workspace), p.slices, count, p.N, p.N, a.bias, a.residual, a.y, a.out_f32, a.bf16);
   }
   return hipGetLastError();
