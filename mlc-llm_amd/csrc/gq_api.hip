@@ -398,10 +398,10 @@ int64_t mi355gq_linear_silu_mul_workspace_bytes(int64_t M, int64_t N, int64_t K,
   const int64_t mid = (bits == 4 && M <= 32 && (M > 8 || (M > 4 && K > 8192)) && (N % 32) == 0)
                           ? gq::midrow_workspace_bytes(M, N, K)
                           : 0;
-  // GEMV / few-row kernels, or a shape that never splits
-  if (M <= 8 || (N % 64) != 0) return mid;
-  if (M <= 16 && !(bits == 4 && N * K >= (40ll << 20) && N * K < (256ll << 20))) return mid;
-  const int64_t gemm = gq::gemm_workspace_bytes(M, N, K, bits, group_size);
+  // GEMV / few-row kernels
+  if (M <= 8 || (N % 2) != 0) return mid;
+  if (M <= 16 && bits == 4 && !(N * K >= (40ll << 20) && N * K < (256ll << 20))) return mid;
+  const int64_t gemm = gq::gemm_workspace_bytes(M, N, K, bits, group_size, 0, 1);
   return gemm > mid ? gemm : mid;
 }
 
@@ -454,7 +454,7 @@ static int linear_impl(const void* x, const void* q_weight, const void* q_scale,
   bool q4_skinny_loses = false;
   if (bits == 4 && M > 8 && M <= 16 && gq::options().gemv_variant < 0 && (K & 7) == 0 && N * K >= (40ll << 20) &&
       N * K < (256ll << 20)) {
-    const int64_t need = gq::gemm_workspace_bytes(M, N, K, bits, group_size);
+    const int64_t need = gq::gemm_workspace_bytes(M, N, K, bits, group_size, 0, paired);
     q4_skinny_loses = need == 0 || (workspace != nullptr && workspace_bytes >= need);
   }
   // q4, 9..16 rows of a K that one phase covers (up to 4096; two phases: below), from about 24 M weights on: the kernel that multiplies
@@ -935,15 +935,14 @@ int mi355gq_linear_dt(const void* x, const void* q_weight, const void* q_scale, 
 int64_t mi355gq_linear_silu_mul_dt_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group_size,
                                                    int model_dtype) {
   if (model_dtype == MI355GQ_F16) return mi355gq_linear_silu_mul_workspace_bytes(M, N, K, bits, group_size);
-  // (the GEMM's partial sums of the fused form need whole 32 + 32 column blocks; the K slices of the kernel on unscaled
-  //  weight operands, 9..16 rows, do not)
-  if ((N % 64) != 0)
-    return (model_dtype == MI355GQ_BF16 && check_scheme(bits, group_size) == MI355GQ_OK && bits == 4 && M <= 16 &&
-            (M > 8 || (M > 4 && K > 8192)) &&
-            N > 0 && K > 0 && N < kMaxDim && K < kMaxDim && (N % 32) == 0)
-               ? gq::midrow_workspace_bytes(M, N, K)
-               : 0;
-  return mi355gq_linear_dt_workspace_bytes(M, N, K, bits, group_size, model_dtype);
+  // bfloat16, as the plain linear (the kernel on unscaled weight operands takes whole 32-row blocks of the fused form); there
+  // is no fused form of float32 models
+  if (model_dtype != MI355GQ_BF16 || check_scheme(bits, group_size) != MI355GQ_OK || M < 2 || N < 0 || K < 0 || M >= kMaxDim ||
+      N >= kMaxDim || K >= kMaxDim || (N % 2) != 0)
+    return 0;
+  const int64_t mid = (bits == 4 && M <= 16 && (M > 8 || (M > 4 && K > 8192)) && (N % 32) == 0) ? gq::midrow_workspace_bytes(M, N, K) : 0;
+  const int64_t gemm = gq::gemm_workspace_bytes(M, N, K, bits, group_size, 1, 1);
+  return gemm > mid ? gemm : mid;
 }
 
 int mi355gq_linear_silu_mul_dt(const void* x, const void* q_weight, const void* q_scale, int64_t M, int64_t N,

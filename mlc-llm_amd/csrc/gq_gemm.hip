@@ -198,6 +198,13 @@ static hipError_t launch_cfg(const GemmParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Columns of the partial sums behind the ones that run first.  The fused gate/up form keeps them in the tile's order, whole blocks of
+// gate and up columns, the last one filled up.
+static int64_t partial_columns(const SplitPlan& plan, int64_t N, int paired) {
+  const int64_t pb = pair_block(plan.bm);
+  return (paired ? (N / 2 + pb - 1) / pb * 2 * pb : N) - plan.n_head;
+}
+
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
   GemmParams p;
   p.x = a.x; p.qw = a.q_weight; p.qs = a.q_scale; p.bias = a.bias; p.residual = a.residual; p.y = a.y;
@@ -227,10 +234,7 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
   if (a.rows == 0 || a.N == 0) return hipSuccess;
   const int variant = options().gemm_variant;
   {
-    // (fused gate/up form: the partial sums keep the tile's column order, which only lines up with
-    //  rows of N floats when the gate half is whole 32-row blocks)
-    const bool may_split = (variant < 0 || a.bf16) && a.workspace != nullptr && (reinterpret_cast<uintptr_t>(a.workspace) & 15) == 0 &&
-                           (!a.paired || (a.N % 64) == 0);
+    const bool may_split = (variant < 0 || a.bf16) && a.workspace != nullptr && (reinterpret_cast<uintptr_t>(a.workspace) & 15) == 0;
     const int64_t scratch = may_split ? a.workspace_bytes : 0;
     const SplitPlan plan = plan_split_k(a.rows, a.N, a.K, a.bits, a.group_size, a.indptr != nullptr, a.bf16, scratch);
     if (plan.n_head > 0 && (variant < 0 || a.bf16)) {
@@ -246,11 +250,11 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
       p.half_lo = head.half_hi;
       p.half_hi = halves ? p.N / 2 : 0;
     }
-    p.part_cols = static_cast<int>(a.N - plan.n_head);
+    p.part_cols = static_cast<int>(partial_columns(plan, a.N, a.paired));
     p.bm_hint = plan.bm;
     p.bn_hint = plan.bn;
     // without (enough) scratch the same tiles run unsplit: slower, never wrong
-    if (plan.bm > 0 && plan.split > 1 && scratch >= static_cast<int64_t>(plan.split) * a.rows * (a.N - plan.n_head) * 4) {
+    if (plan.bm > 0 && plan.split > 1 && scratch >= static_cast<int64_t>(plan.split) * a.rows * p.part_cols * 4) {
       p.partial = static_cast<float*>(a.workspace);
       p.kt_per_split = plan.kt_per_split;
     }
@@ -266,7 +270,7 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
       blocks = blocks < 1 ? 1 : (blocks > 2048 ? 2048 : blocks);
       if (p.paired) {
         hipLaunchKernelGGL(splitk_reduce_silu_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s,
-                           p.partial, split, a.rows, cols, p.N, gemm_pipe_pair_block(p, a.bits),
+                           p.partial, split, a.rows, cols, p.N, p.n_begin, pair_block(p.bm_hint),
                            static_cast<uint16_t*>(p.y), p.bf16);
         return hipGetLastError();
       }
@@ -288,10 +292,10 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
   return launch_cfg<3, 128, 128, 64, 64>(p, s);
 }
 
-int64_t gemm_workspace_bytes(int64_t rows, int64_t N, int64_t K, int bits, int group_size, int bf16) {
+int64_t gemm_workspace_bytes(int64_t rows, int64_t N, int64_t K, int bits, int group_size, int bf16, int paired) {
   if (options().gemm_variant >= 0) return 0;
   const SplitPlan plan = plan_split_k(rows, N, K, bits, group_size, false, bf16, kMaxSplitBytes);
-  return plan.bm > 0 && plan.split > 1 ? static_cast<int64_t>(plan.split) * rows * (N - plan.n_head) * 4 : 0;
+  return plan.bm > 0 && plan.split > 1 ? static_cast<int64_t>(plan.split) * rows * partial_columns(plan, N, paired) * 4 : 0;
 }
 
 }  // namespace gq

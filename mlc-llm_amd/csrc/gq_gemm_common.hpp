@@ -76,12 +76,12 @@ __device__ __forceinline__ int gate_up_row_blk(int c, int N) {
 template <bool HALVES>
 __global__ void splitk_reduce_kernel(const float* partial, int split, int64_t count, int cols, int N,
                                      const uint16_t* bias, const uint16_t* residual, void* y, int out_f32, int bf16);
-// fused gate/up form: partial[split][rows][cols] in the block-interleaved column order -> the last cols / 2 columns of
-// y [rows, N / 2]
-__global__ void splitk_reduce_silu_kernel(const float* partial, int split, int64_t rows, int cols, int N, int pb,
+// fused gate/up form: partial[split][rows][cols] in the block-interleaved column order (its last block filled up) -> the columns of
+// y [rows, N / 2] from n_begin / 2 on
+__global__ void splitk_reduce_silu_kernel(const float* partial, int split, int64_t rows, int cols, int N, int n_begin, int pb,
                                           uint16_t* y, int bf16);
-// gate rows per column block (32 | 16) of the tile launch_gemm_pipe picks for these parameters
-int gemm_pipe_pair_block(const GemmParams& p, int bits);
+// gate rows per column block of the tile planned for a matmul: 16 in the one of 32 rows, whose waves own a single accumulator, else 32
+constexpr int pair_block(int bm) { return bm == 32 ? 16 : 32; }
 
 // How a plain GEMM is cut: its tile and K splits.
 struct SplitPlan {

@@ -459,7 +459,8 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_pipe_kernel(c
     return;
   }
   // (one loop nest per output form keeps each fully unrolled nest small)
-  const int n_lim = second ? p.N : p.N >> 1;  // (the launch of the first columns is whole tiles and stays below either)
+  // (a launch of the first columns is whole tiles and stays below any of these; the fused form comes here with partial sums only)
+  const int n_lim = p.paired ? p.n_begin + p.part_cols : (second ? p.N : p.N >> 1);
   auto for_each = [&](auto&& body) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -475,7 +476,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_pipe_kernel(c
     }
   };
   if (p.partial != nullptr) {
-    const int part_at = second ? p.N - p.part_cols : p.n_begin;  // the column that the sums' first one would be
+    const int part_at = second && !p.paired ? p.N - p.part_cols : p.n_begin;  // the column that the sums' first one would be
     float* part = p.partial + static_cast<int64_t>(blockIdx.z) * p.rows * p.part_cols - part_at;
     for_each([&](int row, int col, float v) { part[static_cast<int64_t>(row) * p.part_cols + col] = v; });
   } else if (p.bias == nullptr && p.residual == nullptr) {
@@ -614,9 +615,9 @@ template __global__ void splitk_reduce_kernel<true>(const float* __restrict__, i
                                                    void*, int, int);
 
 __global__ __launch_bounds__(256) void splitk_reduce_silu_kernel(const float* __restrict__ partial, int split,
-                                                                 int64_t rows, int cols, int N, int pb,
+                                                                 int64_t rows, int cols, int N, int n_begin, int pb,
                                                                  uint16_t* __restrict__ y, int bf16) {
-  const int half = cols >> 1;
+  const int half = (N - n_begin) >> 1;
   const int64_t count = rows * cols, outs = rows * half;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < outs; i += stride) {
@@ -628,7 +629,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_silu_kernel(const float* __
       g += partial[sidx * count + at];
       u += partial[sidx * count + at + pb];
     }
-    y[row * (N >> 1) + ((N - cols) >> 1) + oc] = bf16 ? silu_mul_bf(g, u) : silu_mul_h(g, u);
+    y[row * (N >> 1) + (n_begin >> 1) + oc] = bf16 ? silu_mul_bf(g, u) : silu_mul_h(g, u);
   }
 }
 
@@ -711,12 +712,13 @@ static SplitPlan plan_one(const TileCost* costs, int64_t rows, int64_t N, int nk
 
 // ... or two: a last round of workgroups that is far from full costs about what a full one does, so the columns of the whole rounds run
 // first on one of the large tiles and the rest on whatever suits it (a smaller tile, K split).  Taken where the model puts it 7 % ahead
-// (it is some 5 % too optimistic about two launches).  Measured (us, one launch -> two): 6144 x 4096 at 2700 rows 181 -> 147, 22016 x 4096 at
-// 1536 326 -> 268, 10240 x 8192 at 2048 377 -> 329, 15360 x 5120 at 1200 230 -> 205, 37888 x 3584 at 450 164 -> 145; 28672 x 4096 at 2048 (3.5
+// (it is some 5 % too optimistic about two launches).  Measured (us, one launch -> two): 6144 x 4096 at 2700 rows 181 -> 153, 22016 x 4096 at
+// 1536 326 -> 275, 10240 x 8192 at 2048 377 -> 327, 15360 x 5120 at 1200 230 -> 205, 37888 x 3584 at 450 164 -> 145; 28672 x 4096 at 2048 (3.5
 // rounds) within the noise either way, and left alone by the 7 %.
 // A rest that splits K takes the same columns of both halves of the N (runs = 2): of a gate_up projection those are whole pairs, as
 // the fused form needs them, and either form then adds up an element in the same order.  Unsplit, the order is the same everywhere and the
-// columns adjoin.  (The model puts this 0.1 % behind a rest of adjoining columns that may split.)
+// columns adjoin.  (The model puts this 0.1 % behind a rest of adjoining columns that may split: 9 % where none of the split fits two
+// halves, 5120 x 13824 at 3107 rows 419 -> 456, and mostly nothing, 22016 x 4096 at 380 rows 89.0 -> 87.6.)
 static SplitPlan plan_by_cost(int64_t rows, int64_t N, int nk, int bf16, int64_t scratch_bytes) {
   if (scratch_bytes > kMaxSplitBytes) scratch_bytes = kMaxSplitBytes;
   const TileCost* const costs = bf16 ? kTilesBf16 : kTilesF16;
@@ -781,10 +783,6 @@ SplitPlan plan_split_k(int64_t rows, int64_t N, int64_t K, int bits, int group_s
   plan.kt_per_split = ((nk + split - 1) / split + 3) / 4 * 4;
   plan.split = (nk + plan.kt_per_split - 1) / plan.kt_per_split;
   return plan;
-}
-
-int gemm_pipe_pair_block(const GemmParams& p, int bits) {
-  return p.bm_hint == 32 ? 16 : 32;  // the 32 x 128 tile below
 }
 
 // q3: 128 x 256 tiles rather than 128 x 128 (a K tile is 80 wide and the 256 x 256 tile does not fit LDS)?  A launch costs rounds x

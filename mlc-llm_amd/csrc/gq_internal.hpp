@@ -116,8 +116,8 @@ struct GemmArgs {
   int x_one_row = 0;                    //   when x_one_row is set, row i otherwise
 };
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t s);
-// scratch the split-K form of the GEMM wants for this shape (0 when it does not split)
-int64_t gemm_workspace_bytes(int64_t rows, int64_t N, int64_t K, int bits, int group_size, int bf16 = 0);
+// scratch the split-K form of the GEMM wants for this shape (0 when it does not split); paired: the fused gate/up form
+int64_t gemm_workspace_bytes(int64_t rows, int64_t N, int64_t K, int bits, int group_size, int bf16 = 0, int paired = 0);
 // MFMA kernel for few activation rows per segment (q4 only; hipErrorNotSupported otherwise).
 // rows_max bounds the rows of any one segment.
 hipError_t launch_skinny(const GemmArgs& a, int rows_max, hipStream_t s);

@@ -54,7 +54,7 @@ def test_planned_tiles(dtype, m, n, k, tile, split):
                  ops._MODEL_DTYPES[dtype], ops._MODEL_DTYPES[dtype], out.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream)
     full = want + bias.double()
     assert (out.double() - full).norm() / full.norm() <= tol, gq._lib.last_kernel()
-    if n % 64 == 0:  # the fused gate/up form adds in the same order: the same bits as the two steps
+    if n % 2 == 0:  # the fused gate/up form adds in the same order: the same bits as the two steps
         assert torch.equal(ops.linear_silu_mul(x, qw, qs, 4, 32), ops.silu_mul(ops.linear(x, qw, qs, 4, 32)))
 
 
@@ -91,3 +91,23 @@ def test_fused_form_of_two_launches_adds_in_the_same_order(dtype, m, n, k, secon
     fused = gq._lib.native().linear_silu_mul(x, qw, qs, 4, 32)
     assert isinstance(fused, torch.Tensor) and second in gq._lib.last_kernel(), gq._lib.last_kernel()
     assert torch.equal(fused, steps)
+
+
+@pytest.mark.parametrize("bits", [4, 3])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [
+    (4000, 8208, 1544), (1000, 8208, 1544),  # two launches, the second split
+    (129, 2064, 4096), (300, 4098, 2048), (70, 130, 4096),  # split; halves that are no multiple of 32, odd ones
+    (40, 8208, 1544), (64, 66, 4096), (33, 4112, 1000), (20, 72, 4096), (17, 4110, 2048), (32, 34, 1024),  # tiles of 64 and 32 rows
+    (12, 16400, 4096), (9, 2064, 4096), (200, 8208, 1544), (300, 2, 4096),
+])
+def test_fused_form_of_any_half_adds_in_the_same_order(bits, dtype, m, n, k):
+    """linear_silu_mul equals linear and silu_mul bit for bit also where the halves are not whole 32-column blocks and K is split."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    group = {4: 32, 3: 40}[bits]
+    qw, qs = ops.quantize((torch.randn((n, k), generator=g, device="cuda") * 0.02).to(dtype), bits, group)
+    x = torch.randn((m, k), generator=g, device="cuda").to(dtype)
+    steps = ops.silu_mul(ops.linear(x, qw, qs, bits, group))
+    fused = gq._lib.native().linear_silu_mul(x, qw, qs, bits, group)
+    assert isinstance(fused, torch.Tensor), fused
+    assert torch.equal(fused, steps), gq._lib.last_kernel()

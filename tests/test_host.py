@@ -124,7 +124,9 @@ def test_argument_validation_of_the_later_entry_points():
                                           None) == -1
     assert lib.mi355gq_moe_gemv_silu_mul_dt(P(0x1000), 1, P(0x2000), P(0x3000), P(0x4000), 2, 8, 16, 32, 4, 32, 1,
                                             P(0x5000), None) == _lib.ERR_UNSUPPORTED
-    assert lib.mi355gq_linear_silu_mul_dt_workspace_bytes(40, 100, 4096, 4, 32, 2) == 0  # N % 64 != 0
+    # K split eight ways as in the plain linear; halves of 50 columns, in blocks of 32 + 32 filled up
+    assert lib.mi355gq_linear_silu_mul_dt_workspace_bytes(40, 100, 4096, 4, 32, 2) == 8 * 40 * 128 * 4
+    assert lib.mi355gq_linear_dt_workspace_bytes(40, 100, 4096, 4, 32, 2) == 8 * 40 * 100 * 4
     assert lib.mi355gq_linear_silu_mul_dt_workspace_bytes(40, 128, 4096, 4, 32, 2) > 0
     # routing glue in the other model dtypes
     assert lib.mi355gq_gating_softmax_topk_dt(P(0x1000), 4, 8, 9, P(0x2000), P(0x3000), 2, None) == -1
