@@ -1,6 +1,7 @@
 """Build libmi355gq.so (gfx950 code only) with hipcc and _mi355gq_torch.so (host code only) with g++, in tree.
 
-    python mlc-llm_amd/build.py            # compile every csrc/*.hip and link lib/libmi355gq.so, then csrc/gq_torch.cc
+    python mlc-llm_amd/build.py            # compile every csrc/*.hip and link lib/libmi355gq.so, then
+                                           # csrc/gq_torch.cc where torch and g++ are there
 
 The TVM-FFI adapter (csrc/tvm_ffi_adapter.cc) is compiled in only when the
 `tvm_ffi` Python package (which ships tvm/ffi/c_api.h) is importable.
@@ -67,15 +68,23 @@ def _compile(src: str, extra: list[str]) -> str:
     return obj
 
 
-def _build_torch_ext() -> None:
-    """The native call path of the dense operators: a Python extension module on torch's C++ interface, linked to the library."""
-    import torch
-
+def build_torch_ext() -> str | None:
+    """The native call path of the dense operators: a Python extension module on torch's C++ interface, linked to the library.
+    None where torch or g++ is missing: the Python route then does without it (and one of an earlier build is taken away)."""
+    gxx = shutil.which("g++")
+    try:
+        import torch
+    except ImportError:
+        torch = None
+    if gxx is None or torch is None:
+        if os.path.exists(TORCH_EXT):
+            os.remove(TORCH_EXT)
+        return None
     root = os.path.dirname(torch.__file__)
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
     includes = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
                 os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
-    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+    cmd = [gxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *(f for i in includes for f in ("-isystem", i)), os.path.join(CSRC, "gq_torch.cc"), "-o", TORCH_EXT,
            "-L" + os.path.join(root, "lib"), "-L" + LIBDIR, "-l:libmi355gq.so", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip",
@@ -83,6 +92,7 @@ def _build_torch_ext() -> None:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"g++ failed for gq_torch.cc:\n{r.stdout}\n{r.stderr}")
+    return TORCH_EXT
 
 
 def build(verbose: bool = True) -> str:
@@ -102,9 +112,11 @@ def build(verbose: bool = True) -> str:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
-    _build_torch_ext()
     if verbose:
         print(f"built {LIB} from {len(objs)} objects" + (" (+tvm_ffi adapter)" if ffi_inc else ""))
+    ext = build_torch_ext()
+    if verbose:
+        print(f"built {ext}" if ext else "torch or g++ is missing: without the native call path of the dense operators")
     return LIB
 
 

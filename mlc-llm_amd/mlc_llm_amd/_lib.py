@@ -1,7 +1,7 @@
 """ctypes binding of libmi355gq.so (the C ABI declared in include/mi355gq.h), and the native call path of the dense
-operators beside it (_mi355gq_torch.so, csrc/gq_torch.cc).
+operators beside it (_mi355gq_torch.so, csrc/gq_torch.cc), which only saves interpreter time.
 
-There is no fallback: if the shared library is missing or a call fails, an
+There is no fallback for the library: if it is missing or a call fails, an
 exception is raised.  Tensors are torch tensors on the ROCm device; only their
 `data_ptr()` and the current HIP stream cross the boundary.
 """
@@ -13,6 +13,7 @@ import importlib.machinery
 import importlib.util
 import os
 import re
+import warnings
 from ctypes import c_char_p, c_int, c_int64, c_void_p
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -139,17 +140,20 @@ def lib() -> ctypes.CDLL:
 
 
 def native():
-    """The native call path of the dense operators (loaded once).  Raises if it has not been built."""
+    """The native call path of the dense operators (loaded once), or None where it was not built (no torch or g++ at build time)
+    or does not fit this torch, which is warned of once: the Python route makes the same calls of the C ABI."""
     global _TORCH
     if _TORCH is None:
         lib()  # the library it is linked to
-        if not os.path.exists(TORCH_PATH):
-            raise RuntimeError(f"{TORCH_PATH} is missing: build it with `python mlc-llm_amd/build.py`")
-        loader = importlib.machinery.ExtensionFileLoader("_mi355gq_torch", TORCH_PATH)
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_mi355gq_torch", loader))
-        loader.exec_module(module)
-        _TORCH = module
-    return _TORCH
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("_mi355gq_torch", TORCH_PATH)
+            _TORCH = importlib.util.module_from_spec(importlib.util.spec_from_loader("_mi355gq_torch", loader))
+            loader.exec_module(_TORCH)
+        except ImportError as err:
+            _TORCH = False
+            warnings.warn(f"dense operators take the slower Python route: {err} (python mlc-llm_amd/build.py builds the module)",
+                          RuntimeWarning, stacklevel=2)
+    return _TORCH or None
 
 
 def failed(name: str, rc: int) -> "Mi355gqError":

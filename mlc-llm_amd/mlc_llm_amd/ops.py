@@ -19,7 +19,8 @@ from . import _lib
 
 
 def _stream() -> int:
-    return _lib.native().stream()
+    native = _lib.native()
+    return native.stream() if native is not None else torch.cuda.current_stream().cuda_stream
 
 
 def _chk(t: torch.Tensor, dtype, name: str) -> torch.Tensor:
@@ -98,7 +99,8 @@ def _check_qshapes(q_weight, q_scale, lead, k, bits, group_size):
 
 def embedding_take(ids: torch.Tensor, q_weight: torch.Tensor, q_scale: torch.Tensor, k: int,
                    bits: int, group_size: int) -> torch.Tensor:
-    done = _lib.native().embedding_take(ids, q_weight, q_scale, k, bits, group_size)
+    native = _lib.native()
+    done = native.embedding_take(ids, q_weight, q_scale, k, bits, group_size) if native is not None else None
     if isinstance(done, torch.Tensor):
         return done
     if done is not None:
@@ -126,7 +128,8 @@ def linear(x: torch.Tensor, q_weight: torch.Tensor, q_scale: torch.Tensor, bits:
 
     `residual` (fp16, the shape of y) is added inside the kernel; passing the same tensor as `out`
     updates it in place."""
-    done = _lib.native().linear(x, q_weight, q_scale, bits, group_size, bias, out_dtype, out, residual)
+    native = _lib.native()
+    done = native.linear(x, q_weight, q_scale, bits, group_size, bias, out_dtype, out, residual) if native is not None else None
     if isinstance(done, torch.Tensor):
         return done
     if done is not None:
@@ -293,7 +296,8 @@ def linear_silu_mul(x: torch.Tensor, q_weight: torch.Tensor, q_scale: torch.Tens
     """silu(x1) * x2 with x1, x2 = split(linear(x), 2, axis=-1): the gate_up projection of an MLP
     with its activation folded into the matmul kernel.  Bit-identical to linear then silu_mul;
     shapes without a fused kernel run exactly those two calls."""
-    done = _lib.native().linear_silu_mul(x, q_weight, q_scale, bits, group_size)
+    native = _lib.native()
+    done = native.linear_silu_mul(x, q_weight, q_scale, bits, group_size) if native is not None else None
     if isinstance(done, torch.Tensor):
         return done
     if done is not None and done != _lib.ERR_UNSUPPORTED:

@@ -114,3 +114,60 @@ def test_the_native_path_declines_what_is_not_a_plain_gpu_tensor():
         ops.linear(x, qw, qs, 4, 32)
     with pytest.raises(ValueError, match="GPU"):
         ops.linear_silu_mul(x, qw, qs, 4, 32)
+
+
+@pytest.fixture
+def without_native(tmp_path, monkeypatch):
+    """The package as it is where the extension module was not built, or was built for another torch."""
+    def use(content):
+        path = tmp_path / "_mi355gq_torch.so"
+        if content is not None:
+            path.write_bytes(content)
+        monkeypatch.setattr(gq._lib, "TORCH_PATH", str(path))
+        monkeypatch.setattr(gq._lib, "_TORCH", None)
+        with pytest.warns(RuntimeWarning, match="Python route"):
+            assert gq._lib.native() is None
+        assert gq._lib.native() is None  # (warned of once)
+    return use
+
+
+@pytest.mark.parametrize("content", [None, b"not a shared object"])
+def test_without_the_extension_the_python_route_decides(without_native, content):
+    without_native(content)
+    _, dtype, qw, qs = _weights(8, 64, "q4f16_1", "cpu")
+    with pytest.raises((TypeError, ValueError, RuntimeError)):
+        ops.linear(torch.zeros((1, 64), dtype=dtype), qw, qs, 4, 32)  # (not on a GPU)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scheme", ["q4f16_1", "q4f32_1"])
+def test_every_operator_works_without_the_extension(without_native, scheme):
+    n, k = 96, 320
+    config, dtype, qw, qs = _weights(n, k, scheme, "cuda")
+    x = torch.randn((5, k), device="cuda").to(dtype)
+    ids = torch.randint(0, n, (4,), device="cuda", dtype=torch.int32)
+    indptr = torch.tensor([0, 2, 5], device="cuda", dtype=torch.int32)
+    experts = (torch.stack([qw, qw]), torch.stack([qs, qs]))
+
+    def run():
+        q, s = ops.quantize(x, 4, 32)
+        return [ops.linear(x, qw, qs, 4, 32), ops.linear_silu_mul(x, qw, qs, 4, 32), ops.embedding_take(ids, qw, qs, k, 4, 32), q, s,
+                ops.dequantize(qw, qs, k, 4, 32), ops.moe_group_gemm(x, *experts, indptr, 4, 32), ops.take_rows(x, ids)]
+
+    want = run()
+    without_native(None)
+    for got, w in zip(run(), want):
+        assert torch.equal(got, w)
+
+
+def test_build_leaves_the_extension_out_without_a_compiler(tmp_path, monkeypatch):
+    import importlib.util
+    import os
+    spec = importlib.util.spec_from_file_location("mi355gq_build_test", os.path.join(os.path.dirname(gq._lib.LIB_PATH), os.pardir, "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    stale = tmp_path / "_mi355gq_torch.so"
+    stale.write_bytes(b"")
+    monkeypatch.setattr(build, "TORCH_EXT", str(stale))
+    monkeypatch.setattr(build.shutil, "which", lambda name: None)
+    assert build.build_torch_ext() is None and not stale.exists()
