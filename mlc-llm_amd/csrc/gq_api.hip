@@ -1082,11 +1082,12 @@ static hipError_t moe_row_gemv(const gq::GemmArgs& g, hipStream_t s) {
 // that, up to 24 resp. 16 on average, 32-row passes where K is one phase whose shares of 256 keep most of the waves busy: K = 2048
 // and 3584 (8 of 8, 14 of 16 waves) 58 / 178 against 62 / 219 for the GEMM's tiles, K = 2560 and 768 (10 of 16, 3 of 4) 125 / 47
 // against 102 / 38.  (e2 of Mixtral, K = 14336 in phases, 113-131 against 96-112: the GEMM.)
-static int midrow_rows_per_pass(int64_t rows, int64_t num_experts, int64_t K, int bits) {
+static int midrow_rows_per_pass(int64_t rows, int64_t num_experts, int64_t N, int64_t K, int bits) {
   const int gv = gq::options().gemv_variant;
   if (gv == 10) return 16;  // (forced)
   if (gv == 11) return 32;
-  if (gv >= 0 || bits != 4 || gq::options().gemm_variant >= 0) return 0;
+  // (the fused gate/up form takes whole blocks of 32 columns; other N go elsewhere in either form, which are to add in the same order)
+  if (gv >= 0 || bits != 4 || gq::options().gemm_variant >= 0 || (N & 31) != 0) return 0;
   const bool many = num_experts >= 16;
   const int64_t mid = (many && K < 768 ? 6 : 8) * num_experts;
   if (rows > (many ? 2 : 4) * num_experts && rows <= mid) return 16;
@@ -1144,7 +1145,7 @@ static int moe_group_gemm_impl(const void* x, int64_t rows, const void* q_weight
   //  282 / 292 / 301 / 307 / 343: the skinny kernel, once the step between the two, is behind both since the GEMM reads
   //  its scales in bulk, and only a forced variant runs it on expert segments.  The same rows per expert hold for many
   //  experts: 64 experts x top-6 (2048 x 1408 projections), whole layer at 144 / 192 / 288 / 384 / 432 routed rows
-  if (const int per_pass = midrow_rows_per_pass(rows, num_experts, K, bits)) {
+  if (const int per_pass = midrow_rows_per_pass(rows, num_experts, N, K, bits)) {
     const hipError_t q = gq::launch_midrow(g, per_pass, as_stream(stream));
     if (q != hipErrorNotSupported) return hip_result(q, "moe mid-row launch");
   }
@@ -1359,7 +1360,7 @@ static int moe_group_gemm_dt_impl(const void* x, int64_t rows, const void* q_wei
                               (long long)N, (long long)K);
     }
     // between the few-row kernel and the tiles: as in float16 (the bfloat16 instance)
-    if (const int per_pass = midrow_rows_per_pass(rows, num_experts, K, bits)) {
+    if (const int per_pass = midrow_rows_per_pass(rows, num_experts, N, K, bits)) {
       const hipError_t q = gq::launch_midrow(g, per_pass, as_stream(stream));
       if (q != hipErrorNotSupported) return hip_result(q, "moe_group_gemm_dt mid-row launch");
     }

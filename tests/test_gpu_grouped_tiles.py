@@ -42,3 +42,21 @@ def test_every_row_meets_its_expert(dtype, experts, average):
     assert torch.equal(got, ops.moe_group_gemm(x, qw, qs, indptr.cuda(), 4, 32))
     short = ops.moe_group_gemm(torch.cat([x, x[:5]]), qw, qs, indptr.int().cuda(), 4, 32)  # rows behind the last segment
     assert (short[rows:] == 0).all() and (short[:rows].double() - want).norm() <= 2 * tol * want.norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("experts,n,k,rows", [
+    (64, 176, 2048, 384), (64, 160, 2048, 384),  # N % 32 == 16: the mid-row kernel's blocks do not fit the fused form; 0: they do
+    (16, 80, 2048, 64), (128, 48, 512, 600), (8, 112, 4096, 160), (64, 176, 1408, 300), (8, 98, 1024, 300), (64, 112, 768, 4000),
+])
+def test_fused_expert_segments_equal_the_two_steps(dtype, experts, n, k, rows):
+    g = torch.Generator(device="cuda").manual_seed(experts + n + k)
+    qw, qs = ops.quantize((torch.randn((experts * n, k), generator=g, device="cuda") * 0.02).to(dtype), 4, 32)
+    qw, qs = qw.view(experts, n, -1), qs.view(experts, n, -1)
+    counts = torch.bincount(torch.randint(0, experts, (rows,), generator=torch.Generator().manual_seed(rows)), minlength=experts)
+    indptr = torch.cat([torch.zeros(1, dtype=torch.int64), counts.cumsum(0)]).int().cuda()
+    x = torch.randn((rows, k), generator=g, device="cuda").to(dtype)
+    plain = ops.moe_group_gemm(x, qw, qs, indptr, 4, 32)
+    kernel = gq._lib.last_kernel()
+    fused = ops.moe_group_gemm(x, qw, qs, indptr, 4, 32, silu_mul_halves=True)
+    assert torch.equal(fused, ops.silu_mul(plain)), (kernel, gq._lib.last_kernel())
