@@ -817,13 +817,15 @@ static hipError_t launch_planned_q4(const GemmParams& p, hipStream_t s) {
 // 14336 at r = 20 89.5 / 103, r = 64 183 / 158 / 142 / 170, r = 96 - / 177 / 150 / 185, r = 128 - / 258 / 232 / 189.  Beyond r = 100 a segment no longer fits
 // 128 rows, and 256-row tiles whose waves skip the 32-row blocks past the segment's end are ahead: matrix work is the segment's rows
 // rounded up to 32, and the expert's weights are dequantised once.  bfloat16 the same (64 experts of 5120 x 3584 at r = 128 / 192: 468 / 561
-// against 560 / 728 for 128 rows).
+// against 560 / 728 for 128 rows).  A short K the same: tiles of 128 / 256 rows at r = 64 / 96 on 64 experts of 2048 x 704 38.6 / 46.7, 42.9 / 51.5,
+// on 128 of 1024 x 384 28.9 / 38.1, 34.4 / 41.2, on 32 of 4096 x 640 34.2 / 45.5, 42.4 / 48.9.
 template <bool BF>
 static hipError_t launch_grouped_q4(const GemmParams& p, hipStream_t s) {
   const int64_t rows = p.rows, experts = p.num_experts;
   if (rows <= 24 * experts) return launch_pipe_cfg<4, 32, 128, 32, 32, 4, BF>(p, s);
   if (rows <= 48 * experts) return launch_pipe_cfg<4, 64, 128, 32, 64, 4, BF>(p, s);
-  if (rows <= 100 * experts && p.K >= 768) return launch_pipe_cfg<4, 128, 128, 64, 64, 2, BF>(p, s);  // (the shortest K measured)
+  // (a K of one K tile keeps the 256-row form and its two launches)
+  if (rows <= 100 * experts && p.K > 64) return launch_pipe_cfg<4, 128, 128, 64, 64, 2, BF>(p, s);
   // 256 columns per tile while that gives every CU a workgroup, else 128 (e2 of a Mixtral layer, 128 wide tiles: r = 128 189
   // against 270 us; 16 experts of 4096 x 2048, 256 of them: 53 against 63)
   const int64_t tiles_x = (p.N + 255) / 256, live = experts > rows / 256 ? experts : rows / 256;  // row tiles that hold rows
