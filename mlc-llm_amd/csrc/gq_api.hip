@@ -1077,8 +1077,8 @@ static hipError_t moe_row_gemv(const gq::GemmArgs& g, hipStream_t s) {
 // segment inside one pass: 16-row passes up to 8 rows per expert on average, from 4 on with few experts (Mixtral, e1_e3 / e2
 // in us: 24 tokens 156 / 102 -> 115 / 76, 32 tokens 170 / 106 -> 117 / 78, 16 tokens 118 / 75 against the quad-row kernel's 122 / 74),
 // from 2 on with 16 and more (16 experts of 4096 x 2048 at 4 rows 19.5 against 24.0; 64 of 2816 x 2048, 128 of 1536 x 2048 and of 2048 x 768 at
-// 8 rows 48 / 49 / 32 against 59 / 58 / 46 for 32-row passes and 61 / 64 / 38 for the GEMM's 32-row tiles, at 10 rows 84 / 88 / 55; a K below 768, not measured
-// there, keeps 6).  Beyond
+// 8 rows 48 / 49 / 32 against 59 / 58 / 46 for 32-row passes and 61 / 64 / 38 for the GEMM's 32-row tiles, at 10 rows 84 / 88 / 55; with a K
+// below 768 up to 6: 64 and 128 of 2048 x 512 at 6 rows 13.2 / 19.8 against 14.8 / 26.8 for the GEMM, at 8 rows 21.8 / 34.8 against 14.9 / 26.5).  Beyond
 // that, up to 24 resp. 16 on average, 32-row passes where K is one phase whose shares of 256 keep most of the waves busy: K = 2048
 // and 3584 (8 of 8, 14 of 16 waves) 58 / 178 against 62 / 219 for the GEMM's tiles, K = 2560 and 768 (10 of 16, 3 of 4) 125 / 47
 // against 102 / 38.  (e2 of Mixtral, K = 14336 in phases, 113-131 against 96-112: the GEMM.)
@@ -1140,18 +1140,19 @@ static int moe_group_gemm_impl(const void* x, int64_t rows, const void* q_weight
     if (paired) return fail(MI355GQ_ERR_UNSUPPORTED, "moe_group_gemm_silu_mul: no fused GEMV for N=%lld K=%lld",
                             (long long)N, (long long)K);
   }
-  // (up to about seven rows per expert.  Mixtral layer, 8 experts, whole layer in us at 40 / 48 / 56 / 64 / 80 routed rows:
-  //  this kernel 249 / 258 / 262 / 300 / 319, the GEMM's 32-row tiles 270 / 266 / 276 / 272 / 272, the skinny kernel
-  //  282 / 292 / 301 / 307 / 343: the skinny kernel, once the step between the two, is behind both since the GEMM reads
-  //  its scales in bulk, and only a forced variant runs it on expert segments.  The same rows per expert hold for many
-  //  experts: 64 experts x top-6 (2048 x 1408 projections), whole layer at 144 / 192 / 288 / 384 / 432 routed rows
   if (const int per_pass = midrow_rows_per_pass(rows, num_experts, N, K, bits)) {
     const hipError_t q = gq::launch_midrow(g, per_pass, as_stream(stream));
     if (q != hipErrorNotSupported) return hip_result(q, "moe mid-row launch");
   }
-  //  112 / 115 / 117 / 127 / 142 us against 137 / 141 / 146 / 143 / 144 on the GEMM's tiles as they were; since a tile finds its expert in
-  //  one step, 64 experts of 2048 x 1408 at 4 / 6 rows take 43 / 53 here and 38 / 38 there, and q4 hands over at three from K = 768 on, the shortest K measured)
-  const int64_t quad_per = bits == 4 && num_experts > 16 && K >= 768 ? 3 : 7;
+  // The few-row kernel up to seven rows per expert on average (Mixtral layer, 8 experts, whole layer in us at 40 / 48 / 56 / 64 / 80 routed
+  // rows: this kernel 249 / 258 / 262 / 300 / 319, the GEMM's 32-row tiles 270 / 266 / 276 / 272 / 272, the skinny kernel 282 / 292 / 301 / 307 / 343,
+  // which only a forced variant runs on expert segments).  With more than 16 experts of q4 up to three, and beyond that while rows^2 x N <=
+  // 12100 x K: this kernel's time grows with its passes over the weights, the GEMM's is its walk through K until there are several rounds of
+  // workgroups.  Fitted to 17..96 experts, N 64..2048, K 384..4104 at 4 / 5 / 7 rows per expert (540 pairs of times): 1.9 % behind the better
+  // one on average, always the one or the other 16 / 28 %.  (us at 5 rows, this kernel / the GEMM: 20 experts of 64 x 1408 5.7 / 12.5, of
+  // 1024 x 704 9.8 / 8.4, 40 of 512 x 1408 11.6 / 12.9, of 132 x 640 6.7 / 8.3, 64 of 2048 x 1408 48 / 38, 128 of 1024 x 384 29 / 15.)
+  const bool many_small = bits != 4 || num_experts <= 16 || rows * rows * N <= 12100 * K;
+  const int64_t quad_per = many_small ? 7 : 3;
   const int64_t quad_rows = quad_per * num_experts > 32 ? quad_per * num_experts : 32;
   if ((rows <= 128 || rows <= 8 * num_experts) && gq::options().gemm_variant != 1 &&
       ((gv < 0 && rows <= quad_rows) || (gv >= 6 && gv <= 8))) {

@@ -48,6 +48,7 @@ def test_every_row_meets_its_expert(dtype, experts, average):
 @pytest.mark.parametrize("experts,n,k,rows", [
     (64, 176, 2048, 384), (64, 160, 2048, 384),  # N % 32 == 16: the mid-row kernel's blocks do not fit the fused form; 0: they do
     (16, 80, 2048, 64), (128, 48, 512, 600), (8, 112, 4096, 160), (64, 176, 1408, 300), (8, 98, 1024, 300), (64, 112, 768, 4000),
+    (20, 64, 704, 80), (20, 64, 704, 1200),
 ])
 def test_fused_expert_segments_equal_the_two_steps(dtype, experts, n, k, rows):
     g = torch.Generator(device="cuda").manual_seed(experts + n + k)
@@ -60,3 +61,22 @@ def test_fused_expert_segments_equal_the_two_steps(dtype, experts, n, k, rows):
     kernel = gq._lib.last_kernel()
     fused = ops.moe_group_gemm(x, qw, qs, indptr, 4, 32, silu_mul_halves=True)
     assert torch.equal(fused, ops.silu_mul(plain)), (kernel, gq._lib.last_kernel())
+
+
+@pytest.mark.parametrize("n,rows_per_expert,tile", [
+    (2048, 3, "quad_kernel<"), (2048, 6, "gemm_pipe_kernel<4,32,128,"), (64, 6, "quad_kernel<"), (64, 8, "gemm_pipe_kernel<4,32,128,"),
+    (64, 60, "gemm_pipe_kernel<4,128,128,"), (64, 110, "gemm_pipe_kernel<4,256,")])
+@pytest.mark.parametrize("k", [704, 1408])
+def test_rules_by_rows_per_expert_hold_for_a_short_k_and_a_small_stack(k, n, rows_per_expert, tile):
+    experts = 20
+    rows = experts * rows_per_expert
+    g = torch.Generator(device="cuda").manual_seed(k + rows)
+    qw, qs = ops.quantize((torch.randn((experts * n, k), generator=g, device="cuda") * 0.02).half(), 4, 32)
+    x = torch.randn((rows, k), generator=g, device="cuda").half()
+    indptr = (torch.arange(experts + 1, dtype=torch.int32) * rows_per_expert).cuda()
+    y = ops.moe_group_gemm(x, qw.view(experts, n, -1), qs.view(experts, n, -1), indptr, 4, 32)
+    assert tile in gq._lib.last_kernel(), gq._lib.last_kernel()
+    w = ops.dequantize(qw, qs, k, 4, 32).double().view(experts, n, k)
+    want = torch.cat([x[e * rows_per_expert:(e + 1) * rows_per_expert].double() @ w[e].t().contiguous() for e in range(experts)])
+    # one rounding of the output, and (few-row kernel) of each weight that it does not make
+    assert (y.double() - want).norm() <= (2 * 2.0 ** -11 + 1e-5) * want.norm()
