@@ -1075,10 +1075,11 @@ static hipError_t moe_row_gemv(const gq::GemmArgs& g, hipStream_t s) {
 // 0 where the quad-row kernel (fewer rows) or the GEMM's tiles (more) stay ahead.  A segment longer than a pass takes
 // another pass over its expert's weights while the other experts' workgroups are done, so the bounds keep the longest
 // segment inside one pass: 16-row passes up to 8 rows per expert on average, from 4 on with few experts (Mixtral, e1_e3 / e2
-// in us: 24 tokens 156 / 102 -> 115 / 76, 32 tokens 170 / 106 -> 117 / 78, 16 tokens 118 / 75 against the quad-row kernel's 122 / 74),
-// from 2 on with 16 and more (16 experts of 4096 x 2048 at 4 rows 19.5 against 24.0; 64 of 2816 x 2048, 128 of 1536 x 2048 and of 2048 x 768 at
-// 8 rows 48 / 49 / 32 against 59 / 58 / 46 for 32-row passes and 61 / 64 / 38 for the GEMM's 32-row tiles, at 10 rows 84 / 88 / 55; with a K
-// below 768 up to 6: 64 and 128 of 2048 x 512 at 6 rows 13.2 / 19.8 against 14.8 / 26.8 for the GEMM, at 8 rows 21.8 / 34.8 against 14.9 / 26.5).  Beyond
+// in us: 24 tokens 156 / 102 -> 115 / 76, 32 tokens 170 / 106 -> 117 / 78, 16 tokens 118 / 75 against the quad-row kernel's 122 / 74), with more
+// than 16 from 2 on (64 experts x top-6, 2816 x 2048 / 2048 x 1536 / 5120 x 3584 at 144..384 rows: 55-64 / 46-49 / 142-197 -> 51-53 / 34-35 / 142-145)
+// and, from 25 on, up to 7: the longest of so many random segments passes 16 rows at an average of 8 (32 / 64 / 128 experts of 2048 x 2048 at 7
+// rows 20.7 / 33.8 / 64.1 against 24.9 / 40.8 / 80.0 for 32-row passes, at 8 rows 35.9 / 61.2 / 113 against 25.9 / 42.0 / 79.2), with a K below 768 up to 6 (64 and 128 of 2048 x 512 at 6 rows 13.2 / 19.8 against 14.8 / 26.8
+// for the GEMM).  Beyond
 // that, up to 24 resp. 16 on average, 32-row passes where K is one phase whose shares of 256 keep most of the waves busy: K = 2048
 // and 3584 (8 of 8, 14 of 16 waves) 58 / 178 against 62 / 219 for the GEMM's tiles, K = 2560 and 768 (10 of 16, 3 of 4) 125 / 47
 // against 102 / 38.  (e2 of Mixtral, K = 14336 in phases, 113-131 against 96-112: the GEMM.)
@@ -1088,8 +1089,8 @@ static int midrow_rows_per_pass(int64_t rows, int64_t num_experts, int64_t N, in
   if (gv == 11) return 32;
   // (the fused gate/up form takes whole blocks of 32 columns; other N go elsewhere in either form, which are to add in the same order)
   if (gv >= 0 || bits != 4 || gq::options().gemm_variant >= 0 || (N & 31) != 0) return 0;
-  const bool many = num_experts >= 16;
-  const int64_t mid = (many && K < 768 ? 6 : 8) * num_experts;
+  const bool many = num_experts > 16;
+  const int64_t mid = (!many ? 8 : (K < 768 ? 6 : (num_experts > 24 ? 7 : 8))) * num_experts;
   if (rows > (many ? 2 : 4) * num_experts && rows <= mid) return 16;
   int64_t waves = 1;
   while (waves * 256 < K) waves *= 2;

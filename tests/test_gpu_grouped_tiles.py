@@ -80,3 +80,20 @@ def test_rules_by_rows_per_expert_hold_for_a_short_k_and_a_small_stack(k, n, row
     want = torch.cat([x[e * rows_per_expert:(e + 1) * rows_per_expert].double() @ w[e].t().contiguous() for e in range(experts)])
     # one rounding of the output, and (few-row kernel) of each weight that it does not make
     assert (y.double() - want).norm() <= (2 * 2.0 ** -11 + 1e-5) * want.norm()
+
+
+@pytest.mark.parametrize("experts,rows,kernel", [
+    (16, 64, "quad_kernel<"), (16, 128, "midrow_kernel<1,"), (16, 320, "midrow_kernel<2,"),  # up to 16 experts: 4 to 8, then to 24
+    (17, 40, "midrow_kernel<1,"), (24, 192, "midrow_kernel<1,"), (25, 175, "midrow_kernel<1,"), (25, 176, "midrow_kernel<2,"),
+])
+def test_midrow_bounds_by_experts(experts, rows, kernel):
+    n, k = 64, 1024
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    qw, qs = ops.quantize((torch.randn((experts * n, k), generator=g, device="cuda") * 0.02).half(), 4, 32)
+    x = torch.randn((rows, k), generator=g, device="cuda").half()
+    cuts = torch.linspace(0, rows, experts + 1).int()
+    y = ops.moe_group_gemm(x, qw.view(experts, n, -1), qs.view(experts, n, -1), cuts.cuda(), 4, 32)
+    assert kernel in gq._lib.last_kernel(), gq._lib.last_kernel()
+    w = ops.dequantize(qw, qs, k, 4, 32).double().view(experts, n, k)
+    want = torch.cat([x[cuts[e]:cuts[e + 1]].double() @ w[e].t().contiguous() for e in range(experts)])
+    assert (y.double() - want).norm() <= (2 * 2.0 ** -11 + 1e-5) * want.norm()  # (as above)
