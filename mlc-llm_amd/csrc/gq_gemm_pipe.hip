@@ -829,7 +829,16 @@ static hipError_t launch_grouped_q4(const GemmParams& p, hipStream_t s) {
   // 256 columns per tile while that gives every CU a workgroup, else 128 (e2 of a Mixtral layer, 128 wide tiles: r = 128 189
   // against 270 us; 16 experts of 4096 x 2048, 256 of them: 53 against 63)
   const int64_t tiles_x = (p.N + 255) / 256, live = experts > rows / 256 ? experts : rows / 256;  // row tiles that hold rows
-  if (tiles_x * live < 256) return launch_pipe_cfg<4, 256, 128, 64, 64, 2, BF, true, 2>(p, s);
+  if (tiles_x * live < 256) {
+    // ... and for bfloat16 128 rows where those tiles, one and a half per expert at r = 128, have a CU each or take one round where the tall
+    // ones take two (128 rows / 256: 4 experts of 2048 x 2048 at r = 128 and 256 0.85 and 0.81 of the time, 8 of 64..2048 x 4096 0.84..0.87, 17
+    // of 2048 x 1024 0.69, 12 of 2048 x 4096 at r = 256 0.72; on the other side 12 of 2048 x 2048 at r = 128 1.26, 8 of 4096 x 4096 1.28;
+    // float16 measures alike, 0.78 and 0.69, and keeps the tall tiles it has had there)
+    const int64_t n_tiles = (p.N + 127) / 128, wg128 = (rows / 128 + experts / 2) * n_tiles;
+    const int64_t tall = rows / 256 + experts / 2, wg256 = (tall > experts ? tall : experts) * n_tiles;
+    if (BF && (wg128 <= 256 || (wg256 > 256 && wg128 <= 512))) return launch_pipe_cfg<4, 128, 128, 64, 64, 2, BF>(p, s);
+    return launch_pipe_cfg<4, 256, 128, 64, 64, 2, BF, true, 2>(p, s);
+  }
   // A last round of workgroups that is at most about half full costs a whole round here (the kernel waits on
   // memory, not on the matrix pipe): its columns go to a second launch on the narrow tile, whose workgroups take
   // half as long.  (Mixtral's e1_e3, 112 column tiles x 8 experts = 3.5 rounds of 256.)

@@ -97,3 +97,27 @@ def test_midrow_bounds_by_experts(experts, rows, kernel):
     w = ops.dequantize(qw, qs, k, 4, 32).double().view(experts, n, k)
     want = torch.cat([x[cuts[e]:cuts[e + 1]].double() @ w[e].t().contiguous() for e in range(experts)])
     assert (y.double() - want).norm() <= (2 * 2.0 ** -11 + 1e-5) * want.norm()  # (as above)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("experts,n,average,tile", [
+    # (float16 keeps the 256-row form)
+    (4, 64, 128, "4,128,128,"), (12, 1408, 128, "4,128,128,"), (12, 2048, 128, "4,256,128,"),  # a CU each, or not
+    (12, 2048, 256, "4,128,128,"), (17, 2048, 128, "4,128,128,"),  # one round of pairs against two
+    (16, 4096, 128, "4,256,256,"),
+])
+def test_tall_tiles_of_long_segments(dtype, experts, n, average, tile):
+    k = 128
+    g = torch.Generator(device="cuda").manual_seed(experts + n)
+    rows = experts * average
+    cuts = torch.linspace(0, rows, experts + 1).int()
+    cuts[1:-1] += torch.randint(-60, 60, (experts - 1,), generator=torch.Generator().manual_seed(n))
+    qw, qs = ops.quantize((torch.randn((experts * n, k), generator=g, device="cuda") * 0.02).to(dtype), 4, 32)
+    x = torch.randn((rows, k), generator=g, device="cuda").to(dtype)
+    y = ops.moe_group_gemm(x, qw.view(experts, n, -1), qs.view(experts, n, -1), cuts.cuda(), 4, 32)
+    if dtype == torch.float16 and tile == "4,128,128,":
+        tile = "4,256,128,"
+    assert f"gemm_pipe_kernel<{tile}" in gq._lib.last_kernel(), gq._lib.last_kernel()
+    w = ops.dequantize(qw, qs, k, 4, 32).double().view(experts, n, k)
+    want = torch.cat([x[cuts[e]:cuts[e + 1]].double() @ w[e].t().contiguous() for e in range(experts)])
+    assert (y.double() - want).norm() <= ((2.0 ** -11 if dtype == torch.float16 else 2.0 ** -9) + 1e-5) * want.norm()  # one rounding
