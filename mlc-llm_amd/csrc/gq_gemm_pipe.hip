@@ -683,14 +683,19 @@ static float tile_us(const TileCost& c, int64_t rows, int64_t N, int nk, int kt,
   // (a split has to be 2 % ahead on paper)
   return split > 1 ? (us + c.reduce + c.traffic * static_cast<float>(split) * mn) * 1.02f : us;
 }
-static bool tile_applies(const TileCost& c, int64_t rows) { return c.bm < 256 || (c.skip != 0) == (c.bn == 128 || rows % 256 != 0); }
+static bool tile_applies(const TileCost& c, int64_t rows, int nk) {
+  // (fitted from K = 2048 on: what a workgroup costs before and behind its K loop is not told apart there, and for a short K this tile,
+  //  whose weight loads run four K tiles ahead, looks a quarter of its time: 16272 x 128 at 3596 rows 74 us, 256 x 256 47)
+  if (c.bm == 256 && c.bn == 128 && nk < 16) return false;
+  return c.bm < 256 || (c.skip != 0) == (c.bn == 128 || rows % 256 != 0);
+}
 
 // one launch for all of N columns
 static SplitPlan plan_one(const TileCost* costs, int64_t rows, int64_t N, int nk, int64_t scratch_bytes, int runs, float* best_us) {
   SplitPlan best{0, 0, 1, 1 << 28};
   for (int t = 0; t < 6; ++t) {
     const TileCost& c = costs[t];
-    if (!tile_applies(c, rows)) continue;
+    if (!tile_applies(c, rows, nk)) continue;
     const int64_t tiles = ((rows + c.bm - 1) / c.bm) * column_tiles(N, c.bn, runs);
     int last = 0;
     for (int want = 1; want <= 16; ++want) {
@@ -727,7 +732,7 @@ static SplitPlan plan_by_cost(int64_t rows, int64_t N, int nk, int bf16, int64_t
   float best_us = one_us / 1.07f;
   for (int t = 1; t <= 4; ++t) {  // (the tiles of one workgroup per CU)
     const TileCost& c = costs[t];
-    if (!tile_applies(c, rows)) continue;
+    if (!tile_applies(c, rows, nk)) continue;
     const int64_t mt = (rows + c.bm - 1) / c.bm;
     for (int runs = 1; runs <= (N % 2 == 0 ? 2 : 1); ++runs) {
       const int64_t nt = column_tiles(N, c.bn, runs), head = mt * nt / 256 * 256 / mt / runs * runs;  // column tiles of the whole rounds
@@ -750,12 +755,33 @@ static SplitPlan plan_by_cost(int64_t rows, int64_t N, int nk, int bf16, int64_t
   return best;
 }
 
+// K up to 512 and several rounds of workgroups, where the output's stores weigh as much as the K loop: rounds x (time of one tile), rounds =
+// ceil(tiles / resident workgroups) (256, 512 for 128 x 128, a lone one of which takes 0.72 of a pair's time), tile times from the rates
+// measured with balanced rounds (1035 / 870 / 806 TFLOP/s); the smaller tile has to win by 8 %.  (us, by the cost above / by this: 28800 x 80 at 2734
+// rows 92 / 58, 35712 x 360 at 760 60 / 41, 20120 x 272 at 3751 138 / 99, 27376 x 64 at 1732 55 / 35.)
+constexpr int kShortTiles = 8;
+static SplitPlan plan_by_rounds(int64_t rows, int64_t N) {
+  const int64_t mt = (rows + 127) / 128, big = ((rows + 255) / 256) * ((N + 255) / 256), mid = mt * ((N + 255) / 256), small = mt * ((N + 127) / 128);
+  const int64_t per_cu = (small + 255) / 256;
+  const double t_small = 16384.0 / (806.0 / 512);
+  const double c_big = static_cast<double>((big + 255) / 256) * (65536.0 / (1035.0 / 256)), c_mid = static_cast<double>((mid + 255) / 256) * (32768.0 / (870.0 / 256)),
+               c_small = static_cast<double>(per_cu / 2) * t_small + static_cast<double>(per_cu % 2) * 0.72 * t_small;
+  SplitPlan plan{256, 256, 1, 1 << 28};
+  double best = c_big;
+  if (c_mid < 0.92 * best) { plan.bm = 128; best = c_mid; }
+  if (c_small < 0.92 * best) plan.bm = plan.bn = 128;
+  return plan;
+}
+
 SplitPlan plan_split_k(int64_t rows, int64_t N, int64_t K, int bits, int group_size, bool grouped, int bf16, int64_t scratch_bytes) {
   SplitPlan plan{0, 0, 1, 1 << 28};
   if (grouped || rows <= 0 || N <= 0 || K <= 0 || (K & 7) != 0) return plan;
   const int ng = static_cast<int>((K + group_size - 1) / group_size);
   const int nk = (ng + 1) / 2;
-  if (bits == 4 && rows > 64 && options().gemm_split_k <= 0) return plan_by_cost(rows, N, nk, bf16, scratch_bytes);
+  if (bits == 4 && rows > 64 && options().gemm_split_k <= 0) {
+    if (nk <= kShortTiles && ((rows + 127) / 128) * ((N + 127) / 128) >= 200) return plan_by_rounds(rows, N);
+    return plan_by_cost(rows, N, nk, bf16, scratch_bytes);
+  }
   // few rows: the GEMM is bound by streaming the weights, and 128-wide column tiles alone leave
   // most CUs idle (o_proj / down have 32 of them).  Match the tile height to the rows and cut K
   // until about one workgroup per CU exists.
@@ -807,7 +833,7 @@ static hipError_t launch_planned_q4(const GemmParams& p, hipStream_t s) {
   if (p.bm_hint == 128 && p.bn_hint == 256) return launch_pipe_cfg<4, 128, 256, 64, 64, 2, BF>(p, s);
   if (p.bm_hint == 256 && p.bn_hint == 128) return launch_pipe_cfg<4, 256, 128, 64, 64, 2, BF, true, 2>(p, s);
   if (p.bm_hint == 256)
-    return p.rows % 256 != 0 ? launch_pipe_cfg<4, 256, 256, 128, 64, 2, BF, true, 2>(p, s) : launch_pipe_cfg<4, 256, 256, 128, 64, 2, BF>(p, s);
+    return p.rows % 256 != 0 && (p.ng + 1) / 2 > kShortTiles ? launch_pipe_cfg<4, 256, 256, 128, 64, 2, BF, true, 2>(p, s) : launch_pipe_cfg<4, 256, 256, 128, 64, 2, BF>(p, s);
   return launch_pipe_cfg<4, 128, 128, 64, 64, 2, BF>(p, s);
 }
 

@@ -16,6 +16,8 @@ CASES = [(65, 256, 256, "64,128", False), (65, 256, 1000, "64,128", True), (65, 
          (512, 28680, 512, "256,256", False), (1025, 2056, 4096, None, None),
          # a K shorter than a K tile, whose chunks past K are loaded from the row's start
          (65, 256, 8, None, False), (130, 200, 24, None, False), (300, 130, 56, None, False),
+         # K up to 512: by rounds of workgroups where there are many (ragged rows on the 256-row tile as well), by the cost else
+         (760, 12000, 360, "256,256,128,64,2,false,false", False), (1732, 3400, 64, "128,256", False), (2734, 2880, 80, "128,128", False), (300, 700, 360, "64,128", None),
          # several rounds of workgroups, in one launch (the last one in float16: in two)
          (300, 25000, 2048, None, None), (450, 37888, 1024, None, None), (1536, 12288, 1024, None, None)]
 
