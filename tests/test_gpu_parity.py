@@ -358,7 +358,7 @@ def test_skinny_kernel_forms(mode, m, n, k):
     assert_linear_ok(y32, ref - b.astype(np.float64), x, k, f"skinny mode {mode} fp32 out")
 
 
-@pytest.mark.parametrize("form", [-1, 2, 4])  # ring of two tiles with the offsets kept, four without, three with
+@pytest.mark.parametrize("form", [-1, 2])  # up to 16 rows: a ring of two tiles with the offsets kept, of four without
 @pytest.mark.parametrize("m", [1, 9, 16, 17, 40])  # one pass, a full one, and rows that take two and three passes
 @pytest.mark.parametrize("n,k", [(96, 256), (1000, 1024), (520, 4096), (72, 8192), (256, 14336), (16, 512)])
 def test_midrow_kernel(form, m, n, k):
@@ -378,11 +378,15 @@ def test_midrow_kernel(form, m, n, k):
     finally:
         gq._lib.set_option("gemv_variant", -1)
         gq._lib.set_option("gemv_rows_per_wave", -1)
-    if k > 4096 and form == 2:  # (several phases exist for the default instance only: K slices where the call's scratch
-        #                          holds their partial sums, else the shape falls through)
-        assert not kern.startswith("gq::midrow_kernel") or " phases=1 " in kern, kern
+    # (the instance is asserted, so that an override that selects nothing fails; several phases exist for the default
+    # instances only: K slices, which are one phase each, where the call's scratch holds their partial sums, else the shape falls through)
+    instance = "<2,8,2,0," if m > 16 else "<1,8,4,0," if form == 2 else "<1,8,2,1,"
+    if kern.startswith("gq::midrow_kernel<"):
+        phased = " phases=1 " not in kern
+        assert kern.startswith(f"gq::midrow_kernel{instance}{int(phased)}> "), kern
+        assert not phased or (k > 4096 and form == -1), kern
     else:
-        assert kern.startswith("gq::midrow_kernel<"), kern
+        assert k > 4096 and form == 2, kern
     ref = o.linear_fp32(x, qw, qs, s, b)
     assert_linear_ok(y, ref, x, k, f"mid-row form {form} {m}x{n}x{k} [{kern}]")
     assert_linear_ok(y32, ref - b.astype(np.float64), x, k, f"mid-row form {form} fp32 out")
