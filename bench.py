@@ -577,7 +577,7 @@ def main() -> int:
             ms = timed(lambda: ops.linear(xm_, qwd, qsd, 4, 32), 6 if dt == torch.bfloat16 else 3, 2, False)
             res["gemm_m2048"] = {"us": round(ms * 1e3, 1), "TFLOP/s": round(2.0 * 2048 * n * k / ms / 1e9, 1),
                                  "matrix_instruction": "v_mfma_f32_32x32x16_bf16" if dt == torch.bfloat16
-                                 else "v_mfma_f32_32x32x2_f32 (157 TFLOP/s peak)"}
+                                 else "v_mfma_f32_32x32x16_bf16 on three bfloat16 planes of x"}
             other[label] = res
             del qwd, qsd, x1, x4, xm_
         extra["other_model_dtypes"] = other
