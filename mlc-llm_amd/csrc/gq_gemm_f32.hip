@@ -15,9 +15,10 @@
 // weights global -> registers -> bfloat16 -> LDS, both in the field order in which v_cvt_scalef32_pk_f32_fp8 delivers a
 // storage word ((0, 2) (4, 6) (1, 3) (5, 7)): an order of k is free as long as both operands have it.  LDS rows are 80 bytes
 // apart: eight consecutive rows of a fragment read start 20 banks apart and meet all banks once.  The split of x is done by
-// every workgroup for itself (5.5 vector instructions per element and column tile), which is why the tile is wide: at 128 x
-// 256 a wave's K tile is 24 matrix instructions (768 cycles) next to about 160 vector instructions (640 cycles), 64 of
-// them the scaling of the results.  Interleaving the two by sched_group_barrier (one matrix instruction, 4 / 6 / 8 vector
+// every workgroup for itself (7.5 vector instructions per element and column tile, two of them for infinities), which is why
+// the tile is wide: at 128 x 256 a wave's K tile is 24 matrix instructions (768 cycles) next to 184 to 195 vector instructions (740 to
+// 780 cycles), 64 of them the scaling of the results; over whole launches the matrix pipe is busy for 50 to 54 % of the cycles
+// and the vector pipe for 51 to 52 %, so that the two together, not memory, bound it.  Interleaving the two by sched_group_barrier (one matrix instruction, 4 / 6 / 8 vector
 // instructions) was 4 to 10 % slower than the compiler's own order.
 //
 // Measured against the float32 matrix instruction's kernel it replaced (us; rows, then N x K): 16 x 4096 x 4096 317 -> 18,

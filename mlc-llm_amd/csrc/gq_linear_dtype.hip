@@ -2,7 +2,7 @@
 // of GroupQuantizeLinear.forward / lm_head_forward (group_quantization.py:390-437, 524-556) with
 // x, q_scale and bias in float32 or bfloat16.
 //
-// A first form of the two regimes of the float16 path:
+// Two regimes; bfloat16 and q4 float32 come here where their faster kernels do not apply or lose (one row, K % 8 != 0, q3 float32):
 //  * up to 8 activation rows: a persistent-wave GEMV with x resident in LDS in the model dtype
 //    (fp32 FMAs for float32, v_dot2_f32_bf16 on bf16 pairs for bfloat16);
 //  * more rows: a 128 x 128 tile GEMM on v_mfma_f32_32x32x2_f32 with both operands in LDS as

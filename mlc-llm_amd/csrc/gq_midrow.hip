@@ -203,8 +203,8 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
       };
       // scales: the U of this lane's row c.  float32 (PAIR): of the tiles of rounds r and r + 1 in one load, lane (c, j) taking
       // half j % 2 of row c of tile j / 2, handed round when a tile's turn comes.  A lane's own 32 bytes would be two loads per
-      // tile, which all four lanes of a row make to the same addresses; the texture unit was busy for 67 % of the kernel and
-      // is what the exchange relieves (four rows: 128256 x 4096 88 -> 77 us, 28672 x 4096 28 -> 23, 4096 x 14336 20.1 -> 18.4; the
+      // tile, which all four lanes of a row make to the same addresses; the exchange halves those requests (with it the
+      // texture unit is busy for 48 to 53 % of the cycles, the vector pipe for 44 to 49 %; four rows: 128256 x 4096 88 -> 77 us, 28672 x 4096 28 -> 23, 4096 x 14336 20.1 -> 18.4; the
       // 16-bit scales are one load per tile, and the exchange's registers spill there)
       const int s_lane = (c * p.ng + ga) * EL + (PAIR ? (j & 1) * (U / 2 * EL) : 0);
       constexpr int NS = PAIR ? RT / 2 : RT;
@@ -578,11 +578,11 @@ hipError_t launch_mid(const MidParams& p, int wgx, int experts, hipStream_t s) {
 
 }  // namespace
 
-// q4f16_1 / q4bf16_1 (float16 / bfloat16 activations, scales and results), K % 256 == 0 (a wave's eight groups: 16-byte runs of scales), N % 16 == 0 for expert
+// q4f16_1 / q4bf16_1 / q4f32_1 (activations, scales and results of one type), K % 256 == 0 (a wave's eight groups: 16-byte runs of scales), N % 16 == 0 for expert
 // segments and N % 32 == 0 for the fused gate/up form; any number of rows (more than the batch tiles hold: passes that read
 // the weights again, so callers keep it to few rows per segment).  hipErrorNotSupported otherwise.  Tuning overrides:
 // quad_ksplit (log2 of the waves that share a tile's K, minus one), gemv_waves (workgroups per expert x 16),
-// gemv_rows_per_wave (1, 2: other one-batch-tile instances).
+// gemv_rows_per_wave (2: the float16 instance of one batch tile with a ring of four tiles).
 hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   if (a.bits != 4 || a.group_size != 32) return hipErrorNotSupported;
   if (a.rows < 1 || a.N < 16 || (a.K & 255) != 0 || a.K == 0) return hipErrorNotSupported;
