@@ -20,9 +20,11 @@
 // wave instruction covers 16 rows x 64 contiguous bytes); a 4 x 4 transpose across the four 16-lane rows
 // (v_permlane32_swap, v_permlane16_swap: four instructions) then leaves register m of lane (c, j) with word j of group
 // 4 * step + m.  A operand = 16 activation rows x the same 32 k: lane (i, j) holds x[i][32 g + 8 j ..] in the pair
-// order of the unpack masks, the odd fields' activations divided by 16; it reads those 16 bytes straight from global
-// memory once and keeps them.  The offset term needs no cross-lane sum either: the same matrix instruction on a
-// constant B operand (-1031 for the even fields, -16 * 71 for the odd ones) leaves -(offset) of rows 4 j .. 4 j + 3 in
+// order of the unpack masks, the odd fields' activations divided by 16; x is read once, in whole cache lines, and comes into
+// that order through a wave's own 2 KiB of LDS (against 16-byte reads of sixteen rows at a time: 28672 x 4096 at 16 / 32 rows
+// 22.6 / 30.1 -> 20.5 / 28.2 us, 6144 x 4096 10.6 / 14.8 -> 8.6 / 10.4, 4096 x 4096 9.6 / 13.9 -> 7.5 / 9.9).  The offset
+// term needs no cross-lane sum either: the same matrix instruction on a constant B operand (-1031 for the even fields,
+// -16 * 71 for the odd ones) leaves -(offset) of rows 4 j .. 4 j + 3 in
 // lane (c, j), which is where the C operand wants it.  D: lane (c, j) receives rows 4 j .. 4 j + 3 of column c, four
 // values of the lane's own weight row: its scale of the group multiplies them into the fp32 accumulators.
 //
@@ -272,25 +274,48 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
           xa[0][u][3] = __builtin_amdgcn_perm(v[7], v[5], kHiHi);
         }
       } else {
-        // ---- this wave's share of x goes out first (it is needed first, and loads retire in issue order): lane (i = c, j)
-        //      of batch tile bt reads x[row 16 bt + i][32 g + 8 j .. + 7]
+        // ---- this wave's share of x goes out first (it is needed first, and loads retire in issue order).  Lane (i = c, j) of
+        //      batch tile bt wants x[row 16 bt + i][32 g + 8 j .. + 7], but loads that way would touch sixteen cache lines
+        //      per quarter of a wave: all of x (32 rows of K = 4096) arrives in 5.9 us that way and in 1.7 with eight lanes
+        //      side by side on the 128 bytes of a row (a kernel of these loads alone, less its launch).  So load i of a lane is 16 bytes of row 8 (i % 2) +
+        //      lane / 8, groups 2 (i / 2) and the next, and a tile of LDS of the wave's own (16 rows x 128 bytes, no barrier:
+        //      a wave's LDS instructions execute in order) turns two loads into the operands of two groups.
         uint4 xraw[NBT][U];
         bool x_ok[NBT];
+        int xl = threadIdx.x & 63;
+        asm volatile("" : "+v"(xl));  // (what follows from it is made here, not kept in registers through the walk)
 #pragma unroll
         for (int bt = 0; bt < NBT; ++bt) {
-          const int b = pass_lo + 16 * bt + c;
-          x_ok[bt] = k_live && b < seg_hi;
-          const uint16_t* xrow = p.x + x_row(p.x_rows, p.x_src_rows, x_ok[bt] ? b : seg_lo) * p.K + ga * 32 + 8 * j;
+          x_ok[bt] = k_live && pass_lo + 16 * bt + (xl & 15) < seg_hi;
+          const uint16_t* xrow[2];
 #pragma unroll
-          for (int u = 0; u < U; ++u) xraw[bt][u] = *reinterpret_cast<const uint4*>(xrow + u * 32);
+          for (int h = 0; h < 2; ++h) {
+            const int b = pass_lo + 16 * bt + 8 * h + (xl >> 3);
+            xrow[h] = p.x + x_row(p.x_rows, p.x_src_rows, b < seg_hi ? b : seg_lo) * p.K + ga * 32 + 8 * (xl & 7);
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) xraw[bt][u] = *reinterpret_cast<const uint4*>(xrow[u & 1] + (u >> 1) * 64);
         }
         issue_all();
 
         // ---- x in operand order, (x0, x4) (x2, x6) (x1, x5) / 16 (x3, x7) / 16, and the offset terms
+        // (16-byte chunk k of row r sits at chunk k ^ (r / 2 % 8): the reads of sixteen rows at one k then meet no bank twice)
+        char* const x_lds = reinterpret_cast<char*>(res_lds) + (p.rounds * NBT * 16 + 2 * wave) * 1024;
+        const int x_put = (xl >> 3) * 128, x_get = (xl & 15) * 128;
 #pragma unroll
         for (int bt = 0; bt < NBT; ++bt) {
 #pragma unroll
           for (int u = 0; u < U; ++u) {
+            if (u % 2 == 0) {
+              __builtin_amdgcn_wave_barrier();
+#pragma unroll
+              for (int h = 0; h < 2; ++h)
+                *reinterpret_cast<uint4*>(x_lds + x_put + 1024 * h + (((xl & 7) ^ ((4 * h + (xl >> 4)) & 7)) << 4)) = xraw[bt][u + h];
+              __builtin_amdgcn_wave_barrier();
+#pragma unroll
+              for (int h = 0; h < 2; ++h)
+                xraw[bt][u + h] = *reinterpret_cast<const uint4*>(x_lds + x_get + (((4 * h + (xl >> 4)) ^ ((xl >> 1) & 7)) << 4));
+            }
             uint4 v = xraw[bt][u];
             if (!x_ok[bt]) v = make_uint4(0, 0, 0, 0);
             xa[bt][u][0] = __builtin_amdgcn_perm(v.z, v.x, kLoLo);
@@ -559,7 +584,7 @@ __global__ __launch_bounds__(256) void mid_reduce_silu_kernel(const float* __res
 
 template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16>
 hipError_t launch_mid(const MidParams& p, int wgx, int experts, hipStream_t s) {
-  const size_t lds = static_cast<size_t>(p.rounds) * 16 * NBT * 1024;
+  const size_t lds = (static_cast<size_t>(p.rounds) * NBT + (DT == MODEL_F32 ? 0 : 2)) * 16 * 1024;  // sums, and 2 KiB of x per wave
   if (lds > 160 * 1024) return hipErrorNotSupported;
   if (lds > 64 * 1024) {
     static bool raised = false;  // (idempotent; a race sets the same attribute twice)
