@@ -67,6 +67,7 @@ struct MidParams {
   int phases;              // passes over K (a workgroup covers KW * U groups per phase)
   int slices;              // workgroups along K (plain linears with a workspace: grid z; each covers one phase's worth of
                            // K and leaves fp32 partial sums [slice][rows][N] in y for the reduction kernel)
+  int slice_shares;        // shares of U groups of K in a slice (without slices: kw, the shares of a phase)
   int kw_log2;             // log2 of the waves that share a tile's K
   int out_f32, paired, indptr_i64, x_src_rows;
   int num_experts, x_one_row;  // with ids: experts in the stack; every row reads row 0 of x
@@ -190,9 +191,15 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
 
   for (int pass_lo = seg_lo; pass_lo < seg_hi; pass_lo += BR * NBT) {
     for (int ph = 0; ph < (PHASED ? p.phases : 1); ++ph) {
-      const int ga_raw = ((static_cast<int>(blockIdx.z) + ph) * kw + ks) * U;  // (slices > 1: one phase each)
-      const bool k_live = ga_raw < p.ng;  // (uniform; ng % U == 0: a share is whole or empty)
+      // (slices > 1: each p.slice_shares of K's shares; the phases: kw each.  Uniform; ng % U == 0: a share is whole or empty)
+      const int ga_raw = (static_cast<int>(blockIdx.z) * p.slice_shares + ph * kw + ks) * U;
+      const bool k_live = ga_raw < p.ng && (PHASED || ks < p.slice_shares);
       const int ga = k_live ? ga_raw : p.ng - U;
+      // (a wave without a share of K has descriptors of no bytes: it loads zeros, and no traffic)
+      const __amdgpu_buffer_rsrc_t w_walk = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<uint32_t*>(p.qw + expert * p.expert_w_stride), short(0), k_live ? static_cast<int>(w_bytes) : 0, 0x00020000);
+      const __amdgpu_buffer_rsrc_t s_walk = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<uint16_t*>(p.qs + expert * p.expert_s_stride * (EL / 2)), short(0), k_live ? static_cast<int>(s_bytes) : 0, 0x00020000);
       const int w_lane = (c * p.nw + 4 * (ga + j)) * 4;
       u32x4 w[RT][STEPS];  // (kept as whole register tuples until the point of use, see walk_tile)
       auto issue = [&](int r, u32x4 (&wv)[STEPS]) {
@@ -200,7 +207,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
         const int w_off = static_cast<int>(tile >= 0 ? static_cast<uint32_t>(tile) * w_tile : w_bytes);
 #pragma unroll
         for (int st = 0; st < STEPS; ++st) {
-          wv[st] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_lane + 64 * st, w_off, 0);
+          wv[st] = __builtin_amdgcn_raw_buffer_load_b128(w_walk, w_lane + 64 * st, w_off, 0);
         }
       };
       // scales: the U of this lane's row c.  float32 (PAIR): of the tiles of rounds r and r + 1 in one load, lane (c, j) taking
@@ -219,10 +226,10 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
           const int t1 = tile_of(r + 1);
           const uint32_t o1 = t1 >= 0 ? static_cast<uint32_t>(t1) * s_tile : s_bytes;
           const u32x4 v =
-              __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, s_lane + static_cast<int>(j < 2 ? o0 : o1), 0, 0);
+              __builtin_amdgcn_raw_buffer_load_b128(s_walk, s_lane + static_cast<int>(j < 2 ? o0 : o1), 0, 0);
           sv[0] = v.x; sv[1] = v.y; sv[2] = v.z; sv[3] = v.w;
         } else {
-          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, s_lane, static_cast<int>(o0), 0);
+          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s_walk, s_lane, static_cast<int>(o0), 0);
           sv[0] = v.x; sv[1] = v.y; sv[2] = v.z; sv[3] = v.w;
         }
       };
@@ -435,7 +442,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
           if (tile < 0) break;
           float4_t acc = {0.f, 0.f, 0.f, 0.f}, odd_x = {0.f, 0.f, 0.f, 0.f};  // odd_x: NaN in the rows in question
 #pragma unroll 1
-          for (int g = (static_cast<int>(blockIdx.z) * kw + ks) * U, ph2 = 0; ph2 <= ph && g < p.ng; ++ph2, g += kw * U) {
+          for (int g = ga_raw - ph * kw * U, ph2 = 0; (PHASED || k_live) && ph2 <= ph && g < p.ng; ++ph2, g += kw * U) {
             const uint32_t* const xrow = reinterpret_cast<const uint32_t*>(p.x) + xr * p.K + g * 32 + 8 * j;
 #pragma unroll
             for (int st = 0; st < STEPS; ++st) {
@@ -648,13 +655,18 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   // A plain linear whose K takes several phases and whose caller brings the scratch: one workgroup row per phase's worth of
   // K instead (x stays in registers for all of a workgroup's tiles, the walk comes in chunks), fp32 partial sums in the
   // workspace and a second, small launch that adds them; the fused gate/up form then runs as a plain one and the reduction
-  // folds the activation in.  Tuning override: gemv_ksplit 0 keeps the phases.
+  // folds the activation in.  The slices are as long as one another (K = 14336: four of 14 shares, not three of 16 and one
+  // of 8, whose workgroups would be done first and leave their CUs idle: 15360 x 5120 at 7 / 16 / 32 rows 20.7 / 21.9 / 29.4 -> 18.8 /
+  // 20.1 / 27.5 us, 27648 x 5120 31.9 / 33.4 / 44.4 -> 29.4 / 31.2 / 42.5, 4096 x 14336 16.0 / 16.3 / 20.9 -> 15.5 / 15.6 / 20.2, a K of
+  // whole phases as before).  Tuning override: gemv_ksplit 0 keeps the phases.
   p.slices = 1;
+  p.slice_shares = 1 << kwl;
   bool fold_silu = false;
   if (p.phases > 1 && experts == 1 && !grouped && p.phases <= 64 && options().gemv_ksplit != 0 && a.workspace != nullptr &&
       a.workspace_bytes >= static_cast<int64_t>(p.phases) * p.rows * p.N * 4 &&
       (reinterpret_cast<uintptr_t>(a.workspace) & 15) == 0) {
     p.slices = p.phases;
+    p.slice_shares = (p.ng / U + p.slices - 1) / p.slices;
     p.phases = 1;
     p.y = a.workspace;
     p.bias = nullptr; p.residual = nullptr; p.out_f32 = 1;

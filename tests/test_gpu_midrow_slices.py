@@ -1,0 +1,35 @@
+"""The mid-row kernel's K slices where K is not whole phases: every slice takes the same number of shares, the last one fewer."""
+import numpy as np
+import pytest
+import torch
+
+import mlc_llm_amd as gq
+from mlc_llm_amd import ops
+from oracle import gq_oracle as o
+from test_gpu_parity import SCHEMES, assert_linear_ok, dev, seed_of
+
+pytestmark = pytest.mark.gpu
+
+
+# shares of 256 k in the slices: 9 + 8, 10 + 10, 15 + 14 + 14, 14 each
+@pytest.mark.parametrize("k,slices", [(4352, 2), (5120, 2), (11008, 3), (14336, 4)])
+@pytest.mark.parametrize("m", [5, 16, 17])  # one batch tile, a full one, two
+def test_midrow_kernel_even_slices(m, k, slices):
+    """Against the oracle: the tolerance of every linear test (the products are exact, sums in fp32, one rounding of the result)."""
+    s, n = SCHEMES["q4f16_1"], 544
+    rng = np.random.default_rng(seed_of("even-slices", m, k))
+    qw = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32)
+    qs = (rng.random((n, k // 32)) * 0.02 + 0.001).astype(np.float16)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    out = torch.empty((m, n), dtype=torch.float16, device="cuda")
+    scratch = torch.empty(slices * m * n, dtype=torch.float32, device="cuda")
+    dx, dqw, dqs = dev(x), dev(qw), dev(qs)
+    gq._lib.set_option("gemv_variant", 10)
+    try:
+        gq._lib.call("mi355gq_linear", dx.data_ptr(), dqw.data_ptr(), dqs.data_ptr(), None, m, n, k, 4, 32, gq._lib.F16,
+                     out.data_ptr(), scratch.data_ptr(), scratch.numel() * 4, ops._stream())
+        kern = gq._lib.last_kernel()
+    finally:
+        gq._lib.set_option("gemv_variant", -1)
+    assert kern.startswith("gq::midrow_kernel<") and f"slices={slices} " in kern, kern
+    assert_linear_ok(out, o.linear_fp32(x, qw, qs, s), x, k, f"even slices {m}x{n}x{k} [{kern}]")
