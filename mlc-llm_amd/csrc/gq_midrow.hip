@@ -113,10 +113,10 @@ __device__ __forceinline__ mid_u4 mid_word_bf16(uint32_t w) {
 // PHASED: K takes more than one phase (the sums of all of a wave's rounds stay in LDS between phases: one chunk of rounds);
 // else a wave's rounds come in chunks of p.rounds, each followed by the step that adds the K shares and stores, with x
 // and the ring of loads carried across
-template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16>
-__global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
+template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16, int WV = 16>
+__global__ __launch_bounds__(64 * WV) void midrow_kernel(const MidParams p) {
   constexpr bool BF = DT == MODEL_BF16, F32 = DT == MODEL_F32;
-  static_assert(U == 8 && RT % 2 == 0, "eight scales per row and share; float32 loads them for pairs of tiles");
+  static_assert(U % 8 == 0 && RT % 2 == 0 && (U == 8 || !F32), "scales in whole 16-byte loads; float32 loads them for pairs of tiles");
   constexpr int STEPS = U / 4;
   constexpr int EL = F32 ? 4 : 2;     // bytes of an activation, a scale
   constexpr bool PAIR = F32;        // scales come for pairs of tiles (see issue_scales)
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
   //  then uniform for the compiler as well, which would otherwise wrap every buffer load in a loop over lanes)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, j = lane >> 4;
-  const int kw = 1 << p.kw_log2, tw = 16 >> p.kw_log2;
+  const int kw = 1 << p.kw_log2, tw = WV >> p.kw_log2;
   const int ks = wave & (kw - 1), ti = wave >> p.kw_log2;
   const int tstride = gridDim.x * tw;
   const int base = blockIdx.x * tw + ti;  // this wave's first tile (the fused form: its first gate / up pair)
@@ -229,8 +229,11 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
               __builtin_amdgcn_raw_buffer_load_b128(s_walk, s_lane + static_cast<int>(j < 2 ? o0 : o1), 0, 0);
           sv[0] = v.x; sv[1] = v.y; sv[2] = v.z; sv[3] = v.w;
         } else {
-          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s_walk, s_lane, static_cast<int>(o0), 0);
-          sv[0] = v.x; sv[1] = v.y; sv[2] = v.z; sv[3] = v.w;
+#pragma unroll
+          for (int q = 0; q < SR; q += 4) {
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s_walk, s_lane + 4 * q, static_cast<int>(o0), 0);
+            sv[q] = v.x; sv[q + 1] = v.y; sv[q + 2] = v.z; sv[q + 3] = v.w;
+          }
         }
       };
       auto issue_all = [&]() {
@@ -307,7 +310,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
 
         // ---- x in operand order, (x0, x4) (x2, x6) (x1, x5) / 16 (x3, x7) / 16, and the offset terms
         // (16-byte chunk k of row r sits at chunk k ^ (r / 2 % 8): the reads of sixteen rows at one k then meet no bank twice)
-        char* const x_lds = reinterpret_cast<char*>(res_lds) + (p.rounds * NBT * 16 + 2 * wave) * 1024;
+        char* const x_lds = reinterpret_cast<char*>(res_lds) + (p.rounds * NBT * WV + 2 * wave) * 1024;
         const int x_put = (xl >> 3) * 128, x_get = (xl & 15) * 128;
 #pragma unroll
         for (int bt = 0; bt < NBT; ++bt) {
@@ -472,7 +475,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
               }
             }
           }
-          float* const at = reinterpret_cast<float*>(res_lds + (round * 16 + wave) * 64 + lane_here);
+          float* const at = reinterpret_cast<float*>(res_lds + (round * WV + wave) * 64 + lane_here);
 #pragma unroll
           for (int q = 0; q < 4; ++q)
             if (odd_x[q] != odd_x[q]) at[q] = acc[q];
@@ -493,17 +496,17 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
 #pragma unroll
             for (int pl = 2; pl >= 0; --pl) {
               const int ap = at_row(3 * jq + pl);
-              for (int k = 0; k < kw; ++k) v += res[(((round * 16 + (tl << p.kw_log2) + k) * NBT + bt) << 8) + ap];
+              for (int k = 0; k < kw; ++k) v += res[(((round * WV + (tl << p.kw_log2) + k) * NBT + bt) << 8) + ap];
             }
           } else {
-            for (int k = 0; k < kw; ++k) v += res[(((round * 16 + (tl << p.kw_log2) + k) * NBT + bt) << 8) + at];
+            for (int k = 0; k < kw; ++k) v += res[(((round * WV + (tl << p.kw_log2) + k) * NBT + bt) << 8) + at];
           }
           return F32 ? 512.0f * v : v;
         };
         if (p.paired) {
           const int items = (p.rounds >> 1) * tw * NBT;
           const int half = p.N >> 1;
-          for (int it = threadIdx.x >> 8; it < items; it += 4) {
+          for (int it = threadIdx.x >> 8; it < items; it += WV / 4) {
             const int bt = it % NBT, rest = it / NBT, tl = rest % tw, pr = rest / tw;
             const int pair = blockIdx.x * tw + tl + ((r0 >> 1) + pr) * tstride;
             const int col = pair * 16 + cq, b = pass_lo + BR * bt + jq;
@@ -513,7 +516,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
           }
         } else {
           const int items = p.rounds * tw * NBT;
-          for (int it = threadIdx.x >> 8; it < items; it += 4) {
+          for (int it = threadIdx.x >> 8; it < items; it += WV / 4) {
             const int bt = it % NBT, rest = it / NBT, tl = rest % tw, round = rest / tw;
             const int t = blockIdx.x * tw + tl + (r0 + round) * tstride;
             const int col = t * 16 + cq, b = pass_lo + BR * bt + jq;
@@ -544,7 +547,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
             walk_tile((slot & 1) == 0, r0 + round + slot + RT, w[slot], sraw[PAIR ? slot / 2 : slot], acc);
 #pragma unroll
             for (int bt = 0; bt < NBT; ++bt) {
-              float4* const at = res_lds + (((round + slot) * 16 + wave) * NBT + bt) * 64 + lane;
+              float4* const at = res_lds + (((round + slot) * WV + wave) * NBT + bt) * 64 + lane;
               if constexpr (PHASED) {
                 const float4 old = *at;
                 const bool add = ph > 0;
@@ -559,7 +562,7 @@ __global__ __launch_bounds__(1024) void midrow_kernel(const MidParams p) {
         }
         if (!PHASED || ph + 1 == p.phases) {  // (uniform)
           if constexpr (F32) {
-            const float4 last = res_lds[((p.rounds - 1) * 16 + wave) * 64 + lane];
+            const float4 last = res_lds[((p.rounds - 1) * WV + wave) * 64 + lane];
             const float sum = (last.x + last.y) + (last.z + last.w);
             if (__ballot(sum != sum) != 0) redo_odd_rows(r0);  // (uniform; the sums are this wave's own until the barrier)
           }
@@ -589,14 +592,14 @@ __global__ __launch_bounds__(256) void mid_reduce_silu_kernel(const float* __res
   }
 }
 
-template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16>
+template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16, int WV = 16>
 hipError_t launch_mid(const MidParams& p, int wgx, int experts, hipStream_t s) {
-  const size_t lds = (static_cast<size_t>(p.rounds) * NBT + (DT == MODEL_F32 ? 0 : 2)) * 16 * 1024;  // sums, and 2 KiB of x per wave
+  const size_t lds = (static_cast<size_t>(p.rounds) * NBT + (DT == MODEL_F32 ? 0 : 2)) * WV * 1024;  // sums, and 2 KiB of x per wave
   if (lds > 160 * 1024) return hipErrorNotSupported;
   if (lds > 64 * 1024) {
     static bool raised = false;  // (idempotent; a race sets the same attribute twice)
     if (!raised) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT>),
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT, WV>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
       if (e != hipSuccess) return e;
       raised = true;
@@ -604,7 +607,7 @@ hipError_t launch_mid(const MidParams& p, int wgx, int experts, hipStream_t s) {
   }
   note_kernel("gq::midrow_kernel<%d,%d,%d,%d,%d%s> rounds=%d chunks=%d phases=%d slices=%d kw=%d", NBT, U, RT, int(KEEP_C),
               int(PHASED), DT == MODEL_BF16 ? ",true" : (DT == MODEL_F32 ? ",f32" : ""), p.rounds, p.chunks, p.phases, p.slices, 1 << p.kw_log2);
-  hipLaunchKernelGGL((midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT>), dim3(wgx, experts, p.slices), dim3(1024), lds, s, p);
+  hipLaunchKernelGGL((midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT, WV>), dim3(wgx, experts, p.slices), dim3(64 * WV), lds, s, p);
   return hipGetLastError();
 }
 
@@ -698,6 +701,19 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   wgx = (sets + items - 1) / items;
   int rounds = (items * per_round + unit - 1) / unit * unit;
   p.chunks = (rounds + max_rounds - 1) / max_rounds;
+  // One batch tile and more than one chunk of rounds: eight waves of sixteen groups each instead, whose sums take half the LDS
+  // (twice the rounds per chunk, half as many stops where the shares meet; the sums of half as many shares): 128256 x 4096 at 7 /
+  // 16 rows 63.8 / 67.1 -> 61.1 / 66.5 us, 27648 x 5120 29.4 / 31.2 -> 25.9 / 27.0, 57344 x 8192 61.3 / 65.9 -> 56.7 / 60.9; where one chunk
+  // does, sixteen waves hide more (4096 x 4096 7.4 against 8.1, 28672 x 4096 at 16 rows 19.4 against 19.7).  Two batch tiles lose
+  // with eight waves (128256 x 4096 at 32 rows 81.5 against 86.6).
+  // (The fused gate/up form walks half as many items of two rounds each, so it takes more than one chunk exactly where the plain
+  // form does, and the two add in the same order.)
+  const bool wide = nbt == 1 && !a.f32 && p.phases == 1 && p.chunks > 1 && (a.K & 511) == 0 && options().quad_ksplit < 0 && form < 0;
+  if (wide) {
+    --p.kw_log2;
+    p.slice_shares = p.slices > 1 ? (p.ng / 16 + p.slices - 1) / p.slices : 1 << p.kw_log2;
+    p.chunks = (rounds + 2 * max_rounds - 1) / (2 * max_rounds);
+  }
   p.rounds = ((rounds + p.chunks - 1) / p.chunks + unit - 1) / unit * unit;
   auto run = [&]() -> hipError_t {
     if (a.f32) {
@@ -705,6 +721,9 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
         return launch_mid<1, 8, 2, false, true, MODEL_F32>(p, wgx, experts, s);
       return launch_mid<1, 8, 2, false, false, MODEL_F32>(p, wgx, experts, s);
     }
+    if (wide)
+      return a.bf16 ? launch_mid<1, 16, 2, true, false, MODEL_BF16, 8>(p, wgx, experts, s)
+                    : launch_mid<1, 16, 2, true, false, MODEL_F16, 8>(p, wgx, experts, s);
     if (a.bf16) {  // (the bfloat16 instances: q4bf16_*)
       if (p.phases > 1)
         return nbt == 2 ? launch_mid<2, 8, 2, false, true, MODEL_BF16>(p, wgx, experts, s)

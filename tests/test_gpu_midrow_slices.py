@@ -33,3 +33,34 @@ def test_midrow_kernel_even_slices(m, k, slices):
         gq._lib.set_option("gemv_variant", -1)
     assert kern.startswith("gq::midrow_kernel<") and f"slices={slices} " in kern, kern
     assert_linear_ok(out, o.linear_fp32(x, qw, qs, s), x, k, f"even slices {m}x{n}x{k} [{kern}]")
+
+
+# one batch tile and more than one chunk of rounds (few workgroups): K of one and two shares of sixteen groups, whole, and as slices of five
+# and of seven, eight, ... ; a ragged last tile
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k", [(2600, 512), (1312, 1024), (328, 4096), (552, 5120), (320, 18944)])
+@pytest.mark.parametrize("m", [5, 16])
+def test_midrow_kernel_eight_waves(dtype, m, n, k):
+    """Eight waves of sixteen groups, against the float64 product of the quantised weights (which this kernel does not round): the
+    result's own rounding, 2^-11 / 2^-8 at most and half of it root-mean-square at most, beside sums in fp32 of products around 1031 x."""
+    g = torch.Generator(device="cuda").manual_seed(n + k + m)
+    qw = torch.randint(-2**31, 2**31 - 1, (n, k // 8), device="cuda", dtype=torch.int32, generator=g)
+    qs = (torch.rand((n, k // 32), device="cuda", generator=g) * 0.02 + 0.001).to(dtype)
+    x = torch.randn((m, k), device="cuda", generator=g).to(dtype)
+    q = torch.stack([(qw >> (4 * i)) & 15 for i in range(8)], -1).reshape(n, k).double() - 7
+    ref = x.double() @ (q * qs.double().repeat_interleave(32, 1)).T
+    out = torch.empty((m, n), dtype=dtype, device="cuda")
+    scratch = torch.empty(5 * m * n, dtype=torch.float32, device="cuda")
+    code = gq._lib.F16 if dtype == torch.float16 else gq._lib.BF16
+    gq._lib.set_option("gemv_variant", 10)
+    gq._lib.set_option("gemv_waves", 16)  # one workgroup per slice
+    try:
+        gq._lib.call("mi355gq_linear_dt", x.data_ptr(), qw.data_ptr(), qs.data_ptr(), None, m, n, k, 4, 32, code, code,
+                     out.data_ptr(), scratch.data_ptr(), scratch.numel() * 4, ops._stream())
+        kern = gq._lib.last_kernel()
+    finally:
+        gq._lib.set_option("gemv_variant", -1)
+        gq._lib.set_option("gemv_waves", -1)
+    assert kern.startswith("gq::midrow_kernel<1,16,"), kern
+    err = (out.double() - ref).norm() / ref.norm()
+    assert err <= (2.0**-11 if dtype == torch.float16 else 2.0**-8), (kern, err)
