@@ -320,16 +320,50 @@ int mi355gq_embedding_take_dt(const void* ids, int64_t T, const void* q_weight, 
                     "embedding_take_dt launch");
 }
 
+// Rows and shapes of a q4 linear that run on the kernel on unscaled weight operands (gq_midrow.hip; K % 256 == 0, N % 32 == 0), in
+// us against the kernel that would run otherwise.  slices: K beyond 4096 runs as K slices over workgroups, for which the caller
+// has brought the scratch.  The same rule for the plain and the fused gate/up form: both must add in the same order.
+static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16) {
+  const int64_t weights = N * K;
+  const auto mi = [](int64_t n) { return n << 20; };
+  if (M <= 4 || M > 32) return false;
+  if (M <= 8) {
+    // against the quad-row kernel with x in registers: a K that is not 2048 or 4096 leaves some of its waves without a share
+    // (5 / 8 rows: 4096 x 2560 7.9 / 7.7 -> 6.9 / 6.9, 8192 x 3072 10.2 / 10.4 -> 7.9 / 7.8, 4608 x 3584 9.3 / 9.2 -> 7.4 / 7.5, 37888 x 3584 24.0 / 25.8
+    // -> 20.3 / 20.6); for 4096 it is ahead on the smaller matrices (4096 x 4096 6.4 / 6.1 against 7.6, 12288 x 4096 11.4 / 11.0 against
+    // 11.6 / 11.7, 20480 x 4096 15.3 / 15.4 against 15.2 / 16.2) and behind from about 84 M weights on (22016 x 4096 16.9 / 16.4 -> 16.4 / 16.0,
+    // 28672 x 4096 at 7 rows 21.8 -> 18.4, 128256 x 4096 64.7 / 65.0 -> 62.3 / 63.1; bfloat16 from 112 M, 67.3 / 69.9 -> 62.4 / 63.8)
+    if (K <= 4096) return (K > 2048 && K < 4096 && weights >= mi(10)) || weights >= (bf16 ? mi(112) : mi(84));
+    // K slices: 5120 x 5120 12.3 / 12.0 -> 11.2, 8192 x 5120 15.3 / 15.6 -> 12.5 / 12.9, 8192 x 7168 16.4 / 17.3 -> 13.8 / 14.3, 27648 x 5120 34.9 /
+    // 35.5 -> 25.8 / 26.2; 2048 x 5632 stays (8.4 / 8.1 against 9.3); 57344 x 8192 65.5 / 66.3 -> 58.1 / 58.8, 10240 x 8192 stays (16.9 / 15.9
+    // against 17.8 / 17.5).  Beyond 8192 the quad-row kernel reads x from LDS, once per four rows and K share: 4096 x 11008 14.0 / 14.4 ->
+    // 13.3 / 13.4, 4096 x 14336 15.8 / 16.1 -> 15.4 / 15.5 (bfloat16 16.6 / 17.5 -> 15.5 / 15.6), 8192 x 28672 46.1 / 47.3 -> 34.9 / 35.0; 4096 x 9216
+    // stays (12.1 / 12.2 against 12.5)
+    if (K <= 8192) return slices && ((K < 8192 && weights >= mi(24)) || weights >= mi(256));
+    return slices && weights >= mi(40);
+  }
+  if (M <= 16) {
+    // against the skinny kernel (bfloat16: the GEMM's 32-row tile; 9 / 16 rows): 4096 x 4096 9.4 / 9.4 -> 7.5 / 7.4, 3584 x 3584 9.3 / 9.4 -> 7.2 / 7.4,
+    // 11264 x 2048 11.4 / 11.6 -> 8.4 / 8.5, 2048 x 5632 11.5 / 11.6 -> 9.3 / 9.4, 28672 x 4096 27.8 / 28.1 -> 18.3 / 19.4; 4096 x 2048 (6.9 / 7.0
+    // against 7.1) and smaller stay, in bfloat16 down to 4 M weights they do not (2048 x 2048 at 16 rows 9.4 -> 6.9).  Without the scratch a
+    // K of two phases from 48 M weights on (8192 x 8192 21 -> 17-18.5)
+    return K <= 4096 ? weights >= (bf16 ? mi(4) : mi(10)) : (slices && weights >= mi(10)) || (K <= 8192 && weights >= mi(48));
+  }
+  // 17..32 rows, two batch tiles, against the GEMM's 32-row tile and its split of K (17 / 32 rows): 2048 x 2048 8.9 / 10.0 -> 8.3 / 8.4,
+  // 4096 x 4096 11.8 / 12.4 -> 9.1 / 9.1, 6144 x 4096 12.9 / 13.9 -> 9.3 / 9.7, 12288 x 4096 16.9 / 18.9 -> 14.7 / 16.0, 128256 x 4096 98 / 102 -> 80.6 /
+  // 81.5; bfloat16 4096 x 4096 12.3 / 13.0 -> 9.6 / 9.7, 28672 x 4096 31.6 / 32.4 -> 28.6 / 30.3, 128256 x 4096 99 / 102 -> 87 / 92.  K slices where
+  // they are whole and many: 10240 x 8192 27.5 / 28.5 -> 25.7 / 27.6, 8192 x 28672 50.2 / 52.5 -> 47.2 / 50.4, 57344 x 8192 97 -> 77; half of
+  // the waves without a share loses (27648 x 5120 33.6 / 34.4 against 42)
+  return K <= 4096 ? weights >= mi(4) : slices && ((K % 4096 == 0 && weights >= mi(80)) || weights >= mi(256));
+}
+
 // with_slices false: what the shape needs when the K slices of the kernel on unscaled weight operands go without
 static int64_t linear_workspace_need(int64_t M, int64_t N, int64_t K, int bits, int group_size, bool with_slices) {
   if (check_scheme(bits, group_size) != MI355GQ_OK || M < 0 || N < 0 || K < 0 || M >= kMaxDim ||
       N >= kMaxDim || K >= kMaxDim)
     return 0;
-  // q4 at 9..32 rows of a K beyond 4096, at 5..8 rows of a K beyond 8192: the K slices of the kernel on unscaled weight
-  // operands (see linear_impl)
-  const int64_t mid = (with_slices && bits == 4 && M <= 32 && (M > 8 || (M > 4 && K > 8192)))
-                          ? gq::midrow_workspace_bytes(M, N, K)
-                          : 0;
+  // q4 at 5..32 rows of a K beyond 4096: the K slices of the kernel on unscaled weight operands (see midrow_takes)
+  const int64_t mid = (with_slices && bits == 4 && M <= 32 && M > 4) ? gq::midrow_workspace_bytes(M, N, K) : 0;
   // only the few-row GEMM (more rows than the GEMV / skinny kernels take, at most 256) splits K
   // (q4 at 9..16 rows: the skinny kernel, except on matrices of 40 M to 256 M weights, see linear_impl)
   if (M <= 16 && bits == 4 && !(M > 8 && N * K >= (40ll << 20) && N * K < (256ll << 20))) return mid;
@@ -382,9 +416,9 @@ int64_t mi355gq_linear_dt_workspace_bytes(int64_t M, int64_t N, int64_t K, int b
   if (model_dtype != MI355GQ_BF16 || check_scheme(bits, group_size) != MI355GQ_OK || M < 2 || N < 0 || K < 0 ||
       M >= kMaxDim || N >= kMaxDim || K >= kMaxDim)
     return 0;
-  // bfloat16: every batch from two rows on may run the few-row GEMM (there are no bf16 skinny kernels); 9..16 rows of a
+  // bfloat16: every batch from two rows on may run the few-row GEMM (there are no bf16 skinny kernels); 5..32 rows of a
   // long K: the K slices of the kernel on unscaled weight operands
-  const int64_t mid = (bits == 4 && M <= 16 && (M > 8 || (M > 4 && K > 8192))) ? gq::midrow_workspace_bytes(M, N, K) : 0;
+  const int64_t mid = (bits == 4 && M <= 32 && M > 4) ? gq::midrow_workspace_bytes(M, N, K) : 0;
   const int64_t gemm = gq::gemm_workspace_bytes(M, N, K, bits, group_size, 1);
   return gemm > mid ? gemm : mid;
 }
@@ -393,11 +427,8 @@ int64_t mi355gq_linear_silu_mul_workspace_bytes(int64_t M, int64_t N, int64_t K,
   if (check_scheme(bits, group_size) != MI355GQ_OK || M < 0 || N < 0 || K < 0 || M >= kMaxDim ||
       N >= kMaxDim || K >= kMaxDim)
     return 0;
-  // q4 at 9..32 rows of a K beyond 4096, at 5..8 rows of a K beyond 8192: the K slices of the kernel on unscaled weight
-  // operands (as the plain linear)
-  const int64_t mid = (bits == 4 && M <= 32 && (M > 8 || (M > 4 && K > 8192)) && (N % 32) == 0)
-                          ? gq::midrow_workspace_bytes(M, N, K)
-                          : 0;
+  // q4 at 5..32 rows of a K beyond 4096: the K slices of the kernel on unscaled weight operands (as the plain linear)
+  const int64_t mid = (bits == 4 && M <= 32 && M > 4 && (N % 32) == 0) ? gq::midrow_workspace_bytes(M, N, K) : 0;
   // GEMV / few-row kernels
   if (M <= 8 || (N % 2) != 0) return mid;
   if (M <= 16 && bits == 4 && !(N * K >= (40ll << 20) && N * K < (256ll << 20))) return mid;
@@ -457,31 +488,11 @@ static int linear_impl(const void* x, const void* q_weight, const void* q_scale,
     const int64_t need = gq::gemm_workspace_bytes(M, N, K, bits, group_size, 0, paired);
     q4_skinny_loses = need == 0 || (workspace != nullptr && workspace_bytes >= need);
   }
-  // q4, 9..16 rows of a K that one phase covers (up to 4096; two phases: below), from about 24 M weights on: the kernel that multiplies
-  // unscaled weight operands and scales the matrix instruction's result (28672 x 4096 at 9 / 16 rows 20.0 / 20.3 us
-  // against 27.8-28.1 for the GEMM's 32-row tile, 6144 x 4096 10.4 / 10.9 against 12.2 / 13.1 for the skinny kernel;
-  // 4096 x 4096 stays with the skinny kernel, 9.0-9.4 either way, and a longer K with the GEMM's tiles, 4096 x 14336
-  // 26-27 against 20).  The same test for the plain and the fused gate/up form: both must add in the same order.
-  // (K of two phases, up to 8192, from 48 M weights on: 10240 x 8192 28 -> 21-22 us, 8192 x 8192 21 -> 17-18.5, 57344 x 8192
-  //  100-106 -> 74-78, 15360 x 5120 24.5 -> 21-22, 27648 x 5120 33.4-34.4 -> 32.4-33.8)
-  // 17..32 rows (two batch tiles per pass, the offsets subtracted from the weight operand): one phase and 48 M weights or more
-  // (14336 x 4096 at 17 / 24 / 32 rows 19.4 / 19.9 / 20.4 -> 16.9 / 17.9 / 19.0 us, 28672 x 4096 28.3 / 28.0 / 27.9 -> 26.0 / 26.1 / 27.5, 128256 x
-  //  4096 99-101 -> 84-87; 6144 x 4096 13.4-14.4 against 12.3-14.1 and 4096 x 4096 stay with the GEMM's tile).
-  // A longer K runs as K slices over workgroups where the caller brings the scratch for their partial sums
-  // (mi355gq_linear_workspace_bytes), ahead of the phases everywhere and of the GEMM's tiles at 9..16 rows from 24 M weights
-  // on (4096 x 14336 20.1 / 19.5 -> 16.5 / 17.2 us at 9 / 16 rows, 5120 x 13824 24.2 / 24.7 -> 18.7 / 19.4, 8192 x 28672 49.7 / 51.9 -> 38.7 / 39.8,
-  //  57344 x 8192 72.9 / 77.4 in phases -> 64.5 / 68.1) and at 17..32 rows from 256 M weights on (57344 x 8192 97 -> 85; 4096 x 14336
-  //  20.0 against 22.1 and 8192 x 28672 52 against 52 stay with the tiles).
+  // q4, 5..32 rows: the kernel that multiplies unscaled weight operands and scales the matrix instruction's result; a K beyond 4096
+  // as K slices over workgroups where the caller brings the scratch for their partial sums (mi355gq_linear_workspace_bytes)
   const bool slices_ok = K > 4096 && workspace != nullptr && aligned16(workspace) &&
                          workspace_bytes >= gq::midrow_workspace_bytes(M, N, K) && gq::options().gemv_ksplit != 0;
-  // 5..8 rows of a K beyond 8192 from 64 M weights on, as K slices: the quad-row kernels read x once per four rows and K
-  // share there (8192 x 28672 at 5 / 8 rows 46.1 / 47.3 -> 37.0 us, 5120 x 13824 22.3 / 23.2 -> 18.2 / 18.6; 4096 x 14336 15.3-16.1 against
-  // 15.9-16.2 and up to four rows, 36.6 against 36.5 and 17.2 against 18.4, stay with them)
-  const bool mid_size =
-      (M > 4 && M <= 8 && slices_ok && K > 8192 && N * K >= (64ll << 20)) ||
-      (M > 8 && M <= 16 && N * K >= (24ll << 20) && (K <= 4096 || slices_ok || (K <= 8192 && N * K >= (48ll << 20)))) ||
-      (M > 16 && M <= 32 && ((K <= 4096 && N * K >= (48ll << 20)) || (slices_ok && N * K >= (256ll << 20))));
-  const bool mid_rows = bits == 4 && mid_size && gq::options().gemm_variant < 0 &&
+  const bool mid_rows = bits == 4 && midrow_takes(M, N, K, slices_ok, false) && gq::options().gemm_variant < 0 &&
                         (gq::options().gemv_variant < 0 || gq::options().gemv_variant == 10) && (K & 255) == 0 &&
                         (N & 31) == 0;
   if (mid_rows || gq::options().gemv_variant == 10) {  // (10: forced, whatever the shape)
@@ -882,21 +893,13 @@ static int linear_dt_impl(const void* x, const void* q_weight, const void* q_sca
     g.workspace = workspace; g.workspace_bytes = workspace ? workspace_bytes : 0;
     g.bf16 = 1;
     g.paired = paired;
-    // 9..16 rows of q4: the bfloat16 instance of the float16 linear's kernel for this range (ahead of the few-row kernels
-    // below because a long K takes it from five rows on); K of one phase from 4 M
-    // weights on (there is no bfloat16 skinny kernel: 6144 x 4096 at 16 rows 30.4 -> 10.8 us, 28672 x 4096 31.5 -> 20.3,
-    // 128256 x 4096 105 -> 71, 4096 x 4096 12.2 -> 9.4, 2048 x 2048 9.4 -> 8.8)
+    // 5..32 rows of q4: the bfloat16 instance of the float16 linear's kernel for this range, ahead of the few-row kernels below
+    // (there is no bfloat16 skinny kernel)
     {
       const int gvm = gq::options().gemv_variant;
       const bool slices_ok = K > 4096 && workspace != nullptr && aligned16(workspace) &&
                              workspace_bytes >= gq::midrow_workspace_bytes(M, N, K) && gq::options().gemv_ksplit != 0;
-      // (5..8 rows of a K beyond 8192 from 64 M weights on, as K slices, like the float16 linear: 8192 x 28672 at 5 / 8 rows
-      //  49.1 / 50.6 -> 38.0 / 37.5 us, 5120 x 13824 23.1 / 23.7 -> 18.6 / 18.2; 4096 x 14336 15.5-16.3 against 15.7-16.1 stays)
-      const bool mid_size =
-          (M > 4 && M <= 8 && slices_ok && K > 8192 && N * K >= (64ll << 20)) ||
-          (M > 8 && M <= 16 &&
-           ((K <= 4096 && N * K >= (4ll << 20)) || (slices_ok && N * K >= (24ll << 20)) || (K <= 8192 && N * K >= (48ll << 20))));
-      const bool mid_rows = bits == 4 && mid_size && gq::options().gemm_variant < 0 && gvm < 0 && (K & 255) == 0 && (N & 31) == 0;
+      const bool mid_rows = bits == 4 && midrow_takes(M, N, K, slices_ok, true) && gq::options().gemm_variant < 0 && gvm < 0 && (K & 255) == 0 && (N & 31) == 0;
       if (mid_rows || gvm == 10) {
         const hipError_t e = gq::launch_midrow(g, static_cast<int>(M), as_stream(stream));
         if (e != hipErrorNotSupported) return hip_result(e, "linear_dt mid-row launch");
@@ -940,7 +943,7 @@ int64_t mi355gq_linear_silu_mul_dt_workspace_bytes(int64_t M, int64_t N, int64_t
   if (model_dtype != MI355GQ_BF16 || check_scheme(bits, group_size) != MI355GQ_OK || M < 2 || N < 0 || K < 0 || M >= kMaxDim ||
       N >= kMaxDim || K >= kMaxDim || (N % 2) != 0)
     return 0;
-  const int64_t mid = (bits == 4 && M <= 16 && (M > 8 || (M > 4 && K > 8192)) && (N % 32) == 0) ? gq::midrow_workspace_bytes(M, N, K) : 0;
+  const int64_t mid = (bits == 4 && M <= 32 && M > 4 && (N % 32) == 0) ? gq::midrow_workspace_bytes(M, N, K) : 0;
   const int64_t gemm = gq::gemm_workspace_bytes(M, N, K, bits, group_size, 1, 1);
   return gemm > mid ? gemm : mid;
 }

@@ -113,8 +113,11 @@ __device__ __forceinline__ mid_u4 mid_word_bf16(uint32_t w) {
 // PHASED: K takes more than one phase (the sums of all of a wave's rounds stay in LDS between phases: one chunk of rounds);
 // else a wave's rounds come in chunks of p.rounds, each followed by the step that adds the K shares and stores, with x
 // and the ring of loads carried across
-template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16, int WV = 16>
-__global__ __launch_bounds__(64 * WV) void midrow_kernel(const MidParams p) {
+// ONCE: every tile of a wave is in its first ring of loads (p.rounds == RT): nothing is loaded behind it, and a round without a
+// tile is left out instead of walked over zeros
+template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT, int WV, bool ONCE>
+__device__ __forceinline__ void midrow_body(const MidParams& p) {
+  static_assert(!ONCE || (!PHASED && DT != MODEL_F32), "one chunk, and no look at the last round's sums");
   constexpr bool BF = DT == MODEL_BF16, F32 = DT == MODEL_F32;
   static_assert(U % 8 == 0 && RT % 2 == 0 && (U == 8 || !F32), "scales in whole 16-byte loads; float32 loads them for pairs of tiles");
   constexpr int STEPS = U / 4;
@@ -422,8 +425,10 @@ __global__ __launch_bounds__(64 * WV) void midrow_kernel(const MidParams p) {
         }
         // (after the arithmetic: the loads then land in the very registers the tile has left, with no copies whose
         //  wait would drain the queue)
-        issue(next, wv);
-        if (!PAIR || first) issue_scales(next, sp);
+        if constexpr (!ONCE) {
+          issue(next, wv);
+          if (!PAIR || first) issue_scales(next, sp);
+        }
       };
 
       // (float32) the sums of a chunk of rounds in the rows whose shares of x hold infinities or NaNs, which are then all that
@@ -538,9 +543,10 @@ __global__ __launch_bounds__(64 * WV) void midrow_kernel(const MidParams p) {
       // ---- the walk: p.rounds is a multiple of RT (rounds past the last tile read nothing and leave zeros in LDS slots
       //      that nobody reads).  Later phases add to what the earlier ones left (the read is unconditional and the
       //      first phase drops it: no branch inside the walk).
-      for (int chunk = 0; chunk < p.chunks; ++chunk) {
-        const int r0 = chunk * p.rounds;
-        for (int round = 0; round < p.rounds; round += RT) {
+      const int chunks = ONCE ? 1 : p.chunks, rounds = ONCE ? RT : p.rounds;
+      for (int chunk = 0; chunk < chunks; ++chunk) {
+        const int r0 = chunk * rounds;
+        for (int round = 0; round < rounds; round += RT) {
 #pragma unroll
           for (int slot = 0; slot < RT; ++slot) {
             float4_t acc[NBT];
@@ -573,6 +579,16 @@ __global__ __launch_bounds__(64 * WV) void midrow_kernel(const MidParams p) {
       }
     }
   }
+}
+
+template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT, int WV>
+__global__ __launch_bounds__(64 * WV) void midrow_kernel(const MidParams p) {
+  midrow_body<NBT, U, RT, KEEP_C, PHASED, DT, WV, false>(p);
+}
+
+template <int NBT, int U, int RT, bool KEEP_C, int DT>
+__global__ __launch_bounds__(1024) void midonce_kernel(const MidParams p) {
+  midrow_body<NBT, U, RT, KEEP_C, false, DT, 16, true>(p);
 }
 
 // y[b][j] = silu(sum over slices of part[s][b][j]) * (sum over slices of part[s][b][N / 2 + j]), in the model dtype
@@ -608,6 +624,22 @@ hipError_t launch_mid(const MidParams& p, int wgx, int experts, hipStream_t s) {
   note_kernel("gq::midrow_kernel<%d,%d,%d,%d,%d%s> rounds=%d chunks=%d phases=%d slices=%d kw=%d", NBT, U, RT, int(KEEP_C),
               int(PHASED), DT == MODEL_BF16 ? ",true" : (DT == MODEL_F32 ? ",f32" : ""), p.rounds, p.chunks, p.phases, p.slices, 1 << p.kw_log2);
   hipLaunchKernelGGL((midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT, WV>), dim3(wgx, experts, p.slices), dim3(64 * WV), lds, s, p);
+  return hipGetLastError();
+}
+
+template <int DT>
+hipError_t launch_mid_once(const MidParams& p, int wgx, int experts, hipStream_t s) {
+  constexpr int NBT = 2, RT = 2;
+  constexpr size_t lds = (RT * NBT + 2) * 16 * 1024;  // (96 KiB)
+  static bool raised = false;  // (idempotent; a race sets the same attribute twice)
+  if (!raised) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&midonce_kernel<NBT, 8, RT, false, DT>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e != hipSuccess) return e;
+    raised = true;
+  }
+  note_kernel("gq::midonce_kernel<%d,8,%d,0%s> slices=%d kw=%d", NBT, RT, DT == MODEL_BF16 ? ",true" : "", p.slices, 1 << p.kw_log2);
+  hipLaunchKernelGGL((midonce_kernel<NBT, 8, RT, false, DT>), dim3(wgx, experts, p.slices), dim3(1024), lds, s, p);
   return hipGetLastError();
 }
 
@@ -716,6 +748,8 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   }
   p.rounds = ((rounds + p.chunks - 1) / p.chunks + unit - 1) / unit * unit;
   auto run = [&]() -> hipError_t {
+    if (nbt == 2 && !grouped && p.phases == 1 && p.chunks == 1 && p.rounds == 2 && options().gemv_variant < 0)
+      return a.bf16 ? launch_mid_once<MODEL_BF16>(p, wgx, experts, s) : launch_mid_once<MODEL_F16>(p, wgx, experts, s);
     if (a.f32) {
       if (p.phases > 1)
         return launch_mid<1, 8, 2, false, true, MODEL_F32>(p, wgx, experts, s);

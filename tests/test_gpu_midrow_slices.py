@@ -64,3 +64,31 @@ def test_midrow_kernel_eight_waves(dtype, m, n, k):
     assert kern.startswith("gq::midrow_kernel<1,16,"), kern
     err = (out.double() - ref).norm() / ref.norm()
     assert err <= (2.0**-11 if dtype == torch.float16 else 2.0**-8), (kern, err)
+
+
+# at most two tiles per wave: K of eight, sixteen and fifteen shares (one idle wave); as few tiles as the dispatch sends, two rounds filled to
+# the last tile, one tile more (the walk with a ring)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k,once", [(2048, 2048, True), (16384, 2048, True), (8192, 4096, True), (8224, 4096, False), (1120, 3840, True)])
+@pytest.mark.parametrize("m", [17, 32])
+def test_midrow_kernel_of_two_rounds(dtype, m, n, k, once):
+    """The default dispatch at 17..32 rows, against the float64 product of the quantised weights (tolerance: see above); bias and residual
+    with a float32 result, where what is left are sums in fp32; the fused gate/up form against the two steps."""
+    g = torch.Generator(device="cuda").manual_seed(n + k + m)
+    qw = torch.randint(-2**31, 2**31 - 1, (n, k // 8), device="cuda", dtype=torch.int32, generator=g)
+    qs = (torch.rand((n, k // 32), device="cuda", generator=g) * 0.02 + 0.001).to(dtype)
+    x, b, r = (torch.randn(shape, device="cuda", generator=g).to(dtype) for shape in ((m, k), (n,), (m, n)))
+    q = torch.stack([(qw >> (4 * i)) & 15 for i in range(8)], -1).reshape(n, k).double() - 7
+    ref = x.double() @ (q * qs.double().repeat_interleave(32, 1)).T
+    words = qw.view(torch.uint32)
+    y = ops.linear(x, words, qs, 4, 32)
+    kern = gq._lib.last_kernel()
+    assert kern.startswith("gq::midonce_kernel<2,") == once, kern
+    y32 = ops.linear(x, words, qs, 4, 32, b, torch.float32, residual=r)
+    fused = ops.linear_silu_mul(x, words, qs, 4, 32)
+    err = (y.double() - ref).norm() / ref.norm()
+    assert err <= (2.0**-11 if dtype == torch.float16 else 2.0**-8), (kern, err)
+    want = ref + b.double() + r.double()
+    err32 = (y32.double() - want).norm() / want.norm()
+    assert err32 <= 5e-6 + 1e-7 * k**0.5, (kern, err32)
+    assert torch.equal(fused, ops.silu_mul(y))
