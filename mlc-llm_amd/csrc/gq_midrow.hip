@@ -257,15 +257,46 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
         static_assert(!F32 || (NBT == 1 && !KEEP_C), "one batch tile, offsets from the operand");
         const int b = pass_lo + c / 3;
         const bool ok = k_live && c < 3 * BR && b < seg_hi;
-        const int64_t xr = p.x_one_row ? 0 : x_row(p.x_rows, p.x_src_rows, ok ? b : seg_lo);
-        const float* const xrow = reinterpret_cast<const float*>(p.x) + xr * p.K + ga * 32 + 8 * j;
         uint4 lo[U], hi[U];
+        if constexpr (PHASED) {
+          const int64_t xr = p.x_one_row ? 0 : x_row(p.x_rows, p.x_src_rows, ok ? b : seg_lo);
+          const float* const xrow = reinterpret_cast<const float*>(p.x) + xr * p.K + ga * 32 + 8 * j;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          lo[u] = *reinterpret_cast<const uint4*>(xrow + u * 32);
-          hi[u] = *reinterpret_cast<const uint4*>(xrow + u * 32 + 4);
+          for (int u = 0; u < U; ++u) {
+            lo[u] = *reinterpret_cast<const uint4*>(xrow + u * 32);
+            hi[u] = *reinterpret_cast<const uint4*>(xrow + u * 32 + 4);
+          }
+          issue_all();  // (behind the loads of x: those are needed first, and loads retire in issue order)
+        } else {
+          // Each row's 1 KiB is one load (a lane's own two 16 bytes per group would be sixteen of them, three lanes asking for
+          // the same), and the lanes take theirs from LDS: the wave's own slots for the sums of rounds 0 .. 4, a KiB each,
+          // are free until its walk begins.  Chunk k of row i sits at chunk k + 3 i: five rows at one k meet no bank twice.
+          // (5 rows: 4096 x 4096 11.0 -> 10.3 us, 6144 x 4096 11.4 -> 10.3, 28672 x 4096 23.8 -> 23.2, 128256 x 4096 80.5 -> 78.0, 4096 x 14336
+          // 19.4 -> 18.6.  The phases keep sums in these slots, and a lane's own loads.)
+          int xl = threadIdx.x & 63;
+          asm volatile("" : "+v"(xl));  // (what follows from it is made here, not kept in registers through the walk)
+          const int bl = pass_lo + (xl < BR ? xl : 0);
+          const int row_of_lane = p.x_one_row ? 0 : static_cast<int>(x_row(p.x_rows, p.x_src_rows, bl < seg_hi ? bl : seg_lo));
+          uint4 xw[BR];
+#pragma unroll
+          for (int i = 0; i < BR; ++i) {
+            const int64_t xr = __builtin_amdgcn_readlane(row_of_lane, i);
+            xw[i] = *reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(p.x) + xr * p.K + ga * 32 + 4 * xl);
+          }
+          issue_all();
+          char* const x_lds = reinterpret_cast<char*>(res_lds) + wave * 1024;
+#pragma unroll
+          for (int i = 0; i < BR; ++i) *reinterpret_cast<uint4*>(x_lds + i * 16384 + (((xl + 3 * i) & 63) << 4)) = xw[i];
+          __builtin_amdgcn_wave_barrier();
+          const int xi = min((xl & 15) / 3, BR - 1);
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int at = 8 * u + 2 * (xl >> 4) + 3 * xi;
+            lo[u] = *reinterpret_cast<const uint4*>(x_lds + xi * 16384 + ((at & 63) << 4));
+            hi[u] = *reinterpret_cast<const uint4*>(x_lds + xi * 16384 + (((at + 1) & 63) << 4));
+          }
+          __builtin_amdgcn_wave_barrier();
         }
-        issue_all();  // (behind the loads of x: those are needed first, and loads retire in issue order)
         // (masks: selects become branches behind the loads, which wait for all of them, the ring's included)
         uint32_t live_x = ok ? 0xffffffffu : 0u, minus_h = pl > 0 ? 0xffff0000u : 0u, minus_m = pl > 1 ? 0xffff0000u : 0u;
         asm volatile("" : "+v"(live_x), "+v"(minus_h), "+v"(minus_m));
@@ -610,7 +641,9 @@ __global__ __launch_bounds__(256) void mid_reduce_silu_kernel(const float* __res
 
 template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16, int WV = 16>
 hipError_t launch_mid(const MidParams& p, int wgx, int experts, hipStream_t s) {
-  const size_t lds = (static_cast<size_t>(p.rounds) * NBT + (DT == MODEL_F32 ? 0 : 2)) * WV * 1024;  // sums, and 2 KiB of x per wave
+  // the sums, and 2 KiB of x per wave (float32: x in the slots of five rounds' sums)
+  const int slots = DT == MODEL_F32 ? (PHASED || p.rounds > 5 ? p.rounds : 5) : p.rounds * NBT + 2;
+  const size_t lds = static_cast<size_t>(slots) * WV * 1024;
   if (lds > 160 * 1024) return hipErrorNotSupported;
   if (lds > 64 * 1024) {
     static bool raised = false;  // (idempotent; a race sets the same attribute twice)
