@@ -347,13 +347,15 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
     // 11264 x 2048 11.4 / 11.6 -> 8.4 / 8.5, 2048 x 5632 11.5 / 11.6 -> 9.3 / 9.4, 28672 x 4096 27.8 / 28.1 -> 18.3 / 19.4; 4096 x 2048 (6.9 / 7.0
     // against 7.1) and smaller stay, in bfloat16 down to 4 M weights they do not (2048 x 2048 at 16 rows 9.4 -> 6.9).  Without the scratch a
     // K of two phases from 48 M weights on (8192 x 8192 21 -> 17-18.5)
-    return K <= 4096 ? weights >= (bf16 ? mi(4) : mi(10)) : (slices && weights >= mi(10)) || (K <= 8192 && weights >= mi(48));
+    // (bfloat16 K slices from 24 M: below, the GEMM keeps a row's infinities, which the kept offsets make NaN)
+    return K <= 4096 ? weights >= (bf16 ? mi(4) : mi(10)) : (slices && weights >= (bf16 ? mi(24) : mi(10))) || (K <= 8192 && weights >= mi(48));
   }
   // 17..32 rows, two batch tiles, against the GEMM's 32-row tile and its split of K (17 / 32 rows): 2048 x 2048 8.9 / 10.0 -> 8.3 / 8.4,
   // 4096 x 4096 11.8 / 12.4 -> 9.1 / 9.1, 6144 x 4096 12.9 / 13.9 -> 9.3 / 9.7, 12288 x 4096 16.9 / 18.9 -> 14.7 / 16.0, 128256 x 4096 98 / 102 -> 80.6 /
-  // 81.5; bfloat16 4096 x 4096 12.3 / 13.0 -> 9.6 / 9.7, 28672 x 4096 31.6 / 32.4 -> 28.6 / 30.3, 128256 x 4096 99 / 102 -> 87 / 92.  K slices where
-  // they are whole and many: 10240 x 8192 27.5 / 28.5 -> 25.7 / 27.6, 8192 x 28672 50.2 / 52.5 -> 47.2 / 50.4, 57344 x 8192 97 -> 77; half of
-  // the waves without a share loses (27648 x 5120 33.6 / 34.4 against 42)
+  // 81.5.  K slices where they are whole and many: 10240 x 8192 27.5 / 28.5 -> 25.7 / 27.6, 8192 x 28672 50.2 / 52.5 -> 47.2 / 50.4,
+  // 57344 x 8192 97 -> 77; half of the waves without a share loses (27648 x 5120 33.6 / 34.4 against 42).  bfloat16 stays with the GEMM:
+  // its instance is ahead (4096 x 4096 12.3 / 13.0 -> 9.6 / 9.7) but makes NaN of an infinity, offset included, where the GEMM keeps it
+  if (bf16) return false;
   return K <= 4096 ? weights >= mi(4) : slices && ((K % 4096 == 0 && weights >= mi(80)) || weights >= mi(256));
 }
 
@@ -416,9 +418,9 @@ int64_t mi355gq_linear_dt_workspace_bytes(int64_t M, int64_t N, int64_t K, int b
   if (model_dtype != MI355GQ_BF16 || check_scheme(bits, group_size) != MI355GQ_OK || M < 2 || N < 0 || K < 0 ||
       M >= kMaxDim || N >= kMaxDim || K >= kMaxDim)
     return 0;
-  // bfloat16: every batch from two rows on may run the few-row GEMM (there are no bf16 skinny kernels); 5..32 rows of a
+  // bfloat16: every batch from two rows on may run the few-row GEMM (there are no bf16 skinny kernels); 5..16 rows of a
   // long K: the K slices of the kernel on unscaled weight operands
-  const int64_t mid = (bits == 4 && M <= 32 && M > 4) ? gq::midrow_workspace_bytes(M, N, K) : 0;
+  const int64_t mid = (bits == 4 && M <= 16 && M > 4) ? gq::midrow_workspace_bytes(M, N, K) : 0;
   const int64_t gemm = gq::gemm_workspace_bytes(M, N, K, bits, group_size, 1);
   return gemm > mid ? gemm : mid;
 }
@@ -893,7 +895,7 @@ static int linear_dt_impl(const void* x, const void* q_weight, const void* q_sca
     g.workspace = workspace; g.workspace_bytes = workspace ? workspace_bytes : 0;
     g.bf16 = 1;
     g.paired = paired;
-    // 5..32 rows of q4: the bfloat16 instance of the float16 linear's kernel for this range, ahead of the few-row kernels below
+    // 5..16 rows of q4: the bfloat16 instance of the float16 linear's kernel for this range, ahead of the few-row kernels below
     // (there is no bfloat16 skinny kernel)
     {
       const int gvm = gq::options().gemv_variant;
@@ -943,7 +945,7 @@ int64_t mi355gq_linear_silu_mul_dt_workspace_bytes(int64_t M, int64_t N, int64_t
   if (model_dtype != MI355GQ_BF16 || check_scheme(bits, group_size) != MI355GQ_OK || M < 2 || N < 0 || K < 0 || M >= kMaxDim ||
       N >= kMaxDim || K >= kMaxDim || (N % 2) != 0)
     return 0;
-  const int64_t mid = (bits == 4 && M <= 32 && M > 4 && (N % 32) == 0) ? gq::midrow_workspace_bytes(M, N, K) : 0;
+  const int64_t mid = (bits == 4 && M <= 16 && M > 4 && (N % 32) == 0) ? gq::midrow_workspace_bytes(M, N, K) : 0;
   const int64_t gemm = gq::gemm_workspace_bytes(M, N, K, bits, group_size, 1, 1);
   return gemm > mid ? gemm : mid;
 }

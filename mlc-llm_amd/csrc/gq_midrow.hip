@@ -125,6 +125,8 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
   constexpr bool PAIR = F32;        // scales come for pairs of tiles (see issue_scales)
   constexpr int BR = F32 ? 5 : 16;    // activation rows a batch tile holds
   constexpr int SW = F32 ? U : U / 2; // registers of a row's U scales
+  // the weight operands carry no offset (else it is the C operand's, kept or made anew ahead of each group)
+  constexpr bool SUB = !KEEP_C && DT == MODEL_F16;
   constexpr uint32_t kMagic = BF ? 0x43004300u : 0x64006400u;
   // element i of a tensor in the model dtype
   auto elem = [](const uint16_t* t, int64_t i) -> float {
@@ -366,7 +368,7 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
             xa[bt][u][1] = __builtin_amdgcn_perm(v.w, v.y, kLoLo);
             xa[bt][u][2] = __builtin_amdgcn_perm(v.z, v.x, kHiHi);
             xa[bt][u][3] = __builtin_amdgcn_perm(v.w, v.y, kHiHi);
-            if constexpr (!BF) {
+            if constexpr (!BF && !SUB) {
               xa[bt][u][2] = as_u32(as_half2(xa[bt][u][2]) * r16);
               xa[bt][u][3] = as_u32(as_half2(xa[bt][u][3]) * r16);
             }
@@ -431,16 +433,16 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
               const uint16_t sb = static_cast<uint16_t>((u & 1) ? sv[u >> 1] >> 16 : sv[u >> 1] & 0xffffu);
               s = BF ? bf2f(sb) : h2f(sb);
             }
-            // (float16 without the kept offsets: the offsets come off the weight operand instead, exactly - 1024 + q - 1031
-            //  and 1024 + 16 q - 16 * 71 are small integers -, four packed adds per group whatever the batch tiles, in place
-            //  of one more matrix instruction per group and batch tile)
-            constexpr bool SUB = !KEEP_C && DT == MODEL_F16;
+            // (float16 without the kept offsets: they come off the weight operand instead, exactly, four packed instructions per group
+            //  whatever the batch tiles, in place of one more matrix instruction per group and batch tile: 1024 + q - 1031 and
+            //  (1024 + 16 q) / 16 - 71 are small integers, and x is taken as it is, infinities and the smallest values included)
             mid_u4 bo = bw;
             if constexpr (SUB) {
               const half2_t o_lo = {static_cast<_Float16>(-1031.f), static_cast<_Float16>(-1031.f)};
-              const half2_t o_hi = {static_cast<_Float16>(-1136.f), static_cast<_Float16>(-1136.f)};
+              const half2_t o_hi = {static_cast<_Float16>(-71.f), static_cast<_Float16>(-71.f)};
               bo[0] = as_u32(as_half2(bw[0]) + o_lo); bo[1] = as_u32(as_half2(bw[1]) + o_lo);
-              bo[2] = as_u32(as_half2(bw[2]) + o_hi); bo[3] = as_u32(as_half2(bw[3]) + o_hi);
+              bo[2] = as_u32(__builtin_elementwise_fma(as_half2(bw[2]), r16, o_hi));
+              bo[3] = as_u32(__builtin_elementwise_fma(as_half2(bw[3]), r16, o_hi));
             }
 #pragma unroll
             for (int bt = 0; bt < NBT; ++bt) {
@@ -660,19 +662,21 @@ hipError_t launch_mid(const MidParams& p, int wgx, int experts, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int DT>
-hipError_t launch_mid_once(const MidParams& p, int wgx, int experts, hipStream_t s) {
-  constexpr int NBT = 2, RT = 2;
-  constexpr size_t lds = (RT * NBT + 2) * 16 * 1024;  // (96 KiB)
-  static bool raised = false;  // (idempotent; a race sets the same attribute twice)
-  if (!raised) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&midonce_kernel<NBT, 8, RT, false, DT>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (e != hipSuccess) return e;
-    raised = true;
+template <int NBT>
+hipError_t launch_mid_once(const MidParams& p, int wgx, hipStream_t s) {
+  constexpr int RT = 2;
+  constexpr size_t lds = (RT * NBT + 2) * 16 * 1024;  // (64 or 96 KiB)
+  if (lds > 64 * 1024) {
+    static bool raised = false;  // (idempotent; a race sets the same attribute twice)
+    if (!raised) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&midonce_kernel<NBT, 8, RT, false, MODEL_F16>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+      if (e != hipSuccess) return e;
+      raised = true;
+    }
   }
-  note_kernel("gq::midonce_kernel<%d,8,%d,0%s> slices=%d kw=%d", NBT, RT, DT == MODEL_BF16 ? ",true" : "", p.slices, 1 << p.kw_log2);
-  hipLaunchKernelGGL((midonce_kernel<NBT, 8, RT, false, DT>), dim3(wgx, experts, p.slices), dim3(1024), lds, s, p);
+  note_kernel("gq::midonce_kernel<%d,8,%d,0> slices=%d kw=%d", NBT, RT, p.slices, 1 << p.kw_log2);
+  hipLaunchKernelGGL((midonce_kernel<NBT, 8, RT, false, MODEL_F16>), dim3(wgx, 1, p.slices), dim3(1024), lds, s, p);
   return hipGetLastError();
 }
 
@@ -781,8 +785,13 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   }
   p.rounds = ((rounds + p.chunks - 1) / p.chunks + unit - 1) / unit * unit;
   auto run = [&]() -> hipError_t {
-    if (nbt == 2 && !grouped && p.phases == 1 && p.chunks == 1 && p.rounds == 2 && options().gemv_variant < 0)
-      return a.bf16 ? launch_mid_once<MODEL_BF16>(p, wgx, experts, s) : launch_mid_once<MODEL_F16>(p, wgx, experts, s);
+    // Two rounds of a plain float16 linear.  One batch tile only below 24 M weights: with 24 M and more, rows with an infinity have
+    // always been NaN there (the kept offsets' inf - inf), below they went to a kernel that gave infinities, which this form gives too.
+    const bool once = !a.f32 && !a.bf16 && experts == 1 && !grouped && p.phases == 1 && p.chunks == 1 && p.rounds == 2 &&
+                      options().gemv_variant < 0;
+    if (once && nbt == 2) return launch_mid_once<2>(p, wgx, s);
+    if (a.rows > 8 && !a.bf16 && options().gemv_variant < 0 && !grouped && nbt == 1 && !a.f32 && a.N * a.K < (24ll << 20))
+      return once ? launch_mid_once<1>(p, wgx, s) : hipErrorNotSupported;
     if (a.f32) {
       if (p.phases > 1)
         return launch_mid<1, 8, 2, false, true, MODEL_F32>(p, wgx, experts, s);
