@@ -378,21 +378,13 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void gemm_pipe_kernel(c
     load_scales(0, sc_cur);
     load_scales(1, sc_nxt);
   }
-  // (in the order in which the loop refills the rings: a wait counts the loads behind the one it is for, and the loop's first K
-  //  tile shares its counts with the later ones)
-  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int d = 0; d < WD; ++d) {
-    if (d + DEPTH >= WD) load_a(kt0 + d + DEPTH - WD, ra[d + DEPTH - WD]);
-    __builtin_amdgcn_sched_barrier(0);
-    load_w(kt0 + d, rw[d]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  for (int d = 0; d < DEPTH; ++d) load_a(kt0 + d, ra[d]);
+#pragma unroll
+  for (int d = 0; d < WD; ++d) load_w(kt0 + d, rw[d]);
   store_tile(kt0, ra[0], rw[0], 0, sc_cur, 0);
-  __builtin_amdgcn_sched_barrier(0);
   load_a(kt0 + DEPTH, ra[0]);
   load_w(kt0 + WD, rw[0]);
-  __builtin_amdgcn_sched_barrier(0);
   __syncthreads();
   // (a register stage is refilled right after the MFMA/store block that drains it; a tile past
   //  the end is stored as zeros and adds nothing)
