@@ -1,4 +1,4 @@
-// Matmul for 9..64 activation rows against streamed q4f16_1 (q4bf16_1) weights (batched decode, short prefill chunks):
+// Matmul for 5..64 activation rows against streamed q4f16_1 (q4bf16_1) weights (batched decode, short prefill chunks):
 // v_mfma_f32_16x16x32_f16 on UNSCALED weight operands, the group's scale applied to the matrix instruction's result,
 // the activations resident in registers.
 //
@@ -28,9 +28,12 @@
 // lane (c, j), which is where the C operand wants it.  D: lane (c, j) receives rows 4 j .. 4 j + 3 of column c, four
 // values of the lane's own weight row: its scale of the group multiplies them into the fp32 accumulators.
 //
+// That is the form of one batch tile with the offsets kept (float16).  The float16 forms without them (two batch tiles, and two rounds
+// at most: midonce_kernel) take the offset and the factor 16 off the weight operand, four packed instructions per group, and x as it is.
+//
 // A wave owns U consecutive groups of K (its x: 4 registers per group and batch tile, the offsets as many where they are
-// kept) and walks tiles with RT tiles of loads in flight.  The 16 waves of a workgroup are KW neighbouring K shares x
-// 16 / KW tiles side by side; results wait in LDS until the walk is over (a store inside the walk would turn every wait
+// kept) and walks tiles with RT tiles of loads in flight.  The 16 waves of a workgroup (8 of twice the K where the walk
+// is long) are KW neighbouring K shares x 16 / KW tiles side by side; results wait in LDS until the walk is over (a store inside the walk would turn every wait
 // for a load into a wait for all of them), then the K shares are added and leave.  K beyond a workgroup's KW * U groups
 // is walked in phases: each phase loads its share of x and visits every tile again (its own K range of it: the weights
 // are still read once), adding to the sums in LDS.  Expert segments (moe_matmul.dequantize_group_gemm,
