@@ -185,11 +185,12 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
   // tile's loads a wait for all of them.
   const int pair_shift = p.paired ? 1 : 0;
   const int up_tiles = p.paired ? half_tiles : 0;
-  auto tile_of = [&](int r) -> int {
-    const int item = base + (r >> pair_shift) * tstride;
+  auto tile_from = [&](int first, int r) -> int {
+    const int item = first + (r >> pair_shift) * tstride;
     const int t = item + (r & pair_shift) * up_tiles;
     return item < p.ntiles ? t : -1;
   };
+  auto tile_of = [&](int r) -> int { return tile_from(base, r); };
 
   constexpr uint32_t kLoLo = 0x05040100u, kHiHi = 0x07060302u;
   const half2_t r16 = {static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)};
@@ -203,19 +204,16 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
       const int ga_raw = (static_cast<int>(blockIdx.z) * p.slice_shares + ph * kw + ks) * U;
       const bool k_live = ga_raw < p.ng && (PHASED || ks < p.slice_shares);
       const int ga = k_live ? ga_raw : p.ng - U;
-      // (a wave without a share of K has descriptors of no bytes: it loads zeros, and no traffic)
-      const __amdgpu_buffer_rsrc_t w_walk = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<uint32_t*>(p.qw + expert * p.expert_w_stride), short(0), k_live ? static_cast<int>(w_bytes) : 0, 0x00020000);
-      const __amdgpu_buffer_rsrc_t s_walk = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<uint16_t*>(p.qs + expert * p.expert_s_stride * (EL / 2)), short(0), k_live ? static_cast<int>(s_bytes) : 0, 0x00020000);
+      // (a wave without a share of K walks tiles past the end, see above: it loads zeros, and no traffic)
+      const int walk_base = k_live ? base : p.ntiles;
       const int w_lane = (c * p.nw + 4 * (ga + j)) * 4;
       u32x4 w[RT][STEPS];  // (kept as whole register tuples until the point of use, see walk_tile)
       auto issue = [&](int r, u32x4 (&wv)[STEPS]) {
-        const int tile = tile_of(r);
+        const int tile = tile_from(walk_base, r);
         const int w_off = static_cast<int>(tile >= 0 ? static_cast<uint32_t>(tile) * w_tile : w_bytes);
 #pragma unroll
         for (int st = 0; st < STEPS; ++st) {
-          wv[st] = __builtin_amdgcn_raw_buffer_load_b128(w_walk, w_lane + 64 * st, w_off, 0);
+          wv[st] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_lane + 64 * st, w_off, 0);
         }
       };
       // scales: the U of this lane's row c.  float32 (PAIR): of the tiles of rounds r and r + 1 in one load, lane (c, j) taking
@@ -228,18 +226,18 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
       constexpr int SR = PAIR ? SW / 2 : SW;
       uint32_t sraw[NS][SR];
       auto issue_scales = [&](int r, uint32_t (&sv)[SR]) {
-        const int t0 = tile_of(r);
+        const int t0 = tile_from(walk_base, r);
         const uint32_t o0 = t0 >= 0 ? static_cast<uint32_t>(t0) * s_tile : s_bytes;
         if constexpr (PAIR) {
-          const int t1 = tile_of(r + 1);
+          const int t1 = tile_from(walk_base, r + 1);
           const uint32_t o1 = t1 >= 0 ? static_cast<uint32_t>(t1) * s_tile : s_bytes;
           const u32x4 v =
-              __builtin_amdgcn_raw_buffer_load_b128(s_walk, s_lane + static_cast<int>(j < 2 ? o0 : o1), 0, 0);
+              __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, s_lane + static_cast<int>(j < 2 ? o0 : o1), 0, 0);
           sv[0] = v.x; sv[1] = v.y; sv[2] = v.z; sv[3] = v.w;
         } else {
 #pragma unroll
           for (int q = 0; q < SR; q += 4) {
-            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s_walk, s_lane + 4 * q, static_cast<int>(o0), 0);
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, s_lane + 4 * q, static_cast<int>(o0), 0);
             sv[q] = v.x; sv[q + 1] = v.y; sv[q + 2] = v.z; sv[q + 3] = v.w;
           }
         }

@@ -102,3 +102,44 @@ def test_midrow_kernel_of_two_rounds(m, n, k, once):
     expect = torch.where(w[:, 5] == 0, float("nan"), torch.sign(w[:, 5]) * float("inf")).half()
     assert torch.equal(torch.isnan(y[2]), torch.isnan(expect)) and torch.equal(torch.nan_to_num(y[2]), torch.nan_to_num(expect)), kern
     assert torch.isfinite(y[[0, 1] + list(range(3, m))]).all()
+
+
+# a wave without a share of K, in every form: the walk with a ring (one batch tile, two, eight waves, phases, slices) and the two rounds
+@pytest.mark.parametrize("dtype,m,n,k,form,kernel", [
+    (torch.float16, 5, 2752, 3840, "", "gq::midrow_kernel<1,8,"), (torch.float16, 9, 2752, 3840, "", "gq::midonce_kernel<1,"),
+    (torch.float16, 16, 7040, 3584, "", "gq::midrow_kernel<1,8,"), (torch.float16, 17, 1120, 3840, "", "gq::midonce_kernel<2,"),
+    (torch.float16, 32, 8224, 3840, "", "gq::midrow_kernel<2,8,"), (torch.float16, 5, 552, 5120, "one workgroup", "gq::midrow_kernel<1,16,"),
+    (torch.float16, 6, 544, 14336, "forced", "gq::midrow_kernel<1,8,"), (torch.float16, 7, 544, 4352, "no scratch", "gq::midrow_kernel<1,8,"),
+    (torch.bfloat16, 9, 1120, 3840, "", "gq::midrow_kernel<1,8,"), (torch.bfloat16, 24, 544, 3840, "forced", "gq::midrow_kernel<2,8,"),
+    (torch.float32, 5, 1120, 3840, "", "gq::midrow_kernel<1,8,"), (torch.float32, 3, 1120, 14336, "", "gq::midrow_kernel<1,8,")])
+def test_midrow_kernel_idle_waves_load_nothing(dtype, m, n, k, form, kernel):
+    """Such a wave multiplies by zeros, so only a value that zero times it shows can tell what it has loaded: an infinite scale in the last
+    group of K of some rows, tiles beyond the first among them.  There x is positive and the weights are, so that the group's sum is, of every
+    plane of a float32 x (which meet as rows of their own, each scaled): these results are infinities, not NaN, and the others finite."""
+    g = torch.Generator(device="cuda").manual_seed(n + k + m)
+    qw = torch.randint(-2**31, 2**31 - 1, (n, k // 8), device="cuda", dtype=torch.int32, generator=g)
+    qs = (torch.rand((n, k // 32), device="cuda", generator=g) * 0.02 + 0.001).to(dtype)
+    x = torch.randn((m, k), device="cuda", generator=g).to(dtype)
+    rows = [3, 19, n // 2, n - 1]
+    qs[rows, -1] = float("inf")
+    qw[rows, -4:] |= torch.tensor(0x88888888 - 2**32, dtype=torch.int32, device="cuda")  # (eight at least in every field)
+    x[:, -32:] = x[:, -32:].abs()
+    y = torch.empty((m, n), dtype=dtype, device="cuda")
+    scratch = torch.empty(5 * m * n, dtype=torch.float32, device="cuda")
+    code = {torch.float16: gq._lib.F16, torch.bfloat16: gq._lib.BF16, torch.float32: gq._lib.F32}[dtype]
+    if form:
+        gq._lib.set_option("gemv_variant", 10)
+    if form == "one workgroup":
+        gq._lib.set_option("gemv_waves", 16)
+    try:
+        gq._lib.call("mi355gq_linear_dt", x.data_ptr(), qw.data_ptr(), qs.data_ptr(), None, m, n, k, 4, 32, code, code, y.data_ptr(),
+                     scratch.data_ptr(), 0 if form == "no scratch" else scratch.numel() * 4, ops._stream())
+        kern = gq._lib.last_kernel()
+    finally:
+        gq._lib.set_option("gemv_variant", -1)
+        gq._lib.set_option("gemv_waves", -1)
+    assert kern.startswith(kernel) and (form != "no scratch" or " phases=2 " in kern), kern
+    assert (y[:, rows] == float("inf")).all(), (kern, y[:, rows])
+    rest = torch.ones(n, dtype=torch.bool, device="cuda")
+    rest[rows] = False
+    assert torch.isfinite(y[:, rest]).all(), kern
