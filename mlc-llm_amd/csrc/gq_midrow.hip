@@ -67,6 +67,7 @@ struct MidParams {
   int ntiles;              // tiles of 16 weight rows a walk visits: ceil(N / 16); the fused gate/up form: N / 32 pairs
   int rounds;              // tiles a wave walks per chunk (a multiple of the tiles in flight; the fused form: even)
   int chunks;              // chunks of rounds (1 when K takes phases)
+  int total_rounds;        // rounds in all chunks: the last one may be shorter (a multiple of the tiles in flight too)
   int phases;              // passes over K (a workgroup covers KW * U groups per phase)
   int slices;              // workgroups along K (plain linears with a workspace: grid z; each covers one phase's worth of
                            // K and leaves fp32 partial sums [slice][rows][N] in y for the reduction kernel)
@@ -523,7 +524,7 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
 
       // ---- the K shares of a tile meet: 256 values per (round, tile lane, batch tile); thread (jq, cq) takes row
       //      16 bt + jq of column cq, so that 16 neighbouring threads store 16 neighbouring columns
-      auto finish = [&](int r0) __attribute__((always_inline)) {
+      auto finish = [&](int r0, int rounds) __attribute__((always_inline)) {
         const float* const res = reinterpret_cast<const float*>(res_lds);
         const int sub = threadIdx.x & 255, cq = sub & 15, jq = sub >> 4;
         auto at_row = [&](int r) { return (((r >> 2) * 16 + cq) << 2) + (r & 3); };  // lane (cq, r / 4), value r % 4
@@ -543,7 +544,7 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
           return F32 ? 512.0f * v : v;
         };
         if (p.paired) {
-          const int items = (p.rounds >> 1) * tw * NBT;
+          const int items = (rounds >> 1) * tw * NBT;
           const int half = p.N >> 1;
           for (int it = threadIdx.x >> 8; it < items; it += WV / 4) {
             const int bt = it % NBT, rest = it / NBT, tl = rest % tw, pr = rest / tw;
@@ -554,7 +555,7 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
             if constexpr (!F32) static_cast<uint16_t*>(p.y)[static_cast<int64_t>(b) * half + col] = silu_mul_t<BF>(gate, up);
           }
         } else {
-          const int items = p.rounds * tw * NBT;
+          const int items = rounds * tw * NBT;
           for (int it = threadIdx.x >> 8; it < items; it += WV / 4) {
             const int bt = it % NBT, rest = it / NBT, tl = rest % tw, round = rest / tw;
             const int t = blockIdx.x * tw + tl + (r0 + round) * tstride;
@@ -577,9 +578,10 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
       // ---- the walk: p.rounds is a multiple of RT (rounds past the last tile read nothing and leave zeros in LDS slots
       //      that nobody reads).  Later phases add to what the earlier ones left (the read is unconditional and the
       //      first phase drops it: no branch inside the walk).
-      const int chunks = ONCE ? 1 : p.chunks, rounds = ONCE ? RT : p.rounds;
+      const int chunks = ONCE ? 1 : p.chunks;
       for (int chunk = 0; chunk < chunks; ++chunk) {
-        const int r0 = chunk * rounds;
+        const int r0 = chunk * p.rounds;
+        const int rounds = ONCE ? RT : min(p.rounds, p.total_rounds - r0);
         for (int round = 0; round < rounds; round += RT) {
 #pragma unroll
           for (int slot = 0; slot < RT; ++slot) {
@@ -602,12 +604,12 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
         }
         if (!PHASED || ph + 1 == p.phases) {  // (uniform)
           if constexpr (F32) {
-            const float4 last = res_lds[((p.rounds - 1) * WV + wave) * 64 + lane];
+            const float4 last = res_lds[((rounds - 1) * WV + wave) * 64 + lane];
             const float sum = (last.x + last.y) + (last.z + last.w);
             if (__ballot(sum != sum) != 0) redo_odd_rows(r0);  // (uniform; the sums are this wave's own until the barrier)
           }
           __syncthreads();
-          finish(r0);
+          finish(r0, rounds);
           __syncthreads();  // (the next chunk, or the next pass, writes the same LDS slots)
         }
       }
@@ -769,6 +771,8 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
     wgx = (sets + items - 1) / items;
   }
   wgx = (sets + items - 1) / items;
+  // (chunks of one length, the last one shorter by what is over: walked to its full length as well, 18 rounds of eight waves were 20, and
+  //  66560 x 4096 took 37.5-38.7 us at 5..8 rows where the quad-row kernel takes 36-37; now 35.3-36.4)
   int rounds = (items * per_round + unit - 1) / unit * unit;
   p.chunks = (rounds + max_rounds - 1) / max_rounds;
   // One batch tile and more than one chunk of rounds: eight waves of sixteen groups each instead, whose sums take half the LDS
@@ -785,6 +789,7 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
     p.chunks = (rounds + 2 * max_rounds - 1) / (2 * max_rounds);
   }
   p.rounds = ((rounds + p.chunks - 1) / p.chunks + unit - 1) / unit * unit;
+  p.total_rounds = rounds;
   auto run = [&]() -> hipError_t {
     // Two rounds of a plain float16 linear.  One batch tile only below 24 M weights: with 24 M and more, rows with an infinity have
     // always been NaN there (the kept offsets' inf - inf), below they went to a kernel that gave infinities, which this form gives too.

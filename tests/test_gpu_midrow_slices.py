@@ -143,3 +143,43 @@ def test_midrow_kernel_idle_waves_load_nothing(dtype, m, n, k, form, kernel):
     rest = torch.ones(n, dtype=torch.bool, device="cuda")
     rest[rows] = False
     assert torch.isfinite(y[:, rest]).all(), kern
+
+
+# one workgroup, more rounds than its chunks hold evenly: 18 as 10 + 8 (eight waves), 10 as 6 + 4 (sixteen), 6 as 4 + 2 (two batch tiles)
+@pytest.mark.parametrize("dtype,m,n,k", [(torch.float16, 7, 288, 4096), (torch.float16, 7, 160, 3840), (torch.float16, 24, 96, 4096),
+                                         (torch.bfloat16, 16, 288, 4096), (torch.bfloat16, 24, 96, 4096), (torch.float32, 5, 160, 4096)])
+def test_midrow_kernel_shorter_last_chunk(dtype, m, n, k):
+    """Against the float64 product of the quantised weights (tolerance: see test_midrow_kernel_eight_waves; float32: sums in fp32), and the fused
+    gate/up form against the two steps.  float32: a row with an infinity, which the kernel finds by the sums of the last round walked."""
+    g = torch.Generator(device="cuda").manual_seed(n + k + m)
+    qw = torch.randint(-2**31, 2**31 - 1, (n, k // 8), device="cuda", dtype=torch.int32, generator=g)
+    qs = (torch.rand((n, k // 32), device="cuda", generator=g) * 0.02 + 0.001).to(dtype)
+    x = torch.randn((m, k), device="cuda", generator=g).to(dtype)
+    q = torch.stack([(qw >> (4 * i)) & 15 for i in range(8)], -1).reshape(n, k).double() - 7
+    w = q * qs.double().repeat_interleave(32, 1)
+    words, fused = qw.view(torch.uint32), None
+    gq._lib.set_option("gemv_variant", 10)
+    gq._lib.set_option("gemv_waves", 16)
+    try:
+        y = ops.linear(x, words, qs, 4, 32, None, dtype)
+        kern = gq._lib.last_kernel()
+        if dtype != torch.float32:
+            fused = ops.linear_silu_mul(x, words, qs, 4, 32)
+        else:
+            x[2, 5] = float("inf")
+            odd = ops.linear(x, words, qs, 4, 32, None, dtype)[2]
+            x[2, 5] = 0
+    finally:
+        gq._lib.set_option("gemv_variant", -1)
+        gq._lib.set_option("gemv_waves", -1)
+    assert kern.startswith("gq::midrow_kernel<") and " chunks=2 " in kern, kern
+    if fused is not None:
+        assert torch.equal(fused, ops.silu_mul(y)), kern
+        ref = x.double() @ w.T
+        assert (y.double() - ref).norm() / ref.norm() <= (2.0**-11 if dtype == torch.float16 else 2.0**-8), kern
+    else:
+        expect = torch.where(w[:, 5] == 0, float("nan"), torch.sign(w[:, 5]) * float("inf")).float()
+        assert torch.equal(torch.isnan(odd), torch.isnan(expect)) and torch.equal(torch.nan_to_num(odd), torch.nan_to_num(expect)), kern
+        rows = [0, 1, 3, 4]
+        ref = x[rows].double() @ w.T
+        assert (y[rows].double() - ref).norm() / ref.norm() <= 1e-6, kern
