@@ -331,15 +331,22 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
     // against the quad-row kernel with x in registers: a K that is not 2048 or 4096 leaves some of its waves without a share
     // (5 / 8 rows: 4096 x 2560 7.9 / 7.7 -> 6.9 / 6.9, 8192 x 3072 10.2 / 10.4 -> 7.9 / 7.8, 4608 x 3584 9.3 / 9.2 -> 7.4 / 7.5, 37888 x 3584 24.0 / 25.8
     // -> 20.3 / 20.6); for 4096 it is ahead on the smaller matrices (4096 x 4096 6.4 / 6.1 against 7.6, 12288 x 4096 11.4 / 11.0 against
-    // 11.6 / 11.7, 20480 x 4096 15.3 / 15.4 against 15.2 / 16.2) and behind from about 84 M weights on (22016 x 4096 16.9 / 16.4 -> 16.4 / 16.0,
-    // 28672 x 4096 at 7 rows 21.8 -> 18.4, 128256 x 4096 64.7 / 65.0 -> 62.3 / 63.1; bfloat16 from 112 M, 67.3 / 69.9 -> 62.4 / 63.8)
+    // 11.6 / 11.7, 18432 x 4096 15.1 / 14.8 against 14.8 / 15.1, 20480 x 4096 15.0 / 15.0 against 14.9 / 15.4; four whole rounds of tiles are an
+    // exception, 16384 x 4096 13.3 / 12.9 against 12.3 / 12.4) and behind from about 84 M weights on (21504 x 4096 16.5 / 16.3 -> 15.6 / 15.9,
+    // 28672 x 4096 18.4 / 18.5 -> 18.1 / 18.5, 128256 x 4096 64.4 / 66.6 -> 61.8 / 63.7; 57344 x 2048 21.5 / 22.1 -> 18.2 / 18.5; bfloat16 is ahead from 84 M on as
+    // well, 23552 x 4096 17.1 / 16.7 -> 15.8 / 16.4, and is taken from 112 M: 28672 x 4096 19.1 / 19.2 -> 18.2 / 18.8, 128256 x 4096 67.0 / 69.2 -> 62.0 / 64.0)
     if (K <= 4096) return (K > 2048 && K < 4096 && weights >= mi(10)) || weights >= (bf16 ? mi(112) : mi(84));
     // K slices: 5120 x 5120 12.3 / 12.0 -> 11.2, 8192 x 5120 15.3 / 15.6 -> 12.5 / 12.9, 8192 x 7168 16.4 / 17.3 -> 13.8 / 14.3, 27648 x 5120 34.9 /
-    // 35.5 -> 25.8 / 26.2; 2048 x 5632 stays (8.4 / 8.1 against 9.3); 57344 x 8192 65.5 / 66.3 -> 58.1 / 58.8, 10240 x 8192 stays (16.9 / 15.9
+    // 35.5 -> 25.8 / 26.2; 2048 x 5632 stays (8.4 / 8.1 against 9.3).  Not where the matrix has so many rows that the register kernel has no
+    // room for their sums and the one with x in LDS answers, while the slices leave two fifths of these waves without a share (30720 x 4864
+    // 37.5 / 38.2 -> 28.7 / 29.1, but 32352 x 4864 24.4 / 25.6 against 29.2 / 29.8, 60256 x 4352 39.0 / 40.6 against 48.2 / 48.8; from K = 5120 on that shows later:
+    // 45056 x 5120 38.1 / 39.0 -> 36.3 / 36.7, 51200 x 5120 39.2 / 40.7 against 41.0 / 42.1, 63040 x 6656 51.8 / 54.5 against 58.8 / 59.2).
+    // 57344 x 8192 65.5 / 66.3 -> 58.1 / 58.8, 10240 x 8192 stays (16.9 / 15.9
     // against 17.8 / 17.5).  Beyond 8192 the quad-row kernel reads x from LDS, once per four rows and K share: 4096 x 11008 14.0 / 14.4 ->
     // 13.3 / 13.4, 4096 x 14336 15.8 / 16.1 -> 15.4 / 15.5 (bfloat16 16.6 / 17.5 -> 15.5 / 15.6), 8192 x 28672 46.1 / 47.3 -> 34.9 / 35.0; 4096 x 9216
     // stays (12.1 / 12.2 against 12.5)
-    if (K <= 8192) return slices && ((K < 8192 && weights >= mi(24)) || weights >= mi(256));
+    if (K < 8192) return slices && weights >= mi(24) && N <= (K < 5120 ? 30 : 44) * 1024;
+    if (K == 8192) return slices && weights >= mi(256);
     return slices && weights >= mi(40);
   }
   if (M <= 16) {
@@ -352,11 +359,15 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
   }
   // 17..32 rows, two batch tiles, against the GEMM's 32-row tile and its split of K (17 / 32 rows): 2048 x 2048 8.9 / 10.0 -> 8.3 / 8.4,
   // 4096 x 4096 11.8 / 12.4 -> 9.1 / 9.1, 6144 x 4096 12.9 / 13.9 -> 9.3 / 9.7, 12288 x 4096 16.9 / 18.9 -> 14.7 / 16.0, 128256 x 4096 98 / 102 -> 80.6 /
-  // 81.5.  K slices where they are whole and many: 10240 x 8192 27.5 / 28.5 -> 25.7 / 27.6, 8192 x 28672 50.2 / 52.5 -> 47.2 / 50.4,
+  // 81.5.  A K below 2048 leaves the x that a wave loads (32 rows) less to be used on: 16384 x 256 4.9 / 5.3 against 9.8 / 9.9, 4096 x 1024 7.7 / 8.4
+  // against 8.4 / 8.6, 26240 x 1280 11.3 / 11.7 against 12.7 / 13.4; from K = 1280 on it is ahead up to 24 M weights (16384 x 1536 11.5 / 12.7
+  // -> 9.1 / 9.4), and from 48 M weights on it takes all of them as it has.  K slices where they are whole and many: 10240 x 8192 27.4 / 28.4 -> 22.4 / 24.3,
+  // 5120 x 16384 25.0 / 25.7 -> 22.8 / 24.4 (4096 x 20480 24.2 / 24.6 against 24.4 / 26.3, from 120 M on ahead again: 6656 x 20480 47.5 / 49.8 -> 32.2 / 34.5),
   // 57344 x 8192 97 -> 77; half of the waves without a share loses (27648 x 5120 33.6 / 34.4 against 42).  bfloat16 stays with the GEMM:
   // its instance is ahead (4096 x 4096 12.3 / 13.0 -> 9.6 / 9.7) but makes NaN of an infinity, offset included, where the GEMM keeps it
   if (bf16) return false;
-  return K <= 4096 ? weights >= mi(4) : slices && ((K % 4096 == 0 && weights >= mi(80)) || weights >= mi(256));
+  if (K <= 4096) return weights >= mi(K >= 2048 ? 4 : 48) || (K >= 1280 && weights >= mi(4) && weights <= mi(24));
+  return slices && ((K % 4096 == 0 && weights >= mi(K <= 16384 ? 80 : 120)) || weights >= mi(256));
 }
 
 // with_slices false: what the shape needs when the K slices of the kernel on unscaled weight operands go without

@@ -772,7 +772,7 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   }
   wgx = (sets + items - 1) / items;
   // (chunks of one length, the last one shorter by what is over: walked to its full length as well, 18 rounds of eight waves were 20, and
-  //  66560 x 4096 took 37.5-38.7 us at 5..8 rows where the quad-row kernel takes 36-37; now 35.3-36.4)
+  //  66560 x 4096 took 38.1 / 38.7 us at 5 / 8 rows, where the quad-row kernel takes 36.4 / 37.3; now 35.3 / 36.4)
   int rounds = (items * per_round + unit - 1) / unit * unit;
   p.chunks = (rounds + max_rounds - 1) / max_rounds;
   // One batch tile and more than one chunk of rounds: eight waves of sixteen groups each instead, whose sums take half the LDS

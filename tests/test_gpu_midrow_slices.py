@@ -183,3 +183,35 @@ def test_midrow_kernel_shorter_last_chunk(dtype, m, n, k):
         rows = [0, 1, 3, 4]
         ref = x[rows].double() @ w.T
         assert (y[rows].double() - ref).norm() / ref.norm() <= 1e-6, kern
+
+
+# the default dispatch on both sides of its bounds: (kernel, rows, N, K)
+_QUADREG, _QUAD, _GEMM = "gq::quadreg_kernel<", "gq::quad_kernel<", "gq::gemm_pipe_kernel<"
+_WALK, _WIDE, _WALK2, _ONCE2 = "gq::midrow_kernel<1,8,", "gq::midrow_kernel<1,16,", "gq::midrow_kernel<2,8,", "gq::midonce_kernel<2,"
+_DEFAULTS = [
+    # 17..32 rows of a short K
+    (_GEMM, 32, 16384, 256), (_GEMM, 17, 4096, 1024), (_ONCE2, 17, 3296, 1280), (_GEMM, 17, 3264, 1280), (_GEMM, 24, 20480, 1280), (_WALK2, 17, 39328, 1280),
+    # ... and as K slices
+    (_WALK2, 17, 5120, 16384), (_GEMM, 17, 4096, 20480), (_WALK2, 32, 6144, 20480),
+    # 5..8 rows as K slices, where the quad-row kernel with x in LDS takes the matrices of many rows
+    (_WALK, 8, 30720, 4864), (_QUAD, 5, 32352, 4864), (_WIDE, 5, 45056, 5120), (_QUAD, 8, 51200, 5120),
+]
+
+
+@pytest.mark.parametrize("kernel,m,n,k", _DEFAULTS)
+def test_default_kernel_at_the_bounds(kernel, m, n, k):
+    """Which kernel answers, a sample of the columns against the float64 product of the quantised weights (tolerance: one float16 rounding of the
+    result and, for the kernels that multiply such weights, one of every weight), and the fused gate/up form against the two steps."""
+    g = torch.Generator(device="cuda").manual_seed(n + k + m)
+    qw = torch.randint(-2**31, 2**31 - 1, (n, k // 8), device="cuda", dtype=torch.int32, generator=g)
+    qs = (torch.rand((n, k // 32), device="cuda", generator=g) * 0.02 + 0.001).half()
+    x = torch.randn((m, k), device="cuda", generator=g).half()
+    words = qw.view(torch.uint32)
+    y = ops.linear(x, words, qs, 4, 32)
+    kern = gq._lib.last_kernel()
+    assert kern.startswith(kernel), kern
+    cols = torch.cat([torch.tensor([0, 1, n // 2, n - 1], device="cuda"), torch.randint(0, n, (200,), device="cuda", generator=g)])
+    q = torch.stack([(qw[cols] >> (4 * i)) & 15 for i in range(8)], -1).reshape(len(cols), k).double() - 7
+    ref = x.double() @ (q * qs[cols].double().repeat_interleave(32, 1)).T
+    assert (y[:, cols].double() - ref).norm() / ref.norm() <= 2 * 2.0**-11, kern
+    assert torch.equal(ops.linear_silu_mul(x, words, qs, 4, 32), ops.silu_mul(y)), kern
