@@ -370,13 +370,18 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
   return slices && ((K % 4096 == 0 && weights >= mi(K <= 16384 ? 80 : 120)) || weights >= mi(256));
 }
 
+// Scratch for the K slices of that kernel: what the calls that run on it use, and none for others.  (gemv_variant 10 forces it: 5..32 rows)
+static int64_t midrow_scratch(int64_t M, int64_t N, int64_t K, int bits, bool bf16) {
+  const bool asks = gq::options().gemv_variant == 10 ? M > 4 && M <= (bf16 ? 16 : 32) : (N & 31) == 0 && midrow_takes(M, N, K, true, bf16);
+  return bits == 4 && asks ? gq::midrow_workspace_bytes(M, N, K) : 0;
+}
+
 // with_slices false: what the shape needs when the K slices of the kernel on unscaled weight operands go without
 static int64_t linear_workspace_need(int64_t M, int64_t N, int64_t K, int bits, int group_size, bool with_slices) {
   if (check_scheme(bits, group_size) != MI355GQ_OK || M < 0 || N < 0 || K < 0 || M >= kMaxDim ||
       N >= kMaxDim || K >= kMaxDim)
     return 0;
-  // q4 at 5..32 rows of a K beyond 4096: the K slices of the kernel on unscaled weight operands (see midrow_takes)
-  const int64_t mid = (with_slices && bits == 4 && M <= 32 && M > 4) ? gq::midrow_workspace_bytes(M, N, K) : 0;
+  const int64_t mid = with_slices ? midrow_scratch(M, N, K, bits, false) : 0;
   // only the few-row GEMM (more rows than the GEMV / skinny kernels take, at most 256) splits K
   // (q4 at 9..16 rows: the skinny kernel, except on matrices of 40 M to 256 M weights, see linear_impl)
   if (M <= 16 && bits == 4 && !(M > 8 && N * K >= (40ll << 20) && N * K < (256ll << 20))) return mid;
@@ -429,9 +434,8 @@ int64_t mi355gq_linear_dt_workspace_bytes(int64_t M, int64_t N, int64_t K, int b
   if (model_dtype != MI355GQ_BF16 || check_scheme(bits, group_size) != MI355GQ_OK || M < 2 || N < 0 || K < 0 ||
       M >= kMaxDim || N >= kMaxDim || K >= kMaxDim)
     return 0;
-  // bfloat16: every batch from two rows on may run the few-row GEMM (there are no bf16 skinny kernels); 5..16 rows of a
-  // long K: the K slices of the kernel on unscaled weight operands
-  const int64_t mid = (bits == 4 && M <= 16 && M > 4) ? gq::midrow_workspace_bytes(M, N, K) : 0;
+  // bfloat16: every batch from two rows on may run the few-row GEMM (there are no bf16 skinny kernels)
+  const int64_t mid = midrow_scratch(M, N, K, bits, true);
   const int64_t gemm = gq::gemm_workspace_bytes(M, N, K, bits, group_size, 1);
   return gemm > mid ? gemm : mid;
 }
@@ -440,8 +444,7 @@ int64_t mi355gq_linear_silu_mul_workspace_bytes(int64_t M, int64_t N, int64_t K,
   if (check_scheme(bits, group_size) != MI355GQ_OK || M < 0 || N < 0 || K < 0 || M >= kMaxDim ||
       N >= kMaxDim || K >= kMaxDim)
     return 0;
-  // q4 at 5..32 rows of a K beyond 4096: the K slices of the kernel on unscaled weight operands (as the plain linear)
-  const int64_t mid = (bits == 4 && M <= 32 && M > 4 && (N % 32) == 0) ? gq::midrow_workspace_bytes(M, N, K) : 0;
+  const int64_t mid = (N % 32) == 0 ? midrow_scratch(M, N, K, bits, false) : 0;
   // GEMV / few-row kernels
   if (M <= 8 || (N % 2) != 0) return mid;
   if (M <= 16 && bits == 4 && !(N * K >= (40ll << 20) && N * K < (256ll << 20))) return mid;
@@ -956,7 +959,7 @@ int64_t mi355gq_linear_silu_mul_dt_workspace_bytes(int64_t M, int64_t N, int64_t
   if (model_dtype != MI355GQ_BF16 || check_scheme(bits, group_size) != MI355GQ_OK || M < 2 || N < 0 || K < 0 || M >= kMaxDim ||
       N >= kMaxDim || K >= kMaxDim || (N % 2) != 0)
     return 0;
-  const int64_t mid = (bits == 4 && M <= 16 && M > 4 && (N % 32) == 0) ? gq::midrow_workspace_bytes(M, N, K) : 0;
+  const int64_t mid = (N % 32) == 0 ? midrow_scratch(M, N, K, bits, true) : 0;
   const int64_t gemm = gq::gemm_workspace_bytes(M, N, K, bits, group_size, 1, 1);
   return gemm > mid ? gemm : mid;
 }
