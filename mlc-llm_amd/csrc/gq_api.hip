@@ -355,7 +355,10 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
     // against 7.1) and smaller stay, in bfloat16 down to 4 M weights they do not (2048 x 2048 at 16 rows 9.4 -> 6.9).  Without the scratch a
     // K of two phases from 48 M weights on (8192 x 8192 21 -> 17-18.5)
     // (bfloat16 K slices from 24 M: below, the GEMM keeps a row's infinities, which the kept offsets make NaN)
-    return K <= 4096 ? weights >= (bf16 ? mi(4) : mi(10)) : (slices && weights >= (bf16 ? mi(24) : mi(10))) || (K <= 8192 && weights >= mi(48));
+    // (float16 below 24 M weights: two rounds per wave at most, the form that keeps infinities and the smallest activations as they are)
+    const bool small = bf16 || weights >= mi(24) || gq::midrow_two_rounds(N, K);
+    return K <= 4096 ? small && weights >= (bf16 ? mi(4) : mi(10))
+                     : (slices && small && weights >= (bf16 ? mi(24) : mi(10))) || (K <= 8192 && weights >= mi(48));
   }
   // 17..32 rows, two batch tiles, against the GEMM's 32-row tile and its split of K (17 / 32 rows): 2048 x 2048 8.9 / 10.0 -> 8.3 / 8.4,
   // 4096 x 4096 11.8 / 12.4 -> 9.1 / 9.1, 6144 x 4096 12.9 / 13.9 -> 9.3 / 9.7, 12288 x 4096 16.9 / 18.9 -> 14.7 / 16.0, 128256 x 4096 98 / 102 -> 80.6 /

@@ -134,6 +134,7 @@ hipError_t launch_quadreg(const GemmArgs& a, int rows_max, hipStream_t s);
 // does not fit.
 hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s);
 int64_t midrow_workspace_bytes(int64_t rows, int64_t N, int64_t K);
+bool midrow_two_rounds(int64_t N, int64_t K);
 
 // float32 models (q4f32_1, K % 8 == 0), plain linears and expert segments: three bfloat16 planes of x on the bfloat16
 // matrix cores; hipErrorNotSupported otherwise.  Its split of K wants gemm_f32_workspace_bytes of scratch.

@@ -791,13 +791,13 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   p.rounds = ((rounds + p.chunks - 1) / p.chunks + unit - 1) / unit * unit;
   p.total_rounds = rounds;
   auto run = [&]() -> hipError_t {
-    // Two rounds of a plain float16 linear.  One batch tile only below 24 M weights: with 24 M and more, rows with an infinity have
-    // always been NaN there (the kept offsets' inf - inf), below they went to a kernel that gave infinities, which this form gives too.
+    // Two rounds of a plain float16 linear.  One batch tile only of 9 rows on below 24 M weights: with 24 M and more, rows with an
+    // infinity have always been NaN there (the kept offsets' inf - inf), below they went to a kernel that gave infinities, which this form
+    // gives too (and the dispatch sends no other shapes of those sizes: midrow_two_rounds).
     const bool once = !a.f32 && !a.bf16 && experts == 1 && !grouped && p.phases == 1 && p.chunks == 1 && p.rounds == 2 &&
                       options().gemv_variant < 0;
     if (once && nbt == 2) return launch_mid_once<2>(p, wgx, s);
-    if (a.rows > 8 && !a.bf16 && options().gemv_variant < 0 && !grouped && nbt == 1 && !a.f32 && a.N * a.K < (24ll << 20))
-      return once ? launch_mid_once<1>(p, wgx, s) : hipErrorNotSupported;
+    if (once && a.rows > 8 && a.N * a.K < (24ll << 20)) return launch_mid_once<1>(p, wgx, s);
     if (a.f32) {
       if (p.phases > 1)
         return launch_mid<1, 8, 2, false, true, MODEL_F32>(p, wgx, experts, s);
@@ -839,6 +839,14 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
                        static_cast<const float*>(a.workspace), p.slices, count, p.N, p.N, a.bias, a.residual, a.y, a.out_f32, a.bf16);
   }
   return hipGetLastError();
+}
+
+// whether a dense float16 linear (K a multiple of 256, beyond 4096 as K slices) is two rounds per wave at most
+bool midrow_two_rounds(int64_t N, int64_t K) {
+  const int64_t shares = K / 256, slices = (shares + 15) / 16;
+  int64_t tw = 16;  // tiles side by side in a workgroup
+  while (tw > 1 && 16 / tw < shares) tw /= 2;
+  return slices <= 256 && (N + 15) / 16 <= 2 * tw * (256 / slices);
 }
 
 // scratch for the K slices of a plain linear (0: K is one phase)

@@ -188,6 +188,7 @@ def test_midrow_kernel_shorter_last_chunk(dtype, m, n, k):
 # the default dispatch on both sides of its bounds: (kernel, rows, N, K)
 _QUADREG, _QUAD, _GEMM = "gq::quadreg_kernel<", "gq::quad_kernel<", "gq::gemm_pipe_kernel<"
 _WALK, _WIDE, _WALK2, _ONCE2 = "gq::midrow_kernel<1,8,", "gq::midrow_kernel<1,16,", "gq::midrow_kernel<2,8,", "gq::midonce_kernel<2,"
+_SKINNY, _ONCE = "gq::skinny_q4_", "gq::midonce_kernel<1,"
 _DEFAULTS = [
     # 17..32 rows of a short K
     (_GEMM, 32, 16384, 256), (_GEMM, 17, 4096, 1024), (_ONCE2, 17, 3296, 1280), (_GEMM, 17, 3264, 1280), (_GEMM, 24, 20480, 1280), (_WALK2, 17, 39328, 1280),
@@ -195,6 +196,8 @@ _DEFAULTS = [
     (_WALK2, 17, 5120, 16384), (_GEMM, 17, 4096, 20480), (_WALK2, 32, 6144, 20480),
     # 5..8 rows as K slices, where the quad-row kernel with x in LDS takes the matrices of many rows
     (_WALK, 8, 30720, 4864), (_QUAD, 5, 32352, 4864), (_WIDE, 5, 45056, 5120), (_QUAD, 8, 51200, 5120),
+    # 9..16 rows below 24 M weights, where a wave walks two rounds or the skinny kernel answers
+    (_ONCE, 12, 8192, 2560), (_SKINNY, 12, 9216, 2560), (_ONCE, 9, 4096, 5632), (_SKINNY, 16, 4128, 5632),
 ]
 
 
