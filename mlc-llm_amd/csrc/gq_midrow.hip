@@ -779,10 +779,13 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   // (twice the rounds per chunk, half as many stops where the shares meet; the sums of half as many shares): 128256 x 4096 at 7 /
   // 16 rows 63.8 / 67.1 -> 61.1 / 66.5 us, 27648 x 5120 29.4 / 31.2 -> 25.9 / 27.0, 57344 x 8192 61.3 / 65.9 -> 56.7 / 60.9; where one chunk
   // does, sixteen waves hide more (4096 x 4096 7.4 against 8.1, 28672 x 4096 at 16 rows 19.4 against 19.7).  Two batch tiles lose
-  // with eight waves (128256 x 4096 at 32 rows 81.5 against 86.6).
+  // with eight waves (128256 x 4096 at 32 rows 81.5 against 86.6).  A K of one or two such shares leaves little between the stops
+  // either way, and sixteen waves stay ahead (180224 x 1024 at 7 / 16 rows 25.1 / 26.1 against 26.5 / 28.2).  Expert segments alike (rows per
+  // expert): 8 of 28672 x 4096 at 4..8 106-108 -> 104-107, 64 of 5120 x 3584 at 4.5 147 -> 139, 64 of 5120 x 1536 at 4.5 66.9 -> 65.9, but 64 of
+  // 9952 x 1024 at 4.5 84.4 against 88.0, 64 of 9952 x 512 49.1 against 54.3.
   // (The fused gate/up form walks half as many items of two rounds each, so it takes more than one chunk exactly where the plain
   // form does, and the two add in the same order.)
-  const bool wide = nbt == 1 && !a.f32 && p.phases == 1 && p.chunks > 1 && (a.K & 511) == 0 && options().quad_ksplit < 0 && form < 0;
+  const bool wide = nbt == 1 && !a.f32 && p.phases == 1 && p.chunks > 1 && a.K >= 1536 && (a.K & 511) == 0 && options().quad_ksplit < 0 && form < 0;
   if (wide) {
     --p.kw_log2;
     p.slice_shares = p.slices > 1 ? (p.ng / 16 + p.slices - 1) / p.slices : 1 << p.kw_log2;

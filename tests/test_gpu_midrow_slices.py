@@ -35,10 +35,10 @@ def test_midrow_kernel_even_slices(m, k, slices):
     assert_linear_ok(out, o.linear_fp32(x, qw, qs, s), x, k, f"even slices {m}x{n}x{k} [{kern}]")
 
 
-# one batch tile and more than one chunk of rounds (few workgroups): K of one and two shares of sixteen groups, whole, and as slices of five
-# and of seven, eight, ... ; a ragged last tile
+# one batch tile and more than one chunk of rounds (few workgroups): K of three, four and eight shares of sixteen groups, and as slices of five
+# and of seven, eight, ... ; a ragged last tile; one and two such shares, which sixteen waves of eight groups take
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("n,k", [(2600, 512), (1312, 1024), (328, 4096), (552, 5120), (320, 18944)])
+@pytest.mark.parametrize("n,k", [(2600, 512), (1312, 1024), (872, 1536), (648, 2048), (328, 4096), (552, 5120), (320, 18944)])
 @pytest.mark.parametrize("m", [5, 16])
 def test_midrow_kernel_eight_waves(dtype, m, n, k):
     """Eight waves of sixteen groups, against the float64 product of the quantised weights (which this kernel does not round): the
@@ -61,9 +61,64 @@ def test_midrow_kernel_eight_waves(dtype, m, n, k):
     finally:
         gq._lib.set_option("gemv_variant", -1)
         gq._lib.set_option("gemv_waves", -1)
-    assert kern.startswith("gq::midrow_kernel<1,16,"), kern
+    assert kern.startswith("gq::midrow_kernel<1,16," if k >= 1536 else "gq::midrow_kernel<1,8,"), kern
     err = (out.double() - ref).norm() / ref.norm()
     assert err <= (2.0**-11 if dtype == torch.float16 else 2.0**-8), (kern, err)
+
+
+# the same on expert segments, one workgroup per expert
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k", [(1184, 512), (608, 1024), (608, 1536), (608, 2048), (288, 4096)])
+def test_midrow_kernel_eight_waves_of_expert_segments(dtype, n, k):
+    """An empty expert, one of a single row, one of a whole batch tile, one of two passes and one of three, the gather of the rows folded in, against
+    the float64 products (tolerance: see above); the fused gate/up form against the two steps."""
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    cuts = [0, 1, 1, 17, 36, 76]
+    qw = torch.randint(-2**31, 2**31 - 1, (5, n, k // 8), device="cuda", dtype=torch.int32, generator=g)
+    qs = (torch.rand((5, n, k // 32), device="cuda", generator=g) * 0.02 + 0.001).to(dtype)
+    xs = torch.randn((25, k), device="cuda", generator=g).to(dtype)
+    rows = torch.randint(0, 25, (76,), device="cuda", dtype=torch.int32, generator=g)
+    ip, words = torch.tensor(cuts, dtype=torch.int32, device="cuda"), qw.view(torch.uint32)
+    gq._lib.set_option("gemv_variant", 10)
+    gq._lib.set_option("gemv_waves", 16)
+    try:
+        y = ops.moe_experts(xs, rows, words, qs, ip, 4, 32)
+        kern = gq._lib.last_kernel()
+        fused = ops.moe_experts(xs, rows, words, qs, ip, 4, 32, silu_mul_halves=True)
+        kern_fused = gq._lib.last_kernel()
+    finally:
+        gq._lib.set_option("gemv_variant", -1)
+        gq._lib.set_option("gemv_waves", -1)
+    want = "gq::midrow_kernel<1,16," if k >= 1536 else "gq::midrow_kernel<1,8,"
+    assert kern.startswith(want) and kern_fused.startswith(want) and " chunks=1 " not in kern, (kern, kern_fused)
+    assert torch.equal(fused, ops.silu_mul(y)), kern
+    q = torch.stack([(qw >> (4 * i)) & 15 for i in range(8)], -1).reshape(5, n, k).double() - 7
+    w, x = q * qs.double().repeat_interleave(32, 2), xs[rows.long()].double()
+    ref = torch.cat([x[cuts[e]:cuts[e + 1]] @ w[e].T for e in range(5)])
+    each = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert each.max() <= (2.0**-11 if dtype == torch.float16 else 2.0**-8), (kern, each)
+
+
+def test_default_kernel_of_a_large_expert_stack():
+    """48 rows over 8 experts of 28672 x 4096: eight waves, a sample of the columns against the float64 products (tolerance: see above), the fused
+    gate/up form against the two steps."""
+    e, n, k = 8, 28672, 4096
+    g = torch.Generator(device="cuda").manual_seed(48)
+    cuts = [0, 3, 9, 9, 26, 30, 37, 42, 48]
+    qw = torch.randint(-2**31, 2**31 - 1, (e, n, k // 8), device="cuda", dtype=torch.int32, generator=g)
+    qs = (torch.rand((e, n, k // 32), device="cuda", generator=g) * 0.02 + 0.001).half()
+    x = torch.randn((48, k), device="cuda", generator=g).half()
+    ip, words = torch.tensor(cuts, dtype=torch.int32, device="cuda"), qw.view(torch.uint32)
+    y = ops.moe_experts(x, None, words, qs, ip, 4, 32)
+    kern = gq._lib.last_kernel()
+    fused = ops.moe_experts(x, None, words, qs, ip, 4, 32, silu_mul_halves=True)
+    assert kern.startswith("gq::midrow_kernel<1,16,") and gq._lib.last_kernel().startswith("gq::midrow_kernel<1,16,"), (kern, gq._lib.last_kernel())
+    assert torch.equal(fused, ops.silu_mul(y)), kern
+    cols = torch.cat([torch.tensor([0, n // 2, n - 1], device="cuda"), torch.randint(0, n, (100,), device="cuda", generator=g)])
+    for i in range(e):
+        q = torch.stack([(qw[i, cols] >> (4 * f)) & 15 for f in range(8)], -1).reshape(len(cols), k).double() - 7
+        ref = x[cuts[i]:cuts[i + 1]].double() @ (q * qs[i, cols].double().repeat_interleave(32, 1)).T
+        assert (y[cuts[i]:cuts[i + 1]][:, cols].double() - ref).norm() <= 2.0**-11 * ref.norm(), (kern, i)
 
 
 # at most two tiles per wave: K of eight, sixteen and fifteen shares (one idle wave); as few tiles as the dispatch sends, two rounds filled to
