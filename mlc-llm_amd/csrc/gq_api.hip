@@ -335,17 +335,28 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
     // exception, 16384 x 4096 13.3 / 12.9 against 12.3 / 12.4) and behind from about 84 M weights on (21504 x 4096 16.5 / 16.3 -> 15.6 / 15.9,
     // 28672 x 4096 18.4 / 18.5 -> 18.1 / 18.5, 128256 x 4096 64.4 / 66.6 -> 61.8 / 63.7; 57344 x 2048 21.5 / 22.1 -> 18.2 / 18.5; bfloat16 is ahead from 84 M on as
     // well, 23552 x 4096 17.1 / 16.7 -> 15.8 / 16.4, and is taken from 112 M: 28672 x 4096 19.1 / 19.2 -> 18.2 / 18.8, 128256 x 4096 67.0 / 69.2 -> 62.0 / 64.0)
-    if (K <= 4096) return (K > 2048 && K < 4096 && weights >= mi(10)) || weights >= (bf16 ? mi(112) : mi(84));
+    // K = 3584 and 3840 fill the quad-row kernel's waves but for one or a half: the smaller matrices stay (5 / 8 rows: 3520 x 3584 7.4 / 7.3 against
+    // 7.4 / 7.4, 3552 x 3840 7.1 / 7.6 against 7.5 / 7.5; 4416 x 3584 9.0 / 9.6 -> 8.0 / 8.2, 4384 x 3840 8.4 / 9.0 -> 8.2 / 8.3)
+    if (K <= 4096)
+      return (K > 2048 && K < 4096 && weights >= mi(K > 3584 ? 16 : K > 3328 ? 14 : 10)) || weights >= (bf16 ? mi(112) : mi(84));
     // K slices: 5120 x 5120 12.3 / 12.0 -> 11.2, 8192 x 5120 15.3 / 15.6 -> 12.5 / 12.9, 8192 x 7168 16.4 / 17.3 -> 13.8 / 14.3, 27648 x 5120 34.9 /
     // 35.5 -> 25.8 / 26.2; 2048 x 5632 stays (8.4 / 8.1 against 9.3).  Not where the matrix has so many rows that the register kernel has no
     // room for their sums and the one with x in LDS answers, while the slices leave two fifths of these waves without a share (30720 x 4864
     // 37.5 / 38.2 -> 28.7 / 29.1, but 32352 x 4864 24.4 / 25.6 against 29.2 / 29.8, 60256 x 4352 39.0 / 40.6 against 48.2 / 48.8; from K = 5120 on that shows later:
-    // 45056 x 5120 38.1 / 39.0 -> 36.3 / 36.7, 51200 x 5120 39.2 / 40.7 against 41.0 / 42.1, 63040 x 6656 51.8 / 54.5 against 58.8 / 59.2).
+    // 45056 x 5120 38.1 / 39.0 -> 36.3 / 36.7, 51200 x 5120 39.2 / 40.7 against 41.0 / 42.1, 63040 x 6656 51.8 / 54.5 against 58.8 / 59.2; in bfloat16 45056 x 5120
+    // 37.5 against 38.8, 45056 x 6144 41.1 / 41.9, 40960 x 6144 ahead), nor where 31 to 32 Ki rows fill that kernel's walk (32768 x 5120 24.6 / 26.1 against
+    // 28.3 / 29.2, 32768 x 7168 31.1 / 34.3 against 32.6 / 32.7; bfloat16 32768 x 6144 31.4 against 32.7, 32768 x 6656 34.5 -> 32.5).  And from K = 6144 on the
+    // register kernel's waves have work enough on the smaller matrices (4096 x 6144 10.6 / 10.6 against 10.7 / 10.7, 4800 x 6144 level), from 7680 on
+    // nearly all of them (4672 x 7680 11.8 / 12.0 against 12.3 / 12.4, 6080 x 7936 level, 6560 x 7680 14.8 / 14.6 -> 14.3 / 13.5).
     // 57344 x 8192 65.5 / 66.3 -> 58.1 / 58.8, 10240 x 8192 stays (16.9 / 15.9
     // against 17.8 / 17.5).  Beyond 8192 the quad-row kernel reads x from LDS, once per four rows and K share: 4096 x 11008 14.0 / 14.4 ->
     // 13.3 / 13.4, 4096 x 14336 15.8 / 16.1 -> 15.4 / 15.5 (bfloat16 16.6 / 17.5 -> 15.5 / 15.6), 8192 x 28672 46.1 / 47.3 -> 34.9 / 35.0; 4096 x 9216
     // stays (12.1 / 12.2 against 12.5)
-    if (K < 8192) return slices && weights >= mi(24) && N <= (K < 5120 ? 30 : 44) * 1024;
+    if (K < 8192) {
+      const int64_t ki = 1024, most = (K < 5120 ? 30 : bf16 && K < 6656 ? 40 : 44) * ki;
+      const bool quad_filled = N > 31 * ki && N <= 32 * ki && (!bf16 || K < 6656);
+      return slices && weights >= mi(K >= 7680 ? 48 : K >= 6144 ? 28 : 24) && N <= most && !quad_filled;
+    }
     if (K == 8192) return slices && weights >= mi(256);
     return slices && weights >= mi(40);
   }
@@ -355,9 +366,11 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
     // against 7.1) and smaller stay, in bfloat16 down to 4 M weights they do not (2048 x 2048 at 16 rows 9.4 -> 6.9).  Without the scratch a
     // K of two phases from 48 M weights on (8192 x 8192 21 -> 17-18.5)
     // (bfloat16 K slices from 24 M: below, the GEMM keeps a row's infinities, which the kept offsets make NaN)
+    // (K = 768 leaves one of four waves without a share: 16384 x 768 at 9 / 12 / 16 rows 6.7 / 6.7 / 7.1 against 7.0 / 6.8 / 7.0, 17760 x 768
+    // 7.8 / 7.9 / 8.1 -> 7.7 / 7.5 / 7.8)
     // (float16 below 24 M weights: two rounds per wave at most, the form that keeps infinities and the smallest activations as they are)
     const bool small = bf16 || weights >= mi(24) || gq::midrow_two_rounds(N, K);
-    return K <= 4096 ? small && weights >= (bf16 ? mi(4) : mi(10))
+    return K <= 4096 ? small && weights >= (bf16 ? mi(4) : mi(K == 768 ? 13 : 10))
                      : (slices && small && weights >= (bf16 ? mi(24) : mi(10))) || (K <= 8192 && weights >= mi(48));
   }
   // 17..32 rows, two batch tiles, against the GEMM's 32-row tile and its split of K (17 / 32 rows): 2048 x 2048 8.9 / 10.0 -> 8.3 / 8.4,
@@ -369,6 +382,9 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
   // 57344 x 8192 97 -> 77; half of the waves without a share loses (27648 x 5120 33.6 / 34.4 against 42).  bfloat16 stays with the GEMM:
   // its instance is ahead (4096 x 4096 12.3 / 13.0 -> 9.6 / 9.7) but makes NaN of an infinity, offset included, where the GEMM keeps it
   if (bf16) return false;
+  // (K = 2304 and 2560, where seven and six of sixteen waves have no share, while the GEMM's tiles are one round: 9152 x 2304 at 17 / 32 rows 12.2 / 12.9
+  // against 13.0 / 13.5, 8608 x 2560 12.8 / 14.0 against 13.0 / 13.8)
+  if (K > 2048 && K <= 2560 && weights > mi(17) && weights < mi(26)) return false;
   if (K <= 4096) return weights >= mi(K >= 2048 ? 4 : 48) || (K >= 1280 && weights >= mi(4) && weights <= mi(24));
   return slices && ((K % 4096 == 0 && weights >= mi(K <= 16384 ? 80 : 120)) || weights >= mi(256));
 }

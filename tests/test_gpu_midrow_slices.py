@@ -161,7 +161,7 @@ def test_midrow_kernel_of_two_rounds(m, n, k, once):
 
 # a wave without a share of K, in every form: the walk with a ring (one batch tile, two, eight waves, phases, slices) and the two rounds
 @pytest.mark.parametrize("dtype,m,n,k,form,kernel", [
-    (torch.float16, 5, 2752, 3840, "", "gq::midrow_kernel<1,8,"), (torch.float16, 9, 2752, 3840, "", "gq::midonce_kernel<1,"),
+    (torch.float16, 5, 4416, 3840, "", "gq::midrow_kernel<1,8,"), (torch.float16, 9, 2752, 3840, "", "gq::midonce_kernel<1,"),
     (torch.float16, 16, 7040, 3584, "", "gq::midrow_kernel<1,8,"), (torch.float16, 17, 1120, 3840, "", "gq::midonce_kernel<2,"),
     (torch.float16, 32, 8224, 3840, "", "gq::midrow_kernel<2,8,"), (torch.float16, 5, 552, 5120, "one workgroup", "gq::midrow_kernel<1,16,"),
     (torch.float16, 6, 544, 14336, "forced", "gq::midrow_kernel<1,8,"), (torch.float16, 7, 544, 4352, "no scratch", "gq::midrow_kernel<1,8,"),
@@ -240,36 +240,52 @@ def test_midrow_kernel_shorter_last_chunk(dtype, m, n, k):
         assert (y[rows].double() - ref).norm() / ref.norm() <= 1e-6, kern
 
 
-# the default dispatch on both sides of its bounds: (kernel, rows, N, K)
-_QUADREG, _QUAD, _GEMM = "gq::quadreg_kernel<", "gq::quad_kernel<", "gq::gemm_pipe_kernel<"
-_WALK, _WIDE, _WALK2, _ONCE2 = "gq::midrow_kernel<1,8,", "gq::midrow_kernel<1,16,", "gq::midrow_kernel<2,8,", "gq::midonce_kernel<2,"
-_SKINNY, _ONCE = "gq::skinny_q4_", "gq::midonce_kernel<1,"
+# the default dispatch on both sides of its bounds: (kernel, rows, N, K), float16
+_QUADREG, _QUAD, _GEMM, _SKINNY = "gq::quadreg_kernel<", "gq::quad_kernel<", "gq::gemm_pipe_kernel<", "gq::skinny_q4_"
+_WALK, _WIDE, _WALK2 = "gq::midrow_kernel<1,8,", "gq::midrow_kernel<1,16,", "gq::midrow_kernel<2,8,"
+_ONCE, _ONCE2 = "gq::midonce_kernel<1,", "gq::midonce_kernel<2,"
 _DEFAULTS = [
     # 17..32 rows of a short K
     (_GEMM, 32, 16384, 256), (_GEMM, 17, 4096, 1024), (_ONCE2, 17, 3296, 1280), (_GEMM, 17, 3264, 1280), (_GEMM, 24, 20480, 1280), (_WALK2, 17, 39328, 1280),
+    (_ONCE2, 17, 2048, 2048), (_GEMM, 17, 2016, 2048), (_ONCE2, 24, 7712, 2304), (_GEMM, 17, 7744, 2304), (_GEMM, 32, 11808, 2304), (_WALK2, 32, 11840, 2304),
+    (_GEMM, 17, 8608, 2560), (_WALK2, 17, 8608, 2816),
     # ... and as K slices
-    (_WALK2, 17, 5120, 16384), (_GEMM, 17, 4096, 20480), (_WALK2, 32, 6144, 20480),
-    # 5..8 rows as K slices, where the quad-row kernel with x in LDS takes the matrices of many rows
-    (_WALK, 8, 30720, 4864), (_QUAD, 5, 32352, 4864), (_WIDE, 5, 45056, 5120), (_QUAD, 8, 51200, 5120),
+    (_WALK2, 17, 5120, 16384), (_GEMM, 17, 4096, 20480), (_WALK2, 32, 6144, 20480), (_WALK2, 32, 10240, 8192), (_GEMM, 32, 10208, 8192),
+    # 5..8 rows of one phase of K
+    (_WALK, 5, 4096, 2560), (_QUADREG, 5, 4064, 2560), (_WALK, 8, 4096, 3584), (_QUADREG, 8, 4064, 3584), (_WALK, 5, 4384, 3840), (_QUADREG, 5, 4352, 3840),
+    (_WALK, 6, 21504, 4096), (_QUADREG, 8, 21472, 4096), (_WIDE, 5, 37888, 3584),
+    # ... as K slices
+    (_WALK, 5, 4928, 5120), (_QUADREG, 5, 4896, 5120), (_WALK, 7, 4800, 6144), (_QUADREG, 8, 4768, 6144), (_WALK, 5, 6560, 7680), (_QUADREG, 8, 6528, 7680),
+    (_WIDE, 6, 32768, 8192), (_QUAD, 6, 32736, 8192), (_WALK, 8, 4096, 10240), (_QUAD, 8, 4064, 10240),
+    # ... where the quad-row kernel with x in LDS takes the matrices of many rows
+    (_WALK, 8, 30720, 4864), (_QUAD, 5, 32352, 4864), (_WIDE, 5, 45056, 5120), (_QUAD, 8, 51200, 5120), (_WIDE, 5, 31744, 5120), (_QUAD, 5, 31776, 5120),
+    (_QUAD, 8, 32768, 7168), (_WIDE, 8, 32800, 7168),
     # 9..16 rows below 24 M weights, where a wave walks two rounds or the skinny kernel answers
-    (_ONCE, 12, 8192, 2560), (_SKINNY, 12, 9216, 2560), (_ONCE, 9, 4096, 5632), (_SKINNY, 16, 4128, 5632),
+    (_ONCE, 12, 8192, 2560), (_SKINNY, 12, 9216, 2560), (_ONCE, 9, 4096, 5632), (_SKINNY, 16, 4128, 5632), (_ONCE, 9, 17760, 768), (_SKINNY, 9, 17728, 768),
 ]
 
 
-@pytest.mark.parametrize("kernel,m,n,k", _DEFAULTS)
-def test_default_kernel_at_the_bounds(kernel, m, n, k):
-    """Which kernel answers, a sample of the columns against the float64 product of the quantised weights (tolerance: one float16 rounding of the
+# ... bfloat16, where the bounds are others
+_DEFAULTS_BF16 = [
+    (_WALK, 5, 28672, 4096), (_QUADREG, 8, 28640, 4096), (_WIDE, 5, 40960, 6144), (_QUAD, 8, 40992, 6144), (_WIDE, 7, 45056, 6656), (_QUAD, 6, 32768, 6144),
+    (_WIDE, 6, 32768, 6656), (_WALK, 16, 2048, 2048), (_GEMM, 9, 2016, 2048), (_WALK, 12, 4928, 5120), (_GEMM, 12, 4896, 5120), (_GEMM, 17, 28672, 4096),
+]
+
+
+@pytest.mark.parametrize("kernel,m,n,k,dtype", [(*d, torch.float16) for d in _DEFAULTS] + [(*d, torch.bfloat16) for d in _DEFAULTS_BF16])
+def test_default_kernel_at_the_bounds(kernel, m, n, k, dtype):
+    """Which kernel answers, a sample of the columns against the float64 product of the quantised weights (tolerance: one rounding of the
     result and, for the kernels that multiply such weights, one of every weight), and the fused gate/up form against the two steps."""
     g = torch.Generator(device="cuda").manual_seed(n + k + m)
     qw = torch.randint(-2**31, 2**31 - 1, (n, k // 8), device="cuda", dtype=torch.int32, generator=g)
-    qs = (torch.rand((n, k // 32), device="cuda", generator=g) * 0.02 + 0.001).half()
-    x = torch.randn((m, k), device="cuda", generator=g).half()
+    qs = (torch.rand((n, k // 32), device="cuda", generator=g) * 0.02 + 0.001).to(dtype)
+    x = torch.randn((m, k), device="cuda", generator=g).to(dtype)
     words = qw.view(torch.uint32)
-    y = ops.linear(x, words, qs, 4, 32)
+    y = ops.linear(x, words, qs, 4, 32, None, dtype)
     kern = gq._lib.last_kernel()
     assert kern.startswith(kernel), kern
     cols = torch.cat([torch.tensor([0, 1, n // 2, n - 1], device="cuda"), torch.randint(0, n, (200,), device="cuda", generator=g)])
     q = torch.stack([(qw[cols] >> (4 * i)) & 15 for i in range(8)], -1).reshape(len(cols), k).double() - 7
     ref = x.double() @ (q * qs[cols].double().repeat_interleave(32, 1)).T
-    assert (y[:, cols].double() - ref).norm() / ref.norm() <= 2 * 2.0**-11, kern
+    assert (y[:, cols].double() - ref).norm() / ref.norm() <= 2 * (2.0**-11 if dtype == torch.float16 else 2.0**-8), kern
     assert torch.equal(ops.linear_silu_mul(x, words, qs, 4, 32), ops.silu_mul(y)), kern
