@@ -329,16 +329,17 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
   if (M <= 4 || M > 32) return false;
   if (M <= 8) {
     // against the quad-row kernel with x in registers: a K that is not 2048 or 4096 leaves some of its waves without a share
-    // (5 / 8 rows: 4096 x 2560 7.9 / 7.7 -> 6.9 / 6.9, 8192 x 3072 10.2 / 10.4 -> 7.9 / 7.8, 4608 x 3584 9.3 / 9.2 -> 7.4 / 7.5, 37888 x 3584 24.0 / 25.8
-    // -> 20.3 / 20.6); for 4096 it is ahead on the smaller matrices (4096 x 4096 6.4 / 6.1 against 7.6, 12288 x 4096 11.4 / 11.0 against
-    // 11.6 / 11.7, 18432 x 4096 15.1 / 14.8 against 14.8 / 15.1, 20480 x 4096 15.0 / 15.0 against 14.9 / 15.4; four whole rounds of tiles are an
-    // exception, 16384 x 4096 13.3 / 12.9 against 12.3 / 12.4) and behind from about 84 M weights on (21504 x 4096 16.5 / 16.3 -> 15.6 / 15.9,
-    // 28672 x 4096 18.4 / 18.5 -> 18.1 / 18.5, 128256 x 4096 64.4 / 66.6 -> 61.8 / 63.7; 57344 x 2048 21.5 / 22.1 -> 18.2 / 18.5; bfloat16 is ahead from 84 M on as
-    // well, 23552 x 4096 17.1 / 16.7 -> 15.8 / 16.4, and is taken from 112 M: 28672 x 4096 19.1 / 19.2 -> 18.2 / 18.8, 128256 x 4096 67.0 / 69.2 -> 62.0 / 64.0)
-    // K = 3584 and 3840 fill the quad-row kernel's waves but for one or a half: the smaller matrices stay (5 / 8 rows: 3520 x 3584 7.4 / 7.3 against
-    // 7.4 / 7.4, 3552 x 3840 7.1 / 7.6 against 7.5 / 7.5; 4416 x 3584 9.0 / 9.6 -> 8.0 / 8.2, 4384 x 3840 8.4 / 9.0 -> 8.2 / 8.3)
+    // (5 / 8 rows: 8192 x 3072 10.2 / 10.4 -> 7.9 / 7.8, 4608 x 3584 9.3 / 9.2 -> 7.4 / 7.5, 37888 x 3584 24.0 / 25.8 -> 20.3 / 20.6), of K = 3840 so few that it
+    // takes 22 M weights (4096 x 3840 7.3 / 7.7 against 7.6 / 7.6, 5472 x 3840 folded 8.6 / 9.4 against 8.8 / 9.0, 6560 x 3840 9.6 / 10.3 -> 8.3 / 8.5).  Up to 4096 rows of
+    // weights give the fused form half of the workgroups that the plain one has (4096 x 3072 7.4 / 7.5 against 8.1 / 8.5, 4448 x 3072 9.4 / 9.8 -> 8.4 / 8.6).
+    // For 2048 and 4096 it is ahead on the smaller matrices (4096 x 4096 6.4 / 6.1 against 7.6, 12288 x 4096 11.4 / 11.0 against 11.6 / 11.7, 18432 x 4096 15.1 /
+    // 14.8 against 14.8 / 15.1, 20480 x 4096 15.0 / 15.0 against 14.9 / 15.4; four whole rounds of tiles are an exception, 16384 x 4096 13.3 / 12.9 against
+    // 12.3 / 12.4) and behind from about 84 M weights on (57344 x 2048 21.5 / 22.1 -> 18.2 / 18.5, 43008 x 2048 folded 16.9 / 17.0 -> 15.3 / 15.6), for K = 4096 from
+    // 150 M on: before that the fused form is ahead there too (folded / plain at 8 rows 28672 x 4096 17.1 / 17.5 against 18.4 / 17.8, 36864 x 4096 21.0 / 21.0
+    // against 21.8 / 21.2, 38912 x 4096 22.6 / 22.6 -> 21.9 / 21.7, 128256 x 4096 plain 66.6 -> 63.7).  bfloat16 is ahead from 84 M on as well, 23552 x 4096 17.1 / 16.7
+    // -> 15.8 / 16.4, and is taken from 112 M: 28672 x 4096 19.1 / 19.2 -> 18.2 / 18.8, folded 18.9 -> 18.4, 128256 x 4096 67.0 / 69.2 -> 62.0 / 64.0)
     if (K <= 4096)
-      return (K > 2048 && K < 4096 && weights >= mi(K > 3584 ? 16 : K > 3328 ? 14 : 10)) || weights >= (bf16 ? mi(112) : mi(84));
+      return (K > 2048 && K < 4096 && N > 4096 && weights >= mi(K > 3584 ? 22 : 10)) || weights >= mi(bf16 ? 112 : K == 4096 ? 150 : 84);
     // K slices: 5120 x 5120 12.3 / 12.0 -> 11.2, 8192 x 5120 15.3 / 15.6 -> 12.5 / 12.9, 8192 x 7168 16.4 / 17.3 -> 13.8 / 14.3, 27648 x 5120 34.9 /
     // 35.5 -> 25.8 / 26.2; 2048 x 5632 stays (8.4 / 8.1 against 9.3).  Not where the matrix has so many rows that the register kernel has no
     // room for their sums and the one with x in LDS answers, while the slices leave two fifths of these waves without a share (30720 x 4864
@@ -368,8 +369,11 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
     // (bfloat16 K slices from 24 M: below, the GEMM keeps a row's infinities, which the kept offsets make NaN)
     // (K = 768 leaves one of four waves without a share: 16384 x 768 at 9 / 12 / 16 rows 6.7 / 6.7 / 7.1 against 7.0 / 6.8 / 7.0, 17760 x 768
     // 7.8 / 7.9 / 8.1 -> 7.7 / 7.5 / 7.8)
+    // (K = 1024, whose fused form leaves half of the CUs without a workgroup, where the skinny kernel has more than one tile per workgroup: 13312 x
+    // 1024 at 9 / 16 rows folded 7.4 / 7.8 against 7.6 / 8.1, 12288 x 1024 and 20480 x 1024 ahead)
     // (float16 below 24 M weights: two rounds per wave at most, the form that keeps infinities and the smallest activations as they are)
     const bool small = bf16 || weights >= mi(24) || gq::midrow_two_rounds(N, K);
+    if (!bf16 && K == 1024 && weights > mi(12) && weights < mi(17)) return false;
     return K <= 4096 ? small && weights >= (bf16 ? mi(4) : mi(K == 768 ? 13 : 10))
                      : (slices && small && weights >= (bf16 ? mi(24) : mi(10))) || (K <= 8192 && weights >= mi(48));
   }

@@ -161,7 +161,7 @@ def test_midrow_kernel_of_two_rounds(m, n, k, once):
 
 # a wave without a share of K, in every form: the walk with a ring (one batch tile, two, eight waves, phases, slices) and the two rounds
 @pytest.mark.parametrize("dtype,m,n,k,form,kernel", [
-    (torch.float16, 5, 4416, 3840, "", "gq::midrow_kernel<1,8,"), (torch.float16, 9, 2752, 3840, "", "gq::midonce_kernel<1,"),
+    (torch.float16, 5, 6016, 3840, "", "gq::midrow_kernel<1,8,"), (torch.float16, 9, 2752, 3840, "", "gq::midonce_kernel<1,"),
     (torch.float16, 16, 7040, 3584, "", "gq::midrow_kernel<1,8,"), (torch.float16, 17, 1120, 3840, "", "gq::midonce_kernel<2,"),
     (torch.float16, 32, 8224, 3840, "", "gq::midrow_kernel<2,8,"), (torch.float16, 5, 552, 5120, "one workgroup", "gq::midrow_kernel<1,16,"),
     (torch.float16, 6, 544, 14336, "forced", "gq::midrow_kernel<1,8,"), (torch.float16, 7, 544, 4352, "no scratch", "gq::midrow_kernel<1,8,"),
@@ -252,8 +252,9 @@ _DEFAULTS = [
     # ... and as K slices
     (_WALK2, 17, 5120, 16384), (_GEMM, 17, 4096, 20480), (_WALK2, 32, 6144, 20480), (_WALK2, 32, 10240, 8192), (_GEMM, 32, 10208, 8192),
     # 5..8 rows of one phase of K
-    (_WALK, 5, 4096, 2560), (_QUADREG, 5, 4064, 2560), (_WALK, 8, 4096, 3584), (_QUADREG, 8, 4064, 3584), (_WALK, 5, 4384, 3840), (_QUADREG, 5, 4352, 3840),
-    (_WALK, 6, 21504, 4096), (_QUADREG, 8, 21472, 4096), (_WIDE, 5, 37888, 3584),
+    (_WALK, 6, 4576, 2304), (_QUADREG, 6, 4544, 2304), (_WALK, 5, 4128, 2560), (_QUADREG, 5, 4096, 2560), (_WALK, 8, 4128, 3584), (_QUADREG, 8, 4096, 3584),
+    (_WALK, 5, 6016, 3840), (_QUADREG, 5, 5984, 3840), (_WIDE, 6, 38400, 4096), (_QUADREG, 8, 38368, 4096), (_WALK, 7, 43008, 2048), (_QUADREG, 7, 42976, 2048),
+    (_WIDE, 5, 37888, 3584),
     # ... as K slices
     (_WALK, 5, 4928, 5120), (_QUADREG, 5, 4896, 5120), (_WALK, 7, 4800, 6144), (_QUADREG, 8, 4768, 6144), (_WALK, 5, 6560, 7680), (_QUADREG, 8, 6528, 7680),
     (_WIDE, 6, 32768, 8192), (_QUAD, 6, 32736, 8192), (_WALK, 8, 4096, 10240), (_QUAD, 8, 4064, 10240),
@@ -262,6 +263,7 @@ _DEFAULTS = [
     (_QUAD, 8, 32768, 7168), (_WIDE, 8, 32800, 7168),
     # 9..16 rows below 24 M weights, where a wave walks two rounds or the skinny kernel answers
     (_ONCE, 12, 8192, 2560), (_SKINNY, 12, 9216, 2560), (_ONCE, 9, 4096, 5632), (_SKINNY, 16, 4128, 5632), (_ONCE, 9, 17760, 768), (_SKINNY, 9, 17728, 768),
+    (_ONCE, 12, 12288, 1024), (_SKINNY, 9, 12320, 1024), (_SKINNY, 16, 17376, 1024), (_ONCE, 16, 17408, 1024),
 ]
 
 
