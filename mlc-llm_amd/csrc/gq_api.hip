@@ -320,13 +320,13 @@ int mi355gq_embedding_take_dt(const void* ids, int64_t T, const void* q_weight, 
                     "embedding_take_dt launch");
 }
 
-// Rows and shapes of a q4 linear that run on the kernel on unscaled weight operands (gq_midrow.hip; K % 256 == 0, N % 32 == 0), in
+// Rows and shapes of a q4 linear that run on the kernel on unscaled weight operands (gq_midrow.hip: K % 256 == 0; N % 32 == 0 for the fused form), in
 // us against the kernel that would run otherwise.  slices: K beyond 4096 runs as K slices over workgroups, for which the caller
 // has brought the scratch.  The same rule for the plain and the fused gate/up form: both must add in the same order.
 static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16) {
   const int64_t weights = N * K;
   const auto mi = [](int64_t n) { return n << 20; };
-  if (M <= 4 || M > 32) return false;
+  if (M <= 4 || M > 32 || (K & 255) != 0 || (N & 31) != 0 || K == 0) return false;
   if (M <= 8) {
     // against the quad-row kernel with x in registers: a K that is not 2048 or 4096 leaves some of its waves without a share
     // (5 / 8 rows: 8192 x 3072 10.2 / 10.4 -> 7.9 / 7.8, 4608 x 3584 9.3 / 9.2 -> 7.4 / 7.5, 37888 x 3584 24.0 / 25.8 -> 20.3 / 20.6), of K = 3840 so few that it
@@ -395,7 +395,7 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
 
 // Scratch for the K slices of that kernel: what the calls that run on it use, and none for others.  (gemv_variant 10 forces it: 5..32 rows)
 static int64_t midrow_scratch(int64_t M, int64_t N, int64_t K, int bits, bool bf16) {
-  const bool asks = gq::options().gemv_variant == 10 ? M > 4 && M <= (bf16 ? 16 : 32) : (N & 31) == 0 && midrow_takes(M, N, K, true, bf16);
+  const bool asks = gq::options().gemv_variant == 10 ? M > 4 && M <= (bf16 ? 16 : 32) : midrow_takes(M, N, K, true, bf16);
   return bits == 4 && asks ? gq::midrow_workspace_bytes(M, N, K) : 0;
 }
 
@@ -532,8 +532,7 @@ static int linear_impl(const void* x, const void* q_weight, const void* q_scale,
   const bool slices_ok = K > 4096 && workspace != nullptr && aligned16(workspace) &&
                          workspace_bytes >= gq::midrow_workspace_bytes(M, N, K) && gq::options().gemv_ksplit != 0;
   const bool mid_rows = bits == 4 && midrow_takes(M, N, K, slices_ok, false) && gq::options().gemm_variant < 0 &&
-                        (gq::options().gemv_variant < 0 || gq::options().gemv_variant == 10) && (K & 255) == 0 &&
-                        (N & 31) == 0;
+                        (gq::options().gemv_variant < 0 || gq::options().gemv_variant == 10);
   if (mid_rows || gq::options().gemv_variant == 10) {  // (10: forced, whatever the shape)
     const hipError_t e = gq::launch_midrow(g, static_cast<int>(M), as_stream(stream));
     if (e != hipErrorNotSupported) return hip_result(e, "mid-row launch");
@@ -938,7 +937,7 @@ static int linear_dt_impl(const void* x, const void* q_weight, const void* q_sca
       const int gvm = gq::options().gemv_variant;
       const bool slices_ok = K > 4096 && workspace != nullptr && aligned16(workspace) &&
                              workspace_bytes >= gq::midrow_workspace_bytes(M, N, K) && gq::options().gemv_ksplit != 0;
-      const bool mid_rows = bits == 4 && midrow_takes(M, N, K, slices_ok, true) && gq::options().gemm_variant < 0 && gvm < 0 && (K & 255) == 0 && (N & 31) == 0;
+      const bool mid_rows = bits == 4 && midrow_takes(M, N, K, slices_ok, true) && gq::options().gemm_variant < 0 && gvm < 0;
       if (mid_rows || gvm == 10) {
         const hipError_t e = gq::launch_midrow(g, static_cast<int>(M), as_stream(stream));
         if (e != hipErrorNotSupported) return hip_result(e, "linear_dt mid-row launch");

@@ -314,7 +314,8 @@ def test_activation_chunks_are_loaded_from_inside_their_row():
 @pytest.mark.parametrize("rows,n,k,slices", [
     (5, 5120, 5120, 2), (8, 8192, 28672, 7), (5, 45056, 5120, 2), (12, 2048, 14336, 4), (32, 57344, 8192, 2),  # K slices
     (12, 4096, 5632, 2), (12, 4128, 5632, 0), (16, 5120, 4608, 0),  # two rounds of tiles, or the skinny kernel
-    (5, 2048, 5632, 0), (8, 8192, 8192, 0), (8, 10240, 8192, 0), (7, 4096, 9216, 0), (5, 51200, 5120, 0), (4, 8192, 28672, 0), (8, 8200, 5120, 0)])
+    (5, 2048, 5632, 0), (8, 8192, 8192, 0), (8, 10240, 8192, 0), (7, 4096, 9216, 0), (5, 51200, 5120, 0), (4, 8192, 28672, 0), (8, 8200, 5120, 0),
+    (9, 2100, 72, 0), (12, 64, 0, 0), (16, 0, 5120, 0), (9, 4096, 4360, 0)])  # no such K, N
 def test_scratch_is_asked_for_by_calls_that_use_it(rows, n, k, slices):
     """float16, the plain linear and the fused gate/up form: the partial sums of the K slices where the call runs on them, else none."""
     lib = _lib.lib()
