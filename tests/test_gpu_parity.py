@@ -417,22 +417,22 @@ def test_midrow_kernel_random_shapes():
 @pytest.mark.parametrize("m", [9, 12, 16, 17, 32])
 @pytest.mark.parametrize("n,k", [(6144, 4096), (28672, 4096), (8192, 8192)])
 def test_midrow_kernel_is_the_default_on_large_matrices(m, n, k):
-    """9..16 rows of q4 on matrices of 24 M weights or more with K up to 4096 (48 M with K up to 8192, two phases), 17..32 rows
-    from 48 M weights on with K up to 4096: the default dispatch, against the oracle on a sample of the columns; the fused gate/up form takes the same kernel and equals
-    linear + silu_mul bit for bit."""
+    """9..16 rows of q4 on matrices of 24 M weights or more (8192 x 8192 as two K slices), 17..32 rows of K up to 4096, the smaller matrix in the
+    form of two rounds: the default dispatch, against the oracle on a sample of the columns; the fused gate/up form takes the same kernel and
+    equals linear + silu_mul bit for bit.  17..32 rows of 8192 x 8192 stay with the GEMM."""
     s = SCHEMES["q4f16_1"]
     rng = np.random.default_rng(seed_of("midrow", m, n, k))
     qw = rng.integers(0, 2**32, (n, k // 8), dtype=np.uint32)
     qs = (rng.random((n, k // 32)) * 0.02 + 0.001).astype(np.float16)
     x = rng.standard_normal((m, k)).astype(np.float16)
     cols = np.unique(np.concatenate([[0, 1, n // 2, n - 1], rng.integers(0, n, 300)]))
-    # (17..32 rows: two batch tiles, from 48 M weights on and with K of one phase only)
-    want = m <= 16 or (n * k >= 48 << 20 and k <= 4096)
+    two_tiles = {6144: "gq::midonce_kernel<2,", 28672: "gq::midrow_kernel<2,", 8192: "gq::gemm_pipe_kernel<"}
+    want = "gq::midrow_kernel<1," if m <= 16 else two_tiles[n]
     y = ops.linear(dev(x), dev(qw), dev(qs), 4, 32)
-    assert gq._lib.last_kernel().startswith(f"gq::midrow_kernel<{1 if m <= 16 else 2},") == want, gq._lib.last_kernel()
+    assert gq._lib.last_kernel().startswith(want), gq._lib.last_kernel()
     assert_linear_ok(y[:, torch.from_numpy(cols).to(DEV)], o.linear_fp32(x, qw[cols], qs[cols], s), x, k, f"mid-row {m}x{n}x{k}")
     fused = ops.linear_silu_mul(dev(x), dev(qw), dev(qs), 4, 32)
-    assert gq._lib.last_kernel().startswith("gq::midrow_kernel<") == want, gq._lib.last_kernel()
+    assert gq._lib.last_kernel().startswith(want), gq._lib.last_kernel()
     assert torch.equal(fused, ops.silu_mul(y))
 
 
@@ -440,9 +440,9 @@ def test_midrow_kernel_is_the_default_on_large_matrices(m, n, k):
                                    (9, 10240, 8192), (24, 32768, 8192), (32, 2048, 8192), (5, 5120, 13824), (8, 8192, 28672),
                                    (7, 4096, 14336)])
 def test_midrow_kernel_k_slices(m, n, k):
-    """A K of several phases on a plain linear whose caller brings the scratch: one workgroup row per phase's worth of K,
-    fp32 partial sums, a reduction that adds bias and residual and casts.  The default at 9..16 rows from 24 M weights on, at
-    17..32 rows from 256 M and at 5..8 rows of a K beyond 8192 from 64 M; forced elsewhere.  Against the oracle on a sample of the columns, with bias, residual and
+    """A K of several phases on a plain linear whose caller brings the scratch: as many workgroup rows, each with an equal share of K,
+    fp32 partial sums, a reduction that adds bias and residual and casts.  The default of these calls but for 32 rows of 4096 x 14336 and of
+    2048 x 8192, where it is forced.  Against the oracle on a sample of the columns, with bias, residual and
     float32 output; the fused gate/up form equals linear + silu_mul bit for bit; without the scratch the call still answers
     (phases inside the workgroup, or the GEMM's tiles)."""
     s = SCHEMES["q4f16_1"]
@@ -454,7 +454,7 @@ def test_midrow_kernel_k_slices(m, n, k):
     res = rng.standard_normal((m, n)).astype(np.float16)
     cols = np.unique(np.concatenate([[0, 1, n // 2, n - 1], rng.integers(0, n, 200)]))
     pick = torch.from_numpy(cols).to(DEV)
-    default = (8 < m <= 16 and n * k >= 24 << 20) or (m > 16 and n * k >= 256 << 20) or (m <= 8 and k > 8192 and n * k >= 64 << 20)
+    default = (m, n, k) not in ((32, 4096, 14336), (32, 2048, 8192))
     phases = -(-(k // 32) // 128)
     if not default:
         gq._lib.set_option("gemv_variant", 10)
