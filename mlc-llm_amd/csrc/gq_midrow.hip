@@ -69,8 +69,8 @@ struct MidParams {
   int chunks;              // chunks of rounds (1 when K takes phases)
   int total_rounds;        // rounds in all chunks: the last one may be shorter (a multiple of the tiles in flight too)
   int phases;              // passes over K (a workgroup covers KW * U groups per phase)
-  int slices;              // workgroups along K (plain linears with a workspace: grid z; each covers one phase's worth of
-                           // K and leaves fp32 partial sums [slice][rows][N] in y for the reduction kernel)
+  int slices;              // workgroups along K (plain linears with a workspace: grid z; each covers slice_shares shares of
+                           // K, one phase's worth at most, and leaves fp32 partial sums [slice][rows][N] in y for the reduction kernel)
   int slice_shares;        // shares of U groups of K in a slice (without slices: kw, the shares of a phase)
   int kw_log2;             // log2 of the waves that share a tile's K
   int out_f32, paired, indptr_i64, x_src_rows;
@@ -110,15 +110,17 @@ __device__ __forceinline__ mid_u4 mid_word_bf16(uint32_t w) {
                 __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(t1, 1.0f, true))};
 }
 
-// NBT: batch tiles of 16 rows; U: groups of K a wave owns (4 or 8); RT: tiles of loads in flight per wave;
-// BF: bfloat16 model (x, scales, bias, residual and the 16-bit result are bfloat16): 0x4300 | q is the bfloat16 128 + q, so
+// NBT: batch tiles of 16 rows (float32: of five); U: groups of K a wave owns (8 or, with eight waves, 16); RT: tiles of loads in flight per wave;
+// DT: the model's type (x, scales, bias, residual and the result).  bfloat16: 0x4300 | q is the bfloat16 128 + q, so
 // every field is shifted down to bit 0 of its half (no x16 trick, x is not rescaled) and all carry the offset 128 + 7;
-// KEEP_C: the offset terms stay in registers (else the constant-operand instruction runs again in front of each group);
+// KEEP_C: the offset terms stay in registers (else, in bfloat16 and float32 the constant-operand instruction runs again in front of each group, in float16
+// the weight operand is rid of the offset);
 // PHASED: K takes more than one phase (the sums of all of a wave's rounds stay in LDS between phases: one chunk of rounds);
 // else a wave's rounds come in chunks of p.rounds, each followed by the step that adds the K shares and stores, with x
 // and the ring of loads carried across
-// ONCE: every tile of a wave is in its first ring of loads (p.rounds == RT): nothing is loaded behind it, and a round without a
-// tile is left out instead of walked over zeros
+// WV: waves of a workgroup (16 or 8)
+// ONCE: every tile of a wave is in its first ring of loads (p.rounds == RT): nothing is loaded behind it (a round without a tile is
+// walked over zeros all the same)
 template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT, int WV, bool ONCE>
 __device__ __forceinline__ void midrow_body(const MidParams& p) {
   static_assert(!ONCE || (!PHASED && DT != MODEL_F32), "one chunk, and no look at the last round's sums");
@@ -727,8 +729,8 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   p.kw_log2 = kwl;
   const int phase_groups = (1 << kwl) * U;
   p.phases = (p.ng + phase_groups - 1) / phase_groups;
-  // A plain linear whose K takes several phases and whose caller brings the scratch: one workgroup row per phase's worth of
-  // K instead (x stays in registers for all of a workgroup's tiles, the walk comes in chunks), fp32 partial sums in the
+  // A plain linear whose K takes several phases and whose caller brings the scratch: as many workgroup rows as
+  // phases, each with an equal share of K, instead (x stays in registers for all of a workgroup's tiles, the walk comes in chunks), fp32 partial sums in the
   // workspace and a second, small launch that adds them; the fused gate/up form then runs as a plain one and the reduction
   // folds the activation in.  The slices are as long as one another (K = 14336: four of 14 shares, not three of 16 and one
   // of 8, whose workgroups would be done first and leave their CUs idle: 15360 x 5120 at 7 / 16 / 32 rows 20.7 / 21.9 / 29.4 -> 18.8 /
@@ -844,7 +846,7 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
   return hipGetLastError();
 }
 
-// whether a dense float16 linear (K a multiple of 256, beyond 4096 as K slices) is two rounds per wave at most
+// whether a dense float16 linear (K a positive multiple of 256, beyond 4096 as K slices) is two rounds per wave at most
 bool midrow_two_rounds(int64_t N, int64_t K) {
   const int64_t shares = K / 256, slices = (shares + 15) / 16;
   int64_t tw = 16;  // tiles side by side in a workgroup
