@@ -121,7 +121,8 @@ __device__ __forceinline__ mid_u4 mid_word_bf16(uint32_t w) {
 // WV: waves of a workgroup (16 or 8)
 // ONCE: every tile of a wave is in its first ring of loads (p.rounds == RT): nothing is loaded behind it (a round without a tile is
 // walked over zeros all the same)
-template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT, int WV, bool ONCE>
+// OWN_X (float32; the phases always): a lane loads its own x instead of taking it from LDS
+template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT, int WV, bool ONCE, bool OWN_X>
 __device__ __forceinline__ void midrow_body(const MidParams& p) {
   static_assert(!ONCE || (!PHASED && DT != MODEL_F32), "one chunk, and no look at the last round's sums");
   constexpr bool BF = DT == MODEL_BF16, F32 = DT == MODEL_F32;
@@ -264,7 +265,7 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
         const int b = pass_lo + c / 3;
         const bool ok = k_live && c < 3 * BR && b < seg_hi;
         uint4 lo[U], hi[U];
-        if constexpr (PHASED) {
+        if constexpr (PHASED || OWN_X) {
           const int64_t xr = p.x_one_row ? 0 : x_row(p.x_rows, p.x_src_rows, ok ? b : seg_lo);
           const float* const xrow = reinterpret_cast<const float*>(p.x) + xr * p.K + ga * 32 + 8 * j;
 #pragma unroll
@@ -619,14 +620,14 @@ __device__ __forceinline__ void midrow_body(const MidParams& p) {
   }
 }
 
-template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT, int WV>
+template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT, int WV, bool OWN_X>
 __global__ __launch_bounds__(64 * WV) void midrow_kernel(const MidParams p) {
-  midrow_body<NBT, U, RT, KEEP_C, PHASED, DT, WV, false>(p);
+  midrow_body<NBT, U, RT, KEEP_C, PHASED, DT, WV, false, OWN_X>(p);
 }
 
 template <int NBT, int U, int RT, bool KEEP_C, int DT>
 __global__ __launch_bounds__(1024) void midonce_kernel(const MidParams p) {
-  midrow_body<NBT, U, RT, KEEP_C, false, DT, 16, true>(p);
+  midrow_body<NBT, U, RT, KEEP_C, false, DT, 16, true, false>(p);
 }
 
 // y[b][j] = silu(sum over slices of part[s][b][j]) * (sum over slices of part[s][b][N / 2 + j]), in the model dtype
@@ -646,24 +647,24 @@ __global__ __launch_bounds__(256) void mid_reduce_silu_kernel(const float* __res
   }
 }
 
-template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16, int WV = 16>
+template <int NBT, int U, int RT, bool KEEP_C, bool PHASED, int DT = MODEL_F16, int WV = 16, bool OWN_X = false>
 hipError_t launch_mid(const MidParams& p, int wgx, int experts, hipStream_t s) {
   // the sums, and 2 KiB of x per wave (float32: x in the slots of five rounds' sums)
-  const int slots = DT == MODEL_F32 ? (PHASED || p.rounds > 5 ? p.rounds : 5) : p.rounds * NBT + 2;
+  const int slots = DT == MODEL_F32 ? (PHASED || OWN_X || p.rounds > 5 ? p.rounds : 5) : p.rounds * NBT + 2;
   const size_t lds = static_cast<size_t>(slots) * WV * 1024;
   if (lds > 160 * 1024) return hipErrorNotSupported;
   if (lds > 64 * 1024) {
     static bool raised = false;  // (idempotent; a race sets the same attribute twice)
     if (!raised) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT, WV>),
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT, WV, OWN_X>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
       if (e != hipSuccess) return e;
       raised = true;
     }
   }
-  note_kernel("gq::midrow_kernel<%d,%d,%d,%d,%d%s> rounds=%d chunks=%d phases=%d slices=%d kw=%d", NBT, U, RT, int(KEEP_C),
-              int(PHASED), DT == MODEL_BF16 ? ",true" : (DT == MODEL_F32 ? ",f32" : ""), p.rounds, p.chunks, p.phases, p.slices, 1 << p.kw_log2);
-  hipLaunchKernelGGL((midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT, WV>), dim3(wgx, experts, p.slices), dim3(64 * WV), lds, s, p);
+  note_kernel("gq::midrow_kernel<%d,%d,%d,%d,%d%s> rounds=%d chunks=%d phases=%d slices=%d kw=%d%s", NBT, U, RT, int(KEEP_C),
+              int(PHASED), DT == MODEL_BF16 ? ",true" : (DT == MODEL_F32 ? ",f32" : ""), p.rounds, p.chunks, p.phases, p.slices, 1 << p.kw_log2, OWN_X ? " own x" : "");
+  hipLaunchKernelGGL((midrow_kernel<NBT, U, RT, KEEP_C, PHASED, DT, WV, OWN_X>), dim3(wgx, experts, p.slices), dim3(64 * WV), lds, s, p);
   return hipGetLastError();
 }
 
@@ -806,6 +807,11 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
     if (a.f32) {
       if (p.phases > 1)
         return launch_mid<1, 8, 2, false, true, MODEL_F32>(p, wgx, experts, s);
+      // One or two rows of up to 12 M weights: a lane's own loads of x.  The way through LDS is ahead once more rows or more workgroups want
+      // it (in us, own loads against LDS, 2 rows: 4096 x 768 8.5 / 8.8, 4096 x 2304 10.0 / 10.1, 1 row 1024 x 9216 11.4 / 11.9; 2 rows 4096 x 4096
+      // 10.8 / 10.4, 28672 x 768 10.5 / 10.1, 3 rows 4096 x 768 8.8 / 8.9, 4096 x 1024 9.2 / 8.9).
+      if (!grouped && (a.expert_ids != nullptr || a.rows <= 2) && a.N * a.K * experts < (12ll << 20))
+        return launch_mid<1, 8, 2, false, false, MODEL_F32, 16, true>(p, wgx, experts, s);
       return launch_mid<1, 8, 2, false, false, MODEL_F32>(p, wgx, experts, s);
     }
     if (wide)

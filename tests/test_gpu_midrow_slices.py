@@ -291,3 +291,26 @@ def test_default_kernel_at_the_bounds(kernel, m, n, k, dtype):
     ref = x.double() @ (q * qs[cols].double().repeat_interleave(32, 1)).T
     assert (y[:, cols].double() - ref).norm() / ref.norm() <= 2 * (2.0**-11 if dtype == torch.float16 else 2.0**-8), kern
     assert torch.equal(ops.linear_silu_mul(x, words, qs, 4, 32), ops.silu_mul(y)), kern
+
+
+# float32: one or two rows of a small matrix load their own x, others take it from LDS (whole and idle shares of K, K slices)
+@pytest.mark.parametrize("m,n,k,own", [(2, 48, 256, True), (2, 1120, 3840, True), (1, 1024, 9216, True), (2, 3056, 4096, True), (2, 3072, 4096, False),
+                                       (3, 1120, 3840, False), (1, 1376, 9216, False)])
+def test_float32_rows_that_load_their_own_x(m, n, k, own):
+    """Against the float64 product of the quantised weights (sums in fp32), and a row with an infinity."""
+    g = torch.Generator(device="cuda").manual_seed(n + k + m)
+    qw = torch.randint(-2**31, 2**31 - 1, (n, k // 8), device="cuda", dtype=torch.int32, generator=g)
+    qs = torch.rand((n, k // 32), device="cuda", generator=g) * 0.02 + 0.001
+    x = torch.randn((m, k), device="cuda", generator=g)
+    q = torch.stack([(qw >> (4 * i)) & 15 for i in range(8)], -1).reshape(n, k).double() - 7
+    w = q * qs.double().repeat_interleave(32, 1)
+    y = ops.linear(x, qw.view(torch.uint32), qs, 4, 32, None, torch.float32)
+    kern = gq._lib.last_kernel()
+    assert kern.startswith("gq::midrow_kernel<1,8,2,0,0,f32>") and kern.endswith(" own x") == own, kern
+    ref = x.double() @ w.T
+    assert (y.double() - ref).norm() / ref.norm() <= 1e-6, kern
+    x[m - 1, 5] = float("inf")
+    odd = ops.linear(x, qw.view(torch.uint32), qs, 4, 32, None, torch.float32)
+    expect = torch.where(w[:, 5] == 0, float("nan"), torch.sign(w[:, 5]) * float("inf")).float()
+    assert torch.equal(torch.isnan(odd[m - 1]), torch.isnan(expect)) and torch.equal(torch.nan_to_num(odd[m - 1]), torch.nan_to_num(expect)), kern
+    assert torch.equal(odd[:m - 1], y[:m - 1]), kern
