@@ -809,8 +809,12 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
         return launch_mid<1, 8, 2, false, true, MODEL_F32>(p, wgx, experts, s);
       // One or two rows of up to 12 M weights: a lane's own loads of x.  The way through LDS is ahead once more rows or more workgroups want
       // it (in us, own loads against LDS, 2 rows: 4096 x 768 8.5 / 8.8, 4096 x 2304 10.0 / 10.1, 1 row 1024 x 9216 11.4 / 11.9; 2 rows 4096 x 4096
-      // 10.8 / 10.4, 28672 x 768 10.5 / 10.1, 3 rows 4096 x 768 8.8 / 8.9, 4096 x 1024 9.2 / 8.9).
-      if (!grouped && (a.expert_ids != nullptr || a.rows <= 2) && a.N * a.K * experts < (12ll << 20))
+      // 10.8 / 10.4, 28672 x 768 10.5 / 10.1, 3 rows 4096 x 1024 9.2 / 8.9).  Three and four rows too where a wave has one tile and a quarter
+      // of the waves or more no share of a K below 3072, so that fewer of them load (3 rows 1216 x 1280 8.30 / 8.65, 672 x 2304 9.11 / 9.42,
+      // 4 rows 7360 x 1280 9.01 / 9.22, 192 x 2560 9.07 / 9.24; but two tiles, 3 rows 9408 x 1280 9.29 / 9.14, no such waves, 3 rows 1968 x 2048
+      // 9.28 / 8.98, and 4 rows 160 x 3072 9.31 / 9.22, 5 rows 304 x 2560 level).
+      const bool idle_waves = p.slices == 1 && items == 1 && a.K < 3072 && 4 * (p.ng / U) <= 3 << kwl;
+      if (!grouped && (a.expert_ids != nullptr || a.rows <= (idle_waves ? 4 : 2)) && a.N * a.K * experts < (12ll << 20))
         return launch_mid<1, 8, 2, false, false, MODEL_F32, 16, true>(p, wgx, experts, s);
       return launch_mid<1, 8, 2, false, false, MODEL_F32>(p, wgx, experts, s);
     }

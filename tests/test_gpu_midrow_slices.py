@@ -293,9 +293,12 @@ def test_default_kernel_at_the_bounds(kernel, m, n, k, dtype):
     assert torch.equal(ops.linear_silu_mul(x, words, qs, 4, 32), ops.silu_mul(y)), kern
 
 
-# float32: one or two rows of a small matrix load their own x, others take it from LDS (whole and idle shares of K, K slices)
+# float32: one or two rows of a small matrix load their own x, and three or four where a wave has one tile and a quarter of the waves no share
+# of a short K; others take it from LDS (whole and idle shares of K, K slices)
 @pytest.mark.parametrize("m,n,k,own", [(2, 48, 256, True), (2, 1120, 3840, True), (1, 1024, 9216, True), (2, 3056, 4096, True), (2, 3072, 4096, False),
-                                       (3, 1120, 3840, False), (1, 1376, 9216, False)])
+                                       (3, 1120, 3840, False), (1, 1376, 9216, False), (3, 240, 768, True), (4, 336, 1536, True),
+                                       (3, 8192, 1280, True), (4, 8208, 1280, False), (4, 4096, 2816, True), (3, 4112, 2816, False),
+                                       (4, 160, 3072, False), (3, 256, 2048, False), (5, 304, 2560, False)])
 def test_float32_rows_that_load_their_own_x(m, n, k, own):
     """Against the float64 product of the quantised weights (sums in fp32), and a row with an infinity."""
     g = torch.Generator(device="cuda").manual_seed(n + k + m)
