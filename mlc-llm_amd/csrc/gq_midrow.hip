@@ -813,8 +813,14 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
       // of the waves or more no share of a K below 3072, so that fewer of them load (3 rows 1216 x 1280 8.30 / 8.65, 672 x 2304 9.11 / 9.42,
       // 4 rows 7360 x 1280 9.01 / 9.22, 192 x 2560 9.07 / 9.24; but two tiles, 3 rows 9408 x 1280 9.29 / 9.14, no such waves, 3 rows 1968 x 2048
       // 9.28 / 8.98, and 4 rows 160 x 3072 9.31 / 9.22, 5 rows 304 x 2560 level).
-      const bool idle_waves = p.slices == 1 && items == 1 && a.K < 3072 && 4 * (p.ng / U) <= 3 << kwl;
-      if (!grouped && (a.expert_ids != nullptr || a.rows <= (idle_waves ? 4 : 2)) && a.N * a.K * experts < (12ll << 20))
+      // Expert segments of about one row on average (two with such waves), one tile per wave: own loads as well, ahead while the longest segment
+      // has one or two rows (4 experts at 3 rows: 1056 x 768 8.16 / 8.52, 656 x 1280 8.22 / 8.70, 192 x 2304 8.87 / 9.45, 592 x 3584 9.61 / 10.06; 8 at 5
+      // rows of 176 x 4096 9.21 / 9.63, at 14 of 736 x 1280 9.24 / 9.47; but 8 at 14 of 176 x 4096 10.44 / 9.95, 16 at 24 of 192 x 3072 10.42 / 10.21).
+      const bool one_tile = p.slices == 1 && items == 1;
+      const bool idle_waves = a.K < 3072 && 4 * (p.ng / U) <= 3 << kwl;
+      const bool own_x = grouped ? one_tile && a.rows <= (idle_waves ? 2 * a.num_experts : a.num_experts + 1)
+                                 : (a.expert_ids != nullptr || a.rows <= (one_tile && idle_waves ? 4 : 2)) && a.N * a.K * experts < (12ll << 20);
+      if (own_x)
         return launch_mid<1, 8, 2, false, false, MODEL_F32, 16, true>(p, wgx, experts, s);
       return launch_mid<1, 8, 2, false, false, MODEL_F32>(p, wgx, experts, s);
     }

@@ -317,3 +317,30 @@ def test_float32_rows_that_load_their_own_x(m, n, k, own):
     expect = torch.where(w[:, 5] == 0, float("nan"), torch.sign(w[:, 5]) * float("inf")).float()
     assert torch.equal(torch.isnan(odd[m - 1]), torch.isnan(expect)) and torch.equal(torch.nan_to_num(odd[m - 1]), torch.nan_to_num(expect)), kern
     assert torch.equal(odd[:m - 1], y[:m - 1]), kern
+
+
+# ... and of expert segments, one tile per wave and few rows per expert: a row each, twice as many where a quarter of the waves idle, one row or tile too many
+@pytest.mark.parametrize("rows,experts,n,k,own", [(4, 4, 256, 4096, True), (5, 4, 336, 3840, True), (6, 4, 176, 1792, False), (8, 4, 1056, 768, True),
+                                                  (9, 4, 304, 1280, False), (32, 16, 144, 2304, True), (8, 8, 512, 4096, True), (8, 8, 528, 4096, False)])
+def test_float32_expert_rows_that_load_their_own_x(rows, experts, n, k, own):
+    """Against the float64 products of the quantised weights (sums in fp32); the last expert has no row, and a row has an infinity."""
+    g = torch.Generator(device="cuda").manual_seed(n + k + rows)
+    qw = torch.randint(-2**31, 2**31 - 1, (experts, n, k // 8), device="cuda", dtype=torch.int32, generator=g)
+    qs = torch.rand((experts, n, k // 32), device="cuda", generator=g) * 0.02 + 0.001
+    x = torch.randn((rows, k), device="cuda", generator=g)
+    of = torch.sort(torch.randint(0, experts - 1, (rows,), device="cuda", generator=g))[0]
+    ip = torch.zeros(experts + 1, dtype=torch.int32, device="cuda")
+    ip[1:] = torch.cumsum(torch.bincount(of, minlength=experts), 0).int()
+    y = ops.moe_experts(x, None, qw.view(torch.uint32), qs, ip, 4, 32)
+    kern = gq._lib.last_kernel()
+    assert kern.startswith("gq::midrow_kernel<1,8,2,0,0,f32>") and kern.endswith(" own x") == own, kern
+    q = torch.stack([(qw >> (4 * i)) & 15 for i in range(8)], -1).reshape(experts, n, k).double() - 7
+    w = (q * qs.double().repeat_interleave(32, 2))[of]
+    ref = torch.stack([w[i] @ x[i].double() for i in range(rows)])
+    assert ((y.double() - ref).norm(dim=1) / ref.norm(dim=1)).max() <= 1e-6, kern
+    x[1, 5] = float("inf")
+    odd = ops.moe_experts(x, None, qw.view(torch.uint32), qs, ip, 4, 32)
+    expect = torch.where(w[1, :, 5] == 0, float("nan"), torch.sign(w[1, :, 5]) * float("inf")).float()
+    assert torch.equal(torch.isnan(odd[1]), torch.isnan(expect)) and torch.equal(torch.nan_to_num(odd[1]), torch.nan_to_num(expect)), kern
+    rest = [i for i in range(rows) if i != 1]
+    assert torch.equal(odd[rest], y[rest]), kern
