@@ -351,15 +351,16 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
     // nearly all of them (4672 x 7680 11.8 / 12.0 against 12.3 / 12.4, 6080 x 7936 level, 6560 x 7680 14.8 / 14.6 -> 14.3 / 13.5).
     // 57344 x 8192 65.5 / 66.3 -> 58.1 / 58.8, 10240 x 8192 stays (16.9 / 15.9
     // against 17.8 / 17.5).  Beyond 8192 the quad-row kernel reads x from LDS, once per four rows and K share: 4096 x 11008 14.0 / 14.4 ->
-    // 13.3 / 13.4, 4096 x 14336 15.8 / 16.1 -> 15.4 / 15.5 (bfloat16 16.6 / 17.5 -> 15.5 / 15.6), 8192 x 28672 46.1 / 47.3 -> 34.9 / 35.0; 4096 x 9216
-    // stays (12.1 / 12.2 against 12.5)
+    // 13.3 / 13.4, 4096 x 14336 15.8 / 16.1 -> 15.4 / 15.5 (bfloat16 16.6 / 17.5 -> 15.5 / 15.6), 8192 x 28672 46.1 / 47.3 -> 34.9 / 35.0; up to 4096
+    // rows and K = 10240, one round of its workgroups, it stays (4096 x 9216 12.1 / 12.2 against 12.5, 4096 x 10240 11.9 / 12.1 against 13.1 / 13.2,
+    // while 4128 x 10240 17.6 / 17.7 -> 13.3 / 13.2, 4096 x 10496 13.4 / 13.8 -> 12.1)
     if (K < 8192) {
       const int64_t ki = 1024, most = (K < 5120 ? 30 : bf16 && K < 6656 ? 40 : 44) * ki;
       const bool quad_filled = N > 31 * ki && N <= 32 * ki && (!bf16 || K < 6656);
       return slices && weights >= mi(K >= 7680 ? 48 : K >= 6144 ? 28 : 24) && N <= most && !quad_filled;
     }
     if (K == 8192) return slices && weights >= mi(256);
-    return slices && weights >= mi(40);
+    return slices && weights >= mi(40) && (K > 10240 || N > 4096);
   }
   if (M <= 16) {
     // against the skinny kernel (bfloat16: the GEMM's 32-row tile; 9 / 16 rows): 4096 x 4096 9.4 / 9.4 -> 7.5 / 7.4, 3584 x 3584 9.3 / 9.4 -> 7.2 / 7.4,

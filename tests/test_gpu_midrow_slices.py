@@ -257,7 +257,7 @@ _DEFAULTS = [
     (_WIDE, 5, 37888, 3584),
     # ... as K slices
     (_WALK, 5, 4928, 5120), (_QUADREG, 5, 4896, 5120), (_WALK, 7, 4800, 6144), (_QUADREG, 8, 4768, 6144), (_WALK, 5, 6560, 7680), (_QUADREG, 8, 6528, 7680),
-    (_WIDE, 6, 32768, 8192), (_QUAD, 6, 32736, 8192), (_WALK, 8, 4096, 10240), (_QUAD, 8, 4064, 10240),
+    (_WIDE, 6, 32768, 8192), (_QUAD, 6, 32736, 8192), (_QUAD, 5, 4096, 10240), (_WALK, 8, 4128, 10240), (_WALK, 8, 4096, 10496),
     # ... where the quad-row kernel with x in LDS takes the matrices of many rows
     (_WALK, 8, 30720, 4864), (_QUAD, 5, 32352, 4864), (_WIDE, 5, 45056, 5120), (_QUAD, 8, 51200, 5120), (_WIDE, 5, 31744, 5120), (_QUAD, 5, 31776, 5120),
     (_QUAD, 8, 32768, 7168), (_WIDE, 8, 32800, 7168),
