@@ -329,9 +329,9 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
   if (M <= 4 || M > 32 || (K & 255) != 0 || (N & 31) != 0 || K == 0) return false;
   if (M <= 8) {
     // against the quad-row kernel with x in registers: a K that is not 2048 or 4096 leaves some of its waves without a share
-    // (5 / 8 rows: 8192 x 3072 10.2 / 10.4 -> 7.9 / 7.8, 4608 x 3584 9.3 / 9.2 -> 7.4 / 7.5, 37888 x 3584 24.0 / 25.8 -> 20.3 / 20.6), of K = 3840 so few that it
-    // takes 22 M weights (4096 x 3840 7.3 / 7.7 against 7.6 / 7.6, 5472 x 3840 folded 8.6 / 9.4 against 8.8 / 9.0, 6560 x 3840 9.6 / 10.3 -> 8.3 / 8.5).  Up to 4096 rows of
-    // weights give the fused form half of the workgroups that the plain one has (4096 x 3072 7.4 / 7.5 against 8.1 / 8.5, 4448 x 3072 9.4 / 9.8 -> 8.4 / 8.6).
+    // (5 / 8 rows: 8192 x 3072 10.2 / 10.4 -> 7.9 / 7.8, 4608 x 3584 9.3 / 9.2 -> 7.4 / 7.5, 37888 x 3584 24.0 / 25.8 -> 20.3 / 20.6), of K = 3840 so few that at 5
+    // and 6 rows of float16 it takes 22 M weights (folded at 5 / 7 rows, 4224 x 3840 7.7 / 8.0 against 8.0 / 7.9, 5472 x 3840 7.9 / 8.3 against 8.0 / 8.0, 6560 x 3840 9.6 -> 8.3 at 5;
+    // bfloat16 4224 x 3840 8.1 / 8.4 -> 8.1 / 8.1).  Up to 4096 rows of weights give the fused form half of the workgroups that the plain one has (4096 x 3072 7.4 / 7.5 against 8.1 / 8.5, 4448 x 3072 9.4 / 9.8 -> 8.4 / 8.6).
     // For 2048 and 4096 it is ahead on the smaller matrices (4096 x 4096 6.4 / 6.1 against 7.6, 12288 x 4096 11.4 / 11.0 against 11.6 / 11.7, 18432 x 4096 15.1 /
     // 14.8 against 14.8 / 15.1, 20480 x 4096 15.0 / 15.0 against 14.9 / 15.4; four whole rounds of tiles are an exception, 16384 x 4096 13.3 / 12.9 against
     // 12.3 / 12.4) and behind from about 84 M weights on (57344 x 2048 21.5 / 22.1 -> 18.2 / 18.5, 43008 x 2048 folded 16.9 / 17.0 -> 15.3 / 15.6), for K = 4096 from
@@ -339,25 +339,29 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
     // against 21.8 / 21.2, 38912 x 4096 22.6 / 22.6 -> 21.9 / 21.7, 128256 x 4096 plain 66.6 -> 63.7).  bfloat16 is ahead from 84 M on as well, 23552 x 4096 17.1 / 16.7
     // -> 15.8 / 16.4, and is taken from 112 M: 28672 x 4096 19.1 / 19.2 -> 18.2 / 18.8, folded 18.9 -> 18.4, 128256 x 4096 67.0 / 69.2 -> 62.0 / 64.0)
     if (K <= 4096)
-      return (K > 2048 && K < 4096 && N > 4096 && weights >= mi(K > 3584 ? 22 : 10)) || weights >= mi(bf16 ? 112 : K == 4096 ? 150 : 84);
+      return (K > 2048 && K < 4096 && N > 4096 && weights >= mi(K > 3584 && M < 7 && !bf16 ? 22 : 10)) || weights >= mi(bf16 ? 112 : K == 4096 ? 150 : 84);
     // K slices: 5120 x 5120 12.3 / 12.0 -> 11.2, 8192 x 5120 15.3 / 15.6 -> 12.5 / 12.9, 8192 x 7168 16.4 / 17.3 -> 13.8 / 14.3, 27648 x 5120 34.9 /
-    // 35.5 -> 25.8 / 26.2; 2048 x 5632 stays (8.4 / 8.1 against 9.3).  Not where the matrix has so many rows that the register kernel has no
-    // room for their sums and the one with x in LDS answers, while the slices leave two fifths of these waves without a share (30720 x 4864
-    // 37.5 / 38.2 -> 28.7 / 29.1, but 32352 x 4864 24.4 / 25.6 against 29.2 / 29.8, 60256 x 4352 39.0 / 40.6 against 48.2 / 48.8; from K = 5120 on that shows later:
-    // 45056 x 5120 38.1 / 39.0 -> 36.3 / 36.7, 51200 x 5120 39.2 / 40.7 against 41.0 / 42.1, 63040 x 6656 51.8 / 54.5 against 58.8 / 59.2; in bfloat16 45056 x 5120
-    // 37.5 against 38.8, 45056 x 6144 41.1 / 41.9, 40960 x 6144 ahead), nor where 31 to 32 Ki rows fill that kernel's walk (32768 x 5120 24.6 / 26.1 against
-    // 28.3 / 29.2, 32768 x 7168 31.1 / 34.3 against 32.6 / 32.7; bfloat16 32768 x 6144 31.4 against 32.7, 32768 x 6656 34.5 -> 32.5).  And from K = 6144 on the
-    // register kernel's waves have work enough on the smaller matrices (4096 x 6144 10.6 / 10.6 against 10.7 / 10.7, 4800 x 6144 level), from 7680 on
-    // nearly all of them (4672 x 7680 11.8 / 12.0 against 12.3 / 12.4, 6080 x 7936 level, 6560 x 7680 14.8 / 14.6 -> 14.3 / 13.5).
+    // 35.5 -> 25.8 / 26.2; 2048 x 5632 stays (8.4 / 8.1 against 9.3).  From K = 6144 on the register kernel's waves have work enough on the smaller
+    // matrices (4096 x 6144 10.6 / 10.6 against 10.7 / 10.7, 4800 x 6144 level), from 7680 on up to 6144 rows of weights (4672 x 7680 11.8 / 12.0 against 12.3 / 12.4, 6144 x
+    // 7680 12.1 / 12.3 against 12.0 / 12.2, 6176 x 7680 13.2 / 13.4 -> 11.9 / 12.0).  From 31 Ki rows on the register kernel has no room for their sums and
+    // the one with x in LDS answers (31744 x 4352 39 / 40 -> 28.5, but 31776 x 4352 25.4 / 25.8 against 27.2 / 28.1): its walk is full at 31 to 32 Ki rows, where the slices are
+    // ahead of it from K = 7680 on only (32768 x 5120 24.6 / 26.1 against 28.3 / 29.2, 32768 x 7168 31.1 / 34.3 against 32.6 / 32.7, 32768 x 7680 37.3 / 39.8 -> 34.9 /
+    // 35.7; bfloat16 32768 x 6144 31.4 against 32.7 or 32.7 against 31.2 by the card, 32768 x 6656 34.5 -> 32.5), and has caught up again by 40 Ki rows of a short K, which
+    // leaves two fifths of the slices' waves without a share (36864 x 4608 33.1 / 33.7 -> 30.6 / 30.4, 45088 x 4608 34.7 / 36.6 against 37.3 / 37.1, 60256 x 4352 39.0 / 40.6
+    // against 48.2 / 48.8), by 44 Ki of K = 5120 (45056 x 5120 38.1 / 39.0 -> 36.3 / 36.7, 51200 x 5120 39.2 / 40.7 against 41.0 / 42.1; bfloat16 45056 x 5120 37.5 against
+    // 38.8, 45056 x 6144 41.1 / 41.9) and by 52 Ki from 6144 on (53248 x 6144 47.8 / 50.9 -> 45.9 / 46.4, 63040 x 6656 51.8 / 54.5 against 58.8 / 59.2); in bfloat16 from K =
+    // 6656 on nowhere (45088 x 6656 48.5 / 50.7 -> 43.5 / 44.6, 131072 x 6656 118 / 123 -> 112 / 116).
     // 57344 x 8192 65.5 / 66.3 -> 58.1 / 58.8, 10240 x 8192 stays (16.9 / 15.9
     // against 17.8 / 17.5).  Beyond 8192 the quad-row kernel reads x from LDS, once per four rows and K share: 4096 x 11008 14.0 / 14.4 ->
     // 13.3 / 13.4, 4096 x 14336 15.8 / 16.1 -> 15.4 / 15.5 (bfloat16 16.6 / 17.5 -> 15.5 / 15.6), 8192 x 28672 46.1 / 47.3 -> 34.9 / 35.0; up to 4096
     // rows and K = 10240, one round of its workgroups, it stays (4096 x 9216 12.1 / 12.2 against 12.5, 4096 x 10240 11.9 / 12.1 against 13.1 / 13.2,
     // while 4128 x 10240 17.6 / 17.7 -> 13.3 / 13.2, 4096 x 10496 13.4 / 13.8 -> 12.1)
     if (K < 8192) {
-      const int64_t ki = 1024, most = (K < 5120 ? 30 : bf16 && K < 6656 ? 40 : 44) * ki;
-      const bool quad_filled = N > 31 * ki && N <= 32 * ki && (!bf16 || K < 6656);
-      return slices && weights >= mi(K >= 7680 ? 48 : K >= 6144 ? 28 : 24) && N <= most && !quad_filled;
+      const int64_t ki = 1024;
+      if (!slices || (K >= 7680 ? N <= 6 * ki : weights < mi(K >= 6144 ? 28 : 24))) return false;
+      if (N <= 31 * ki) return true;
+      if (N <= 32 * ki) return K >= (bf16 ? 6656 : 7680);
+      return bf16 ? K >= 6656 || N <= 40 * ki : N <= (K < 5120 ? 40 : K < 6144 ? 44 : 52) * ki;
     }
     if (K == 8192) return slices && weights >= mi(256);
     return slices && weights >= mi(40) && (K > 10240 || N > 4096);

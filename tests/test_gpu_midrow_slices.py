@@ -253,14 +253,14 @@ _DEFAULTS = [
     (_WALK2, 17, 5120, 16384), (_GEMM, 17, 4096, 20480), (_WALK2, 32, 6144, 20480), (_WALK2, 32, 10240, 8192), (_GEMM, 32, 10208, 8192),
     # 5..8 rows of one phase of K
     (_WALK, 6, 4576, 2304), (_QUADREG, 6, 4544, 2304), (_WALK, 5, 4128, 2560), (_QUADREG, 5, 4096, 2560), (_WALK, 8, 4128, 3584), (_QUADREG, 8, 4096, 3584),
-    (_WALK, 5, 6016, 3840), (_QUADREG, 5, 5984, 3840), (_WIDE, 6, 38400, 4096), (_QUADREG, 8, 38368, 4096), (_WALK, 7, 43008, 2048), (_QUADREG, 7, 42976, 2048),
+    (_WALK, 5, 6016, 3840), (_QUADREG, 6, 5984, 3840), (_WALK, 7, 4128, 3840), (_QUADREG, 7, 4096, 3840), (_WIDE, 6, 38400, 4096), (_QUADREG, 8, 38368, 4096), (_WALK, 7, 43008, 2048), (_QUADREG, 7, 42976, 2048),
     (_WIDE, 5, 37888, 3584),
     # ... as K slices
-    (_WALK, 5, 4928, 5120), (_QUADREG, 5, 4896, 5120), (_WALK, 7, 4800, 6144), (_QUADREG, 8, 4768, 6144), (_WALK, 5, 6560, 7680), (_QUADREG, 8, 6528, 7680),
+    (_WALK, 5, 4928, 5120), (_QUADREG, 5, 4896, 5120), (_WALK, 7, 4800, 6144), (_QUADREG, 8, 4768, 6144), (_WALK, 5, 6176, 7680), (_QUADREG, 8, 6144, 7680),
     (_WIDE, 6, 32768, 8192), (_QUAD, 6, 32736, 8192), (_QUAD, 5, 4096, 10240), (_WALK, 8, 4128, 10240), (_WALK, 8, 4096, 10496),
     # ... where the quad-row kernel with x in LDS takes the matrices of many rows
-    (_WALK, 8, 30720, 4864), (_QUAD, 5, 32352, 4864), (_WIDE, 5, 45056, 5120), (_QUAD, 8, 51200, 5120), (_WIDE, 5, 31744, 5120), (_QUAD, 5, 31776, 5120),
-    (_QUAD, 8, 32768, 7168), (_WIDE, 8, 32800, 7168),
+    (_WALK, 8, 31744, 4864), (_QUAD, 5, 31776, 4864), (_WALK, 8, 32800, 4864), (_QUAD, 5, 40992, 4864), (_WIDE, 5, 45056, 5120), (_QUAD, 8, 51200, 5120), (_WIDE, 5, 31744, 5120), (_QUAD, 5, 31776, 5120),
+    (_QUAD, 8, 32768, 7168), (_WIDE, 8, 32800, 7168), (_WIDE, 5, 32768, 7680), (_WIDE, 8, 53248, 6144), (_QUAD, 5, 53280, 6144),
     # 9..16 rows below 24 M weights, where a wave walks two rounds or the skinny kernel answers
     (_ONCE, 12, 8192, 2560), (_SKINNY, 12, 9216, 2560), (_ONCE, 9, 4096, 5632), (_SKINNY, 16, 4128, 5632), (_ONCE, 9, 17760, 768), (_SKINNY, 9, 17728, 768),
     (_ONCE, 12, 12288, 1024), (_SKINNY, 9, 12320, 1024), (_SKINNY, 16, 17376, 1024), (_ONCE, 16, 17408, 1024),
@@ -270,7 +270,7 @@ _DEFAULTS = [
 # ... bfloat16, where the bounds are others
 _DEFAULTS_BF16 = [
     (_WALK, 5, 28672, 4096), (_QUADREG, 8, 28640, 4096), (_WIDE, 5, 40960, 6144), (_QUAD, 8, 40992, 6144), (_WIDE, 7, 45056, 6656), (_QUAD, 6, 32768, 6144),
-    (_WIDE, 6, 32768, 6656), (_WALK, 16, 2048, 2048), (_GEMM, 9, 2016, 2048), (_WALK, 12, 4928, 5120), (_GEMM, 12, 4896, 5120), (_GEMM, 17, 28672, 4096),
+    (_WIDE, 6, 32768, 6656), (_WIDE, 5, 61440, 6656), (_WALK, 5, 4128, 3840), (_WALK, 16, 2048, 2048), (_GEMM, 9, 2016, 2048), (_WALK, 12, 4928, 5120), (_GEMM, 12, 4896, 5120), (_GEMM, 17, 28672, 4096),
 ]
 
 
