@@ -374,28 +374,32 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
     // (bfloat16 K slices from 24 M: below, the GEMM keeps a row's infinities, which the kept offsets make NaN)
     // (K = 768 leaves one of four waves without a share: 16384 x 768 at 9 / 12 / 16 rows 6.7 / 6.7 / 7.1 against 7.0 / 6.8 / 7.0, 17760 x 768
     // 7.8 / 7.9 / 8.1 -> 7.7 / 7.5 / 7.8)
-    // (K = 1024, whose fused form leaves half of the CUs without a workgroup, where the skinny kernel has more than one tile per workgroup: 13312 x
-    // 1024 at 9 / 16 rows folded 7.4 / 7.8 against 7.6 / 8.1, 12288 x 1024 and 20480 x 1024 ahead)
+    // (K = 1024, whose fused form leaves half of the CUs without a workgroup, up to 12 rows where the skinny kernel runs two tiles per workgroup, from 800 tiles on, in two
+    // rounds of them: 13312 x 1024 at 9 / 12 / 16 rows folded 7.3 / 7.4 / 7.8 against 7.6 / 7.6 / 7.6; 12576 x 1024 13.6 -> 7.0, 16416 x 1024 8.3 -> 7.9)
     // (float16 below 24 M weights: two rounds per wave at most, the form that keeps infinities and the smallest activations as they are)
     const bool small = bf16 || weights >= mi(24) || gq::midrow_two_rounds(N, K);
-    if (!bf16 && K == 1024 && weights > mi(12) && weights < mi(17)) return false;
+    if (!bf16 && K == 1024 && M <= 12 && N >= 800 * 16 && N <= 1024 * 16) return false;
     return K <= 4096 ? small && weights >= (bf16 ? mi(4) : mi(K == 768 ? 13 : 10))
                      : (slices && small && weights >= (bf16 ? mi(24) : mi(10))) || (K <= 8192 && weights >= mi(48));
   }
   // 17..32 rows, two batch tiles, against the GEMM's 32-row tile and its split of K (17 / 32 rows): 2048 x 2048 8.9 / 10.0 -> 8.3 / 8.4,
   // 4096 x 4096 11.8 / 12.4 -> 9.1 / 9.1, 6144 x 4096 12.9 / 13.9 -> 9.3 / 9.7, 12288 x 4096 16.9 / 18.9 -> 14.7 / 16.0, 128256 x 4096 98 / 102 -> 80.6 /
-  // 81.5.  A K below 2048 leaves the x that a wave loads (32 rows) less to be used on: 16384 x 256 4.9 / 5.3 against 9.8 / 9.9, 4096 x 1024 7.7 / 8.4
-  // against 8.4 / 8.6, 26240 x 1280 11.3 / 11.7 against 12.7 / 13.4; from K = 1280 on it is ahead up to 24 M weights (16384 x 1536 11.5 / 12.7
-  // -> 9.1 / 9.4), and from 48 M weights on it takes all of them as it has.  K slices where they are whole and many: 10240 x 8192 27.4 / 28.4 -> 22.4 / 24.3,
-  // 5120 x 16384 25.0 / 25.7 -> 22.8 / 24.4 (4096 x 20480 24.2 / 24.6 against 24.4 / 26.3, from 120 M on ahead again: 6656 x 20480 47.5 / 49.8 -> 32.2 / 34.5),
+  // 81.5.  A K below 2048 leaves the x that a wave loads (32 rows) less to be used on: the GEMM stays ahead of it once it fills the chip without its split of
+  // K, with 200 tiles of 128 columns (25600 x 768 at 17 / 32 rows 8.7 / 8.9 against 9.7 / 10.0, 25600 x 1280 11.4 / 11.7 against 13.0 / 13.1, 25600 x 1536 level; 25600 x
+  // 1792 14.3 / 14.8 -> 13.0 / 13.6), and with the split up to about 10 M weights (16384 x 256 4.9 / 5.3 against 9.8 / 9.9, 16384 x 512 8.0 / 9.8 against 9.2 / 9.4, 4096 x 1024 7.7 /
+  // 8.4 against 8.4 / 8.6; 25472 x 512 10.9 / 12.5 -> 9.7 / 9.8, 16384 x 768 10.2 / 11.5 -> 9.2 / 9.5, 25472 x 1024 13.3 / 15.0 -> 10.2 / 10.5), from K = 1280 on up to 4 M (16384 x
+  // 1536 11.5 / 12.7 -> 9.1 / 9.4); from 48 M weights on it takes all of them as it has.  K slices where they are whole and many: 10240 x 8192 27.4 / 28.4 -> 22.4 / 24.3,
+  // 5120 x 16384 25.0 / 25.7 -> 22.8 / 24.4 (up to 4096 rows of weights of 20480 and 24576 the GEMM is one round: 4096 x 20480 24.2 / 24.6 against 24.4 / 26.3, 4096 x 24576 29.4 /
+  // 28.9 against 29.9 / 30.6, but 4128 x 20480 33.0 / 33.9 -> 24.4 / 26.1, 3072 x 28672 27.9 / 29.2 -> 24.8 / 26.6),
   // 57344 x 8192 97 -> 77; half of the waves without a share loses (27648 x 5120 33.6 / 34.4 against 42).  bfloat16 stays with the GEMM:
   // its instance is ahead (4096 x 4096 12.3 / 13.0 -> 9.6 / 9.7) but makes NaN of an infinity, offset included, where the GEMM keeps it
   if (bf16) return false;
-  // (K = 2304 and 2560, where seven and six of sixteen waves have no share, while the GEMM's tiles are one round: 9152 x 2304 at 17 / 32 rows 12.2 / 12.9
-  // against 13.0 / 13.5, 8608 x 2560 12.8 / 14.0 against 13.0 / 13.8)
-  if (K > 2048 && K <= 2560 && weights > mi(17) && weights < mi(26)) return false;
-  if (K <= 4096) return weights >= mi(K >= 2048 ? 4 : 48) || (K >= 1280 && weights >= mi(4) && weights <= mi(24));
-  return slices && ((K % 4096 == 0 && weights >= mi(K <= 16384 ? 80 : 120)) || weights >= mi(256));
+  // (K = 2304 and 2560, where seven and six of sixteen waves have no share, past the two rounds per wave of 8192 rows: 8192 x 2304 at 17 / 32 rows 11.4 / 12.4 -> 9.5 / 9.8,
+  // but 9152 x 2304 12.2 / 12.9 against 13.0 / 13.5, 8608 x 2560 12.8 / 14.0 against 13.0 / 13.8; 11744 x 2304 14.9 / 16.3 -> 12.8 / 13.4, 8960 x 2560 12.9 / 14.0 -> 12.5 / 12.9)
+  if (K > 2048 && K <= 2560 && N > 8192 && weights < mi(K == 2304 ? 24 : 22)) return false;
+  const bool gemm_splits = N <= 199 * 128;
+  if (K <= 4096) return weights >= mi(K >= 1792 ? 4 : 48) || (gemm_splits && K >= 512 && weights >= mi(K >= 1280 ? 4 : 10));
+  return slices && ((K % 4096 == 0 && weights >= mi(80) && (K <= 16384 || K > 24576 || N > 4096)) || weights >= mi(256));
 }
 
 // Scratch for the K slices of that kernel: what the calls that run on it use, and none for others.  (gemv_variant 10 forces it: 5..32 rows)

@@ -246,11 +246,12 @@ _WALK, _WIDE, _WALK2 = "gq::midrow_kernel<1,8,", "gq::midrow_kernel<1,16,", "gq:
 _ONCE, _ONCE2 = "gq::midonce_kernel<1,", "gq::midonce_kernel<2,"
 _DEFAULTS = [
     # 17..32 rows of a short K
-    (_GEMM, 32, 16384, 256), (_GEMM, 17, 4096, 1024), (_ONCE2, 17, 3296, 1280), (_GEMM, 17, 3264, 1280), (_GEMM, 24, 20480, 1280), (_WALK2, 17, 39328, 1280),
-    (_ONCE2, 17, 2048, 2048), (_GEMM, 17, 2016, 2048), (_ONCE2, 24, 7712, 2304), (_GEMM, 17, 7744, 2304), (_GEMM, 32, 11808, 2304), (_WALK2, 32, 11840, 2304),
-    (_GEMM, 17, 8608, 2560), (_WALK2, 17, 8608, 2816),
+    (_GEMM, 32, 16384, 256), (_GEMM, 17, 10208, 1024), (_ONCE2, 17, 10240, 1024), (_ONCE2, 32, 20480, 512), (_GEMM, 17, 20448, 512), (_ONCE2, 17, 25472, 1024),
+    (_GEMM, 17, 25504, 1024), (_ONCE2, 17, 3296, 1280), (_GEMM, 17, 3264, 1280), (_WALK2, 24, 20480, 1280), (_GEMM, 32, 25504, 1536), (_WALK2, 17, 39328, 1280),
+    (_ONCE2, 17, 2048, 2048), (_GEMM, 17, 2016, 2048), (_WALK2, 17, 25504, 1792), (_ONCE2, 24, 8192, 2304), (_GEMM, 17, 8224, 2304), (_GEMM, 32, 10912, 2304),
+    (_WALK2, 32, 10944, 2304), (_GEMM, 17, 8992, 2560), (_WALK2, 17, 9024, 2560), (_WALK2, 17, 8608, 2816),
     # ... and as K slices
-    (_WALK2, 17, 5120, 16384), (_GEMM, 17, 4096, 20480), (_WALK2, 32, 6144, 20480), (_WALK2, 32, 10240, 8192), (_GEMM, 32, 10208, 8192),
+    (_WALK2, 17, 5120, 16384), (_GEMM, 17, 4096, 20480), (_WALK2, 32, 4128, 20480), (_GEMM, 17, 4096, 24576), (_WALK2, 17, 3072, 28672), (_WALK2, 32, 10240, 8192), (_GEMM, 32, 10208, 8192),
     # 5..8 rows of one phase of K
     (_WALK, 6, 4576, 2304), (_QUADREG, 6, 4544, 2304), (_WALK, 5, 4128, 2560), (_QUADREG, 5, 4096, 2560), (_WALK, 8, 4128, 3584), (_QUADREG, 8, 4096, 3584),
     (_WALK, 5, 6016, 3840), (_QUADREG, 6, 5984, 3840), (_WALK, 7, 4128, 3840), (_QUADREG, 7, 4096, 3840), (_WIDE, 6, 38400, 4096), (_QUADREG, 8, 38368, 4096), (_WALK, 7, 43008, 2048), (_QUADREG, 7, 42976, 2048),
@@ -263,7 +264,7 @@ _DEFAULTS = [
     (_QUAD, 8, 32768, 7168), (_WIDE, 8, 32800, 7168), (_WIDE, 5, 32768, 7680), (_WIDE, 8, 53248, 6144), (_QUAD, 5, 53280, 6144),
     # 9..16 rows below 24 M weights, where a wave walks two rounds or the skinny kernel answers
     (_ONCE, 12, 8192, 2560), (_SKINNY, 12, 9216, 2560), (_ONCE, 9, 4096, 5632), (_SKINNY, 16, 4128, 5632), (_ONCE, 9, 17760, 768), (_SKINNY, 9, 17728, 768),
-    (_ONCE, 12, 12288, 1024), (_SKINNY, 9, 12320, 1024), (_SKINNY, 16, 17376, 1024), (_ONCE, 16, 17408, 1024),
+    (_ONCE, 9, 12768, 1024), (_SKINNY, 12, 12800, 1024), (_SKINNY, 9, 16384, 1024), (_ONCE, 12, 16416, 1024), (_ONCE, 13, 13312, 1024),
 ]
 
 
