@@ -334,12 +334,13 @@ static bool midrow_takes(int64_t M, int64_t N, int64_t K, bool slices, bool bf16
     // bfloat16 4224 x 3840 8.1 / 8.4 -> 8.1 / 8.1).  Up to 4096 rows of weights give the fused form half of the workgroups that the plain one has (4096 x 3072 7.4 / 7.5 against 8.1 / 8.5, 4448 x 3072 9.4 / 9.8 -> 8.4 / 8.6).
     // For 2048 and 4096 it is ahead on the smaller matrices (4096 x 4096 6.4 / 6.1 against 7.6, 12288 x 4096 11.4 / 11.0 against 11.6 / 11.7, 18432 x 4096 15.1 /
     // 14.8 against 14.8 / 15.1, 20480 x 4096 15.0 / 15.0 against 14.9 / 15.4; four whole rounds of tiles are an exception, 16384 x 4096 13.3 / 12.9 against
-    // 12.3 / 12.4) and behind from about 84 M weights on (57344 x 2048 21.5 / 22.1 -> 18.2 / 18.5, 43008 x 2048 folded 16.9 / 17.0 -> 15.3 / 15.6), for K = 4096 from
-    // 150 M on: before that the fused form is ahead there too (folded / plain at 8 rows 28672 x 4096 17.1 / 17.5 against 18.4 / 17.8, 36864 x 4096 21.0 / 21.0
-    // against 21.8 / 21.2, 38912 x 4096 22.6 / 22.6 -> 21.9 / 21.7, 128256 x 4096 plain 66.6 -> 63.7).  bfloat16 is ahead from 84 M on as well, 23552 x 4096 17.1 / 16.7
+    // 12.3 / 12.4) and behind from about 84 M weights on (57344 x 2048 21.5 / 22.1 -> 18.2 / 18.5, 43008 x 2048 folded 16.9 / 17.0 -> 15.3 / 15.6, 21504 x 4096 folded 16.8 /
+    // 16.3 -> 15.8 / 15.8, 32768 x 4096 21.6 / 21.2 -> 20.0 / 19.8, folded 21.8 / 21.6 -> 20.1 / 20.4, 128256 x 4096 plain 66.6 -> 63.7), but for 24 to 28 Ki rows of K = 4096, whose
+    // tiles are 7 rounds at most and walked as 8 (28672 x 4096 19.2 / 19.4 against 19.2 / 19.2; in a decode step, folded, at 7 rows 0.4 us less on the quad-row kernel).  bfloat16 is ahead from 84 M on as well, 23552 x 4096 17.1 / 16.7
     // -> 15.8 / 16.4, and is taken from 112 M: 28672 x 4096 19.1 / 19.2 -> 18.2 / 18.8, folded 18.9 -> 18.4, 128256 x 4096 67.0 / 69.2 -> 62.0 / 64.0)
     if (K <= 4096)
-      return (K > 2048 && K < 4096 && N > 4096 && weights >= mi(K > 3584 && M < 7 && !bf16 ? 22 : 10)) || weights >= mi(bf16 ? 112 : K == 4096 ? 150 : 84);
+      return (K > 2048 && K < 4096 && N > 4096 && weights >= mi(K > 3584 && M < 7 && !bf16 ? 22 : 10)) ||
+             (weights >= mi(bf16 ? 112 : 84) && (bf16 || K < 4096 || N <= 24 << 10 || N > 28 << 10));
     // K slices: 5120 x 5120 12.3 / 12.0 -> 11.2, 8192 x 5120 15.3 / 15.6 -> 12.5 / 12.9, 8192 x 7168 16.4 / 17.3 -> 13.8 / 14.3, 27648 x 5120 34.9 /
     // 35.5 -> 25.8 / 26.2; 2048 x 5632 stays (8.4 / 8.1 against 9.3).  From K = 6144 on the register kernel's waves have work enough on the smaller
     // matrices (4096 x 6144 10.6 / 10.6 against 10.7 / 10.7, 4800 x 6144 level), from 7680 on up to 6144 rows of weights (4672 x 7680 11.8 / 12.0 against 12.3 / 12.4, 6144 x

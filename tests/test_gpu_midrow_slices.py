@@ -254,7 +254,8 @@ _DEFAULTS = [
     (_WALK2, 17, 5120, 16384), (_GEMM, 17, 4096, 20480), (_WALK2, 32, 4128, 20480), (_GEMM, 17, 4096, 24576), (_WALK2, 17, 3072, 28672), (_WALK2, 32, 10240, 8192), (_GEMM, 32, 10208, 8192),
     # 5..8 rows of one phase of K
     (_WALK, 6, 4576, 2304), (_QUADREG, 6, 4544, 2304), (_WALK, 5, 4128, 2560), (_QUADREG, 5, 4096, 2560), (_WALK, 8, 4128, 3584), (_QUADREG, 8, 4096, 3584),
-    (_WALK, 5, 6016, 3840), (_QUADREG, 6, 5984, 3840), (_WALK, 7, 4128, 3840), (_QUADREG, 7, 4096, 3840), (_WIDE, 6, 38400, 4096), (_QUADREG, 8, 38368, 4096), (_WALK, 7, 43008, 2048), (_QUADREG, 7, 42976, 2048),
+    (_WALK, 5, 6016, 3840), (_QUADREG, 6, 5984, 3840), (_WALK, 7, 4128, 3840), (_QUADREG, 7, 4096, 3840), (_WALK, 6, 21504, 4096), (_QUADREG, 8, 21472, 4096),
+    (_WALK, 5, 24576, 4096), (_QUADREG, 7, 24608, 4096), (_QUADREG, 8, 28672, 4096), (_WALK, 8, 28704, 4096), (_WIDE, 6, 38400, 4096), (_WALK, 7, 43008, 2048), (_QUADREG, 7, 42976, 2048),
     (_WIDE, 5, 37888, 3584),
     # ... as K slices
     (_WALK, 5, 4928, 5120), (_QUADREG, 5, 4896, 5120), (_WALK, 7, 4800, 6144), (_QUADREG, 8, 4768, 6144), (_WALK, 5, 6176, 7680), (_QUADREG, 8, 6144, 7680),
