@@ -812,7 +812,7 @@ hipError_t launch_midrow(const GemmArgs& a, int rows_max, hipStream_t s) {
       // 10.8 / 10.4, 28672 x 768 10.5 / 10.1, 3 rows 4096 x 1024 9.2 / 8.9).  Three and four rows too where a wave has one tile and a quarter
       // of the waves or more no share of a K below 3072, so that fewer of them load (3 rows 1216 x 1280 8.30 / 8.65, 672 x 2304 9.11 / 9.42,
       // 4 rows 7360 x 1280 9.01 / 9.22, 192 x 2560 9.07 / 9.24; but two tiles, 3 rows 9408 x 1280 9.29 / 9.14, no such waves, 3 rows 1968 x 2048
-      // 9.28 / 8.98, and 4 rows 160 x 3072 9.31 / 9.22, 5 rows 304 x 2560 level).
+      // 9.28 / 8.98, and 4 rows 160 x 3072 9.31 / 9.22, 5 rows 336 x 2560 level).
       // Expert segments of about one row on average (two with such waves), one tile per wave: own loads as well, ahead while the longest segment
       // has one or two rows (4 experts at 3 rows: 1056 x 768 8.16 / 8.52, 656 x 1280 8.22 / 8.70, 192 x 2304 8.87 / 9.45, 592 x 3584 9.61 / 10.06; 8 at 5
       // rows of 176 x 4096 9.21 / 9.63, at 14 of 736 x 1280 9.24 / 9.47; but 8 at 14 of 176 x 4096 10.44 / 9.95, 16 at 24 of 192 x 3072 10.42 / 10.21).
